@@ -60,7 +60,8 @@ def _check_i32(x: torch.Tensor, name: str) -> None:
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    # torch.cuda.current_stream().cuda_stream without building the Stream object (1.5 us a call)
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _ptr(x: Optional[torch.Tensor]) -> Optional[int]:

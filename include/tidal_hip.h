@@ -439,6 +439,21 @@ int td_prefill_attn(const td_paged_kv* kv, const int32_t* page_table, int32_t n_
                     float sm_scale, int32_t causal, void* stream);
 
 /*
+ * td_prefill_attn with scratch: where a few query rows leave the chip idle (a further turn on a long
+ * cache, a short prompt) their keys are cut into pieces that several workgroups walk side by side and
+ * a second launch adds up.  workspace: td_prefill_workspace_bytes(...) bytes of device memory (16-byte
+ * aligned, any contents; 0 bytes: the call does not split), to be used by one call at a time.  With less
+ * or NULL it runs as td_prefill_attn does.  Interface replaced: bsk_ops.h:80-88; the reference's kernel
+ * splits the keys through its handler's workspace (kernels/include/prefill/prefill.cuh:674-870).
+ */
+int64_t td_prefill_workspace_bytes(const td_paged_kv* kv, int32_t kv_len, int32_t n_q,
+                                   int32_t num_qo_heads, int32_t causal);
+int td_prefill_attn_split(const td_paged_kv* kv, const int32_t* page_table, int32_t n_pages,
+                          int32_t kv_len, const void* q, void* o, int32_t n_q, int32_t num_qo_heads,
+                          float sm_scale, int32_t causal, void* workspace, int64_t workspace_bytes,
+                          void* stream);
+
+/*
  * Matrix-vector product of a batch-1 decode step: y[rows] = W[rows, cols] . f(x) (+ residual),
  * 16-bit storage, fp32 accumulation.  x_mode 0: f(x) = x[cols]; 1: f(x) = RMSNorm(x) * norm_weight
  * (eps); 2: f(x) = silu(x[:cols]) * x[cols:2 cols] (gated MLP).  residual (or NULL) is added to

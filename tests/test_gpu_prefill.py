@@ -152,3 +152,34 @@ def test_random_configurations(cuda, seed):
     got = _run(cuda, case, q, causal, dtype)
     ok = (got.float().cpu() - want).abs() <= ATOL[dtype] * want.abs().clamp(min=1.0)
     assert ok.all(), (dtype, d, hq, hkv, page, layout, causal, kv_len, n_q)
+
+
+@pytest.mark.parametrize("dtype,hq,hkv,d,page,kv_len,n_q,pieces,rise", [
+    # one to six key tiles around the rings of four and five, keys that end inside and on a tile
+    (torch.bfloat16, 2, 2, 128, 16, 64, 64, False, 0.0), (torch.float16, 2, 2, 128, 16, 65, 65, False, 0.0),
+    (torch.bfloat16, 2, 1, 128, 8, 192, 33, False, 12.0), (torch.float16, 1, 1, 64, 16, 257, 257, False, 12.0),
+    (torch.bfloat16, 3, 3, 64, 5, 320, 256, False, 0.0), (torch.float16, 2, 2, 128, 1, 383, 300, False, 12.0),
+    # packed rows of a group of seven: tokens cross waves and workgroup tiles
+    (torch.bfloat16, 7, 1, 128, 16, 300, 37, False, 0.0), (torch.float16, 14, 2, 64, 3, 111, 74, False, 12.0),
+    # keys cut into pieces: a last piece of one key, pieces past the end of the first rows, page sizes
+    (torch.bfloat16, 8, 8, 128, 16, 20481, 16, True, 0.0), (torch.float16, 8, 2, 128, 16, 9000, 300, True, 12.0),
+    (torch.float16, 4, 4, 64, 16, 6401, 257, True, 12.0), (torch.bfloat16, 4, 1, 128, 3, 5000, 1, True, 0.0),
+    (torch.bfloat16, 2, 1, 256, 16, 4100, 70, True, 12.0), (torch.bfloat16, 4, 4, 128, 16, 2000, 2000, True, 0.0),
+])
+def test_row_packing_rings_and_pieces(cuda, dtype, hq, hkv, d, page, kv_len, n_q, pieces, rise):
+    """The edges of the work split: key tiles of 64, rings, packed query rows, pieces and their merge.
+    `rise`: queries grow to this many times their size, so that later keys exceed the first tile's by
+    more than the factor of 2^14 that a row's reference point may lag, and accumulators are rescaled late.  Tolerance as above: weights are rounded
+    relative to their own size whatever the reference point is."""
+    from tidaldecode_amd import _kernels
+    from tidaldecode_amd._lib import lib
+
+    case = PagedCase(kv_len, hkv, d, page, dtype, seed=kv_len + n_q)
+    q = randn((n_q, hq, d), kv_len * 3 + n_q, dtype)
+    if rise:
+        q = (q * torch.linspace(0.5, rise, n_q)[:, None, None]).to(dtype).float()
+    planned = lib.td_prefill_workspace_bytes(_kernels._pool(case.pool.to(cuda), case.layout), kv_len, n_q, hq, 1)
+    assert (planned > 0) == pieces
+    got = _run(cuda, case, q, True, dtype).float().cpu()
+    want = _dense(q, case.k, case.v, True)
+    assert ((got - want).abs() <= ATOL[dtype] * want.abs().clamp(min=1.0)).all()

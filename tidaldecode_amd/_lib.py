@@ -165,6 +165,12 @@ SIGNATURES = {
         [POINTER(PagedKV), c_void_p, c_int32, c_int32, c_void_p, c_void_p, c_int32, c_int32,
          c_float, c_int32, c_void_p],
     ),
+    "td_prefill_workspace_bytes": (c_int64, [POINTER(PagedKV), c_int32, c_int32, c_int32, c_int32]),
+    "td_prefill_attn_split": (
+        c_int32,
+        [POINTER(PagedKV), c_void_p, c_int32, c_int32, c_void_p, c_void_p, c_int32, c_int32,
+         c_float, c_int32, c_void_p, c_int64, c_void_p],
+    ),
     "td_gemv": (
         c_int32,
         [c_void_p, c_int64, c_int32, c_int32, c_void_p, c_int32, c_void_p, c_float, c_void_p,

@@ -280,6 +280,23 @@ __device__ __forceinline__ f32x4 mfma_16x16x32<F16>(u32x4 a, u32x4 b, f32x4 c) {
                                                 __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
 }
 
+// gfx950: D(32x32, fp32) += A(32x16) * B(16x32); a lane holds A[lane % 32][8h .. 8h+7] and
+// B[8h .. 8h+7][lane % 32] (h = lane / 32) as four packed dwords, and element v of the result is
+// D[8 (v / 4) + 4h + v % 4][lane % 32].
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+template <typename T>
+__device__ __forceinline__ f32x16 mfma_32x32x16(u32x4 a, u32x4 b, f32x16 c);
+template <>
+__device__ __forceinline__ f32x16 mfma_32x32x16<BF16>(u32x4 a, u32x4 b, f32x16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a),
+                                                 __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+template <>
+__device__ __forceinline__ f32x16 mfma_32x32x16<F16>(u32x4 a, u32x4 b, f32x16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a),
+                                                __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+}
+
 constexpr float kNegBig = -1.0e30f;  // finite stand-in for -inf in running maxima
 
 __host__ __device__ __forceinline__ int64_t ceil_div64(int64_t a, int64_t b) {

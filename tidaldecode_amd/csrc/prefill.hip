@@ -2,24 +2,34 @@
 // gfx950 (MI355X), on the matrix cores.  Replaces BatchPrefillWithPagedKVCache of the reference
 // (kernels/include/prefill/prefill.cuh:674-870, bound in tidal/ops/csrc/batch_prefill.cu:27-117).
 //
-// One workgroup of NW = 4 or 8 wavefronts per (16 MT NW query rows, query head); a wavefront owns
-// 16 MT query rows as MT = 2 16-row tiles: every K/V operand read from LDS feeds two matrix
-// instructions (head_dim 256: MT = 1, key tiles of 32 tokens).  The loop walks
-// the keys in tiles of 64 tokens that the workgroup stages in LDS, two buffers per matrix (one
-// barrier per tile) and two tiles in flight in registers.  LDS rows are padded by 32 bytes
-// (288 for head_dim 128): gfx950 serves a 16-byte LDS read of lane 0 in one cycle with lanes
-// 1-3, 12-15 and 20-27 (measured), and with that grouping a pitch of 16 (4k + 2) bytes is free of
-// bank conflicts for the K operand reads and for the transposed V reads.  Per key tile:
-//   S^T = K Q^T   mfma_f32_16x16x32, A = K rows from LDS, B = Q rows kept in registers: an operand
-//                 is a 16-byte piece of a row;
-//   softmax       base-2, online; the result tile has the query row in lane % 16 and four
-//                 tokens per lane, which is the A-operand layout of the next product; the row
-//                 maximum crosses the four lane groups with v_permlane16/32_swap;
-//   O += P V      per 32 tokens: A = P (rounded to the KV type), B = V read with
-//                 ds_read_b64_tr_b16, which hands lane r dimension 16 a + r of four tokens.
-// Pages are looked up per staged row, one tile ahead; rows past the end of the sequence are
-// clamped (never out of the pool) and masked.  All query tiles of the heads that share a KV head
-// are placed on one XCD (see the block-index mapping in the kernel).
+// What bounds it.  A long prompt is a contraction (4 n^2 / 2 flops per head dimension and head), so the
+// matrix cores; but per 64 keys and 32 query rows the softmax costs a wave about as long as the two
+// products (1000 cycles of exp2, fma and pack against 1030 of MFMA), so the two have to run at the same
+// time.  A short prompt or a further turn on a long cache has few query rows and is bound by how many
+// CUs have work at all.  Hence:
+//   - The query rows of all heads of a KV head are packed into one list of rows (token * group + head),
+//     cut into workgroup tiles of up to 256: grouped heads share every staged key, and 16 new tokens of four
+//     heads fill 64 rows instead of four quarter-empty tiles.
+//   - The keys of a row tile are cut into pieces when the tiles alone leave CUs idle (plan_prefill);
+//     prefill_merge_kernel adds the pieces up.
+//   - Eight waves of 32 rows, two per SIMD in opposite phases: one multiplies while the other forms
+//     weights (see "the steps" in the kernel).  S^T = K Q^T and O^T = V^T P^T with 32x32x16 MFMA: the
+//     query row is the lane in both results, so P stays in registers and the row maximum and sum cross
+//     one pair of lanes.
+//   - Key tiles go from memory to LDS without passing through registers, into rings of four (K) and five
+//     (V) tiles; a piece is asked for three to four tiles before it is needed.
+// LDS layout: gfx950 serves 256 bytes a cycle, and lanes {0-3, 12-15, 20-27} of a 16-byte read together
+// (measured), so those 16 lanes must hit 16 different bank groups.  head_dim 128: four rows form a block
+// of 1024 + 16 bytes and piece p of row r lies at p ^ 4 (r % 4); head_dim 64: rows of 128 bytes, pieces
+// of K at p ^ ((r / 2) % 8), of V (read transposed, eight bytes a lane) at p ^ 4 ((r / 2) % 2).
+// Measured (bf16, pages of 16, us, before with one 128- or 256-row tile per query head and 16x16x32
+// MFMA -> now): prompt of 32768 x 32 heads 9168 -> 7059 (1246 TFLOP/s; the largest library GEMM reaches
+// 1560 here), 8192 x 32 over 8 KV heads 586 -> 462, 1000 x 32 38 -> 23, 300 x 32 14.7 -> 10.2 (bound by
+// the latency of its five key tiles and cold code); 500 new tokens on 32768 cached ones, 32 heads
+// 992 -> 254, over 8 KV heads 992 -> 242; 16 tokens, 8 KV heads 794 -> 32.
+// Rows past the end of the sequence are clamped (never out of the pool) and masked.
+
+#include <type_traits>
 
 #include "common.cuh"
 #include "../../include/tidal_hip.h"
@@ -36,10 +46,28 @@ __device__ __forceinline__ u32x2 lds_read_tr16(const uint16_t* at) {
   return __builtin_bit_cast(u32x2, v);
 }
 
+// 16 bytes per lane from memory (scalar base + lane offset, or a lane address) to LDS bytes
+// lds + 16 lane.  As asm: the compiler would wait for the load before every later LDS read.
+__device__ __forceinline__ void load_lds(uint32_t lds, uint64_t base, uint32_t offset) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+               :: "s"(lds), "v"(offset), "s"(base) : "memory");
+}
+__device__ __forceinline__ void load_lds(uint32_t lds, uint64_t at) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" :: "s"(lds), "v"(at) : "memory");
+}
+
+constexpr float kTopWeight = 16384.f;  // a lane's share of a tile's row sum: every weight fits fp16 as well
+
+constexpr int kSgMfma = 0x8, kSgRead = 0x100;  // instruction classes of sched_group_barrier
+
+constexpr float kRowFloor = -1.0e20f;  // below every score, far above a masked one (kNegBig)
+
 struct PrefillParams {
   const uint16_t* kv;
   int64_t page_stride, v_offset;  // elements
   int32_t entry_stride, head_stride, page_size, page_shift;
+  uint32_t entry_stride_b;                 // bytes
+  uint32_t page_magic, page_down;  // t / page_size == (2 t * page_magic >> 32) >> page_down for t < 2^30
   uint32_t max_page;
   const int32_t* page_table;
   int32_t n_pages, kv_len;
@@ -48,18 +76,472 @@ struct PrefillParams {
   int32_t n_q, num_qo_heads, q_per_kv;
   float scale_log2;
   int32_t causal;
+  // The work of a KV head: n_rows = n_q * q_per_kv query rows (row = token * q_per_kv + head of the
+  // group), n_tiles workgroup tiles of bm of them, each cut into n_splits pieces of `chunk` keys.
+  int32_t n_kv, n_rows, bm, n_tiles, n_splits, chunk, head_major;
+  float* part_o;   // [n_splits][n_kv * n_rows][D]: un-normalised partial results (n_splits > 1)
+  float* part_ml;  // [n_splits][n_kv * n_rows][2]: running maximum (base 2) and denominator
 };
 
-// BN tokens per key tile (a multiple of 32), NW wavefronts per workgroup (4 or 8: a staged K/V
-// tile serves 16 MT NW query rows, so eight waves halve the global -> LDS traffic per flop)
+// keys that the rows of a tile see together: up to the position of its last query row
+__device__ __forceinline__ int tile_kv_end(const PrefillParams& p, int qtile) {
+  int last_row = (qtile + 1) * p.bm - 1;
+  last_row = last_row < p.n_rows ? last_row : p.n_rows - 1;
+  return p.causal ? p.kv_len - p.n_q + last_row / p.q_per_kv + 1 : p.kv_len;
+}
+
+// Where a workgroup's piece of the work lies.
+struct PrefillPiece {
+  int kvh, split, q0;      // KV head, piece of the keys, first query row
+  int k_begin, k_end;      // keys of the piece
+  bool whole;              // the tile has this piece alone: the result goes to o
+};
+__device__ __forceinline__ bool prefill_piece(const PrefillParams& p, PrefillPiece& w) {
+  // Workgroups go to the eight XCDs round-robin by linear id, and each XCD has its own L2.  Many
+  // tiles (head_major): all tiles of a KV head go to one XCD, one head after the other, so that its L2
+  // streams one head's K/V.  Few tiles: the heads alternate and all of them start with their longest
+  // tile, so that no long tile starts last.  (Placement only decides what the L2 holds and when a
+  // workgroup starts; results do not depend on it.)
+  const int lin = blockIdx.x;
+  int rem;
+  if (p.head_major) {
+    const int per_head = p.n_tiles * p.n_splits, slot = lin >> 3;
+    w.kvh = slot / per_head * 8 + (lin & 7);
+    rem = slot % per_head;
+  } else {
+    w.kvh = lin % p.n_kv;
+    rem = lin / p.n_kv;
+  }
+  const int qtile = p.n_tiles - 1 - rem / p.n_splits;
+  w.split = rem % p.n_splits;
+  w.q0 = qtile * p.bm;
+  const int end = tile_kv_end(p, qtile);
+  w.k_begin = __builtin_amdgcn_readfirstlane(w.split * p.chunk);
+  w.k_end = end - w.k_begin > p.chunk ? w.k_begin + p.chunk : end;
+  w.whole = end <= p.chunk;
+  return w.k_begin < end;  // false: this tile has fewer pieces
+}
+
+// head_dim 64 and 128: eight waves, 32 query rows each, key tiles of 64 tokens.
+// OCT: pages hold a multiple of eight tokens, so eight aligned tokens share a page: one page lookup per
+// wave and tile, made 64 tiles at a time.  Other page sizes look up a page per row (8192 x 28 heads
+// over 4: 480 us at pages of 1 and 454 at 4 against 403 at 16).
+template <typename T, int D, bool OCT>
+__global__ __launch_bounds__(512, 2) void prefill_attn_kernel(const PrefillParams p) {
+  constexpr int BN = 64, NS = D / 16, DB = D / 32;
+  // LDS: rings of RK key tiles and RV value tiles (values are read half a step later than keys)
+  constexpr int RK = 4, RV = 5, NL = D / 64;         // NL: loads per lane, tile and matrix
+  constexpr int BLK = D == 128 ? 1040 : 1024;        // bytes from one load's block to the next
+  constexpr int TILE_B = BN / (512 / D) * BLK;       // a block holds 512 / D rows
+  __shared__ __attribute__((aligned(16))) char smem[(RK + RV) * TILE_B];
+
+  // the wave index is made scalar: the activity tests below must be real branches, because matrix
+  // instructions do not honour the EXEC mask of a masked-off region
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c = lane & 31, h = lane >> 5;
+  const int late = wave >> 2;  // 0: the first of the two waves of a SIMD, 1: the second, a phase behind
+
+  PrefillPiece w;
+  if (!prefill_piece(p, w)) return;  // uniform
+  const int q_off = p.kv_len - p.n_q;     // position of query token 0
+  const int row0 = w.q0 + wave * 32;      // first query row of the wave
+  const int row_end = w.q0 + p.bm < p.n_rows ? w.q0 + p.bm : p.n_rows;  // behind the last of the workgroup
+
+  // ---- Q operand: row (row0 + c), pieces [16 s + 8 h, +8) --------------------------------------
+  int row = row0 + c;
+  row = row < row_end ? row : row_end - 1;
+  const int tok = row / p.q_per_kv;
+  const int64_t o_at = ((int64_t)tok * p.num_qo_heads + w.kvh * p.q_per_kv + (row - tok * p.q_per_kv)) * D;
+  int row_lim = p.kv_len - 1;  // last token this row sees
+  if (p.causal && q_off + tok < row_lim) row_lim = q_off + tok;
+  u32x4 qb[NS];
+#pragma unroll
+  for (int s = 0; s < NS; ++s) qb[s] = *reinterpret_cast<const u32x4*>(p.q + o_at + 16 * s + 8 * h);
+  const int wave_first_pos = q_off + row0 / p.q_per_kv;  // position of the wave's first query row
+
+  // ---- staging: rows go from memory straight into LDS -------------------------------------------
+  // A wave brings rows 8 wave .. 8 wave + 7 of a tile, one KB (a block) per load: lane l fills bytes
+  // 16 l .. 16 l + 15 of the block and so chooses, by what it fetches, which piece of which row lies
+  // there (the swizzle).
+  constexpr int RPB = 512 / D, CPR = D / 8;  // rows per block, 16-byte pieces per row
+  const int rb = lane / CPR;                 // row of the block that this lane fetches a piece of
+  uint32_t piece_k, piece_v;                 // and the byte offset of the piece
+  if constexpr (D == 128) {
+    piece_k = piece_v = (uint32_t)((lane & 15) ^ (4 * rb)) * 16;
+  } else {
+    piece_k = (uint32_t)((lane & 7) ^ ((4 * wave + (rb >> 1)) & 7)) * 16;
+    piece_v = (uint32_t)((lane & 7) ^ (4 * ((rb >> 1) & 1))) * 16;
+  }
+  const uint32_t smem_at = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
+  const uint64_t k_base = (uint64_t)(uintptr_t)(p.kv + (int64_t)w.kvh * p.head_stride);
+  const int last_tok = p.kv_len - 1;
+  auto page_of = [&](int t) { return (int)(__umulhi(2u * (uint32_t)t, p.page_magic) >> p.page_down); };
+  // first token of the wave's rows of tile j (tiles past the end repeat the last tokens: the loads need
+  // no branch and what they bring is masked)
+  auto first_tok = [&](int j) {
+    const int t = w.k_begin + j * BN + 8 * wave;
+    return t < last_tok ? t : last_tok & ~7;
+  };
+  // Row addresses are formed for several tiles at once, one per lane.  OCT (the wave's eight rows of a
+  // tile share a page): lane l holds the offset of the first row of tile (j & ~63) + l, which is
+  // broadcast when that tile is brought; the other rows lie at fixed distances, except in the tiles from
+  // `tail_from` on, whose rows end with the sequence.  Otherwise lane l holds the page of row l % 8 of
+  // tile (j & ~7) + l / 8, and `ahead` those of the eight tiles after that.
+  uint32_t addr_lo = 0, addr_hi = 0;
+  int pages = 0, ahead = 0;
+  const int tail_from = (last_tok - 7 - w.k_begin - 8 * wave + BN) >> 6;
+  uint32_t row_at[NL];
+#pragma unroll
+  for (int x = 0; x < NL; ++x) row_at[x] = (uint32_t)(RPB * x + rb) * p.entry_stride_b;
+  auto page_at = [&](int t) {
+    const uint32_t page = (uint32_t)p.page_table[page_of(t)];
+    return page > p.max_page ? p.max_page : page;
+  };
+  // brings tile j to the ring slots at LDS bytes k_to and v_to
+  auto bring = [&](int j, uint32_t k_to, uint32_t v_to) __attribute__((always_inline)) {
+    k_to += NL * wave * BLK;
+    v_to += NL * wave * BLK;
+    if constexpr (OCT) {
+      if ((j & 63) == 0) {
+        const int t = first_tok(j + lane);
+        const uint64_t at = k_base + (uint64_t)page_at(t) * (uint64_t)(p.page_stride * 2) +
+                            (uint64_t)(uint32_t)(t - page_of(t) * p.page_size) * p.entry_stride_b;
+        addr_lo = (uint32_t)at;
+        addr_hi = (uint32_t)(at >> 32);
+      }
+      const uint64_t k_row = (uint64_t)(uint32_t)__builtin_amdgcn_readlane(addr_lo, j & 63) |
+                             (uint64_t)(uint32_t)__builtin_amdgcn_readlane(addr_hi, j & 63) << 32;
+      const uint64_t v_row = k_row + (uint64_t)p.v_offset * 2;
+      uint32_t at[NL];
+#pragma unroll
+      for (int x = 0; x < NL; ++x) at[x] = row_at[x];
+      if (__builtin_expect(j >= tail_from, 0)) {
+        const int lim = last_tok - first_tok(j);
+#pragma unroll
+        for (int x = 0; x < NL; ++x)
+          at[x] = (uint32_t)(RPB * x + rb < lim ? RPB * x + rb : lim) * p.entry_stride_b;
+      }
+#pragma unroll
+      for (int x = 0; x < NL; ++x) {
+        load_lds(k_to + x * BLK, k_row, at[x] + piece_k);
+        load_lds(v_to + x * BLK, v_row, at[x] + piece_v);
+      }
+    } else {
+      auto page_of_lane = [&](int j8) {
+        const int t = w.k_begin + (j8 + (lane >> 3)) * BN + 8 * wave + (lane & 7);
+        return (int)page_at(t < last_tok ? t : last_tok);
+      };
+      if ((j & 7) == 0) {
+        pages = j == 0 ? page_of_lane(0) : ahead;
+        asm volatile("" : "+v"(pages));  // waited for here and not, with everything else, in every step
+        ahead = page_of_lane(j + 8);
+      }
+      const int t0 = first_tok(j), lim = last_tok - t0;
+#pragma unroll
+      for (int x = 0; x < NL; ++x) {
+        const int t = RPB * x + rb < lim ? t0 + RPB * x + rb : last_tok;
+        const uint32_t page = (uint32_t)__shfl(pages, 8 * (j & 7) + RPB * x + rb, 64);
+        const uint64_t row = (uint64_t)page * (uint64_t)(p.page_stride * 2) +
+                             (uint64_t)(uint32_t)(t - page_of(t) * p.page_size) * p.entry_stride_b;
+        load_lds(k_to + x * BLK, k_base + row + piece_k);
+        load_lds(v_to + x * BLK, k_base + (uint64_t)p.v_offset * 2 + row + piece_v);
+      }
+    }
+  };
+
+  // ---- the two matrix products and the softmax between them --------------------------------------
+  f32x16 st[2], oacc[DB];
+  u32x4 pa[4];
+#pragma unroll
+  for (int b = 0; b < DB; ++b)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) oacc[b][v] = 0.f;
+  float m_run = kNegBig, l_run = 0.f;
+
+  // S^T = K Q^T, two halves of 32 tokens; the first PRE operands were read in the phase before
+  constexpr int PRE = 4;
+  u32x4 kpre[PRE];
+  uint32_t k_lane[4], v_lane[DB];  // byte offsets of this lane's pieces in a tile
+  {
+    const int r = c & 3, vr = (lane & 15) >> 2, q = 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1);
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+      k_lane[a] = D == 128 ? (c >> 2) * BLK + r * 256 + 16 * h + 64 * (a ^ r)
+                           : c * 128 + ((16 * h + 32 * a) ^ (16 * ((c >> 1) & 7)));
+#pragma unroll
+    for (int b = 0; b < DB; ++b)
+      v_lane[b] = 16 * q + 8 * (lane & 1) +
+                  (D == 128 ? h * BLK + vr * 256 + 64 * (b ^ vr) : (4 * h + vr) * 128 + 64 * (b ^ (vr >> 1)));
+  }
+  // operand x of the scores: 16 dimensions (x / 2) of 32 keys (x % 2)
+  auto k_operand = [&](const uint32_t (&at)[4], int x) {
+    const int s = x >> 1, t = x & 1;
+    const uint32_t off = D == 128 ? at[s >> 1] + 32 * (s & 1) + 8 * BLK * t : at[s & 3] + 4096 * t;
+    return *reinterpret_cast<const u32x4*>(smem + off);
+  };
+  auto prefetch = [&](uint32_t kslot) {
+    uint32_t at[4];
+#pragma unroll
+    for (int a = 0; a < 4; ++a) at[a] = k_lane[a] + kslot;
+#pragma unroll
+    for (int x = 0; x < PRE; ++x) kpre[x] = k_operand(at, x);
+  };
+  auto scores = [&](uint32_t kslot) {
+    uint32_t at[4];
+#pragma unroll
+    for (int a = 0; a < 4; ++a) at[a] = k_lane[a] + kslot;
+    const f32x16 zero = {};
+#pragma unroll
+    for (int x = 0; x < 2 * NS; ++x) {
+      const u32x4 ka = x < PRE ? kpre[x] : k_operand(at, x);
+      st[x & 1] = mfma_32x32x16<T>(ka, qb[x >> 1], x < 2 ? zero : st[x & 1]);
+    }
+  };
+  // O^T += V^T P^T
+  auto weigh = [&](uint32_t vslot) {
+    uint32_t at[DB];
+#pragma unroll
+    for (int b = 0; b < DB; ++b) at[b] = v_lane[b] + vslot;
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int b = 0; b < DB; ++b) {
+        const uint32_t off = at[b] + s * (16 / RPB) * BLK;
+        const u32x2 t0 = lds_read_tr16(reinterpret_cast<const uint16_t*>(smem + off));
+        const u32x2 t1 = lds_read_tr16(reinterpret_cast<const uint16_t*>(smem + off + 8 / RPB * BLK));
+        oacc[b] = mfma_32x32x16<T>(u32x4{t0.x, t0.y, t1.x, t1.y}, pa[s], oacc[b]);
+      }
+  };
+  // Order of a matrix phase: operands are read LEAD matrix instructions ahead of their use (left to
+  // itself the compiler reads them one instruction ahead and waits).
+  auto order_scores = [&]() {
+    __builtin_amdgcn_sched_group_barrier(kSgRead, 2, 0);
+#pragma unroll
+    for (int x = 0; x < 2 * NS - PRE - 2; ++x) {
+      __builtin_amdgcn_sched_group_barrier(kSgMfma, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(kSgRead, 1, 0);
+    }
+  };
+  auto order_weigh = [&]() {
+    __builtin_amdgcn_sched_group_barrier(kSgRead, 8, 0);
+#pragma unroll
+    for (int x = 0; x < 4 * DB - 4; ++x) {
+      __builtin_amdgcn_sched_group_barrier(kSgMfma, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(kSgRead, 2, 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(kSgMfma, 4, 0);
+  };
+  auto order_both = [&]() {
+    __builtin_amdgcn_sched_group_barrier(kSgRead, 2, 0);
+#pragma unroll
+    for (int x = 0; x < 2 * NS - PRE - 2; ++x) {
+      __builtin_amdgcn_sched_group_barrier(kSgMfma, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(kSgRead, 1, 0);
+    }
+#pragma unroll
+    for (int x = 0; x < PRE + 4 * DB - 2; ++x) {  // the scores' last products, then the weights'
+      __builtin_amdgcn_sched_group_barrier(kSgMfma, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(kSgRead, 2, 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(kSgMfma, 4, 0);
+  };
+  // first tile in which a row of the wave sees less than all keys
+  int mask_from = (p.kv_len - BN - w.k_begin) >> 6;
+  if (p.causal) {
+    const int m = (wave_first_pos - (BN - 1) - w.k_begin) >> 6;
+    mask_from = m < mask_from ? m : mask_from;
+  }
+  mask_from += 1;
+  auto first_key = [&](int i) { return w.k_begin + i * BN; };
+  // P = 2^(s scale - m_run), its row sums (of this lane's half of the keys)
+  auto weights = [&]() __attribute__((always_inline)) {
+    float sum[2] = {0.f, 0.f};
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        uint32_t pk[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float a = fast_exp2(fmaf(st[t][8 * u + 2 * e], p.scale_log2, -m_run));
+          const float b = fast_exp2(fmaf(st[t][8 * u + 2 * e + 1], p.scale_log2, -m_run));
+          pk[e] = pack2<T>(a, b);
+          sum[0] += a;
+          sum[1] += b;
+        }
+        pa[2 * t + u] = u32x4{pk[0], pk[1], pk[2], pk[3]};
+      }
+    float all = sum[0] + sum[1];
+    asm volatile("" : "+v"(all));  // here, not where the next phase would have to keep its summands
+    return all;
+  };
+  // The reference point m_run is the row's maximum of some earlier tile: softmax does not depend on it,
+  // and weights of up to kTopWeight are as exact as weights of up to 1.  So a tile's maximum is formed
+  // only when its weights turn out larger (and in the first tile, where m_run is no score yet); then the
+  // accumulators are rescaled and the weights formed again.
+  auto softmax = [&](int i) __attribute__((always_inline)) {
+    if (__builtin_expect(i >= mask_from, 0)) {
+      int lim = row_lim - first_key(i) - 4 * h;
+      asm volatile("" : "+v"(lim));  // keeps the 32 differences of the comparisons out of the loop's registers
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int v = 0; v < 16; ++v)
+          st[t][v] = 32 * t + 8 * (v / 4) + v % 4 <= lim ? st[t][v] : kNegBig;
+    }
+    float l_tile = weights();
+    if (__builtin_expect(__ballot(!(l_tile <= kTopWeight)) != 0, 0)) {
+      float mx = kRowFloor;
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int v = 0; v < 16; v += 2) mx = fmaxf(fmaxf(st[t][v], st[t][v + 1]), mx);
+      float lo, hi;
+      swap_halves32(mx, lo, hi);
+      const float m_new = fmaxf(fmaxf(lo, hi) * p.scale_log2, m_run);
+      const float alpha = fast_exp2(m_run - m_new);
+      m_run = m_new;
+      l_run *= alpha;
+#pragma unroll
+      for (int b = 0; b < DB; ++b)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) oacc[b][v] *= alpha;
+      l_tile = weights();
+    }
+    l_run += l_tile;
+  };
+
+  const int nt = __builtin_amdgcn_readfirstlane((w.k_end - w.k_begin + BN - 1) / BN);
+  // tiles that hold keys for the wave's own rows; a wave goes through one even if it has none
+  int own = nt;
+  if (p.causal) {
+    const int last_row = row0 + 31 < row_end ? row0 + 31 : row_end - 1;
+    const int mine = (q_off + last_row / p.q_per_kv - w.k_begin) / BN + 1;
+    own = mine < nt ? mine : nt;
+  }
+  if (row0 >= row_end || own < 1) own = 1;
+  own = __builtin_amdgcn_readfirstlane(own);
+  auto phase_end = [&]() {
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
+
+  // ---- the steps ----------------------------------------------------------------------------------
+  // The two waves of a SIMD take turns, half a step apart: while one forms the scores of its next tile
+  // and the weighted values of its last one (matrix phase), the other turns scores into weights (vector
+  // phase); a barrier ends every half step.  Both walk the same tiles in LDS:
+  //   half step      2i            2i + 1         2i + 2
+  //   early wave     matrix i      vector i       matrix i + 1        matrix i: scores i, values i - 1
+  //   late wave      vector i - 1  matrix i       vector i
+  // A wave asks for its rows of tile i + 3 (late: i + 4) in vector phase i, which is when the last
+  // reader has left the ring slots that they go to, and has them by the end of matrix phase i + 2
+  // (late: i + 2), before the early waves read the first operands of tile i + 3 at the end of vector
+  // phase i + 2.  A wave stops computing after its own last tile (a causal workgroup tile has four to go
+  // on its diagonal) and then only brings its share of the rows: 15.2 -> 13.5 us for 300 tokens x 32 heads.
+  constexpr uint32_t K_END = RK * TILE_B, V_END = K_END + RV * TILE_B;
+  uint32_t kr = 0, vr = V_END - TILE_B;  // ring slots of K(i) and V(i - 1)
+  // ring slots of the tile that is asked for next
+  uint32_t kw = (3 + late) % RK * TILE_B, vw = K_END + (3 + late) % RV * TILE_B;
+  auto next_k = [&](uint32_t slot) { return slot == K_END - TILE_B ? 0u : slot + TILE_B; };
+  auto next_v = [&](uint32_t slot) { return slot == V_END - TILE_B ? K_END : slot + TILE_B; };
+  auto matrix_done = [&]() {
+    __builtin_amdgcn_s_setprio(0);
+    // the wave's operands have been read, and all rows it asked for but those of the youngest tile are there
+    if constexpr (NL == 2)
+      asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)" ::: "memory");
+    else
+      asm volatile("s_waitcnt vmcnt(2) lgkmcnt(0)" ::: "memory");
+    phase_end();
+  };
+  auto bring_next = [&](int i) __attribute__((always_inline)) {  // of vector phase i
+    bring(i + 3 + late, smem_at + kw, smem_at + vw);
+    kw = next_k(kw);
+    vw = next_v(vw);
+  };
+#pragma unroll
+  for (int j = 0; j < 3; ++j) bring(j, smem_at + j * TILE_B, smem_at + K_END + j * TILE_B);
+  if (late) bring(3, smem_at + 3 * TILE_B, smem_at + K_END + 3 * TILE_B);
+  if constexpr (NL == 2)
+    asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+  else
+    asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
+  phase_end();
+  prefetch(0);
+  if (late) phase_end();
+  scores(0);
+  order_scores();
+  matrix_done();
+  for (int i = 0; i < own - 1; ++i) {
+    kr = next_k(kr);
+    vr = next_v(vr);
+    bring_next(i);
+    prefetch(kr);
+    softmax(i);
+    phase_end();
+    __builtin_amdgcn_s_setprio(1);
+    scores(kr);
+    weigh(vr);
+    order_both();
+    matrix_done();
+  }
+  vr = next_v(vr);
+  if (own < nt) bring_next(own - 1);
+  softmax(own - 1);
+  if (own < nt || !late) phase_end();
+  weigh(vr);
+  order_weigh();
+  if (own < nt) {  // the other waves still need this one's share of the rows
+    matrix_done();
+    for (int i = own; i < nt - 1; ++i) {
+      bring_next(i);
+      phase_end();
+      matrix_done();
+    }
+    if (!late) phase_end();
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // nothing is on its way to LDS when the workgroup ends
+
+  // ---- normalise and store (or leave the piece's partial result): a lane holds dimensions
+  //      32 b + 8 (v / 4) + 4 h + v % 4 of its row ---------------------------------------------------
+  float l0, l1;
+  swap_halves32(l_run, l0, l1);
+  const float l = l0 + l1;
+  if (row0 + c >= row_end) return;
+  if (w.whole) {
+    const float inv = l > 0.f ? 1.f / l : 0.f;
+#pragma unroll
+    for (int b = 0; b < DB; ++b)
+#pragma unroll
+      for (int v = 0; v < 16; v += 4)
+        *reinterpret_cast<u32x2*>(p.o + o_at + 32 * b + 2 * v + 4 * h) =
+            u32x2{pack2<T>(oacc[b][v] * inv, oacc[b][v + 1] * inv),
+                  pack2<T>(oacc[b][v + 2] * inv, oacc[b][v + 3] * inv)};
+  } else {
+    const int64_t part = ((int64_t)w.split * p.n_kv + w.kvh) * p.n_rows + row0 + c;
+#pragma unroll
+    for (int b = 0; b < DB; ++b)
+#pragma unroll
+      for (int v = 0; v < 16; v += 4)
+        *reinterpret_cast<f32x4*>(p.part_o + part * D + 32 * b + 2 * v + 4 * h) =
+            f32x4{oacc[b][v], oacc[b][v + 1], oacc[b][v + 2], oacc[b][v + 3]};
+    if (h == 0) *reinterpret_cast<f32x2*>(p.part_ml + part * 2) = f32x2{m_run, l};
+  }
+}
+
+// head_dim 256, whose output alone would take 128 registers of a wave in the kernel above: 16 MT query
+// rows per wave and 16x16x32 MFMA, BN tokens per key tile (a multiple of 32), NW waves per workgroup.
+// K/V tiles pass through registers into two LDS buffers per matrix, one barrier per tile; LDS rows are
+// padded by 32 bytes, which keeps the 16-byte K reads and the transposed V reads free of bank conflicts.
 template <typename T, int D, int MT, int BN, int NW>
-__global__ __launch_bounds__(64 * NW, MT == 2 ? 2 : 1) void prefill_attn_kernel(const PrefillParams p) {
+__global__ __launch_bounds__(64 * NW, 1) void prefill_attn_staged_kernel(const PrefillParams p) {
   constexpr int kThreads = 64 * NW;
-  constexpr int kPfBM = 16 * MT * NW;  // query rows per workgroup
   constexpr int WR = 16 * MT;       // query rows per wavefront
   constexpr int NS = D / 32;        // 16-byte pieces of a Q/K row per lane (one MFMA each)
   constexpr int DC = D / 16;        // head dimensions per lane in the P.V product
-  constexpr int PITCH = D + 16;     // LDS row pitch in elements: +32 bytes (see the layout note)
+  constexpr int PITCH = D + 16;     // LDS row pitch in elements: +32 bytes
   constexpr int CPR = D / 8;        // 16-byte chunks per row
   constexpr int kPfBN = BN;
   constexpr int NSUB = BN / 16;     // 16-token sub-tiles per key tile
@@ -67,7 +549,7 @@ __global__ __launch_bounds__(64 * NW, MT == 2 ? 2 : 1) void prefill_attn_kernel(
   constexpr int RPT = BN / SR;      // staging: rows per thread (row = tid / 8 + SR jr)
   constexpr int CCT = CPR / 8;      // staging: chunks per thread and row (chunk = tid % 8 + 8 jc)
   constexpr int CPT = RPT * CCT;    // chunks a thread stages per tile and matrix
-  static_assert(D == 64 || D == 128 || D == 256, "head dimensions of the prefill kernel");
+  static_assert(D % 64 == 0, "a thread stages whole pieces");
   static_assert(BN % 32 == 0 && RPT >= 1 && CPT * kThreads == BN * CPR, "key tile");
   // two buffers per matrix: tile t + 1 is written while tile t is still being read
   constexpr int TILE = kPfBN * PITCH;
@@ -78,37 +560,23 @@ __global__ __launch_bounds__(64 * NW, MT == 2 ? 2 : 1) void prefill_attn_kernel(
   // matrix instructions do not honour the EXEC mask of a masked-off region
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 15, g = lane >> 4;
-  // Workgroups go to the eight XCDs round-robin by linear id, and each XCD has its own L2.  When
-  // the KV heads divide evenly, all query tiles of the heads that share a KV head are given to one
-  // XCD, so that its L2 streams one head's K/V instead of every head's.  (Placement only decides
-  // what the L2 holds; results do not depend on it.)  Longest rows first in either order.
-  int qtile, qh;
-  {
-    const int n_tiles = gridDim.x, n_heads = gridDim.y;
-    const int lin = blockIdx.x + n_tiles * blockIdx.y;
-    const int n_kv = n_heads / p.q_per_kv;
-    if (n_kv % 8 == 0) {
-      const int xcd = lin & 7, slot = lin >> 3;
-      const int idx = slot / n_tiles;  // which of this XCD's heads
-      qtile = n_tiles - 1 - slot % n_tiles;
-      qh = ((idx / p.q_per_kv) * 8 + xcd) * p.q_per_kv + idx % p.q_per_kv;
-    } else {
-      qtile = n_tiles - 1 - blockIdx.x;
-      qh = blockIdx.y;
-    }
-  }
-  const int kvh = qh / p.q_per_kv;
-  const int q0 = qtile * kPfBM;
-  const int q_off = p.kv_len - p.n_q;  // position of query row 0
+  PrefillPiece w;
+  if (!prefill_piece(p, w)) return;  // uniform
+  const int kvh = w.kvh, split = w.split, q0 = w.q0, k_begin = w.k_begin, kv_end = w.k_end;
+  const bool whole = w.whole;
+  const int q_off = p.kv_len - p.n_q;  // position of query token 0
 
   // ---- Q operands: row (q0 + WR wave + 16 mt + r), pieces [32 s + 8 g, +8) ----------------------
   u32x4 qb[MT][NS];
+  int qpos_of[MT];  // position of this lane's query row
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
     int row = q0 + wave * WR + mt * 16 + r;
-    row = row < p.n_q ? row : p.n_q - 1;
-    const u32x4* src =
-        reinterpret_cast<const u32x4*>(p.q + ((int64_t)row * p.num_qo_heads + qh) * D);
+    row = row < p.n_rows ? row : p.n_rows - 1;
+    const int tok = row / p.q_per_kv;
+    qpos_of[mt] = q_off + tok;
+    const u32x4* src = reinterpret_cast<const u32x4*>(
+        p.q + ((int64_t)tok * p.num_qo_heads + kvh * p.q_per_kv + (row - tok * p.q_per_kv)) * D);
 #pragma unroll
     for (int s = 0; s < NS; ++s) qb[mt][s] = src[4 * s + g];
   }
@@ -122,11 +590,6 @@ __global__ __launch_bounds__(64 * NW, MT == 2 ? 2 : 1) void prefill_attn_kernel(
 #pragma unroll
     for (int d = 0; d < DC; ++d) oacc[mt][d] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
-
-  // keys this workgroup needs: up to the position of its last query row
-  int last_row = q0 + kPfBM - 1;
-  last_row = last_row < p.n_q ? last_row : p.n_q - 1;
-  const int kv_end = p.causal ? (q_off + last_row + 1) : p.kv_len;
 
   // ---- staging: thread -> CPT chunks of K and of V per tile --------------------------------------
   // eight adjacent lanes move 128 contiguous bytes of one row (one cache line in, one conflict-free
@@ -183,13 +646,16 @@ __global__ __launch_bounds__(64 * NW, MT == 2 ? 2 : 1) void prefill_attn_kernel(
       }
   };
 
-  const int wave_first_pos = q_off + q0 + wave * WR;  // position of the wave's first query row
+  // positions of the wave's first and last query row (a wave without rows sees no key tile)
+  const int wave_row0 = q0 + wave * WR;
+  const int wave_first_pos = q_off + wave_row0 / p.q_per_kv;
+  const int wave_last_pos = wave_row0 < p.n_rows ? (p.causal ? q_off + (wave_row0 + WR - 1) / p.q_per_kv : p.kv_len) : -1;
   auto compute = [&](int kt, int buf) {
     // A wave whose last query row lies before the key tile sees none of it (causal).  Inside an
     // active wave every query tile is computed: a tile that lies wholly before the key tile is
     // masked to zero weight below, which happens once per wave, and the loop body stays free of
     // branches around the matrix instructions.
-    if (!p.causal || kt <= wave_first_pos + WR - 1) {
+    if (kt <= wave_last_pos) {
       // ---- S^T: each K operand is read once and used by every active query tile -----------------
       // (the two matrix phases run at raised wave priority: while one wave of a SIMD is in its
       // softmax arithmetic, the other's matrix instructions are issued first and keep the matrix
@@ -215,21 +681,24 @@ __global__ __launch_bounds__(64 * NW, MT == 2 ? 2 : 1) void prefill_attn_kernel(
       uint32_t pa[MT][NSUB][2];
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) {
-        const int qpos = wave_first_pos + mt * 16 + r;  // position of this lane's query row
+        const int qpos = qpos_of[mt];
         // the test of the wave's first query tile covers the second: masking a tile that does
         // not need it changes nothing, and one rare branch keeps the position arithmetic out of
         // the common path
         const bool need_mask =
             (p.causal && kt + kPfBN - 1 > wave_first_pos) || kt + kPfBN > p.kv_len;
         if (need_mask) {
+          // the last token this row sees, counted from the lane's first one of the tile (opaque: the
+          // compiler would keep the 32 differences of the comparisons below in registers for the loop)
+          int lim = p.kv_len - 1;
+          if (p.causal && qpos < lim) lim = qpos;
+          lim -= kt + 4 * g;
+          asm volatile("" : "+v"(lim));
 #pragma unroll
           for (int sub = 0; sub < NSUB; ++sub)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              const int tpos = kt + sub * 16 + 4 * g + i;
-              const bool ok = tpos < p.kv_len && (!p.causal || tpos <= qpos);
-              st[mt][sub][i] = ok ? st[mt][sub][i] : kNegBig;
-            }
+            for (int i = 0; i < 4; ++i)
+              st[mt][sub][i] = sub * 16 + i <= lim ? st[mt][sub][i] : kNegBig;
         }
         float mt_max = kNegBig;
 #pragma unroll
@@ -237,12 +706,13 @@ __global__ __launch_bounds__(64 * NW, MT == 2 ? 2 : 1) void prefill_attn_kernel(
 #pragma unroll
           for (int i = 0; i < 4; ++i) mt_max = fmaxf(mt_max, st[mt][sub][i]);
         mt_max = rows_max(mt_max);
-        // m_run is kept in the scaled base-2 domain.  A masked entry (kNegBig) gives exp2(-huge) = 0
-        // by itself: every query row sees token 0 in its first tile, so m_new is a real maximum.
+        // m_run is kept in the scaled base-2 domain.  A masked entry (kNegBig) gives exp2(-huge) = 0 by
+        // itself, also in a tile that masks the whole row (a later piece of the keys may begin with
+        // one): the reference point never falls to where kNegBig lies.
         // The running maximum only moves when the tile's maximum exceeds it by more than 2^8:
         // softmax does not depend on the reference point, weights up to 256 are exact to the same
         // relative precision, and the accumulator rescale below becomes rare.
-        const float m_tile = mt_max * p.scale_log2;
+        const float m_tile = fmaxf(mt_max, kRowFloor) * p.scale_log2;
         const float m_new = m_tile > m_run[mt] + 8.f ? m_tile : m_run[mt];
         const float alpha = fast_exp2(m_run[mt] - m_new);
         m_run[mt] = m_new;
@@ -295,18 +765,18 @@ __global__ __launch_bounds__(64 * NW, MT == 2 ? 2 : 1) void prefill_attn_kernel(
     }
   };
 
-  // tile 0 into buffer 0, tile 1 into register set a
-  lookup(0);
-  fetch(0, kreg_a, vreg_a);
-  lookup(kPfBN);
+  // first tile into buffer 0, second tile into register set a
+  lookup(k_begin);
+  fetch(k_begin, kreg_a, vreg_a);
+  lookup(k_begin + kPfBN);
   stash(0, kreg_a, vreg_a);
-  if (kPfBN < kv_end) {
-    fetch(kPfBN, kreg_a, vreg_a);
-    lookup(2 * kPfBN);
+  if (k_begin + kPfBN < kv_end) {
+    fetch(k_begin + kPfBN, kreg_a, vreg_a);
+    lookup(k_begin + 2 * kPfBN);
   }
   // One barrier per tile: it makes tile kt visible in its buffer, and it tells that every wave has
   // finished reading the other buffer, which the end of the step overwrites with tile kt + BN.
-  for (int kt = 0; kt < kv_end; kt += 2 * kPfBN) {
+  for (int kt = k_begin; kt < kv_end; kt += 2 * kPfBN) {
     __syncthreads();
     if (kt + 2 * kPfBN < kv_end) {
       fetch(kt + 2 * kPfBN, kreg_b, vreg_b);
@@ -324,51 +794,150 @@ __global__ __launch_bounds__(64 * NW, MT == 2 ? 2 : 1) void prefill_attn_kernel(
     if (kt + 2 * kPfBN < kv_end) stash(0, kreg_b, vreg_b);
   }
 
-  // ---- normalise and store: lane holds rows 4g + i, dimensions 16 a + r ---------------------------
+  // ---- normalise and store (or leave the piece's partial result): lane holds rows 4g + i,
+  //      dimensions 16 a + r ------------------------------------------------------------------------
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
     const float l = rows_sum(l_run[mt]);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const float li = __shfl(l, 4 * g + i, 64);
-      const float inv = li > 0.f ? 1.f / li : 0.f;
-      const int row = q0 + wave * WR + mt * 16 + 4 * g + i;
-      if (row < p.n_q) {
-        uint16_t* dst = p.o + ((int64_t)row * p.num_qo_heads + qh) * D + r;
+      const int row = wave_row0 + mt * 16 + 4 * g + i;
+      if (whole) {
+        const float inv = li > 0.f ? 1.f / li : 0.f;
+        if (row < p.n_rows) {
+          const int tok = row / p.q_per_kv;
+          uint16_t* dst =
+              p.o + ((int64_t)tok * p.num_qo_heads + kvh * p.q_per_kv + (row - tok * p.q_per_kv)) * D + r;
 #pragma unroll
-        for (int a = 0; a < DC; ++a) dst[16 * a] = from_float<T>(oacc[mt][a][i] * inv);
+          for (int a = 0; a < DC; ++a) dst[16 * a] = from_float<T>(oacc[mt][a][i] * inv);
+        }
+      } else {
+        const float mi = __shfl(m_run[mt], 4 * g + i, 64);
+        if (row < p.n_rows) {
+          const int64_t part = ((int64_t)split * p.n_kv + kvh) * p.n_rows + row;
+          float* dst = p.part_o + part * D + r;
+#pragma unroll
+          for (int a = 0; a < DC; ++a) dst[16 * a] = oacc[mt][a][i];
+          if (r == 0) {
+            p.part_ml[part * 2] = mi;
+            p.part_ml[part * 2 + 1] = li;
+          }
+        }
       }
     }
   }
 }
 
+// Adds up the pieces of every row whose keys were split: D / 4 adjacent threads own a row, four
+// dimensions each.  A piece in which a row sees no key carries a maximum far below any real one and
+// so a weight of zero; the piece that holds token 0 is seen by every row.
+template <typename T, int D>
+__global__ __launch_bounds__(256) void prefill_merge_kernel(const PrefillParams p) {
+  constexpr int TPR = D / 4;
+  const int64_t at = (int64_t)blockIdx.x * (256 / TPR) + threadIdx.x / TPR;
+  if (at >= (int64_t)p.n_kv * p.n_rows) return;
+  const int kvh = (int)(at / p.n_rows), row = (int)(at - (int64_t)kvh * p.n_rows);
+  const int kv_end = tile_kv_end(p, row / p.bm);
+  const int n_parts = (kv_end + p.chunk - 1) / p.chunk;
+  if (n_parts <= 1) return;  // the attention kernel wrote the result
+  const int c = threadIdx.x % TPR;
+  const int64_t stride = (int64_t)p.n_kv * p.n_rows;
+  float M = kNegBig, L = 0.f;
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  for (int s0 = 0; s0 < n_parts; s0 += 4) {  // four pieces in flight
+    f32x4 v[4];
+    float m[4], l[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int64_t part = (int64_t)(s0 + u < n_parts ? s0 + u : n_parts - 1) * stride + at;
+      v[u] = *reinterpret_cast<const f32x4*>(p.part_o + part * D + 4 * c);
+      const f32x2 ml = *reinterpret_cast<const f32x2*>(p.part_ml + part * 2);
+      m[u] = s0 + u < n_parts ? ml.x : 2.f * kNegBig;
+      l[u] = s0 + u < n_parts ? ml.y : 0.f;
+    }
+    const float m_new = fmaxf(fmaxf(fmaxf(m[0], m[1]), fmaxf(m[2], m[3])), M);
+    const float alpha = fast_exp2(M - m_new);
+    M = m_new;
+    L *= alpha;
+    acc *= alpha;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const float f = s0 + u < n_parts ? fast_exp2(m[u] - m_new) : 0.f;
+      L = fmaf(l[u], f, L);
+#pragma unroll
+      for (int d = 0; d < 4; ++d) acc[d] = fmaf(v[u][d], f, acc[d]);
+    }
+  }
+  const float inv = L > 0.f ? 1.f / L : 0.f;
+  const int tok = row / p.q_per_kv;
+  uint16_t* dst = p.o + ((int64_t)tok * p.num_qo_heads + kvh * p.q_per_kv + (row - tok * p.q_per_kv)) * D + 4 * c;
+  *reinterpret_cast<u32x2*>(dst) = u32x2{pack2<T>(acc[0] * inv, acc[1] * inv), pack2<T>(acc[2] * inv, acc[3] * inv)};
+}
+
+// Rows per workgroup tile and pieces per tile.  A workgroup walks its keys one tile after the other, so a
+// few query rows on a long cache (a further turn of a conversation) leave most of the chip idle however
+// many keys there are, and so do a short prompt and a prompt of few heads.  Pieces shorten the walk for the
+// price of a merge; smaller row tiles (waves without rows compute nothing) give more workgroups, each with a
+// SIMD per wave, and so a shorter step.  The estimate, in steps of a full workgroup (64 keys, 1.2 us): the
+// chip runs `slots` workgroups at a time (one of eight waves per CU, two of four); a workgroup of 256, 128
+// or 64 rows costs 1, 0.87 or 0.83 per key tile and 6.5 or 4.5 to start (page table, queries, first tiles,
+// cold code, diagonal), all measured; causal tiles start longest first, which leaves a tail of about a
+// quarter of the longest; pieces cost the merge launch (two) and their fp32 round trip through memory.
+// Measured at head_dim 128, pages of 16, us for tiles of 256 / 128 / 64 rows, whole: prompts of 32 heads
+// over 8 KV heads, 100 tokens 9.6 / 8.7 / 7.5, 300 14.0 / 11.7 / 10.5, 640 21 / 17.0 / 15.5, 1000 27 / 23 / 27,
+// 2000 48 / 47 / 80, 2900 75 / 92 / 152.  Pieces against whole tiles of 256: 500 rows of 32 heads on 32768
+// keys 254 against 600.
+static double prefill_cost(const PrefillParams& p, int head_dim, int kv_len, double tile, int splits) {
+  const int bn = head_dim == 256 ? 32 : 64;
+  const int64_t slots = (int64_t)td_num_cus() * (head_dim == 256 ? 2 : 1);
+  const double start = p.bm == 256 ? 6.5 : 4.5, merge = 2.0;
+  const int max_tiles = (kv_len + bn - 1) / bn, c = (max_tiles + splits - 1) / splits;
+  int64_t jobs = 0, total = 0;
+  for (int t = 0; t < p.n_tiles; ++t) {
+    int last = (t + 1) * p.bm - 1;
+    last = last < p.n_rows ? last : p.n_rows - 1;
+    const int end = p.causal ? kv_len - p.n_q + last / p.q_per_kv + 1 : kv_len;
+    const int k = (end + bn - 1) / bn;
+    jobs += (k + c - 1) / c;
+    total += k;
+  }
+  jobs *= p.n_kv;
+  total *= p.n_kv;
+  const double mean = tile * (double)total / jobs + start, longest = tile * c + start;
+  const double share = mean * jobs / slots + 0.25 * longest, rounds = (double)((jobs + slots - 1) / slots) * mean;
+  const double cost = share < rounds ? share : rounds;
+  const double pieces = merge + (double)p.n_kv * p.n_rows * head_dim * 4e-6 * splits / 4.0;
+  return (cost > longest ? cost : longest) + (splits > 1 ? pieces : 0.0);
+}
+
 template <typename T>
-static int launch_prefill(const PrefillParams& p, int head_dim, hipStream_t st) {
-  // Two query tiles per wavefront and 64-token key tiles keep the kernel within 256 registers
-  // (two waves per SIMD).  Staging a K/V tile (global loads, page lookups, LDS stores) costs a
-  // quarter of the kernel's time, so head_dim 128 runs eight waves per workgroup: one staged tile
-  // serves 256 query rows (8.9 -> 8.4 ms per layer at 32K x 32 heads); prompts of up to 128 rows
-  // keep four.  (Four query tiles per wavefront halve the LDS traffic per flop but need twice
-  // the registers: one wave per SIMD with every latency exposed, 2.5x slower.)  head_dim 256 has
-  // twice the accumulators and twice the LDS per token: one query tile per wavefront, 32-token
-  // key tiles.
-  const dim3 block(256);
-  if (head_dim == 128 && p.n_q > 128)
-    hipLaunchKernelGGL((prefill_attn_kernel<T, 128, 2, 64, 8>), dim3((p.n_q + 255) / 256, p.num_qo_heads),
-                       dim3(512), 0, st, p);
+static int launch_prefill(const PrefillParams& p, int head_dim, bool oct, hipStream_t st) {
+  const dim3 grid(p.n_tiles * p.n_kv * p.n_splits), block(head_dim == 256 ? 256 : 512);
+  if (head_dim == 128 && oct)
+    hipLaunchKernelGGL((prefill_attn_kernel<T, 128, true>), grid, block, 0, st, p);
   else if (head_dim == 128)
-    hipLaunchKernelGGL((prefill_attn_kernel<T, 128, 2, 64, 4>), dim3((p.n_q + 127) / 128, p.num_qo_heads),
-                       block, 0, st, p);
+    hipLaunchKernelGGL((prefill_attn_kernel<T, 128, false>), grid, block, 0, st, p);
+  else if (head_dim == 64 && oct)
+    hipLaunchKernelGGL((prefill_attn_kernel<T, 64, true>), grid, block, 0, st, p);
   else if (head_dim == 64)
-    hipLaunchKernelGGL((prefill_attn_kernel<T, 64, 2, 64, 4>), dim3((p.n_q + 127) / 128, p.num_qo_heads),
-                       block, 0, st, p);
+    hipLaunchKernelGGL((prefill_attn_kernel<T, 64, false>), grid, block, 0, st, p);
   else if (head_dim == 256)
-    hipLaunchKernelGGL((prefill_attn_kernel<T, 256, 1, 32, 4>), dim3((p.n_q + 63) / 64, p.num_qo_heads),
-                       block, 0, st, p);
+    hipLaunchKernelGGL((prefill_attn_staged_kernel<T, 256, 1, 32, 4>), grid, block, 0, st, p);
   else
     return fail(TD_ERR_UNSUPPORTED,
                 "BatchPrefillWithPagedKVCache failed to dispatch with head_dim %d (supported: 64, 128, 256)",
                 head_dim);
+  if (p.n_splits > 1) {
+    const int rows_per_block = 256 / (head_dim / 4);
+    const dim3 mgrid((unsigned)(((int64_t)p.n_kv * p.n_rows + rows_per_block - 1) / rows_per_block));
+    if (head_dim == 128)
+      hipLaunchKernelGGL((prefill_merge_kernel<T, 128>), mgrid, dim3(256), 0, st, p);
+    else if (head_dim == 64)
+      hipLaunchKernelGGL((prefill_merge_kernel<T, 64>), mgrid, dim3(256), 0, st, p);
+    else
+      hipLaunchKernelGGL((prefill_merge_kernel<T, 256>), mgrid, dim3(256), 0, st, p);
+  }
   return TD_OK;
 }
 
@@ -376,23 +945,84 @@ static int launch_prefill(const PrefillParams& p, int head_dim, hipStream_t st) 
 
 using namespace tidal;
 
-extern "C" int td_prefill_attn(const td_paged_kv* kv, const int32_t* page_table, int32_t n_pages,
-                               int32_t kv_len, const void* q, void* o, int32_t n_q,
-                               int32_t num_qo_heads, float sm_scale, int32_t causal, void* stream) {
-  TD_REQUIRE(kv && kv->data && page_table && q && o, "td_prefill_attn: NULL argument");
+static int check_prefill(const td_paged_kv* kv, int32_t n_pages, int32_t kv_len, int32_t n_q,
+                         int32_t num_qo_heads) {
   TD_REQUIRE(kv->page_size >= 1 && kv->num_kv_heads >= 1 && kv->max_pages >= 1,
              "td_prefill_attn: bad pool geometry");
   TD_REQUIRE(num_qo_heads >= kv->num_kv_heads && num_qo_heads % kv->num_kv_heads == 0,
              "td_prefill_attn: num_qo_heads %d is not a multiple of num_kv_heads %d", num_qo_heads,
              kv->num_kv_heads);
-  TD_REQUIRE(n_q >= 0 && kv_len >= n_q, "td_prefill_attn: n_q %d, kv_len %d", n_q, kv_len);
+  TD_REQUIRE(n_q >= 0 && kv_len >= n_q && kv_len < (1 << 30), "td_prefill_attn: n_q %d, kv_len %d", n_q,
+             kv_len);
   TD_REQUIRE((int64_t)n_pages * kv->page_size >= kv_len,
              "td_prefill_attn: %d pages of %d entries do not hold %d tokens", n_pages,
              kv->page_size, kv_len);
   TD_REQUIRE(kv->layout == TD_NHD || kv->layout == TD_HND, "td_prefill_attn: layout %d", kv->layout);
+  TD_REQUIRE((int64_t)n_q * (num_qo_heads / kv->num_kv_heads) < ((int64_t)1 << 30),
+             "td_prefill_attn: %d queries of %d heads", n_q, num_qo_heads);
+  return TD_OK;
+}
+
+// shape of the launch for a call that passed check_prefill
+static void plan_prefill(const td_paged_kv* kv, int32_t kv_len, int32_t n_q, int32_t num_qo_heads,
+                         int32_t causal, bool may_split, PrefillParams& p) {
+  const int H = kv->num_kv_heads, D = kv->head_dim;
+  p.n_kv = H;
+  p.q_per_kv = num_qo_heads / H;
+  p.n_rows = n_q * p.q_per_kv;
+  p.n_q = n_q;
+  p.causal = causal;
+  const int bn = D == 256 ? 32 : 64, max_tiles = (kv_len + bn - 1) / bn;
+  double best = 0.0;
+  PrefillParams c = p;
+  for (c.bm = D == 256 ? 64 : 256; c.bm >= 64; c.bm /= 2) {
+    c.n_tiles = (c.n_rows + c.bm - 1) / c.bm;
+    for (int s = 1; s <= 64; s = s < 8 ? s + 1 : (s < 16 ? s + 2 : s * 2)) {
+      const int chunk = (max_tiles + s - 1) / s;
+      if (s > 1 && (!may_split || chunk < 4 || (int64_t)c.n_tiles * H >= 8 * (int64_t)td_num_cus())) break;
+      const double cost = prefill_cost(c, D, kv_len, D == 256 || c.bm == 256 ? 1.0 : c.bm == 128 ? 0.87 : 0.83, s);
+      if (best == 0.0 || cost < best) {
+        best = cost;
+        p.bm = c.bm;
+        p.n_tiles = c.n_tiles;
+        p.chunk = chunk * bn;
+        p.n_splits = (kv_len + p.chunk - 1) / p.chunk;
+      }
+    }
+  }
+  // one head after the other on its XCD once there are enough tiles for the last head to end evenly
+  p.head_major = H % 8 == 0 && (int64_t)p.n_tiles * p.n_splits * H > 4 * (int64_t)td_num_cus();
+}
+
+static int64_t prefill_ws_bytes(const PrefillParams& p, int head_dim) {
+  return p.n_splits > 1 ? (int64_t)p.n_splits * p.n_kv * p.n_rows * (head_dim + 2) * 4 : 0;
+}
+
+extern "C" int64_t td_prefill_workspace_bytes(const td_paged_kv* kv, int32_t kv_len, int32_t n_q,
+                                              int32_t num_qo_heads, int32_t causal) {
+  if (!kv || n_q <= 0 || check_prefill(kv, kv->page_size >= 1 ? kv_len / kv->page_size + 1 : 0, kv_len, n_q,
+                                       num_qo_heads) != TD_OK)
+    return 0;  // the call itself reports what is wrong
+  PrefillParams p;
+  plan_prefill(kv, kv_len, n_q, num_qo_heads, causal, true, p);
+  return prefill_ws_bytes(p, kv->head_dim);
+}
+
+extern "C" int td_prefill_attn_split(const td_paged_kv* kv, const int32_t* page_table, int32_t n_pages,
+                                     int32_t kv_len, const void* q, void* o, int32_t n_q,
+                                     int32_t num_qo_heads, float sm_scale, int32_t causal,
+                                     void* workspace, int64_t workspace_bytes, void* stream) {
+  TD_REQUIRE(kv && kv->data && page_table && q && o, "td_prefill_attn: NULL argument");
+  const int crc = check_prefill(kv, n_pages, kv_len, n_q, num_qo_heads);
+  if (crc != TD_OK) return crc;
   if (n_q == 0) return TD_OK;
   const int P = kv->page_size, H = kv->num_kv_heads, D = kv->head_dim;
   PrefillParams p;
+  plan_prefill(kv, kv_len, n_q, num_qo_heads, causal, true, p);
+  if (workspace == nullptr || workspace_bytes < prefill_ws_bytes(p, D))
+    plan_prefill(kv, kv_len, n_q, num_qo_heads, causal, false, p);
+  p.part_o = reinterpret_cast<float*>(workspace);
+  p.part_ml = p.part_o ? p.part_o + (int64_t)p.n_splits * p.n_kv * p.n_rows * D : nullptr;
   p.kv = reinterpret_cast<const uint16_t*>(kv->data);
   p.page_stride = (int64_t)2 * P * H * D;
   p.v_offset = (int64_t)P * H * D;
@@ -400,27 +1030,37 @@ extern "C" int td_prefill_attn(const td_paged_kv* kv, const int32_t* page_table,
   p.head_stride = kv->layout == TD_NHD ? D : P * D;
   p.page_size = P;
   p.page_shift = (P & (P - 1)) == 0 ? __builtin_ctz(P) : -1;
+  p.entry_stride_b = (uint32_t)(p.entry_stride * 2);
+  const bool oct = P % 8 == 0;
+  // round-up division by a constant: magic = ceil(2^(31 + down) / P), down = ceil(log2 P)
+  p.page_down = 0;
+  while (((int64_t)1 << p.page_down) < P) ++p.page_down;
+  p.page_magic = (uint32_t)((((uint64_t)1 << (31 + p.page_down)) + (uint64_t)P - 1) / (uint64_t)P);
   p.max_page = (uint32_t)(kv->max_pages - 1);
   p.page_table = page_table;
   p.n_pages = n_pages;
   p.kv_len = kv_len;
   p.q = reinterpret_cast<const uint16_t*>(q);
   p.o = reinterpret_cast<uint16_t*>(o);
-  p.n_q = n_q;
   p.num_qo_heads = num_qo_heads;
-  p.q_per_kv = num_qo_heads / H;
   p.scale_log2 = sm_scale * 1.4426950408889634f;
-  p.causal = causal;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   int rc;
   if (kv->dtype == TD_F16)
-    rc = launch_prefill<F16>(p, D, st);
+    rc = launch_prefill<F16>(p, D, oct, st);
   else if (kv->dtype == TD_BF16)
-    rc = launch_prefill<BF16>(p, D, st);
+    rc = launch_prefill<BF16>(p, D, oct, st);
   else
     return fail(TD_ERR_UNSUPPORTED, "BatchPrefillWithPagedKVCache failed to dispatch with dtype %d",
                 kv->dtype);
   if (rc != TD_OK) return rc;
   TD_HIP_CHECK(hipGetLastError());
   return TD_OK;
+}
+
+extern "C" int td_prefill_attn(const td_paged_kv* kv, const int32_t* page_table, int32_t n_pages,
+                               int32_t kv_len, const void* q, void* o, int32_t n_q,
+                               int32_t num_qo_heads, float sm_scale, int32_t causal, void* stream) {
+  return td_prefill_attn_split(kv, page_table, n_pages, kv_len, q, o, n_q, num_qo_heads, sm_scale, causal,
+                               nullptr, 0, stream);
 }

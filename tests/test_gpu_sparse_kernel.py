@@ -469,3 +469,32 @@ def test_pages_of_any_size(cuda, dtype, page, hq, hkv, rows):
     assert torch.equal(pool_f[page_f, 1, entry_f].cpu(), v_new[0].to(dtype))
     pool_f[page_f, :, entry_f] = pool[page_f, :, entry_f]
     assert torch.equal(pool_f, pool)
+
+
+@pytest.mark.parametrize("k", [1, 31, 48, 130])
+@pytest.mark.parametrize("hq,hkv,rows,page", [(8, 8, 8, 16), (8, 2, 2, 16), (8, 8, 8, 6)])
+def test_slots_outside_the_list_are_never_used(cuda, k, hq, hkv, rows, page):
+    """The last tile of a list is rarely full; what the rest of the pool holds (here NaN) must not reach
+    the result through the lanes without a token."""
+    from oracle import tidal_oracle as orc
+    from tidaldecode_amd import _kernels
+
+    d, dtype, n_pages = 128, torch.float16, 64
+    g = torch.Generator().manual_seed(k)
+    pool = torch.full((n_pages, 2, page, hkv, d), float("nan"), dtype=dtype)
+    flat_k, flat_v = torch.randn((2, n_pages * page, hkv, d), generator=g).to(dtype)
+    slots = torch.stack([torch.randperm(n_pages * page - 1, generator=g)[:k] + 1 for _ in range(rows)]).int()
+    used = slots.long().unique()
+    pool[used // page, 0, used % page] = flat_k[used]
+    pool[used // page, 1, used % page] = flat_v[used]
+    q = torch.randn((1, hq, d), generator=g).to(dtype)
+    w = _kernels.BatchDecodeWithPagedKVCachePyTorchWrapper(0)
+    w.begin_forward(None, hq, hkv, d, page, torch.empty(0, dtype=dtype))
+    o = torch.empty((1, hq, d), dtype=dtype, device=cuda)
+    w.forward(q.to(cuda), o, pool.to(cuda), slots.to(cuda), None, 0, 0, None, index_kind="slots")
+    assert _kernels.last_decode_kernel().startswith("short-list")
+    for h in range(hq):
+        s, kvh = slots[h * rows // hq].long(), h * hkv // hq
+        logits = orc.attn_logits(q[0, h: h + 1].float(), flat_k[s, kvh: kvh + 1].float())
+        want = orc.softmax_pv(logits, flat_v[s, kvh: kvh + 1].float())
+        assert (o[0, h].float().cpu() - want.view(-1)).abs().max().item() <= 2e-3

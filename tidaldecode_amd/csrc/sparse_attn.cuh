@@ -408,7 +408,10 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(1, U ==
       for (int u = 0; u < U; ++u)
         vb[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(ka[u] + p.v_offset * 2));
     } else {
-      off_own = valid ? off_own : (uint32_t)__builtin_amdgcn_readfirstlane((int)off_own);
+      // in a statement of its own: inside the conditional the first lane would be the first one
+      // WITHOUT a token
+      const uint32_t off_first = (uint32_t)__builtin_amdgcn_readfirstlane((int)off_own);
+      off_own = valid ? off_own : off_first;
       uint32_t offs[U];
 #define TD_ROW_OFF(N) \
   if constexpr (N < U) offs[N] = row_bcast_u32<N>(off_own) + head_byte_off;

@@ -416,6 +416,23 @@ int td_rms_norm(const void* x, const void* weight, void* out, int32_t rows, int3
                 float eps, int32_t dtype, void* stream);
 
 /*
+ * The passes around a layer's matrix products over a prompt.  td_add_rms_norm: x += delta (rounded to
+ * the storage type, x updated in place), out = RMSNorm(x) * weight.  td_silu_mul: gate_up holds
+ * [gate | up] per row, out[r, :] = silu(gate[r, :]) * up[r, :] for cols columns.
+ * td_rope_append_prompt: the rows of qkv hold a token's query heads, key heads and value heads; rotated
+ * queries go to q_out [n, num_qo_heads, head_dim], rotated keys and the values to the cache slots of
+ * the sequence's newest n_tokens positions (page list as in td_append_kv).  No metadata is kept.
+ */
+int td_add_rms_norm(void* x, const void* delta, const void* weight, void* out, int32_t rows,
+                    int32_t cols, float eps, int32_t dtype, void* stream);
+int td_silu_mul(const void* gate_up, void* out, int32_t rows, int32_t cols, int32_t dtype,
+                void* stream);
+int td_rope_append_prompt(const td_paged_kv* kv, const void* qkv, int64_t qkv_stride, void* q_out,
+                          int32_t n_tokens, int32_t num_qo_heads, int64_t past_kv_len,
+                          const int32_t* kv_indices, const int32_t* kv_indptr, int32_t last_page_len,
+                          float rope_scale, float rope_theta, void* stream);
+
+/*
  * Measurement aid without a counterpart in the reference: the memory side of a sparse layer
  * alone.  Same grid and the same list -> slot -> K / V row loads as td_decode_attn for
  * token-slot lists (the launch that replaces BatchDecodeWithPagedKVCacheKernel,

@@ -420,3 +420,73 @@ def test_page_score_estimator_reference_grid(cuda, head_dim, page_size):
         want = orc.page_score_bound(q[0].float(), kf, page_size)[:, :n_out]
         tol = 2.0 ** -10 * want.abs().clamp(min=1.0) + 1e-3
         assert ((o[:, :n_out].float().cpu() - want).abs() <= tol).all(), (n, page_size, head_dim)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("d,hq,hkv,n,shift", [
+    (128, 5, 1, 3, 0), (64, 3, 2, 2 * 8192 + 5, 0), (128, 1, 1, 8192 + 3, 0), (256, 17, 2, 4096 + 1, 0),
+    (64, 70, 1, 2, 0), (128, 5, 3, 7, 1)])
+def test_rope_workgroup_edges(cuda, dtype, d, hq, hkv, n, shift):
+    """Rows that end inside a pass, several tokens per workgroup with a remainder, unaligned rows."""
+    from oracle import tidal_oracle as orc
+    from tidaldecode_amd import _kernels
+
+    def odd(x):  # the same values, `shift` elements off alignment
+        buf = torch.zeros(x.numel() + 8, dtype=dtype, device=cuda)
+        view = buf[shift: shift + x.numel()].view(x.shape)
+        return view.copy_(x)
+
+    q, k = randn((n, hq, d), 1, dtype), randn((n, hkv, d), 2, dtype)
+    qd, kd = odd(q), odd(k)
+    _kernels.apply_rope_in_place(qd, kd, 1000, 1.0, 1e4)
+    pos = np.arange(1000, 1000 + n)
+    for got, x in ((qd, q), (kd, k)):
+        want = torch.from_numpy(orc.rope_closed_form(x.numpy(), pos, 1e4, 1.0))
+        assert ((got.double().cpu() - want).abs() <= _rope_tol(want, dtype)).all()
+
+
+@pytest.mark.parametrize("layout", [0, 1])
+@pytest.mark.parametrize("d,hq,hkv,page,past,n", [
+    (128, 32, 8, 16, 0, 33), (64, 5, 1, 7, 20, 1), (256, 3, 3, 1, 5, 9), (128, 2, 1, 16, 11, 8192 + 5)])
+def test_rope_append_prompt_equals_the_separate_calls(cuda, layout, d, hq, hkv, page, past, n):
+    from tidaldecode_amd import _kernels
+
+    dtype, total = torch.bfloat16, past + n
+    n_pages = (total + page - 1) // page
+    table = torch.randperm(n_pages + 2, generator=torch.Generator().manual_seed(n))[:n_pages].int().to(cuda)
+    indptr = torch.tensor([0, n_pages], dtype=torch.int32, device=cuda)
+    shape = (n_pages + 2, 2, page, hkv, d) if layout == _kernels.TD_NHD else (n_pages + 2, 2, hkv, page, d)
+    pool = randn(shape, 3, dtype).to(dtype).to(cuda)
+    want_pool = pool.clone()
+    qkv = randn((n, (hq + 2 * hkv) * d), 4, dtype).to(dtype).to(cuda)
+    before, last = qkv.clone(), (total - 1) % page + 1
+    q, k, v = (t.reshape(n, -1, d).clone() for t in qkv.split([hq * d, hkv * d, hkv * d], dim=1))
+    _kernels.apply_rope_in_place(q, k, past, 1.0, 1e4)
+    _kernels.append_kv_cache_prefill(k, v, want_pool, table, indptr, last, int(table[-1]), None, None, None, 0, 0,
+                                     layout)
+    got = _kernels.rope_append_prompt(qkv, hq, past, pool, table, indptr, last, layout)
+    assert torch.equal(got, q) and torch.equal(pool, want_pool) and torch.equal(qkv, before)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rows,cols", [(1, 1), (3, 7), (5, 8), (2, 2056), (300, 4096), (3, 11008), (2, 20000)])
+def test_add_rms_norm_and_silu_mul(cuda, dtype, rows, cols):
+    from tidaldecode_amd import _kernels
+
+    x, delta, w = (randn(s, i, dtype).to(dtype).to(cuda) for i, s in
+                   enumerate(((rows, cols), (rows, cols), (cols,))))
+    want_x = x + delta
+    f = want_x.double()
+    want = f * torch.rsqrt(f.pow(2).mean(-1, keepdim=True) + 1e-5) * w.double()
+    got = _kernels.add_rms_norm(x, delta, w, 1e-5)
+    assert torch.equal(x, want_x)
+    ulp = 2.0 ** -10 if dtype == torch.float16 else 2.0 ** -7   # one rounding is half of it
+    tiny = 2.0 ** -24 if dtype == torch.float16 else 1e-30      # spacing of the smallest fp16 values
+    assert ((got.double() - want).abs() <= want.abs() * ulp * 0.51 + tiny).all()
+
+    gu = (4 * randn((rows, 2 * cols), 9, dtype)).to(dtype).to(cuda)
+    gu[0, 0] = -1e4                                             # exp overflows: silu is -0
+    gate, up = gu[:, :cols].double(), gu[:, cols:].double()
+    want = gate / (1 + (-gate).exp()) * up
+    got = _kernels.silu_mul(gu)                                 # two roundings
+    assert ((got.double() - want).abs() <= want.abs() * ulp * 1.02 + up.abs() * tiny + tiny).all()

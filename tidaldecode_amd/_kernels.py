@@ -115,6 +115,55 @@ def rms_norm_forward(input: torch.Tensor, weight: torch.Tensor, output: torch.Te
                           _dtype_code(input.dtype, "rms_norm_forward"), _stream()))
 
 
+def add_rms_norm(x: torch.Tensor, delta: torch.Tensor, weight: torch.Tensor, epsilon: float) -> torch.Tensor:
+    """Extension: ``x += delta`` in place, returns ``RMSNorm(x) * weight``; ``[..., C]``, one launch."""
+    for t, n in ((x, "x"), (delta, "delta"), (weight, "weight")):
+        _check_input(t, n)
+    cols = x.size(-1)
+    if weight.numel() != cols or delta.shape != x.shape or not (x.dtype == delta.dtype == weight.dtype):
+        raise RuntimeError("add_rms_norm: shape or dtype mismatch")
+    out = torch.empty_like(x)
+    check(lib.td_add_rms_norm(x.data_ptr(), delta.data_ptr(), weight.data_ptr(), out.data_ptr(),
+                              x.numel() // cols, cols, float(epsilon), _dtype_code(x.dtype, "add_rms_norm"),
+                              _stream()))
+    return out
+
+
+def silu_mul(gate_up: torch.Tensor) -> torch.Tensor:
+    """Extension: ``silu(gate) * up`` of rows ``[gate | up]``, ``[..., 2 I]`` -> ``[..., I]``."""
+    _check_input(gate_up, "gate_up")
+    cols = gate_up.size(-1) // 2
+    if gate_up.size(-1) != 2 * cols or cols == 0:
+        raise RuntimeError("silu_mul: the last dimension must be even")
+    out = torch.empty((*gate_up.shape[:-1], cols), dtype=gate_up.dtype, device=gate_up.device)
+    check(lib.td_silu_mul(gate_up.data_ptr(), out.data_ptr(), out.numel() // cols, cols,
+                          _dtype_code(gate_up.dtype, "silu_mul"), _stream()))
+    return out
+
+
+def rope_append_prompt(qkv: torch.Tensor, num_qo_heads: int, past_kv_len: int, kv_data: torch.Tensor,
+                       kv_indices: torch.Tensor, kv_indptr: torch.Tensor, kv_last_page_len: int, layout: int,
+                       rope_scale: float = 1.0, rope_theta: float = 1e4) -> torch.Tensor:
+    """Extension: ``apply_rope_in_place`` + ``append_kv_cache_prefill`` in one launch on the stacked
+    projection.  ``qkv [N, (H_q + 2 H_kv) D]`` is read only; rotated k and v go to the sequence's newest
+    N positions, rotated q ``[N, H_q, D]`` is returned."""
+    _check_input(qkv, "qkv")
+    _check_dim(2, qkv, "qkv")
+    _check_input(kv_indices, "kv_indices")
+    _check_dim(1, kv_indices, "kv_indices")
+    _check_i32(kv_indices, "kv_indices")
+    _check_i32(kv_indptr, "kv_indptr")
+    pool = _pool(kv_data, int(layout))
+    n, d = qkv.size(0), pool.head_dim
+    if qkv.size(1) != (num_qo_heads + 2 * pool.num_kv_heads) * d or qkv.dtype != kv_data.dtype:
+        raise RuntimeError("rope_append_prompt: qkv does not match kv_data in heads, head_dim or dtype")
+    q = torch.empty((n, num_qo_heads, d), dtype=qkv.dtype, device=qkv.device)
+    check(lib.td_rope_append_prompt(pool, qkv.data_ptr(), qkv.stride(0), q.data_ptr(), n, num_qo_heads,
+                                    int(past_kv_len), kv_indices.data_ptr(), kv_indptr.data_ptr(),
+                                    int(kv_last_page_len), float(rope_scale), float(rope_theta), _stream()))
+    return q
+
+
 def gemv(weight: torch.Tensor, x: torch.Tensor, *, norm_weight: Optional[torch.Tensor] = None,
          eps: float = 1e-5, gated: bool = False, residual: Optional[torch.Tensor] = None,
          pair_gated: bool = False, out: Optional[torch.Tensor] = None) -> torch.Tensor:

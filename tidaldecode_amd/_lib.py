@@ -180,6 +180,16 @@ SIGNATURES = {
         c_int32,
         [c_void_p, c_void_p, c_void_p, c_int32, c_int32, c_float, c_int32, c_void_p],
     ),
+    "td_add_rms_norm": (
+        c_int32,
+        [c_void_p, c_void_p, c_void_p, c_void_p, c_int32, c_int32, c_float, c_int32, c_void_p],
+    ),
+    "td_silu_mul": (c_int32, [c_void_p, c_void_p, c_int32, c_int32, c_int32, c_void_p]),
+    "td_rope_append_prompt": (
+        c_int32,
+        [POINTER(PagedKV), c_void_p, c_int64, c_void_p, c_int32, c_int32, c_int64, c_void_p, c_void_p, c_int32,
+         c_float, c_float, c_void_p],
+    ),
 }
 
 

@@ -57,15 +57,139 @@ __device__ __forceinline__ void rope_sincos(double pos_over_scale, double log2_t
   sincospif((float)(2.0 * turns), &sn, &cs);
 }
 
-template <typename T>
-__device__ __forceinline__ void rotate_pair(uint16_t* row, int j, int half, float sn, float cs) {
-  const float lo = to_float<T>(row[j]);
-  const float hi = to_float<T>(row[j + half]);
-  row[j] = from_float<T>(lo * cs - hi * sn);
-  row[j + half] = from_float<T>(hi * cs + lo * sn);
+// one pair turned; every kernel rounds the same two products, so their results agree bit by bit
+__device__ __forceinline__ void turn(float lo, float hi, float sn, float cs, float& out_lo, float& out_hi) {
+  out_lo = fmaf(lo, cs, -(hi * sn));
+  out_hi = fmaf(lo, sn, hi * cs);
 }
 
-// grid: n_tokens; block: 256 threads = (D/2 pair columns) x (512/D head slots)
+template <typename T>
+__device__ __forceinline__ void rotate_pair(uint16_t* row, int j, int half, float sn, float cs) {
+  float lo, hi;
+  turn(to_float<T>(row[j]), to_float<T>(row[j + half]), sn, cs, lo, hi);
+  row[j] = from_float<T>(lo);
+  row[j + half] = from_float<T>(hi);
+}
+
+// RoPE of a prompt, and with APPEND the cache append in the same pass over the projections.
+// Bound by memory for long prompts and by latency for short ones: a lane holds eight pairs of a head
+// row (two 16-byte accesses), so a workgroup covers 512 / (D / 8) rows at a time and has the next rows
+// in flight while it turns the present ones; the angles, which need double precision, are formed once
+// per token and shared through LDS.  TOK tokens per workgroup: as many as 256 threads form angles for
+// at once when the tokens fill the chip anyway, one otherwise.
+struct RopePrompt {
+  const uint16_t *q, *k, *v;  // token rows, heads adjacent; v with APPEND only
+  int64_t q_stride, k_stride, v_stride;
+  uint16_t *q_out, *k_out;    // [n, H, D]; k_out without APPEND only.  q_out == q and k_out == k: in place
+  int32_t n_tokens, Hq, Hkv;
+  double past_len, inv_scale, log2_theta;
+  const int32_t *indices, *indptr;  // APPEND: the sequence's pages, as append_copy_kernel takes them
+  int32_t last_page_len;
+};
+
+template <typename T, int D, bool APPEND, int TOK>
+__global__ __launch_bounds__(256) void rope_prompt_kernel(PoolGeom g, RopePrompt p) {
+  constexpr int kHalf = D / 2, kLanes = kHalf / 8, kRows = 256 / kLanes;
+  __shared__ __attribute__((aligned(16))) float sm_cos[TOK][kHalf], sm_sin[TOK][kHalf];
+  const int tid = threadIdx.x, c = (tid % kLanes) * 8, slot = tid / kLanes;
+  const int tok0 = blockIdx.x * TOK;
+  const int turned = p.Hq + p.Hkv, rows = APPEND ? turned + p.Hkv : turned;
+  auto source = [&](int tok, int h) {
+    if (h < p.Hq) return p.q + (int64_t)tok * p.q_stride + (int64_t)h * D;
+    if (!APPEND || h < turned) return p.k + (int64_t)tok * p.k_stride + (int64_t)(h - p.Hq) * D;
+    return p.v + (int64_t)tok * p.v_stride + (int64_t)(h - turned) * D;
+  };
+  u32x4 lo, hi;  // the next row's halves: asked for before the row in hand is stored
+  auto load = [&](int tok, int h) {
+    const uint16_t* row = source(tok, h) + c;
+    lo = *reinterpret_cast<const u32x4*>(row);
+    hi = *reinterpret_cast<const u32x4*>(row + kHalf);
+  };
+  if (slot < rows) load(tok0, slot);
+  if (TOK > 1 || tid < kHalf) {  // TOK * kHalf is 256 where TOK > 1
+    const int t = tid / kHalf, j = tid % kHalf;
+    rope_sincos((p.past_len + (double)(tok0 + t)) * p.inv_scale, p.log2_theta, j, D, sm_sin[t][j], sm_cos[t][j]);
+  }
+  __syncthreads();
+#pragma unroll 1
+  for (int t = 0; t < TOK; ++t) {
+    const int tok = tok0 + t;
+    if (tok >= p.n_tokens) return;
+    uint16_t* kdst = nullptr;  // APPEND: the token's slot in the pool, head 0
+    if constexpr (APPEND) {
+      const int n_pages = p.indptr[1] - p.indptr[0];
+      const int pos = (n_pages - 1) * g.page_size + p.last_page_len - p.n_tokens + tok;
+      if (pos >= 0 && n_pages > 0) {
+        const int pg = pos / g.page_size;
+        kdst = reinterpret_cast<uint16_t*>(g.data) +
+               k_offset(g, (uint32_t)p.indices[p.indptr[0] + pg], pos - pg * g.page_size, 0);
+      }
+    }
+    float cs[8], sn[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      cs[i] = sm_cos[t][c + i];
+      sn[i] = sm_sin[t][c + i];
+    }
+    for (int h = slot; h < rows; h += kRows) {
+      uint32_t a[4] = {lo.x, lo.y, lo.z, lo.w}, b[4] = {hi.x, hi.y, hi.z, hi.w};
+      if (h + kRows < rows)
+        load(tok, h + kRows);
+      else if (t + 1 < TOK && tok + 1 < p.n_tokens)
+        load(tok + 1, slot);
+      if (!APPEND || h < turned) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          float l0, l1, h0, h1;
+          unpack2<T>(a[i], l0, l1);
+          unpack2<T>(b[i], h0, h1);
+          turn(l0, h0, sn[2 * i], cs[2 * i], l0, h0);
+          turn(l1, h1, sn[2 * i + 1], cs[2 * i + 1], l1, h1);
+          a[i] = pack2<T>(l0, l1);
+          b[i] = pack2<T>(h0, h1);
+        }
+      }
+      uint16_t* dst;
+      if (h < p.Hq)
+        dst = p.q_out + ((int64_t)tok * p.Hq + h) * D;
+      else if constexpr (!APPEND)
+        dst = p.k_out + ((int64_t)tok * p.Hkv + (h - p.Hq)) * D;
+      else if (kdst == nullptr)
+        continue;
+      else
+        dst = h < turned ? kdst + (int64_t)(h - p.Hq) * g.head_stride
+                         : kdst + g.v_offset + (int64_t)(h - turned) * g.head_stride;
+      *reinterpret_cast<u32x4*>(dst + c) = u32x4{a[0], a[1], a[2], a[3]};
+      *reinterpret_cast<u32x4*>(dst + c + kHalf) = u32x4{b[0], b[1], b[2], b[3]};
+    }
+  }
+}
+
+template <typename T, int D, bool APPEND>
+static void launch_rope_prompt(const PoolGeom& g, const RopePrompt& p, hipStream_t st) {
+  constexpr int TOK = 512 / D;
+  // below eight workgroups per compute unit tokens are better spread out
+  if (p.n_tokens >= TOK * 2048)
+    hipLaunchKernelGGL((rope_prompt_kernel<T, D, APPEND, TOK>), dim3((p.n_tokens + TOK - 1) / TOK), dim3(256), 0,
+                       st, g, p);
+  else
+    hipLaunchKernelGGL((rope_prompt_kernel<T, D, APPEND, 1>), dim3(p.n_tokens), dim3(256), 0, st, g, p);
+}
+
+template <bool APPEND>
+static void launch_rope_prompt(const PoolGeom& g, const RopePrompt& p, int D, int32_t dtype, hipStream_t st) {
+#define TD_ROPE(T)                                                \
+  {                                                               \
+    if (D == 64) launch_rope_prompt<T, 64, APPEND>(g, p, st);     \
+    else if (D == 128) launch_rope_prompt<T, 128, APPEND>(g, p, st); \
+    else launch_rope_prompt<T, 256, APPEND>(g, p, st);            \
+  }
+  if (dtype == TD_F16) TD_ROPE(F16) else TD_ROPE(BF16)
+#undef TD_ROPE
+}
+
+// Rows that are not 16-byte aligned.  grid: n_tokens; block: 256 threads = (D/2 pair columns) x
+// (512/D head slots)
 template <typename T>
 __global__ __launch_bounds__(256) void rope_kernel(uint16_t* q, uint16_t* k, int n_tokens, int Hq,
                                                    int Hkv, int D, double past_len,
@@ -121,10 +245,10 @@ __global__ __launch_bounds__(256) void rope_append_decode_kernel(
       const uint16_t* krow = k + ((int64_t)b * Hkv + hk) * D;
       const uint16_t* vrow = v + ((int64_t)b * Hkv + hk) * D;
       uint16_t* kdst = pool + k_offset(g, page, entry, hk);
-      const float lo = to_float<T>(krow[j]);
-      const float hi = to_float<T>(krow[j + half]);
-      kdst[j] = from_float<T>(lo * cs - hi * sn);
-      kdst[j + half] = from_float<T>(hi * cs + lo * sn);
+      float lo, hi;
+      turn(to_float<T>(krow[j]), to_float<T>(krow[j + half]), sn, cs, lo, hi);
+      kdst[j] = from_float<T>(lo);
+      kdst[j + half] = from_float<T>(hi);
       kdst[g.v_offset + j] = vrow[j];
       kdst[g.v_offset + j + half] = vrow[j + half];
     }
@@ -247,15 +371,18 @@ __device__ __forceinline__ float rms_block_sum(float ss) {
 // 16-byte loads per thread issued back to back, and stays in registers between the two passes.
 // Threads past the end of the row reload the row's last chunk (an unconditional load keeps all
 // loads in flight together; a predicated one is waited for inside its branch) and drop it.
-template <typename T, int CH>
-__global__ __launch_bounds__(256) void rms_norm_vec_kernel(const uint16_t* x, const uint16_t* w,
+// ADD: x + delta, rounded to the storage type, goes back to x and is what the norm is taken of; the
+// residual addition of a layer so costs no pass of its own.
+template <typename T, int CH, bool ADD>
+__global__ __launch_bounds__(256) void rms_norm_vec_kernel(uint16_t* x, const uint16_t* delta, const uint16_t* w,
                                                            uint16_t* out, int cols, float eps) {
   const int64_t base = (int64_t)blockIdx.x * cols;
-  uint4 xv[CH], wv[CH];
+  uint4 xv[CH], wv[CH], dv[ADD ? CH : 1];
 #pragma unroll
   for (int i = 0; i < CH; ++i) {
     const int c = min((i * 256 + (int)threadIdx.x) * 8, cols - 8);
     xv[i] = *reinterpret_cast<const uint4*>(x + base + c);
+    if constexpr (ADD) dv[i] = *reinterpret_cast<const uint4*>(delta + base + c);
   }
 #pragma unroll
   for (int i = 0; i < CH; ++i) {
@@ -266,7 +393,20 @@ __global__ __launch_bounds__(256) void rms_norm_vec_kernel(const uint16_t* x, co
   float ss = 0.f;
 #pragma unroll
   for (int i = 0; i < CH; ++i) {
-    const uint32_t xw[4] = {xv[i].x, xv[i].y, xv[i].z, xv[i].w};
+    uint32_t xw[4] = {xv[i].x, xv[i].y, xv[i].z, xv[i].w};
+    if constexpr (ADD) {
+      const uint32_t dw[4] = {dv[i].x, dv[i].y, dv[i].z, dv[i].w};
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        float x0, x1, d0, d1;
+        unpack2<T>(xw[j], x0, x1);
+        unpack2<T>(dw[j], d0, d1);
+        xw[j] = pack2<T>(x0 + d0, x1 + d1);
+      }
+      // a thread past the row's end loaded its last chunk, perhaps after the sum went there: it drops it
+      const int c = (i * 256 + (int)threadIdx.x) * 8;
+      if (c < cols) *reinterpret_cast<uint4*>(x + base + c) = make_uint4(xw[0], xw[1], xw[2], xw[3]);
+    }
 #pragma unroll
     for (int j = 0; j < 4; ++j) unpack2<T>(xw[j], xf[i][2 * j], xf[i][2 * j + 1]);
     if ((i * 256 + (int)threadIdx.x) * 8 < cols) {
@@ -293,40 +433,81 @@ __global__ __launch_bounds__(256) void rms_norm_vec_kernel(const uint16_t* x, co
 }
 
 // Any other row length or alignment: two passes of 2-byte accesses.
-template <typename T>
-__global__ __launch_bounds__(256) void rms_norm_kernel(const uint16_t* x, const uint16_t* w,
+template <typename T, bool ADD>
+__global__ __launch_bounds__(256) void rms_norm_kernel(uint16_t* x, const uint16_t* delta, const uint16_t* w,
                                                        uint16_t* out, int cols, float eps) {
-  const int row = blockIdx.x;
-  const uint16_t* xr = x + (int64_t)row * cols;
-  uint16_t* orow = out + (int64_t)row * cols;
+  const int64_t base = (int64_t)blockIdx.x * cols;
+  uint16_t* xr = x + base;
   float ss = 0.f;
 #pragma unroll 4
   for (int c = threadIdx.x; c < cols; c += 256) {
+    if constexpr (ADD) xr[c] = from_float<T>(to_float<T>(xr[c]) + to_float<T>(delta[base + c]));
     const float f = to_float<T>(xr[c]);
     ss = fmaf(f, f, ss);
   }
   const float inv = rsqrtf(rms_block_sum(ss) / (float)cols + eps);
 #pragma unroll 4
   for (int c = threadIdx.x; c < cols; c += 256)
-    orow[c] = from_float<T>(to_float<T>(xr[c]) * inv * to_float<T>(w[c]));
+    out[base + c] = from_float<T>(to_float<T>(xr[c]) * inv * to_float<T>(w[c]));
 }
 
-template <typename T>
-static void launch_rms_norm(const void* x, const void* weight, void* out, int rows, int cols,
+template <typename T, bool ADD>
+static void launch_rms_norm(void* x, const void* delta, const void* weight, void* out, int rows, int cols,
                             float eps, hipStream_t st) {
-  const uint16_t* xp = (const uint16_t*)x;
+  uint16_t* xp = (uint16_t*)x;
+  const uint16_t* dp = (const uint16_t*)delta;
   const uint16_t* wp = (const uint16_t*)weight;
   uint16_t* op = (uint16_t*)out;
   const bool vec = cols % 8 == 0 && cols <= 8 * 2048 &&
-                   (((uintptr_t)x | (uintptr_t)weight | (uintptr_t)out) & 15) == 0;
-#define TD_RMS(CH) \
-  hipLaunchKernelGGL((rms_norm_vec_kernel<T, CH>), dim3(rows), dim3(256), 0, st, xp, wp, op, cols, eps)
-  if (!vec) hipLaunchKernelGGL(rms_norm_kernel<T>, dim3(rows), dim3(256), 0, st, xp, wp, op, cols, eps);
-  else if (cols <= 2048) TD_RMS(1);
-  else if (cols <= 2 * 2048) TD_RMS(2);
-  else if (cols <= 4 * 2048) TD_RMS(4);
-  else TD_RMS(8);
+                   (((uintptr_t)x | (uintptr_t)delta | (uintptr_t)weight | (uintptr_t)out) & 15) == 0;
+#define TD_RMS(K) hipLaunchKernelGGL((K), dim3(rows), dim3(256), 0, st, xp, dp, wp, op, cols, eps)
+  if (!vec) TD_RMS((rms_norm_kernel<T, ADD>));
+  else if (cols <= 2048) TD_RMS((rms_norm_vec_kernel<T, 1, ADD>));
+  else if (cols <= 2 * 2048) TD_RMS((rms_norm_vec_kernel<T, 2, ADD>));
+  else if (cols <= 4 * 2048) TD_RMS((rms_norm_vec_kernel<T, 4, ADD>));
+  else TD_RMS((rms_norm_vec_kernel<T, 8, ADD>));
 #undef TD_RMS
+}
+
+// The gated MLP's activation over a prompt: out = silu(gate) * up, silu rounded to the storage type
+// first as the model does it.  Bound by memory: [gate | up] is read once and the product written once,
+// where element-wise operators write silu(gate) and read it again.  VEC: eight elements per thread.
+template <typename T, bool VEC>
+__global__ __launch_bounds__(256) void silu_mul_kernel(const uint16_t* gate_up, uint16_t* out, int cols) {
+  const uint16_t* gate = gate_up + (int64_t)blockIdx.x * 2 * cols;
+  uint16_t* o = out + (int64_t)blockIdx.x * cols;
+  const int c = ((int)blockIdx.y * 256 + (int)threadIdx.x) * (VEC ? 8 : 1);
+  if (c >= cols) return;
+  auto silu = [](float x) { return x / (1.f + expf(-x)); };
+  if constexpr (VEC) {
+    const u32x4 gv = *reinterpret_cast<const u32x4*>(gate + c);
+    const u32x4 uv = *reinterpret_cast<const u32x4*>(gate + cols + c);
+    const uint32_t gw[4] = {gv.x, gv.y, gv.z, gv.w}, uw[4] = {uv.x, uv.y, uv.z, uv.w};
+    uint32_t ow[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      float g0, g1, u0, u1;
+      unpack2<T>(gw[i], g0, g1);
+      unpack2<T>(uw[i], u0, u1);
+      unpack2<T>(pack2<T>(silu(g0), silu(g1)), g0, g1);
+      ow[i] = pack2<T>(g0 * u0, g1 * u1);
+    }
+    *reinterpret_cast<u32x4*>(o + c) = u32x4{ow[0], ow[1], ow[2], ow[3]};
+  } else {
+    const float s = to_float<T>(from_float<T>(silu(to_float<T>(gate[c]))));
+    o[c] = from_float<T>(s * to_float<T>(gate[cols + c]));
+  }
+}
+
+template <typename T>
+static void launch_silu_mul(const void* gate_up, void* out, int rows, int cols, hipStream_t st) {
+  const uint16_t* g = (const uint16_t*)gate_up;
+  if (cols % 8 == 0 && (((uintptr_t)gate_up | (uintptr_t)out) & 15) == 0)
+    hipLaunchKernelGGL((silu_mul_kernel<T, true>), dim3(rows, (cols / 8 + 255) / 256), dim3(256), 0, st, g,
+                       (uint16_t*)out, cols);
+  else
+    hipLaunchKernelGGL((silu_mul_kernel<T, false>), dim3(rows, (cols + 255) / 256), dim3(256), 0, st, g,
+                       (uint16_t*)out, cols);
 }
 
 static int check_pool(const td_paged_kv* kv, const char* who) {
@@ -358,18 +539,30 @@ extern "C" int td_rope_in_place(void* q, void* k, int32_t n_tokens, int32_t num_
   TD_REQUIRE(past_kv_len >= 0, "apply_rope_in_place: past_kv_len %lld", (long long)past_kv_len);
   if (n_tokens == 0) return TD_OK;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  if (dtype != TD_F16 && dtype != TD_BF16)
+    return fail(TD_ERR_UNSUPPORTED, "apply_rope_in_place failed to dispatch with dtype %d", dtype);
   const double inv_scale = 1.0 / (double)rope_scale;
   const double log2_theta = log2((double)rope_theta);
-  if (dtype == TD_F16)
-    hipLaunchKernelGGL(rope_kernel<F16>, dim3(n_tokens), dim3(256), 0, st, (uint16_t*)q,
-                       (uint16_t*)k, n_tokens, num_qo_heads, num_kv_heads, head_dim,
-                       (double)past_kv_len, inv_scale, log2_theta);
-  else if (dtype == TD_BF16)
-    hipLaunchKernelGGL(rope_kernel<BF16>, dim3(n_tokens), dim3(256), 0, st, (uint16_t*)q,
-                       (uint16_t*)k, n_tokens, num_qo_heads, num_kv_heads, head_dim,
-                       (double)past_kv_len, inv_scale, log2_theta);
+  uint16_t *qp = (uint16_t*)q, *kp = (uint16_t*)k;
+  if ((((uintptr_t)q | (uintptr_t)k) & 15) == 0) {
+    RopePrompt p = {};
+    p.q = p.q_out = qp;
+    p.k = p.k_out = kp;
+    p.q_stride = (int64_t)num_qo_heads * head_dim;
+    p.k_stride = (int64_t)num_kv_heads * head_dim;
+    p.n_tokens = n_tokens;
+    p.Hq = num_qo_heads;
+    p.Hkv = num_kv_heads;
+    p.past_len = (double)past_kv_len;
+    p.inv_scale = inv_scale;
+    p.log2_theta = log2_theta;
+    launch_rope_prompt<false>(PoolGeom{}, p, head_dim, dtype, st);
+  } else if (dtype == TD_F16)
+    hipLaunchKernelGGL(rope_kernel<F16>, dim3(n_tokens), dim3(256), 0, st, qp, kp, n_tokens, num_qo_heads,
+                       num_kv_heads, head_dim, (double)past_kv_len, inv_scale, log2_theta);
   else
-    return fail(TD_ERR_UNSUPPORTED, "apply_rope_in_place failed to dispatch with dtype %d", dtype);
+    hipLaunchKernelGGL(rope_kernel<BF16>, dim3(n_tokens), dim3(256), 0, st, qp, kp, n_tokens, num_qo_heads,
+                       num_kv_heads, head_dim, (double)past_kv_len, inv_scale, log2_theta);
   TD_HIP_CHECK(hipGetLastError());
   return TD_OK;
 }
@@ -711,18 +904,90 @@ extern "C" int td_estimate_score(const td_paged_kv* meta, const int32_t* meta_in
   return TD_OK;
 }
 
+static int rms_norm_any(void* x, const void* delta, const void* weight, void* out, int32_t rows, int32_t cols,
+                        float eps, int32_t dtype, void* stream, const char* who) {
+  TD_REQUIRE(rows >= 0 && cols >= 1, "%s: rows %d cols %d", who, rows, cols);
+  if (rows == 0) return TD_OK;
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  if (dtype != TD_F16 && dtype != TD_BF16)
+    return fail(TD_ERR_UNSUPPORTED, "%s failed to dispatch with dtype %d", who, dtype);
+  if (delta) {
+    if (dtype == TD_F16) launch_rms_norm<F16, true>(x, delta, weight, out, rows, cols, eps, st);
+    else launch_rms_norm<BF16, true>(x, delta, weight, out, rows, cols, eps, st);
+  } else {
+    if (dtype == TD_F16) launch_rms_norm<F16, false>(x, nullptr, weight, out, rows, cols, eps, st);
+    else launch_rms_norm<BF16, false>(x, nullptr, weight, out, rows, cols, eps, st);
+  }
+  TD_HIP_CHECK(hipGetLastError());
+  return TD_OK;
+}
+
 extern "C" int td_rms_norm(const void* x, const void* weight, void* out, int32_t rows,
                            int32_t cols, float eps, int32_t dtype, void* stream) {
   TD_REQUIRE(x && weight && out, "rms_norm_forward: NULL argument");
-  TD_REQUIRE(rows >= 0 && cols >= 1, "rms_norm_forward: rows %d cols %d", rows, cols);
+  return rms_norm_any(const_cast<void*>(x), nullptr, weight, out, rows, cols, eps, dtype, stream,
+                      "rms_norm_forward");  // without delta x is only read
+}
+
+extern "C" int td_add_rms_norm(void* x, const void* delta, const void* weight, void* out, int32_t rows,
+                               int32_t cols, float eps, int32_t dtype, void* stream) {
+  TD_REQUIRE(x && delta && weight && out, "add_rms_norm: NULL argument");
+  return rms_norm_any(x, delta, weight, out, rows, cols, eps, dtype, stream, "add_rms_norm");
+}
+
+extern "C" int td_silu_mul(const void* gate_up, void* out, int32_t rows, int32_t cols, int32_t dtype,
+                           void* stream) {
+  TD_REQUIRE(gate_up && out, "silu_mul: NULL argument");
+  TD_REQUIRE(rows >= 0 && cols >= 1 && cols <= (1 << 23), "silu_mul: rows %d cols %d", rows, cols);
   if (rows == 0) return TD_OK;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  if (dtype == TD_F16)
-    launch_rms_norm<F16>(x, weight, out, rows, cols, eps, st);
-  else if (dtype == TD_BF16)
-    launch_rms_norm<BF16>(x, weight, out, rows, cols, eps, st);
-  else
-    return fail(TD_ERR_UNSUPPORTED, "rms_norm_forward failed to dispatch with dtype %d", dtype);
+  if (dtype == TD_F16) launch_silu_mul<F16>(gate_up, out, rows, cols, st);
+  else if (dtype == TD_BF16) launch_silu_mul<BF16>(gate_up, out, rows, cols, st);
+  else return fail(TD_ERR_UNSUPPORTED, "silu_mul failed to dispatch with dtype %d", dtype);
+  TD_HIP_CHECK(hipGetLastError());
+  return TD_OK;
+}
+
+extern "C" int td_rope_append_prompt(const td_paged_kv* kv, const void* qkv, int64_t qkv_stride, void* q_out,
+                                     int32_t n_tokens, int32_t num_qo_heads, int64_t past_kv_len,
+                                     const int32_t* kv_indices, const int32_t* kv_indptr, int32_t last_page_len,
+                                     float rope_scale, float rope_theta, void* stream) {
+  const int rc = check_pool(kv, "rope_append_prompt");
+  if (rc) return rc;
+  TD_REQUIRE(qkv && q_out && kv_indices && kv_indptr, "rope_append_prompt: NULL argument");
+  TD_REQUIRE(n_tokens >= 0 && num_qo_heads >= 1, "rope_append_prompt: n_tokens %d heads %d", n_tokens,
+             num_qo_heads);
+  TD_REQUIRE(last_page_len >= 1 && last_page_len <= kv->page_size,
+             "rope_append_prompt: last_page_len %d not in [1, %d]", last_page_len, kv->page_size);
+  const int D = kv->head_dim, Hkv = kv->num_kv_heads;
+  if (D != 64 && D != 128 && D != 256)
+    return fail(TD_ERR_UNSUPPORTED, "rope_append_prompt: head_dim %d (supported: 64, 128, 256)", D);
+  if (kv->dtype != TD_F16 && kv->dtype != TD_BF16)
+    return fail(TD_ERR_UNSUPPORTED, "rope_append_prompt failed to dispatch with dtype %d", kv->dtype);
+  TD_REQUIRE(rope_scale > 0.f && rope_theta > 0.f, "rope_append_prompt: scale %g theta %g", rope_scale,
+             rope_theta);
+  TD_REQUIRE(past_kv_len >= 0, "rope_append_prompt: past_kv_len %lld", (long long)past_kv_len);
+  TD_REQUIRE(qkv_stride >= (int64_t)(num_qo_heads + 2 * Hkv) * D && qkv_stride % 8 == 0,
+             "rope_append_prompt: row stride %lld", (long long)qkv_stride);
+  TD_REQUIRE((((uintptr_t)qkv | (uintptr_t)q_out | (uintptr_t)kv->data) & 15) == 0,
+             "rope_append_prompt: qkv, q_out and the pool must be 16-byte aligned");
+  if (n_tokens == 0) return TD_OK;
+  RopePrompt p = {};
+  p.q = (const uint16_t*)qkv;
+  p.k = p.q + (int64_t)num_qo_heads * D;
+  p.v = p.k + (int64_t)Hkv * D;
+  p.q_stride = p.k_stride = p.v_stride = qkv_stride;
+  p.q_out = (uint16_t*)q_out;
+  p.n_tokens = n_tokens;
+  p.Hq = num_qo_heads;
+  p.Hkv = Hkv;
+  p.past_len = (double)past_kv_len;
+  p.inv_scale = 1.0 / (double)rope_scale;
+  p.log2_theta = log2((double)rope_theta);
+  p.indices = kv_indices;
+  p.indptr = kv_indptr;
+  p.last_page_len = last_page_len;
+  launch_rope_prompt<true>(geom_of(kv), p, D, kv->dtype, reinterpret_cast<hipStream_t>(stream));
   TD_HIP_CHECK(hipGetLastError());
   return TD_OK;
 }

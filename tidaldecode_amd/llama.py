@@ -129,10 +129,7 @@ class TidalLlama:
         return tidal_utils.rms_norm_forward(x, weight, self.config.rms_norm_eps)
 
     def _mlp(self, layer, x):
-        c = self.config
-        gu = x @ layer["w_gate_up"].t()
-        gate, up = gu[..., : c.intermediate_size], gu[..., c.intermediate_size:]
-        return (torch.nn.functional.silu(gate) * up) @ layer["w_down"].t()
+        return _kernels.silu_mul(x @ layer["w_gate_up"].t()) @ layer["w_down"].t()
 
     def _qkv(self, layer, h):
         c = self.config
@@ -145,6 +142,19 @@ class TidalLlama:
         v = qkv[:, k_end:].reshape(n, c.num_kv_heads, c.head_dim).contiguous()
         return q, k, v
 
+    def _qkv_to_cache(self, layer, h, idx, past):
+        """Projections of the prompt rows h; k and v go to the cache, rotated q is returned."""
+        c, ctrl = self.config, self.iController
+        if ctrl.metadata_cache is None:
+            return _kernels.rope_append_prompt(
+                h @ layer["wqkv"].t(), c.num_heads, past, ctrl.kv_cache.buf_layer(idx),
+                ctrl.kv_indices_with_last, ctrl.kv_indptr_for_append, ctrl.kv_cache.last_page_len,
+                ctrl.layout, c.rope_scale, c.rope_theta)
+        q, k, v = self._qkv(layer, h)  # the page bounds come from the append of its own
+        tidal_utils.apply_rope_in_place(q, k, past, c.rope_scale, c.rope_theta)
+        tidal_utils.append_kv(k, v, ctrl, idx)
+        return q
+
     # ----- prefill ----------------------------------------------------------------------------
     @torch.no_grad()
     def prefill(self, input_ids: torch.Tensor) -> torch.Tensor:
@@ -156,17 +166,17 @@ class TidalLlama:
         t0 = time.perf_counter()
         ctrl.prepare_metadata(n)
         ctrl.begin_forward(n)
-        x = self.embed[input_ids.to(self.device)]
+        x = self.embed[input_ids.to(self.device)]  # a copy: the residual stream, updated in place
+        mlp = None                                 # the previous layer's, not yet added to x
         for idx, layer in enumerate(self.layers):
-            h = self._rms(x, layer["ln1"])
-            q, k, v = self._qkv(layer, h)
-            tidal_utils.apply_rope_in_place(q, k, past, c.rope_scale, c.rope_theta)
-            tidal_utils.append_kv(k, v, ctrl, idx)
+            h = self._rms(x, layer["ln1"]) if mlp is None else \
+                _kernels.add_rms_norm(x, mlp, layer["ln1"], c.rms_norm_eps)
+            q = self._qkv_to_cache(layer, h, idx, past)
             o = tidal_utils.prefill_forward(q, ctrl, idx)
-            x = x + o.reshape(n, -1) @ layer["wo"].t()
-            x = x + self._mlp(layer, self._rms(x, layer["ln2"]))
+            h = _kernels.add_rms_norm(x, o.view(n, -1) @ layer["wo"].t(), layer["ln2"], c.rms_norm_eps)
+            mlp = self._mlp(layer, h)
         ctrl.end_forward()
-        logits = self._rms(x[-1:], self.norm) @ self.lm_head.t()
+        logits = _kernels.add_rms_norm(x[-1:], mlp[-1:], self.norm, c.rms_norm_eps) @ self.lm_head.t()
         torch.cuda.synchronize()
         ctrl.prefill_latency.append(time.perf_counter() - t0)
         return logits[0]

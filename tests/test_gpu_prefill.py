@@ -183,3 +183,37 @@ def test_row_packing_rings_and_pieces(cuda, dtype, hq, hkv, d, page, kv_len, n_q
     got = _run(cuda, case, q, True, dtype).float().cpu()
     want = _dense(q, case.k, case.v, True)
     assert ((got - want).abs() <= ATOL[dtype] * want.abs().clamp(min=1.0)).all()
+
+
+def _planned_bytes(case, q, causal):
+    from tidaldecode_amd import _kernels
+    from tidaldecode_amd._lib import lib
+
+    # the CPU pool: the plan depends on the geometry alone
+    pool = _kernels.PagedKV(1, case.max_pages, case.hkv, case.d, case.page_size, case.layout,
+                            _kernels._dtype_code(case.dtype, "pool"))
+    return lib.td_prefill_workspace_bytes(pool, case.n, q.size(0), q.size(1), int(causal))
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+@pytest.mark.parametrize("dtype,hq,hkv,d,past,n_q", [
+    (torch.bfloat16, 8, 8, 128, 0, 4000), (torch.float16, 16, 16, 64, 0, 2900), (torch.bfloat16, 14, 2, 128, 0, 1500),
+    (torch.float16, 4, 4, 128, 2048, 1000), (torch.bfloat16, 4, 2, 256, 0, 1500)])
+def test_rows_that_see_no_key_of_a_piece_take_nothing_from_it(cuda, dtype, hq, hkv, d, past, n_q, bad):
+    """Keys cut into pieces: everything from a key tile's first token on is infinite or NaN.  The rows
+    before that token see none of it, whichever piece it lies in; their 32-token wave ends before it."""
+    kv_len = past + n_q
+    case = PagedCase(kv_len, hkv, d, 16, dtype, seed=kv_len)
+    q = randn((n_q, hq, d), kv_len + 1, dtype)
+    assert _planned_bytes(case, q, True) > 0
+    want = _dense(q, case.k, case.v, True)
+    q_d, pool, table = q.to(dtype).to(cuda), case.pool.to(cuda), case.page_table.to(cuda)
+    from tidaldecode_amd import _kernels
+
+    for t0 in range(kv_len // 64 * 64, past, -64):    # the clean part shrinks
+        pool[table[t0 // 16:], 1] = bad
+        got = _kernels.prefill_with_paged_kv_cache(q_d, pool, table.int(), case.last_page_len, True, 0, False, 1.0,
+                                                   1e4)[: t0 - past].float().cpu()
+        ref = want[: t0 - past]
+        ok = (got - ref).abs() <= ATOL[dtype] * ref.abs().clamp(min=1.0)   # False for NaN
+        assert ok.all(), (t0, (~ok).any(-1).any(-1).nonzero().flatten()[[0, -1]] + past)

@@ -830,8 +830,9 @@ __global__ __launch_bounds__(64 * NW, 1) void prefill_attn_staged_kernel(const P
 }
 
 // Adds up the pieces of every row whose keys were split: D / 4 adjacent threads own a row, four
-// dimensions each.  A piece in which a row sees no key carries a maximum far below any real one and
-// so a weight of zero; the piece that holds token 0 is seen by every row.
+// dimensions each.  The piece that holds token 0 is seen by every row; a piece in which a row sees no key
+// has denominator 0 and its partial result is not used (a wave that sees none of a piece walks its first tile
+// with weights 0, and 0 * V is NaN where a value behind the row is infinite or NaN).
 template <typename T, int D>
 __global__ __launch_bounds__(256) void prefill_merge_kernel(const PrefillParams p) {
   constexpr int TPR = D / 4;
@@ -855,6 +856,7 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(const PrefillParams 
       const f32x2 ml = *reinterpret_cast<const f32x2*>(p.part_ml + part * 2);
       m[u] = s0 + u < n_parts ? ml.x : 2.f * kNegBig;
       l[u] = s0 + u < n_parts ? ml.y : 0.f;
+      if (l[u] == 0.f) v[u] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
     const float m_new = fmaxf(fmaxf(fmaxf(m[0], m[1]), fmaxf(m[2], m[3])), M);
     const float alpha = fast_exp2(M - m_new);

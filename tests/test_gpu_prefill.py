@@ -217,3 +217,26 @@ def test_rows_that_see_no_key_of_a_piece_take_nothing_from_it(cuda, dtype, hq, h
         ref = want[: t0 - past]
         ok = (got - ref).abs() <= ATOL[dtype] * ref.abs().clamp(min=1.0)   # False for NaN
         assert ok.all(), (t0, (~ok).any(-1).any(-1).nonzero().flatten()[[0, -1]] + past)
+
+
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("layout", [0, 1])
+@pytest.mark.parametrize("d", [64, 128, 256])
+@pytest.mark.parametrize("page", [1, 2, 3, 4, 5, 6, 7, 8, 12, 16])
+def test_slots_outside_the_sequence_are_never_used(cuda, page, d, layout, causal):
+    """The tail of the last page and every other page of the pool hold NaN, which weight 0 would not undo."""
+    dtype, hq, hkv = torch.bfloat16, 4, 2
+    for kv_len, n_q, pieces in ((5, 5, False), (37, 37, False), (70, 33, False), (1000, 1, True), (1001, 900, None),
+                                (5000, 18, True)):
+        case = PagedCase(kv_len, hkv, d, page, dtype, layout=layout, seed=kv_len + page)
+        outside = torch.ones(case.max_pages * page, dtype=torch.bool)
+        outside[case.slots_of(torch.arange(kv_len))] = False
+        pages, entries = outside.view(-1, page).nonzero(as_tuple=True)
+        view = case.pool if layout == 0 else case.pool.transpose(2, 3)   # [pages, 2, page, heads, d]
+        view[pages, :, entries] = float("nan")
+        q = randn((n_q, hq, d), kv_len, dtype)
+        if pieces is not None:
+            assert (_planned_bytes(case, q, causal) > 0) == pieces
+        want = _dense(q, case.k, case.v, causal)
+        got = _run(cuda, case, q, causal, dtype).float().cpu()
+        assert ((got - want).abs() <= ATOL[dtype] * want.abs().clamp(min=1.0)).all(), (kv_len, n_q)

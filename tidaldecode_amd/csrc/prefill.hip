@@ -176,7 +176,7 @@ __global__ __launch_bounds__(512, 2) void prefill_attn_kernel(const PrefillParam
   const uint64_t k_base = (uint64_t)(uintptr_t)(p.kv + (int64_t)w.kvh * p.head_stride);
   const int last_tok = p.kv_len - 1;
   auto page_of = [&](int t) { return (int)(__umulhi(2u * (uint32_t)t, p.page_magic) >> p.page_down); };
-  // first token of the wave's rows of tile j (tiles past the end repeat the last tokens: the loads need
+  // OCT: first token of the wave's rows of tile j (tiles past the end repeat the last tokens: the loads need
   // no branch and what they bring is masked)
   auto first_tok = [&](int j) {
     const int t = w.k_begin + j * BN + 8 * wave;
@@ -236,10 +236,11 @@ __global__ __launch_bounds__(512, 2) void prefill_attn_kernel(const PrefillParam
         asm volatile("" : "+v"(pages));  // waited for here and not, with everything else, in every step
         ahead = page_of_lane(j + 8);
       }
-      const int t0 = first_tok(j), lim = last_tok - t0;
+      const int t0 = w.k_begin + j * BN + 8 * wave;
 #pragma unroll
       for (int x = 0; x < NL; ++x) {
-        const int t = RPB * x + rb < lim ? t0 + RPB * x + rb : last_tok;
+        // the token whose page page_of_lane looked up: rows past the end are the last token's
+        const int t = t0 + RPB * x + rb < last_tok ? t0 + RPB * x + rb : last_tok;
         const uint32_t page = (uint32_t)__shfl(pages, 8 * (j & 7) + RPB * x + rb, 64);
         const uint64_t row = (uint64_t)page * (uint64_t)(p.page_stride * 2) +
                              (uint64_t)(uint32_t)(t - page_of(t) * p.page_size) * p.entry_stride_b;

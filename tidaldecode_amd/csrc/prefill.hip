@@ -50,10 +50,11 @@ __device__ __forceinline__ u32x2 lds_read_tr16(const uint16_t* at) {
 // lds + 16 lane.  As asm: the compiler would wait for the load before every later LDS read.
 __device__ __forceinline__ void load_lds(uint32_t lds, uint64_t base, uint32_t offset) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-               :: "s"(lds), "v"(offset), "s"(base) : "memory");
+               :: "s"(lds), "v"(offset), "s"(base) : "memory", "m0");
 }
 __device__ __forceinline__ void load_lds(uint32_t lds, uint64_t at) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" :: "s"(lds), "v"(at) : "memory");
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
+               :: "s"(lds), "v"(at) : "memory", "m0");
 }
 
 constexpr float kTopWeight = 16384.f;  // a lane's share of a tile's row sum: every weight fits fp16 as well

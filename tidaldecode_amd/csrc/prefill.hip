@@ -48,8 +48,10 @@ __device__ __forceinline__ u32x2 lds_read_tr16(const uint16_t* at) {
 
 // 16 bytes per lane from memory (scalar base + lane offset, or a lane address) to LDS bytes
 // lds + 16 lane.  As asm: the compiler would wait for the load before every later LDS read.
+// It inserts no wait states inside the asm, so they stand there: one between m0 and the load, and five
+// between a scalar register that a vector instruction (v_readlane) wrote and the load that reads it.
 __device__ __forceinline__ void load_lds(uint32_t lds, uint64_t base, uint32_t offset) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %1, %2"
                :: "s"(lds), "v"(offset), "s"(base) : "memory", "m0");
 }
 __device__ __forceinline__ void load_lds(uint32_t lds, uint64_t at) {

@@ -314,3 +314,13 @@ def test_step_state_words(cuda):
     assert out.tolist() == [100, 101, 102, 103, 104]          # recording stops at the capacity
     with pytest.raises(RuntimeError):
         _kernels.step_advance(state, table, 4, 10, token, None)
+
+
+def test_prefill_without_layers(cuda):
+    """Embedding, final norm and vocabulary head alone."""
+    from tidaldecode_amd.llama import TidalLlama
+
+    model = TidalLlama(_small(num_layers=0), cuda, seed=2, init_std=0.05)
+    model.tidal_init(page_size=16, max_seq_len=64)
+    ids = torch.randint(0, 1000, (9,), device=cuda)
+    assert _close(model.prefill(ids), _reference_logits(model, ids))

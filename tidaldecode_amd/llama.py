@@ -176,7 +176,9 @@ class TidalLlama:
             h = _kernels.add_rms_norm(x, o.view(n, -1) @ layer["wo"].t(), layer["ln2"], c.rms_norm_eps)
             mlp = self._mlp(layer, h)
         ctrl.end_forward()
-        logits = _kernels.add_rms_norm(x[-1:], mlp[-1:], self.norm, c.rms_norm_eps) @ self.lm_head.t()
+        h = self._rms(x[-1:], self.norm) if mlp is None else \
+            _kernels.add_rms_norm(x[-1:], mlp[-1:], self.norm, c.rms_norm_eps)
+        logits = h @ self.lm_head.t()
         torch.cuda.synchronize()
         ctrl.prefill_latency.append(time.perf_counter() - t0)
         return logits[0]

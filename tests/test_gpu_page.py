@@ -490,3 +490,16 @@ def test_add_rms_norm_and_silu_mul(cuda, dtype, rows, cols):
     want = gate / (1 + (-gate).exp()) * up
     got = _kernels.silu_mul(gu)                                 # two roundings
     assert ((got.double() - want).abs() <= want.abs() * ulp * 1.02 + up.abs() * tiny + tiny).all()
+
+
+def test_rope_append_prompt_refuses_a_page_list_it_cannot_read(cuda):
+    from tidaldecode_amd import _kernels
+
+    pool = torch.zeros((2, 2, 16, 1, 64), dtype=torch.float16, device=cuda)
+    qkv = torch.zeros((4, 3 * 64), dtype=torch.float16, device=cuda)
+    table = torch.arange(1, dtype=torch.int32, device=cuda)
+    ends = torch.tensor([0, 1], dtype=torch.int32)
+    with pytest.raises(RuntimeError, match="kv_indptr must be a CUDA tensor"):
+        _kernels.rope_append_prompt(qkv, 1, 0, pool, table, ends, 4, 0)
+    with pytest.raises(RuntimeError, match="ends of the page list"):
+        _kernels.rope_append_prompt(qkv, 1, 0, pool, table, ends[:1].to(cuda), 4, 0)

@@ -152,7 +152,10 @@ def rope_append_prompt(qkv: torch.Tensor, num_qo_heads: int, past_kv_len: int, k
     _check_input(kv_indices, "kv_indices")
     _check_dim(1, kv_indices, "kv_indices")
     _check_i32(kv_indices, "kv_indices")
+    _check_input(kv_indptr, "kv_indptr")
     _check_i32(kv_indptr, "kv_indptr")
+    if kv_indptr.numel() < 2:
+        raise RuntimeError("rope_append_prompt: kv_indptr must hold the ends of the page list")
     pool = _pool(kv_data, int(layout))
     n, d = qkv.size(0), pool.head_dim
     if qkv.size(1) != (num_qo_heads + 2 * pool.num_kv_heads) * d or qkv.dtype != kv_data.dtype:

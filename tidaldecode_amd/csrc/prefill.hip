@@ -50,6 +50,10 @@ __device__ __forceinline__ u32x2 lds_read_tr16(const uint16_t* at) {
 // lds + 16 lane.  As asm: the compiler would wait for the load before every later LDS read.
 // It inserts no wait states inside the asm, so they stand there: one between m0 and the load, and five
 // between a scalar register that a vector instruction (v_readlane) wrote and the load that reads it.
+// (m0 is a register the compiler allocates to no variable, which it warns about; it does set m0 for
+// instructions of its own, and the list tells it that the value is gone.)
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
 __device__ __forceinline__ void load_lds(uint32_t lds, uint64_t base, uint32_t offset) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %1, %2"
                :: "s"(lds), "v"(offset), "s"(base) : "memory", "m0");
@@ -58,6 +62,7 @@ __device__ __forceinline__ void load_lds(uint32_t lds, uint64_t at) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
                :: "s"(lds), "v"(at) : "memory", "m0");
 }
+#pragma clang diagnostic pop
 
 constexpr float kTopWeight = 16384.f;  // a lane's share of a tile's row sum: every weight fits fp16 as well
 

@@ -169,7 +169,7 @@ def test_random_configurations(cuda, seed):
 def test_row_packing_rings_and_pieces(cuda, dtype, hq, hkv, d, page, kv_len, n_q, pieces, rise):
     """The edges of the work split: key tiles of 64, rings, packed query rows, pieces and their merge.
     `rise`: queries grow to this many times their size, so that later keys exceed the first tile's by
-    more than the factor of 2^14 that a row's reference point may lag, and accumulators are rescaled late.  Tolerance as above: weights are rounded
+    more than the factor of 2^8 that a row's reference point may lag, and accumulators are rescaled late.  Tolerance as above: weights are rounded
     relative to their own size whatever the reference point is."""
     from tidaldecode_amd import _kernels
     from tidaldecode_amd._lib import lib
@@ -240,3 +240,26 @@ def test_slots_outside_the_sequence_are_never_used(cuda, page, d, layout, causal
         want = _dense(q, case.k, case.v, causal)
         got = _run(cuda, case, q, causal, dtype).float().cpu()
         assert ((got - want).abs() <= ATOL[dtype] * want.abs().clamp(min=1.0)).all(), (kv_len, n_q)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("d", [64, 128, 256])
+def test_a_weight_far_above_the_first_tile_is_not_rounded_again(cuda, dtype, d):
+    """One key outweighs all others, which a row's first tile does not show: its weight is the row's
+    reference and so exactly 1, up to which power of two the others are smaller.  What is left are the roundings
+    (u) of the result and of the small weights."""
+    n_q = kv_len = 128
+    top = 100
+    k = torch.zeros(kv_len, 1, d)
+    k[top] = 1.0
+    case = PagedCase(kv_len, 1, d, 16, dtype, seed=d, kv=(k, randn((kv_len, 1, d), d, dtype)))
+    q = (torch.linspace(8.5, 13.9, n_q) / (math.sqrt(d) * math.log2(math.e)))[:, None, None].expand(n_q, 1, d)
+    q = q.to(dtype).float()
+    p = ((q[:, 0].double() @ k[:, 0].double().t()) / math.sqrt(d)).softmax(-1)
+    v = case.v[:, 0].double()
+    want = p @ v
+    p[:, top] = 0.0
+    u = 2.0 ** -11 if dtype == torch.float16 else 2.0 ** -8     # half a unit in the last place, relative
+    tol = 1.01 * u * (want.abs() + p @ v.abs()) + 1e-5          # 1e-5: sums and exponentials in 32 bits
+    got = _run(cuda, case, q, False, dtype)[:, 0].double().cpu()
+    assert ((got - want).abs() <= tol).all()

@@ -320,7 +320,8 @@ def test_prefill_without_layers(cuda):
     """Embedding, final norm and vocabulary head alone."""
     from tidaldecode_amd.llama import TidalLlama
 
-    model = TidalLlama(_small(num_layers=0), cuda, seed=2, init_std=0.05)
-    model.tidal_init(page_size=16, max_seq_len=64)
+    model = TidalLlama(_small(num_layers=1), cuda, seed=2, init_std=0.05)
+    model.tidal_init(page_size=16, max_seq_len=64)   # a cache has at least one layer
+    model.layers.clear()
     ids = torch.randint(0, 1000, (9,), device=cuda)
     assert _close(model.prefill(ids), _reference_logits(model, ids))

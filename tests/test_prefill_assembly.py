@@ -1,5 +1,5 @@
-"""CPU: hazards that the compiler leaves to hand-written instructions, checked in the assembly of
-csrc/prefill.hip (compiled here, about four seconds).
+"""CPU: hazards that the compiler leaves to hand-written instructions, and the registers of the kernels,
+checked in the assembly of csrc/prefill.hip (compiled here, about four seconds).
 
 Inside an asm statement the compiler inserts no wait states.  gfx950 needs five between a vector
 instruction that writes a scalar register (v_readlane, v_readfirstlane) and a memory instruction that
@@ -16,7 +16,7 @@ HIPCC = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
 
 
 @pytest.fixture(scope="module")
-def asm_blocks(tmp_path_factory):
+def assembly(tmp_path_factory):
     if not os.path.exists(HIPCC):
         pytest.skip("no hipcc")
     out = str(tmp_path_factory.mktemp("asm") / "prefill.s")
@@ -24,8 +24,13 @@ def asm_blocks(tmp_path_factory):
                     "-packed-fp32-ops", "--cuda-device-only", "-S", os.path.join(CSRC, "prefill.hip"), "-o", out],
                    check=True, stderr=subprocess.DEVNULL)
     with open(out) as f:
-        return [[i.strip() for i in b.split("\n") if i.strip()]
-                for b in re.findall(r";;#ASMSTART\n(.*?);;#ASMEND", f.read(), re.S)]
+        return f.read()
+
+
+@pytest.fixture(scope="module")
+def asm_blocks(assembly):
+    return [[i.strip() for i in b.split("\n") if i.strip()]
+            for b in re.findall(r";;#ASMSTART\n(.*?);;#ASMEND", assembly, re.S)]
 
 
 def _wait_states(instructions):
@@ -48,3 +53,14 @@ def test_m0_is_named_as_overwritten():
         statements = re.findall(r"asm volatile\((.*?)\);", f.read(), re.S)
     writes = [s for s in statements if "s_mov_b32 m0" in s]
     assert len(writes) == 2 and all('"m0"' in s.split(":")[-1] for s in writes)
+
+
+def test_two_waves_of_an_attention_kernel_share_a_simd(assembly):
+    """Eight waves of 64 / 128 dimensions and two workgroups of 256 dimensions per compute unit need kernels
+    of at most 256 registers; more puts the accumulators into the second register file, with copies in
+    every step."""
+    kernels = re.findall(r"^(\S*prefill_attn\S*):[^\n]*\n(.*?)\.end_amdhsa_kernel", assembly, re.S | re.M)
+    assert len(kernels) == 10
+    for name, body in kernels:
+        assert int(re.search(r"\.amdhsa_next_free_vgpr (\d+)", body).group(1)) <= 256, name
+        assert "scratch_" not in body and "v_accvgpr" not in body, name

@@ -548,8 +548,12 @@ __global__ __launch_bounds__(512, 2) void prefill_attn_kernel(const PrefillParam
 // rows per wave and 16x16x32 MFMA, BN tokens per key tile (a multiple of 32), NW waves per workgroup.
 // K/V tiles pass through registers into two LDS buffers per matrix, one barrier per tile; LDS rows are
 // padded by 32 bytes, which keeps the 16-byte K reads and the transposed V reads free of bank conflicts.
+// A step is a serial chain (scores, weights, values, barrier), so two workgroups share a compute unit: within
+// 256 registers (186) instead of 328 with accumulators copied between register files, whole tiles of 16
+// heads, bf16, take 45.1 us instead of 47.1 for 1000 tokens, 142 instead of 202 for 2900, 497 instead of
+// 751 for 6000.
 template <typename T, int D, int MT, int BN, int NW>
-__global__ __launch_bounds__(64 * NW, 1) void prefill_attn_staged_kernel(const PrefillParams p) {
+__global__ __launch_bounds__(64 * NW, 2) void prefill_attn_staged_kernel(const PrefillParams p) {
   constexpr int kThreads = 64 * NW;
   constexpr int WR = 16 * MT;       // query rows per wavefront
   constexpr int NS = D / 32;        // 16-byte pieces of a Q/K row per lane (one MFMA each)
@@ -607,13 +611,15 @@ __global__ __launch_bounds__(64 * NW, 1) void prefill_attn_staged_kernel(const P
   // ---- staging: thread -> CPT chunks of K and of V per tile --------------------------------------
   // eight adjacent lanes move 128 contiguous bytes of one row (one cache line in, one conflict-free
   // LDS write out); a thread looks up the page of each of its RPT rows once
-  // Two register sets: the loads of tile t + 2 are issued while tile t + 1 still waits in the
-  // other set for its turn to be written to LDS, so a tile has two iterations to arrive.
-  u32x4 kreg_a[CPT], vreg_a[CPT], kreg_b[CPT], vreg_b[CPT];
+  // Two register sets for keys: the loads of tile t + 2 are issued while tile t + 1 still waits in the
+  // other set for its turn to be written to LDS, so its rows have two iterations to arrive.  Values have
+  // one set and one iteration: a second set would not fit 256 registers, and with more a compute unit
+  // holds one workgroup instead of two and accumulators are moved between register files in every step.
+  u32x4 kreg_a[CPT], kreg_b[CPT], vreg[CPT];
   const int srow = tid >> 3, sl8 = tid & 7;
-  // page ids are looked up one tile ahead of the rows they address, so that a tile's K/V loads
-  // never wait for a page-table load issued in the same iteration
-  uint32_t pg[RPT];
+  // page ids are looked up one tile ahead of the rows they address, so that a tile's loads never wait
+  // for a page-table load issued in the same iteration
+  uint32_t pg[RPT], pg_v[RPT];  // of the next tile of keys, of values
   auto split_tok = [&](int kt, int jr, int& pg_i, int& entry) {
     int tok = kt + srow + SR * jr;
     tok = tok < p.kv_len ? tok : p.kv_len - 1;
@@ -633,22 +639,26 @@ __global__ __launch_bounds__(64 * NW, 1) void prefill_attn_staged_kernel(const P
       pg[jr] = (uint32_t)p.page_table[pg_i];
     }
   };
-  auto fetch = [&](int kt, u32x4 (&kreg)[CPT], u32x4 (&vreg)[CPT]) {  // needs lookup(kt) before it
+  auto fetch = [&](int kt, const uint32_t (&pages)[RPT], int64_t matrix, u32x4 (&reg)[CPT]) {
 #pragma unroll
     for (int jr = 0; jr < RPT; ++jr) {
       int pg_i, entry;
       split_tok(kt, jr, pg_i, entry);
-      const uint32_t page = pg[jr] > p.max_page ? p.max_page : pg[jr];
-      const uint16_t* src = p.kv + ((int64_t)page * p.page_stride + (int64_t)entry * p.entry_stride +
+      const uint32_t page = pages[jr] > p.max_page ? p.max_page : pages[jr];
+      const uint16_t* src = p.kv + (matrix + (int64_t)page * p.page_stride + (int64_t)entry * p.entry_stride +
                                     (int64_t)kvh * p.head_stride + sl8 * 8);
 #pragma unroll
-      for (int jc = 0; jc < CCT; ++jc) {
-        kreg[jr * CCT + jc] = *reinterpret_cast<const u32x4*>(src + jc * 64);
-        vreg[jr * CCT + jc] = *reinterpret_cast<const u32x4*>(src + jc * 64 + p.v_offset);
-      }
+      for (int jc = 0; jc < CCT; ++jc) reg[jr * CCT + jc] = *reinterpret_cast<const u32x4*>(src + jc * 64);
     }
   };
-  auto stash = [&](int buf, const u32x4 (&kreg)[CPT], const u32x4 (&vreg)[CPT]) {
+  auto fetch_v = [&](int kt) { fetch(kt, pg_v, p.v_offset, vreg); };
+  auto fetch_k = [&](int kt, u32x4 (&kreg)[CPT]) {  // needs lookup(kt) before it; fetch_v(kt) comes after it
+    fetch(kt, pg, 0, kreg);
+#pragma unroll
+    for (int jr = 0; jr < RPT; ++jr) pg_v[jr] = pg[jr];
+    lookup(kt + kPfBN);
+  };
+  auto stash = [&](int buf, const u32x4 (&kreg)[CPT]) {
 #pragma unroll
     for (int jr = 0; jr < RPT; ++jr)
 #pragma unroll
@@ -778,33 +788,26 @@ __global__ __launch_bounds__(64 * NW, 1) void prefill_attn_staged_kernel(const P
     }
   };
 
-  // first tile into buffer 0, second tile into register set a
+  // first tile into buffer 0, keys of the second into register set a
   lookup(k_begin);
-  fetch(k_begin, kreg_a, vreg_a);
-  lookup(k_begin + kPfBN);
-  stash(0, kreg_a, vreg_a);
-  if (k_begin + kPfBN < kv_end) {
-    fetch(k_begin + kPfBN, kreg_a, vreg_a);
-    lookup(k_begin + 2 * kPfBN);
-  }
+  fetch_k(k_begin, kreg_a);
+  fetch_v(k_begin);
+  stash(0, kreg_a);
+  if (k_begin + kPfBN < kv_end) fetch_k(k_begin + kPfBN, kreg_a);
   // One barrier per tile: it makes tile kt visible in its buffer, and it tells that every wave has
   // finished reading the other buffer, which the end of the step overwrites with tile kt + BN.
   for (int kt = k_begin; kt < kv_end; kt += 2 * kPfBN) {
     __syncthreads();
-    if (kt + 2 * kPfBN < kv_end) {
-      fetch(kt + 2 * kPfBN, kreg_b, vreg_b);
-      lookup(kt + 3 * kPfBN);
-    }
+    if (kt + kPfBN < kv_end) fetch_v(kt + kPfBN);
+    if (kt + 2 * kPfBN < kv_end) fetch_k(kt + 2 * kPfBN, kreg_b);
     compute(kt, 0);
     if (kt + kPfBN >= kv_end) break;
-    stash(1, kreg_a, vreg_a);
+    stash(1, kreg_a);
     __syncthreads();
-    if (kt + 3 * kPfBN < kv_end) {
-      fetch(kt + 3 * kPfBN, kreg_a, vreg_a);
-      lookup(kt + 4 * kPfBN);
-    }
+    if (kt + 2 * kPfBN < kv_end) fetch_v(kt + 2 * kPfBN);
+    if (kt + 3 * kPfBN < kv_end) fetch_k(kt + 3 * kPfBN, kreg_a);
     compute(kt + kPfBN, 1);
-    if (kt + 2 * kPfBN < kv_end) stash(0, kreg_b, vreg_b);
+    if (kt + 2 * kPfBN < kv_end) stash(0, kreg_b);
   }
 
   // ---- normalise and store (or leave the piece's partial result): lane holds rows 4g + i,

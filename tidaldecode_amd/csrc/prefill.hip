@@ -125,8 +125,11 @@ __device__ __forceinline__ bool prefill_piece(const PrefillParams& p, PrefillPie
     w.kvh = lin % p.n_kv;
     rem = lin / p.n_kv;
   }
-  const int qtile = p.n_tiles - 1 - rem / p.n_splits;
-  w.split = rem % p.n_splits;
+  // The first pieces of all tiles before the second ones: full-length pieces come first and the shortest
+  // last.  (Tile by tile, a short tile's only piece starts last and is as long as any: 16 heads of 256,
+  // pieces of half the keys, 1400 tokens 63 -> 55 us, 2000 119 -> 81; 28 / 4 heads of 64, 2000 50 -> 38.)
+  w.split = rem / p.n_tiles;
+  const int qtile = p.n_tiles - 1 - rem % p.n_tiles;
   w.q0 = qtile * p.bm;
   const int end = tile_kv_end(p, qtile);
   w.k_begin = __builtin_amdgcn_readfirstlane(w.split * p.chunk);

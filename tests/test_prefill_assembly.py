@@ -64,3 +64,9 @@ def test_two_waves_of_an_attention_kernel_share_a_simd(assembly):
     for name, body in kernels:
         assert int(re.search(r"\.amdhsa_next_free_vgpr (\d+)", body).group(1)) <= 256, name
         assert "scratch_" not in body and "v_accvgpr" not in body, name
+
+
+def test_attention_kernels_divide_by_multiplication(assembly):
+    """A division by a run-time number starts with v_rcp_iflag_f32 and is a chain of some 20 instructions."""
+    for name, body in re.findall(r"^(\S*prefill_attn\S*):[^\n]*\n(.*?)\.end_amdhsa_kernel", assembly, re.S | re.M):
+        assert "v_rcp_iflag" not in body, name

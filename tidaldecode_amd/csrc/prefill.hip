@@ -926,27 +926,42 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(const PrefillParams 
 // over 8 KV heads, 100 tokens 9.6 / 8.7 / 7.5, 300 14.0 / 11.7 / 10.5, 640 21 / 17.0 / 15.5, 1000 27 / 23 / 27,
 // 2000 48 / 47 / 80, 2900 75 / 92 / 152.  Pieces against whole tiles of 256: 500 rows of 32 heads on 32768
 // keys 254 against 600.
-static double prefill_cost(const PrefillParams& p, int head_dim, int kv_len, double tile, int splits) {
-  const int bn = head_dim == 256 ? 32 : 64;
+static double prefill_cost(const PrefillParams& p, int head_dim, double tile, int64_t tiles, int64_t jobs,
+                           int64_t c) {
   const int64_t slots = (int64_t)td_num_cus() * (head_dim == 256 ? 2 : 1);
-  const double start = p.bm == 256 ? 6.5 : 4.5, merge = 2.0;
-  const int max_tiles = (kv_len + bn - 1) / bn, c = (max_tiles + splits - 1) / splits;
-  int64_t jobs = 0, total = 0;
-  for (int t = 0; t < p.n_tiles; ++t) {
-    int last = (t + 1) * p.bm - 1;
-    last = last < p.n_rows ? last : p.n_rows - 1;
-    const int end = p.causal ? kv_len - p.n_q + last / p.q_per_kv + 1 : kv_len;
-    const int k = (end + bn - 1) / bn;
-    jobs += (k + c - 1) / c;
-    total += k;
-  }
-  jobs *= p.n_kv;
-  total *= p.n_kv;
-  const double mean = tile * (double)total / jobs + start, longest = tile * c + start;
+  const double start = p.bm == 256 ? 6.5 : 4.5;
+  const double mean = tile * (double)tiles / jobs + start, longest = tile * c + start;
   const double share = mean * jobs / slots + 0.25 * longest, rounds = (double)((jobs + slots - 1) / slots) * mean;
   const double cost = share < rounds ? share : rounds;
-  const double pieces = merge + (double)p.n_kv * p.n_rows * head_dim * 4e-6 * splits / 4.0;
-  return (cost > longest ? cost : longest) + (splits > 1 ? pieces : 0.0);
+  return cost > longest ? cost : longest;
+}
+
+// sum of (a i + b) / m over 0 <= i < n, in as many steps as Euclid's algorithm takes for a and m: whole
+// multiples of m come out of a and b, and what is left counts the lattice points under a line of slope below
+// one, which is the same sum with the axes exchanged (Graham, Knuth, Patashnik, Concrete Mathematics, 3.5)
+static int64_t floor_sum(int64_t n, int64_t m, int64_t a, int64_t b) {
+  int64_t sum = 0;
+  while (true) {
+    sum += n * (n - 1) / 2 * (a / m) + n * (b / m);
+    a %= m;
+    b %= m;
+    const int64_t top = a * n + b;
+    if (top < m) return sum;
+    n = top / m;
+    b = top % m;
+    const int64_t slope = a;
+    a = m;
+    m = slope;
+  }
+}
+
+// sum of ceil(key tiles / c) over a KV head's row tiles: its key tiles (c = 1), its pieces of c key tiles
+static int64_t key_pieces(const PrefillParams& p, int kv_len, int bn, int64_t c) {
+  if (!p.causal) return p.n_tiles * ((((int64_t)kv_len + bn - 1) / bn + c - 1) / c);
+  // a tile's last row r sees the keys up to kv_len - n_q + r / group, so that it has
+  // (r + group (kv_len - n_q + bn)) / (group bn) key tiles; r = (i + 1) bm - 1 in all row tiles but the last
+  const int64_t g = p.q_per_kv, m = g * bn * c, b = g * (kv_len - p.n_q + bn) + g * bn * (c - 1);
+  return floor_sum(p.n_tiles - 1, m, p.bm, b + p.bm - 1) + (p.n_rows - 1 + b) / m;
 }
 
 template <typename T>
@@ -1011,14 +1026,21 @@ static void plan_prefill(const td_paged_kv* kv, int32_t kv_len, int32_t n_q, int
   p.n_q = n_q;
   p.causal = causal;
   const int bn = D == 256 ? 32 : 64, max_tiles = (kv_len + bn - 1) / bn;
+  const int64_t cus = td_num_cus();
   double best = 0.0;
   PrefillParams c = p;
   for (c.bm = D == 256 ? 64 : 256; c.bm >= 64; c.bm /= 2) {
     c.n_tiles = (c.n_rows + c.bm - 1) / c.bm;
+    const double tile = D == 256 || c.bm == 256 ? 1.0 : c.bm == 128 ? 0.87 : 0.83;
+    const int64_t tiles = H * key_pieces(c, kv_len, bn, 1);
     for (int s = 1; s <= 64; s = s < 8 ? s + 1 : (s < 16 ? s + 2 : s * 2)) {
       const int chunk = (max_tiles + s - 1) / s;
-      if (s > 1 && (!may_split || chunk < 4 || (int64_t)c.n_tiles * H >= 8 * (int64_t)td_num_cus())) break;
-      const double cost = prefill_cost(c, D, kv_len, D == 256 || c.bm == 256 ? 1.0 : c.bm == 128 ? 0.87 : 0.83, s);
+      if (s > 1 && (!may_split || chunk < 4 || (int64_t)c.n_tiles * H >= 8 * cus)) break;
+      const double pieces = s > 1 ? 2.0 + (double)H * c.n_rows * D * 4e-6 * s / 4.0 : 0.0;
+      // no cost is below that of the longest piece alone
+      if (s > 1 && tile * chunk + pieces >= best) continue;
+      const int64_t jobs = H * (s > 1 ? key_pieces(c, kv_len, bn, chunk) : c.n_tiles);
+      const double cost = prefill_cost(c, D, tile, tiles, jobs, chunk) + pieces;
       if (best == 0.0 || cost < best) {
         best = cost;
         p.bm = c.bm;

@@ -11,6 +11,7 @@ import pytest
 from tidaldecode_amd import _kernels
 from tidaldecode_amd._lib import PagedKV, lib
 
+LIMIT = 256 << 20      # bytes
 CUS = lib.td_num_cus()
 
 
@@ -33,6 +34,10 @@ def bytes_tile_by_tile(hq, hkv, d, kv_len, n_q, causal):
             chunk = ceil(max_tiles, s)
             if s > 1 and (chunk < 4 or len(tiles) * hkv >= 8 * CUS):
                 break
+            n = ceil(kv_len, chunk * bn)
+            scratch = n * hkv * rows * (d + 2) * 4 if n > 1 else 0
+            if scratch > LIMIT:
+                break
             jobs = hkv * sum(ceil(t, chunk) for t in tiles)
             mean, longest = step * (hkv * sum(tiles) / jobs) + start, step * chunk + start
             slots = CUS * (2 if d == 256 else 1)
@@ -40,8 +45,7 @@ def bytes_tile_by_tile(hq, hkv, d, kv_len, n_q, causal):
             if s > 1:
                 cost += 2.0 + hkv * rows * d * 4e-6 * s / 4.0
             if best is None or cost < best[0] * (1 - 1e-12):
-                n = ceil(kv_len, chunk * bn)
-                best = (cost, n * hkv * rows * (d + 2) * 4 if n > 1 else 0)
+                best = (cost, scratch)
     return best[1]
 
 
@@ -74,3 +78,14 @@ def test_a_plan_takes_the_host_microseconds(hq, hkv, d, past, n_q):
             lib.td_prefill_workspace_bytes(pool, past + n_q, n_q, hq, 1)
         best = min(best, (time.perf_counter() - t) / 20)
     assert best < 8e-6
+
+
+def test_scratch_is_bounded():
+    """The largest plans: many rows of many heads on long caches."""
+    rng = random.Random(0)
+    used = []
+    for d, hq, hkv in ((128, 40, 40), (256, 32, 32), (256, 64, 8), (64, 16, 16)):
+        for _ in range(200):
+            n_q = int(2 ** rng.uniform(9, 15))
+            used.append(scratch_bytes(hq, hkv, d, n_q + rng.choice([0, int(2 ** rng.uniform(9, 18))]), n_q))
+    assert LIMIT // 2 < max(used) <= LIMIT

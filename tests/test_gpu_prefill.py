@@ -263,3 +263,23 @@ def test_a_weight_far_above_the_first_tile_is_not_rounded_again(cuda, dtype, d):
     tol = 1.01 * u * (want.abs() + p @ v.abs()) + 1e-5          # 1e-5: sums and exponentials in 32 bits
     got = _run(cuda, case, q, False, dtype)[:, 0].double().cpu()
     assert ((got - want).abs() <= tol).all()
+
+
+def test_memory_too_short_for_scratch(cuda):
+    """Keys cut into pieces want 33 MB of partial results; where the allocator has 24 MB left, a call runs whole."""
+    from tidaldecode_amd import _kernels
+
+    dtype, past, n_q, h, d = torch.bfloat16, 8192, 500, 32, 128
+    case = PagedCase(past + n_q, 8, d, 16, dtype, seed=3)
+    q = randn((n_q, h, d), 4, dtype)
+    assert _planned_bytes(case, q, True) > (24 << 20)
+    want = _dense(q, case.k, case.v, True)
+    q_d, pool, table = q.to(dtype).to(cuda), case.pool.to(cuda), case.page_table.int().to(cuda)
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(cuda).total_memory
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (24 << 20)) / total)
+    try:
+        got = _kernels.prefill_with_paged_kv_cache(q_d, pool, table, case.last_page_len, True, 0, False, 1.0, 1e4)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert ((got.float().cpu() - want).abs() <= ATOL[dtype] * want.abs().clamp(min=1.0)).all()

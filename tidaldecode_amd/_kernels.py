@@ -524,7 +524,12 @@ def prefill_with_paged_kv_cache(q, kv_data, kv_indices, kv_last_page_len, causal
     causal = int(bool(causal))
     # scratch of this call alone (torch's allocator hands it out again in stream order)
     ws_bytes = lib.td_prefill_workspace_bytes(pool, kv_len, q.size(0), q.size(1), causal)
-    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device) if ws_bytes > 0 else None
+    ws = None
+    if ws_bytes > 0:
+        try:
+            ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device)
+        except torch.OutOfMemoryError:  # slower without, but a call needs none
+            ws_bytes = 0
     check(lib.td_prefill_attn_split(pool, kv_indices.data_ptr(), n_pages, kv_len, q.data_ptr(),
                                     o.data_ptr(), q.size(0), q.size(1),
                                     1.0 / math.sqrt(pool.head_dim), causal,

@@ -9,7 +9,7 @@ import time
 import pytest
 
 from tidaldecode_amd import _kernels
-from tidaldecode_amd._lib import PagedKV, lib
+from tidaldecode_amd._lib import TD_ERR_INVALID_ARG, PagedKV, last_error, lib
 
 LIMIT = 256 << 20      # bytes
 CUS = lib.td_num_cus()
@@ -89,3 +89,13 @@ def test_scratch_is_bounded():
             n_q = int(2 ** rng.uniform(9, 15))
             used.append(scratch_bytes(hq, hkv, d, n_q + rng.choice([0, int(2 ** rng.uniform(9, 18))]), n_q))
     assert LIMIT // 2 < max(used) <= LIMIT
+
+
+def test_workspace_that_is_not_aligned_is_refused():
+    """16-byte accesses to the partial results; the host refuses before anything is launched."""
+    pool = PagedKV(4096, 2049, 8, 128, 16, 0, _kernels.TD_BF16)             # addresses that nothing touches
+    n_bytes = lib.td_prefill_workspace_bytes(pool, 32768, 16, 32, 1)
+    assert n_bytes > 0
+    for off in (1, 4, 8):
+        rc = lib.td_prefill_attn_split(pool, 4096, 2048, 32768, 4096, 4096, 16, 32, 0.1, 1, 4096 + off, n_bytes, None)
+        assert rc == TD_ERR_INVALID_ARG and "16-byte aligned" in last_error()

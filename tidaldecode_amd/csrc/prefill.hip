@@ -1089,6 +1089,8 @@ extern "C" int td_prefill_attn_split(const td_paged_kv* kv, const int32_t* page_
   plan_prefill(kv, kv_len, n_q, num_qo_heads, causal, true, p);
   if (workspace == nullptr || workspace_bytes < prefill_ws_bytes(p, D))
     plan_prefill(kv, kv_len, n_q, num_qo_heads, causal, false, p);
+  TD_REQUIRE(p.n_splits == 1 || ((uintptr_t)workspace & 15) == 0,
+             "td_prefill_attn: the workspace must be 16-byte aligned");
   p.part_o = reinterpret_cast<float*>(workspace);
   p.part_ml = p.part_o ? p.part_o + (int64_t)p.n_splits * p.n_kv * p.n_rows * D : nullptr;
   p.kv = reinterpret_cast<const uint16_t*>(kv->data);

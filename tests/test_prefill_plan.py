@@ -9,7 +9,7 @@ import time
 import pytest
 
 from tidaldecode_amd import _kernels
-from tidaldecode_amd._lib import TD_ERR_INVALID_ARG, PagedKV, last_error, lib
+from tidaldecode_amd._lib import TD_ERR_INVALID_ARG, TD_ERR_UNSUPPORTED, PagedKV, last_error, lib
 
 LIMIT = 256 << 20      # bytes
 CUS = lib.td_num_cus()
@@ -99,3 +99,13 @@ def test_workspace_that_is_not_aligned_is_refused():
     for off in (1, 4, 8):
         rc = lib.td_prefill_attn_split(pool, 4096, 2048, 32768, 4096, 4096, 16, 32, 0.1, 1, 4096 + off, n_bytes, None)
         assert rc == TD_ERR_INVALID_ARG and "16-byte aligned" in last_error()
+
+
+def test_lengths_that_only_memory_limits():
+    """2^30 tokens of one head of 64 dimensions, and 2^30 packed query rows, fit 288 GB."""
+    n = (1 << 30) + 5
+    assert scratch_bytes(4, 1, 64, n, 16) > 0
+    # a head_dim without a kernel: refused for that, after the sizes were accepted and before any launch
+    pool = PagedKV(4096, 1 << 22, 1, 32, 16, 0, _kernels.TD_BF16)
+    rows = lib.td_prefill_attn(pool, 4096, 1 << 21, 1 << 25, 4096, 4096, 1 << 25, 32, 0.1, 1, None)
+    assert rows == TD_ERR_UNSUPPORTED and "head_dim" in last_error()

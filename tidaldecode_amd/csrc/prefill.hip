@@ -1005,13 +1005,14 @@ static int check_prefill(const td_paged_kv* kv, int32_t n_pages, int32_t kv_len,
   TD_REQUIRE(num_qo_heads >= kv->num_kv_heads && num_qo_heads % kv->num_kv_heads == 0,
              "td_prefill_attn: num_qo_heads %d is not a multiple of num_kv_heads %d", num_qo_heads,
              kv->num_kv_heads);
-  TD_REQUIRE(n_q >= 0 && kv_len >= n_q && kv_len < (1 << 30), "td_prefill_attn: n_q %d, kv_len %d", n_q,
-             kv_len);
+  // 32-bit positions and rows, of which the kernels look up to 80 key tiles and a row tile past the end
+  TD_REQUIRE(n_q >= 0 && kv_len >= n_q && kv_len <= INT32_MAX - (1 << 14), "td_prefill_attn: n_q %d, kv_len %d",
+             n_q, kv_len);
   TD_REQUIRE((int64_t)n_pages * kv->page_size >= kv_len,
              "td_prefill_attn: %d pages of %d entries do not hold %d tokens", n_pages,
              kv->page_size, kv_len);
   TD_REQUIRE(kv->layout == TD_NHD || kv->layout == TD_HND, "td_prefill_attn: layout %d", kv->layout);
-  TD_REQUIRE((int64_t)n_q * (num_qo_heads / kv->num_kv_heads) < ((int64_t)1 << 30),
+  TD_REQUIRE((int64_t)n_q * (num_qo_heads / kv->num_kv_heads) <= INT32_MAX - (1 << 9),
              "td_prefill_attn: %d queries of %d heads", n_q, num_qo_heads);
   return TD_OK;
 }

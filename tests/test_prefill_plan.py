@@ -103,8 +103,9 @@ def test_workspace_that_is_not_aligned_is_refused():
 
 def test_lengths_that_only_memory_limits():
     """2^30 tokens of one head of 64 dimensions, and 2^30 packed query rows, fit 288 GB."""
-    n = (1 << 30) + 5
-    assert scratch_bytes(4, 1, 64, n, 16) > 0
+    for n in ((1 << 30) + 5, (1 << 31) - (1 << 14) - 1):
+        assert scratch_bytes(4, 1, 64, n, 16) == bytes_tile_by_tile(4, 1, 64, n, 16, 1) > 0
+        assert scratch_bytes(32, 32, 64, n, 1 << 16) == 0           # whole tiles
     # a head_dim without a kernel: refused for that, after the sizes were accepted and before any launch
     pool = PagedKV(4096, 1 << 22, 1, 32, 16, 0, _kernels.TD_BF16)
     rows = lib.td_prefill_attn(pool, 4096, 1 << 21, 1 << 25, 4096, 4096, 1 << 25, 32, 0.1, 1, None)

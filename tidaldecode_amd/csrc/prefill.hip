@@ -876,7 +876,7 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(const PrefillParams 
   if (at >= (int64_t)p.n_kv * p.n_rows) return;
   const int kvh = (int)(at / p.n_rows), row = (int)(at - (int64_t)kvh * p.n_rows);
   const int kv_end = tile_kv_end(p, row / p.bm);
-  const int n_parts = (kv_end + p.chunk - 1) / p.chunk;
+  const int n_parts = 1 + (kv_end - 1) / p.chunk;
   if (n_parts <= 1) return;  // the attention kernel wrote the result
   const int c = threadIdx.x % TPR;
   const int64_t stride = (int64_t)p.n_kv * p.n_rows;
@@ -1047,7 +1047,7 @@ static void plan_prefill(const td_paged_kv* kv, int32_t kv_len, int32_t n_q, int
       const int chunk = (max_tiles + s - 1) / s;
       if (s > 1 && (!may_split || chunk < 4 || (int64_t)c.n_tiles * H >= 8 * cus)) break;
       c.chunk = chunk * bn;
-      c.n_splits = (kv_len + c.chunk - 1) / c.chunk;
+      c.n_splits = 1 + (kv_len - 1) / c.chunk;
       if (prefill_ws_bytes(c, D) > kMaxScratch) break;
       const double pieces = s > 1 ? 2.0 + (double)H * c.n_rows * D * 4e-6 * s / 4.0 : 0.0;
       // no cost is below that of the longest piece alone

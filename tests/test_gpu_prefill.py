@@ -189,8 +189,8 @@ def _planned_bytes(case, q, causal):
     from tidaldecode_amd import _kernels
     from tidaldecode_amd._lib import lib
 
-    # the CPU pool: the plan depends on the geometry alone
-    pool = _kernels.PagedKV(1, case.max_pages, case.hkv, case.d, case.page_size, case.layout,
+    # no pool: the plan depends on the geometry alone (and on whether the address is aligned)
+    pool = _kernels.PagedKV(16, case.max_pages, case.hkv, case.d, case.page_size, case.layout,
                             _kernels._dtype_code(case.dtype, "pool"))
     return lib.td_prefill_workspace_bytes(pool, case.n, q.size(0), q.size(1), int(causal))
 
@@ -283,3 +283,22 @@ def test_memory_too_short_for_scratch(cuda):
     finally:
         torch.cuda.set_per_process_memory_fraction(1.0)
     assert ((got.float().cpu() - want).abs() <= ATOL[dtype] * want.abs().clamp(min=1.0)).all()
+
+
+@pytest.mark.parametrize("off", [1, 2, 4, 7])
+@pytest.mark.parametrize("d,page,causal", [(64, 16, True), (64, 3, False), (128, 16, True), (128, 1, False), (256, 16, True)])
+def test_pool_that_is_not_16_byte_aligned(cuda, d, page, causal, off):
+    """A pool inside a wider buffer, `off` elements from its start: whole tiles and pieces."""
+    from tidaldecode_amd import _kernels
+
+    dtype, hq, hkv = torch.bfloat16, 4, 2
+    for kv_len, n_q in ((37, 37), (700, 333), (5000, 18)):
+        case = PagedCase(kv_len, hkv, d, page, dtype, seed=kv_len + d)
+        q = randn((n_q, hq, d), kv_len + off, dtype)
+        wide = torch.zeros(case.pool.numel() + 8, dtype=dtype, device=cuda)
+        pool = wide[off: off + case.pool.numel()].view(case.pool.shape).copy_(case.pool)
+        assert pool.data_ptr() % 16 == 2 * off
+        got = _kernels.prefill_with_paged_kv_cache(q.to(dtype).to(cuda), pool, case.page_table.int().to(cuda),
+                                                   case.last_page_len, causal, 0, False, 1.0, 1e4).float().cpu()
+        want = _dense(q, case.k, case.v, causal)
+        assert ((got - want).abs() <= ATOL[dtype] * want.abs().clamp(min=1.0)).all(), (kv_len, n_q)

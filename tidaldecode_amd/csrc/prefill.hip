@@ -109,6 +109,7 @@ struct PrefillParams {
   // The work of a KV head: n_rows = n_q * q_per_kv query rows (row = token * q_per_kv + head of the
   // group), n_tiles workgroup tiles of bm of them, each cut into n_splits pieces of `chunk` keys.
   int32_t n_kv, n_rows, bm, n_tiles, n_splits, chunk, head_major;
+  bool staged;     // prefill_attn_staged_kernel
   float* part_o;   // [n_splits][n_kv * n_rows][D]: un-normalised partial results (n_splits > 1)
   float* part_ml;  // [n_splits][n_kv * n_rows][2]: running maximum (base 2) and denominator
 };
@@ -564,7 +565,8 @@ __global__ __launch_bounds__(512, 2) void prefill_attn_kernel(const PrefillParam
   }
 }
 
-// head_dim 256, whose output alone would take 128 registers of a wave in the kernel above: 16 MT query
+// head_dim 256, whose output alone would take 128 registers of a wave in the kernel above, and pools that are
+// not 16-byte aligned, which direct loads to LDS are not specified for: 16 MT query
 // rows per wave and 16x16x32 MFMA, BN tokens per key tile (a multiple of 32), NW waves per workgroup.
 // K/V tiles pass through registers into two LDS buffers per matrix, one barrier per tile; LDS rows are
 // padded by 32 bytes, which keeps the 16-byte K reads and the transposed V reads free of bank conflicts.
@@ -926,9 +928,8 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(const PrefillParams 
 // over 8 KV heads, 100 tokens 9.6 / 8.7 / 7.5, 300 14.0 / 11.7 / 10.5, 640 21 / 17.0 / 15.5, 1000 27 / 23 / 27,
 // 2000 48 / 47 / 80, 2900 75 / 92 / 152.  Pieces against whole tiles of 256: 500 rows of 32 heads on 32768
 // keys 254 against 600.
-static double prefill_cost(const PrefillParams& p, int head_dim, double tile, int64_t tiles, int64_t jobs,
-                           int64_t c) {
-  const int64_t slots = (int64_t)td_num_cus() * (head_dim == 256 ? 2 : 1);
+static double prefill_cost(const PrefillParams& p, double tile, int64_t tiles, int64_t jobs, int64_t c) {
+  const int64_t slots = (int64_t)td_num_cus() * (p.staged ? 2 : 1);
   const double start = p.bm == 256 ? 6.5 : 4.5;
   const double mean = tile * (double)tiles / jobs + start, longest = tile * c + start;
   const double share = mean * jobs / slots + 0.25 * longest, rounds = (double)((jobs + slots - 1) / slots) * mean;
@@ -966,8 +967,14 @@ static int64_t key_pieces(const PrefillParams& p, int kv_len, int bn, int64_t c)
 
 template <typename T>
 static int launch_prefill(const PrefillParams& p, int head_dim, bool oct, hipStream_t st) {
-  const dim3 grid(p.n_tiles * p.n_kv * p.n_splits), block(head_dim == 256 ? 256 : 512);
-  if (head_dim == 128 && oct)
+  const dim3 grid(p.n_tiles * p.n_kv * p.n_splits), block(p.staged ? 256 : 512);
+  if (head_dim == 256)
+    hipLaunchKernelGGL((prefill_attn_staged_kernel<T, 256, 1, 32, 4>), grid, block, 0, st, p);
+  else if (head_dim == 128 && p.staged)
+    hipLaunchKernelGGL((prefill_attn_staged_kernel<T, 128, 1, 32, 4>), grid, block, 0, st, p);
+  else if (head_dim == 64 && p.staged)
+    hipLaunchKernelGGL((prefill_attn_staged_kernel<T, 64, 1, 32, 4>), grid, block, 0, st, p);
+  else if (head_dim == 128 && oct)
     hipLaunchKernelGGL((prefill_attn_kernel<T, 128, true>), grid, block, 0, st, p);
   else if (head_dim == 128)
     hipLaunchKernelGGL((prefill_attn_kernel<T, 128, false>), grid, block, 0, st, p);
@@ -975,8 +982,6 @@ static int launch_prefill(const PrefillParams& p, int head_dim, bool oct, hipStr
     hipLaunchKernelGGL((prefill_attn_kernel<T, 64, true>), grid, block, 0, st, p);
   else if (head_dim == 64)
     hipLaunchKernelGGL((prefill_attn_kernel<T, 64, false>), grid, block, 0, st, p);
-  else if (head_dim == 256)
-    hipLaunchKernelGGL((prefill_attn_staged_kernel<T, 256, 1, 32, 4>), grid, block, 0, st, p);
   else
     return fail(TD_ERR_UNSUPPORTED,
                 "BatchPrefillWithPagedKVCache failed to dispatch with head_dim %d (supported: 64, 128, 256)",
@@ -1035,13 +1040,14 @@ static void plan_prefill(const td_paged_kv* kv, int32_t kv_len, int32_t n_q, int
   p.n_rows = n_q * p.q_per_kv;
   p.n_q = n_q;
   p.causal = causal;
-  const int bn = D == 256 ? 32 : 64, max_tiles = (kv_len + bn - 1) / bn;
+  p.staged = D == 256 || ((uintptr_t)kv->data & 15) != 0;
+  const int bn = p.staged ? 32 : 64, max_tiles = (kv_len + bn - 1) / bn;
   const int64_t cus = td_num_cus();
   double best = 0.0;
   PrefillParams c = p;
-  for (c.bm = D == 256 ? 64 : 256; c.bm >= 64; c.bm /= 2) {
+  for (c.bm = p.staged ? 64 : 256; c.bm >= 64; c.bm /= 2) {
     c.n_tiles = (c.n_rows + c.bm - 1) / c.bm;
-    const double tile = D == 256 || c.bm == 256 ? 1.0 : c.bm == 128 ? 0.87 : 0.83;
+    const double tile = p.staged || c.bm == 256 ? 1.0 : c.bm == 128 ? 0.87 : 0.83;
     const int64_t tiles = H * key_pieces(c, kv_len, bn, 1);
     for (int s = 1; s <= 64; s = s < 8 ? s + 1 : (s < 16 ? s + 2 : s * 2)) {
       const int chunk = (max_tiles + s - 1) / s;
@@ -1053,7 +1059,7 @@ static void plan_prefill(const td_paged_kv* kv, int32_t kv_len, int32_t n_q, int
       // no cost is below that of the longest piece alone
       if (s > 1 && tile * chunk + pieces >= best) continue;
       const int64_t jobs = H * (s > 1 ? key_pieces(c, kv_len, bn, chunk) : c.n_tiles);
-      const double cost = prefill_cost(c, D, tile, tiles, jobs, chunk) + pieces;
+      const double cost = prefill_cost(c, tile, tiles, jobs, chunk) + pieces;
       if (best == 0.0 || cost < best) {
         best = cost;
         p.bm = c.bm;

@@ -95,7 +95,7 @@ __device__ __forceinline__ int operator/(int n, const Divisor& f) {
 struct PrefillParams {
   const uint16_t* kv;
   int64_t page_stride, v_offset;  // elements
-  int32_t entry_stride, head_stride, page_size, page_shift;
+  int32_t entry_stride, head_stride, page_size;
   uint32_t entry_stride_b;                 // bytes
   Divisor by_page, by_group, by_kv, by_tiles, by_head;  // page_size, q_per_kv, n_kv, n_tiles, n_tiles * n_splits
   uint32_t max_page;
@@ -566,32 +566,28 @@ __global__ __launch_bounds__(512, 2) void prefill_attn_kernel(const PrefillParam
 }
 
 // head_dim 256, whose output alone would take 128 registers of a wave in the kernel above, and pools that are
-// not 16-byte aligned, which direct loads to LDS are not specified for: 16 MT query
-// rows per wave and 16x16x32 MFMA, BN tokens per key tile (a multiple of 32), NW waves per workgroup.
+// not 16-byte aligned, which direct loads to LDS are not specified for: four waves of 16 query rows and
+// 16x16x32 MFMA, 32 tokens per key tile.
 // K/V tiles pass through registers into two LDS buffers per matrix, one barrier per tile; LDS rows are
 // padded by 32 bytes, which keeps the 16-byte K reads and the transposed V reads free of bank conflicts.
 // A step is a serial chain (scores, weights, values, barrier), so two workgroups share a compute unit: within
 // 256 registers (186) instead of 328 with accumulators copied between register files, whole tiles of 16
 // heads, bf16, take 45.1 us instead of 47.1 for 1000 tokens, 142 instead of 202 for 2900, 497 instead of
 // 751 for 6000.
-template <typename T, int D, int MT, int BN, int NW>
-__global__ __launch_bounds__(64 * NW, 2) void prefill_attn_staged_kernel(const PrefillParams p) {
-  constexpr int kThreads = 64 * NW;
-  constexpr int WR = 16 * MT;       // query rows per wavefront
+template <typename T, int D>
+__global__ __launch_bounds__(256, 2) void prefill_attn_staged_kernel(const PrefillParams p) {
+  constexpr int WR = 16;            // query rows per wavefront
   constexpr int NS = D / 32;        // 16-byte pieces of a Q/K row per lane (one MFMA each)
   constexpr int DC = D / 16;        // head dimensions per lane in the P.V product
   constexpr int PITCH = D + 16;     // LDS row pitch in elements: +32 bytes
   constexpr int CPR = D / 8;        // 16-byte chunks per row
-  constexpr int kPfBN = BN;
+  constexpr int BN = 32;            // tokens per key tile
   constexpr int NSUB = BN / 16;     // 16-token sub-tiles per key tile
-  constexpr int SR = kThreads / 8;  // staging: rows per pass (8 lanes per row piece)
-  constexpr int RPT = BN / SR;      // staging: rows per thread (row = tid / 8 + SR jr)
-  constexpr int CCT = CPR / 8;      // staging: chunks per thread and row (chunk = tid % 8 + 8 jc)
-  constexpr int CPT = RPT * CCT;    // chunks a thread stages per tile and matrix
+  constexpr int CPT = CPR / 8;      // staging: chunks per thread, tile and matrix (row = tid / 8,
+                                    // chunk = tid % 8 + 8 jc)
   static_assert(D % 64 == 0, "a thread stages whole pieces");
-  static_assert(BN % 32 == 0 && RPT >= 1 && CPT * kThreads == BN * CPR, "key tile");
   // two buffers per matrix: tile t + 1 is written while tile t is still being read
-  constexpr int TILE = kPfBN * PITCH;
+  constexpr int TILE = BN * PITCH;
   __shared__ __attribute__((aligned(16))) uint16_t ks[2 * TILE];
   __shared__ __attribute__((aligned(16))) uint16_t vs[2 * TILE];
 
@@ -605,34 +601,25 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_attn_staged_kernel(const P
   const bool whole = w.whole;
   const int q_off = p.kv_len - p.n_q;  // position of query token 0
 
-  // ---- Q operands: row (q0 + WR wave + 16 mt + r), pieces [32 s + 8 g, +8) ----------------------
-  u32x4 qb[MT][NS];
-  int qpos_of[MT];  // position of this lane's query row
+  // ---- Q operand: row (q0 + 16 wave + r), pieces [32 s + 8 g, +8) -------------------------------
+  int q_row = q0 + wave * WR + r;
+  q_row = q_row < p.n_rows ? q_row : p.n_rows - 1;
+  const int q_tok = q_row / p.by_group;
+  const int qpos = q_off + q_tok;  // position of this lane's query row
+  const u32x4* q_src = reinterpret_cast<const u32x4*>(
+      p.q + ((int64_t)q_tok * p.num_qo_heads + kvh * p.q_per_kv + (q_row - q_tok * p.q_per_kv)) * D);
+  u32x4 qb[NS];
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt) {
-    int row = q0 + wave * WR + mt * 16 + r;
-    row = row < p.n_rows ? row : p.n_rows - 1;
-    const int tok = row / p.by_group;
-    qpos_of[mt] = q_off + tok;
-    const u32x4* src = reinterpret_cast<const u32x4*>(
-        p.q + ((int64_t)tok * p.num_qo_heads + kvh * p.q_per_kv + (row - tok * p.q_per_kv)) * D);
-#pragma unroll
-    for (int s = 0; s < NS; ++s) qb[mt][s] = src[4 * s + g];
-  }
+  for (int s = 0; s < NS; ++s) qb[s] = q_src[4 * s + g];
 
-  f32x4 oacc[MT][DC];
-  float m_run[MT], l_run[MT];
+  f32x4 oacc[DC];
+  float m_run = kNegBig, l_run = 0.f;
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt) {
-    m_run[mt] = kNegBig;
-    l_run[mt] = 0.f;
-#pragma unroll
-    for (int d = 0; d < DC; ++d) oacc[mt][d] = f32x4{0.f, 0.f, 0.f, 0.f};
-  }
+  for (int d = 0; d < DC; ++d) oacc[d] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   // ---- staging: thread -> CPT chunks of K and of V per tile --------------------------------------
   // eight adjacent lanes move 128 contiguous bytes of one row (one cache line in, one conflict-free
-  // LDS write out); a thread looks up the page of each of its RPT rows once
+  // LDS write out); a thread looks up the page of its row once
   // Two register sets for keys: the loads of tile t + 2 are issued while tile t + 1 still waits in the
   // other set for its turn to be written to LDS, so its rows have two iterations to arrive.  Values have
   // one set and one iteration: a second set would not fit 256 registers, and with more a compute unit
@@ -641,54 +628,40 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_attn_staged_kernel(const P
   const int srow = tid >> 3, sl8 = tid & 7;
   // page ids are looked up one tile ahead of the rows they address, so that a tile's loads never wait
   // for a page-table load issued in the same iteration
-  uint32_t pg[RPT], pg_v[RPT];  // of the next tile of keys, of values
-  auto split_tok = [&](int kt, int jr, int& pg_i, int& entry) {
-    int tok = kt + srow + SR * jr;
+  uint32_t pg, pg_v;  // of the next tile of keys, of values
+  auto split_tok = [&](int kt, int& pg_i, int& entry) {
+    int tok = kt + srow;
     tok = tok < p.kv_len ? tok : p.kv_len - 1;
-    if (p.page_shift >= 0) {
-      pg_i = tok >> p.page_shift;
-      entry = tok & (p.page_size - 1);
-    } else {
-      pg_i = tok / p.by_page;
-      entry = tok - pg_i * p.page_size;
-    }
+    pg_i = tok / p.by_page;
+    entry = tok - pg_i * p.page_size;
   };
   auto lookup = [&](int kt) {
-#pragma unroll
-    for (int jr = 0; jr < RPT; ++jr) {
-      int pg_i, entry;
-      split_tok(kt, jr, pg_i, entry);
-      pg[jr] = (uint32_t)p.page_table[pg_i];
-    }
+    int pg_i, entry;
+    split_tok(kt, pg_i, entry);
+    pg = (uint32_t)p.page_table[pg_i];
   };
-  auto fetch = [&](int kt, const uint32_t (&pages)[RPT], int64_t matrix, u32x4 (&reg)[CPT]) {
+  auto fetch = [&](int kt, uint32_t page, int64_t matrix, u32x4 (&reg)[CPT]) {
+    int pg_i, entry;
+    split_tok(kt, pg_i, entry);
+    page = page > p.max_page ? p.max_page : page;
+    const uint16_t* src = p.kv + (matrix + (int64_t)page * p.page_stride + (int64_t)entry * p.entry_stride +
+                                  (int64_t)kvh * p.head_stride + sl8 * 8);
 #pragma unroll
-    for (int jr = 0; jr < RPT; ++jr) {
-      int pg_i, entry;
-      split_tok(kt, jr, pg_i, entry);
-      const uint32_t page = pages[jr] > p.max_page ? p.max_page : pages[jr];
-      const uint16_t* src = p.kv + (matrix + (int64_t)page * p.page_stride + (int64_t)entry * p.entry_stride +
-                                    (int64_t)kvh * p.head_stride + sl8 * 8);
-#pragma unroll
-      for (int jc = 0; jc < CCT; ++jc) reg[jr * CCT + jc] = *reinterpret_cast<const u32x4*>(src + jc * 64);
-    }
+    for (int jc = 0; jc < CPT; ++jc) reg[jc] = *reinterpret_cast<const u32x4*>(src + jc * 64);
   };
   auto fetch_v = [&](int kt) { fetch(kt, pg_v, p.v_offset, vreg); };
   auto fetch_k = [&](int kt, u32x4 (&kreg)[CPT]) {  // needs lookup(kt) before it; fetch_v(kt) comes after it
     fetch(kt, pg, 0, kreg);
-#pragma unroll
-    for (int jr = 0; jr < RPT; ++jr) pg_v[jr] = pg[jr];
-    lookup(kt + kPfBN);
+    pg_v = pg;
+    lookup(kt + BN);
   };
   auto stash = [&](int buf, const u32x4 (&kreg)[CPT]) {
 #pragma unroll
-    for (int jr = 0; jr < RPT; ++jr)
-#pragma unroll
-      for (int jc = 0; jc < CCT; ++jc) {
-        const int at = buf * TILE + (srow + SR * jr) * PITCH + (sl8 + 8 * jc) * 8;
-        *reinterpret_cast<u32x4*>(&ks[at]) = kreg[jr * CCT + jc];
-        *reinterpret_cast<u32x4*>(&vs[at]) = vreg[jr * CCT + jc];
-      }
+    for (int jc = 0; jc < CPT; ++jc) {
+      const int at = buf * TILE + srow * PITCH + (sl8 + 8 * jc) * 8;
+      *reinterpret_cast<u32x4*>(&ks[at]) = kreg[jc];
+      *reinterpret_cast<u32x4*>(&vs[at]) = vreg[jc];
+    }
   };
 
   // positions of the wave's first and last query row (a wave without rows sees no key tile)
@@ -696,92 +669,76 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_attn_staged_kernel(const P
   const int wave_first_pos = q_off + wave_row0 / p.by_group;
   const int wave_last_pos = wave_row0 < p.n_rows ? (p.causal ? q_off + (wave_row0 + WR - 1) / p.by_group : p.kv_len) : -1;
   auto compute = [&](int kt, int buf) {
-    // A wave whose last query row lies before the key tile sees none of it (causal).  Inside an
-    // active wave every query tile is computed: a tile that lies wholly before the key tile is
-    // masked to zero weight below, which happens once per wave, and the loop body stays free of
-    // branches around the matrix instructions.
+    // A wave whose last query row lies before the key tile sees none of it (causal).  In an active wave a
+    // row that lies wholly before the key tile is masked to zero weight below.
     if (kt <= wave_last_pos) {
-      // ---- S^T: each K operand is read once and used by every active query tile -----------------
+      // ---- S^T = K Q^T ---------------------------------------------------------------------------
       // (the two matrix phases run at raised wave priority: while one wave of a SIMD is in its
       // softmax arithmetic, the other's matrix instructions are issued first and keep the matrix
       // pipeline busy)
       __builtin_amdgcn_s_setprio(2);
-      f32x4 st[MT][NSUB];
+      f32x4 st[NSUB];  // raw q.k; the softmax scale is folded into the exponent below
 #pragma unroll
       for (int sub = 0; sub < NSUB; ++sub) {
         u32x4 ka[NS];
         const uint16_t* krow = &ks[buf * TILE + (sub * 16 + r) * PITCH + 8 * g];
 #pragma unroll
         for (int s = 0; s < NS; ++s) ka[s] = *reinterpret_cast<const u32x4*>(krow + 32 * s);
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt) {
-          f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-          for (int s = 0; s < NS; ++s) acc = mfma_16x16x32<T>(ka[s], qb[mt][s], acc);
-          st[mt][sub] = acc;  // raw q.k; the softmax scale is folded into the exponent below
-        }
+        for (int s = 0; s < NS; ++s) acc = mfma_16x16x32<T>(ka[s], qb[s], acc);
+        st[sub] = acc;
       }
       __builtin_amdgcn_s_setprio(0);
       // ---- online softmax of query row r (lanes r, r+16, r+32, r+48 share the row) ---------------
-      uint32_t pa[MT][NSUB][2];
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt) {
-        const int qpos = qpos_of[mt];
-        // the test of the wave's first query tile covers the second: masking a tile that does
-        // not need it changes nothing, and one rare branch keeps the position arithmetic out of
-        // the common path
-        const bool need_mask =
-            (p.causal && kt + kPfBN - 1 > wave_first_pos) || kt + kPfBN > p.kv_len;
-        if (need_mask) {
-          // the last token this row sees, counted from the lane's first one of the tile (opaque: the
-          // compiler would keep the 32 differences of the comparisons below in registers for the loop)
-          int lim = p.kv_len - 1;
-          if (p.causal && qpos < lim) lim = qpos;
-          lim -= kt + 4 * g;
-          asm volatile("" : "+v"(lim));
-#pragma unroll
-          for (int sub = 0; sub < NSUB; ++sub)
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-              st[mt][sub][i] = sub * 16 + i <= lim ? st[mt][sub][i] : kNegBig;
-        }
-        float mt_max = kNegBig;
+      if ((p.causal && kt + BN - 1 > wave_first_pos) || kt + BN > p.kv_len) {
+        // the last token this row sees, counted from the lane's first one of the tile (opaque: the
+        // compiler would keep the differences of the comparisons below in registers for the loop)
+        int lim = p.kv_len - 1;
+        if (p.causal && qpos < lim) lim = qpos;
+        lim -= kt + 4 * g;
+        asm volatile("" : "+v"(lim));
 #pragma unroll
         for (int sub = 0; sub < NSUB; ++sub)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) mt_max = fmaxf(mt_max, st[mt][sub][i]);
-        mt_max = rows_max(mt_max);
-        // m_run is kept in the scaled base-2 domain.  A masked entry (kNegBig) gives exp2(-huge) = 0 by
-        // itself, also in a tile that masks the whole row (a later piece of the keys may begin with
-        // one): the reference point never falls to where kNegBig lies.
-        // The running maximum only moves when the tile's maximum exceeds it by more than 2^8:
-        // softmax does not depend on the reference point, weights up to 256 are exact to the same
-        // relative precision, and the accumulator rescale below becomes rare.
-        const float m_tile = fmaxf(mt_max, kRowFloor) * p.scale_log2;
-        const float m_new = m_tile > m_run[mt] + 8.f ? m_tile : m_run[mt];
-        const float alpha = fast_exp2(m_run[mt] - m_new);
-        m_run[mt] = m_new;
-        float psum = 0.f;
+          for (int i = 0; i < 4; ++i) st[sub][i] = sub * 16 + i <= lim ? st[sub][i] : kNegBig;
+      }
+      float t_max = kNegBig;
 #pragma unroll
-        for (int sub = 0; sub < NSUB; ++sub) {
-          float pr[4];
+      for (int sub = 0; sub < NSUB; ++sub)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            pr[i] = fast_exp2(fmaf(st[mt][sub][i], p.scale_log2, -m_new));
-            psum += pr[i];
-          }
-          pa[mt][sub][0] = pack2<T>(pr[0], pr[1]);
-          pa[mt][sub][1] = pack2<T>(pr[2], pr[3]);
+        for (int i = 0; i < 4; ++i) t_max = fmaxf(t_max, st[sub][i]);
+      t_max = rows_max(t_max);
+      // m_run is kept in the scaled base-2 domain.  A masked entry (kNegBig) gives exp2(-huge) = 0 by
+      // itself, also in a tile that masks the whole row (a later piece of the keys may begin with
+      // one): the reference point never falls to where kNegBig lies.
+      // The running maximum only moves when the tile's maximum exceeds it by more than 2^8: softmax
+      // does not depend on the reference point, and the accumulator rescale below becomes rare.
+      const float m_tile = fmaxf(t_max, kRowFloor) * p.scale_log2;
+      const float m_new = m_tile > m_run + 8.f ? m_tile : m_run;
+      const float alpha = fast_exp2(m_run - m_new);
+      m_run = m_new;
+      uint32_t pa[NSUB][2];
+      float psum = 0.f;
+#pragma unroll
+      for (int sub = 0; sub < NSUB; ++sub) {
+        float pr[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          pr[i] = fast_exp2(fmaf(st[sub][i], p.scale_log2, -m_new));
+          psum += pr[i];
         }
-        l_run[mt] = fmaf(l_run[mt], alpha, psum);
-        // rescale: accumulator row 4g + i is query row 4g + i, whose factor sits in lane 4g + i
-        if (__ballot(alpha != 1.f)) {
+        pa[sub][0] = pack2<T>(pr[0], pr[1]);
+        pa[sub][1] = pack2<T>(pr[2], pr[3]);
+      }
+      l_run = fmaf(l_run, alpha, psum);
+      // rescale: accumulator row 4g + i is query row 4g + i, whose factor sits in lane 4g + i
+      if (__ballot(alpha != 1.f)) {
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const float f = __shfl(alpha, 4 * g + i, 64);
+        for (int i = 0; i < 4; ++i) {
+          const float f = __shfl(alpha, 4 * g + i, 64);
 #pragma unroll
-            for (int d = 0; d < DC; ++d) oacc[mt][d][i] *= f;
-          }
+          for (int d = 0; d < DC; ++d) oacc[d][i] *= f;
         }
       }
       __builtin_amdgcn_s_setprio(2);
@@ -791,20 +748,12 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_attn_staged_kernel(const P
       // block inside every 16 lanes: lane r points at the 8-byte piece r % 4 of token row r / 4
       // and receives dimension r of the four rows.
       const uint16_t* vlane = &vs[buf * TILE + (4 * g + (r >> 2)) * PITCH + 4 * (r & 3)];
+      const u32x4 pp = {pa[0][0], pa[0][1], pa[1][0], pa[1][1]};
 #pragma unroll
-      for (int pair = 0; pair < NSUB / 2; ++pair) {
-#pragma unroll
-        for (int a = 0; a < DC; ++a) {
-          const u32x2 t0 = lds_read_tr16(vlane + (32 * pair) * PITCH + 16 * a);
-          const u32x2 t1 = lds_read_tr16(vlane + (32 * pair + 16) * PITCH + 16 * a);
-          const u32x4 vb = {t0.x, t0.y, t1.x, t1.y};
-#pragma unroll
-          for (int mt = 0; mt < MT; ++mt) {
-            const u32x4 pp = {pa[mt][2 * pair][0], pa[mt][2 * pair][1], pa[mt][2 * pair + 1][0],
-                              pa[mt][2 * pair + 1][1]};
-            oacc[mt][a] = mfma_16x16x32<T>(pp, vb, oacc[mt][a]);
-          }
-        }
+      for (int a = 0; a < DC; ++a) {
+        const u32x2 t0 = lds_read_tr16(vlane + 16 * a);
+        const u32x2 t1 = lds_read_tr16(vlane + 16 * PITCH + 16 * a);
+        oacc[a] = mfma_16x16x32<T>(pp, u32x4{t0.x, t0.y, t1.x, t1.y}, oacc[a]);
       }
       __builtin_amdgcn_s_setprio(0);
     }
@@ -815,52 +764,48 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_attn_staged_kernel(const P
   fetch_k(k_begin, kreg_a);
   fetch_v(k_begin);
   stash(0, kreg_a);
-  if (k_begin + kPfBN < kv_end) fetch_k(k_begin + kPfBN, kreg_a);
+  if (k_begin + BN < kv_end) fetch_k(k_begin + BN, kreg_a);
   // One barrier per tile: it makes tile kt visible in its buffer, and it tells that every wave has
   // finished reading the other buffer, which the end of the step overwrites with tile kt + BN.
-  for (int kt = k_begin; kt < kv_end; kt += 2 * kPfBN) {
+  for (int kt = k_begin; kt < kv_end; kt += 2 * BN) {
     __syncthreads();
-    if (kt + kPfBN < kv_end) fetch_v(kt + kPfBN);
-    if (kt + 2 * kPfBN < kv_end) fetch_k(kt + 2 * kPfBN, kreg_b);
+    if (kt + BN < kv_end) fetch_v(kt + BN);
+    if (kt + 2 * BN < kv_end) fetch_k(kt + 2 * BN, kreg_b);
     compute(kt, 0);
-    if (kt + kPfBN >= kv_end) break;
+    if (kt + BN >= kv_end) break;
     stash(1, kreg_a);
     __syncthreads();
-    if (kt + 2 * kPfBN < kv_end) fetch_v(kt + 2 * kPfBN);
-    if (kt + 3 * kPfBN < kv_end) fetch_k(kt + 3 * kPfBN, kreg_a);
-    compute(kt + kPfBN, 1);
-    if (kt + 2 * kPfBN < kv_end) stash(0, kreg_b);
+    if (kt + 2 * BN < kv_end) fetch_v(kt + 2 * BN);
+    if (kt + 3 * BN < kv_end) fetch_k(kt + 3 * BN, kreg_a);
+    compute(kt + BN, 1);
+    if (kt + 2 * BN < kv_end) stash(0, kreg_b);
   }
 
   // ---- normalise and store (or leave the piece's partial result): lane holds rows 4g + i,
   //      dimensions 16 a + r ------------------------------------------------------------------------
+  const float l = rows_sum(l_run);
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt) {
-    const float l = rows_sum(l_run[mt]);
+  for (int i = 0; i < 4; ++i) {
+    const float li = __shfl(l, 4 * g + i, 64);
+    const int row = wave_row0 + 4 * g + i;
+    if (whole) {
+      const float inv = li > 0.f ? 1.f / li : 0.f;
+      if (row < p.n_rows) {
+        const int tok = row / p.by_group;
+        uint16_t* dst = p.o + ((int64_t)tok * p.num_qo_heads + kvh * p.q_per_kv + (row - tok * p.q_per_kv)) * D + r;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float li = __shfl(l, 4 * g + i, 64);
-      const int row = wave_row0 + mt * 16 + 4 * g + i;
-      if (whole) {
-        const float inv = li > 0.f ? 1.f / li : 0.f;
-        if (row < p.n_rows) {
-          const int tok = row / p.by_group;
-          uint16_t* dst =
-              p.o + ((int64_t)tok * p.num_qo_heads + kvh * p.q_per_kv + (row - tok * p.q_per_kv)) * D + r;
+        for (int a = 0; a < DC; ++a) dst[16 * a] = from_float<T>(oacc[a][i] * inv);
+      }
+    } else {
+      const float mi = __shfl(m_run, 4 * g + i, 64);
+      if (row < p.n_rows) {
+        const int64_t part = ((int64_t)split * p.n_kv + kvh) * p.n_rows + row;
+        float* dst = p.part_o + part * D + r;
 #pragma unroll
-          for (int a = 0; a < DC; ++a) dst[16 * a] = from_float<T>(oacc[mt][a][i] * inv);
-        }
-      } else {
-        const float mi = __shfl(m_run[mt], 4 * g + i, 64);
-        if (row < p.n_rows) {
-          const int64_t part = ((int64_t)split * p.n_kv + kvh) * p.n_rows + row;
-          float* dst = p.part_o + part * D + r;
-#pragma unroll
-          for (int a = 0; a < DC; ++a) dst[16 * a] = oacc[mt][a][i];
-          if (r == 0) {
-            p.part_ml[part * 2] = mi;
-            p.part_ml[part * 2 + 1] = li;
-          }
+        for (int a = 0; a < DC; ++a) dst[16 * a] = oacc[a][i];
+        if (r == 0) {
+          p.part_ml[part * 2] = mi;
+          p.part_ml[part * 2 + 1] = li;
         }
       }
     }
@@ -969,11 +914,11 @@ template <typename T>
 static int launch_prefill(const PrefillParams& p, int head_dim, bool oct, hipStream_t st) {
   const dim3 grid(p.n_tiles * p.n_kv * p.n_splits), block(p.staged ? 256 : 512);
   if (head_dim == 256)
-    hipLaunchKernelGGL((prefill_attn_staged_kernel<T, 256, 1, 32, 4>), grid, block, 0, st, p);
+    hipLaunchKernelGGL((prefill_attn_staged_kernel<T, 256>), grid, block, 0, st, p);
   else if (head_dim == 128 && p.staged)
-    hipLaunchKernelGGL((prefill_attn_staged_kernel<T, 128, 1, 32, 4>), grid, block, 0, st, p);
+    hipLaunchKernelGGL((prefill_attn_staged_kernel<T, 128>), grid, block, 0, st, p);
   else if (head_dim == 64 && p.staged)
-    hipLaunchKernelGGL((prefill_attn_staged_kernel<T, 64, 1, 32, 4>), grid, block, 0, st, p);
+    hipLaunchKernelGGL((prefill_attn_staged_kernel<T, 64>), grid, block, 0, st, p);
   else if (head_dim == 128 && oct)
     hipLaunchKernelGGL((prefill_attn_kernel<T, 128, true>), grid, block, 0, st, p);
   else if (head_dim == 128)
@@ -1106,7 +1051,6 @@ extern "C" int td_prefill_attn_split(const td_paged_kv* kv, const int32_t* page_
   p.entry_stride = kv->layout == TD_NHD ? H * D : D;
   p.head_stride = kv->layout == TD_NHD ? D : P * D;
   p.page_size = P;
-  p.page_shift = (P & (P - 1)) == 0 ? __builtin_ctz(P) : -1;
   p.entry_stride_b = (uint32_t)(p.entry_stride * 2);
   const bool oct = P % 8 == 0;
   p.by_page = divisor(P);

@@ -302,3 +302,17 @@ def test_pool_that_is_not_16_byte_aligned(cuda, d, page, causal, off):
                                                    case.last_page_len, causal, 0, False, 1.0, 1e4).float().cpu()
         want = _dense(q, case.k, case.v, causal)
         assert ((got - want).abs() <= ATOL[dtype] * want.abs().clamp(min=1.0)).all(), (kv_len, n_q)
+
+
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("hq,hkv,d,page", [(4, 4, 128, 16), (14, 2, 64, 3), (8, 1, 128, 1), (3, 1, 64, 32)])
+def test_caches_of_one_key_tile(cuda, hq, hkv, d, page, causal):
+    """Around 32 and 64 keys, where the kernel changes: fresh prompts, and a few rows on cached tokens."""
+    dtype = torch.float16
+    for kv_len in (1, 2, 15, 31, 32, 33, 63, 64, 65):
+        case = PagedCase(kv_len, hkv, d, page, dtype, seed=kv_len)
+        for n_q in {kv_len, 1, min(kv_len, 17)}:
+            q = randn((n_q, hq, d), kv_len * 3 + n_q, dtype)
+            got = _run(cuda, case, q, causal, dtype).float().cpu()
+            want = _dense(q, case.k, case.v, causal)
+            assert ((got - want).abs() <= ATOL[dtype] * want.abs().clamp(min=1.0)).all(), (kv_len, n_q)

@@ -565,8 +565,8 @@ __global__ __launch_bounds__(512, 2) void prefill_attn_kernel(const PrefillParam
   }
 }
 
-// head_dim 256, whose output alone would take 128 registers of a wave in the kernel above, and pools that are
-// not 16-byte aligned, which direct loads to LDS are not specified for: four waves of 16 query rows and
+// head_dim 256, whose output alone would take 128 registers of a wave in the kernel above; caches of up to 64
+// tokens; and pools that are not 16-byte aligned, which direct loads to LDS are not specified for: four waves of 16 query rows and
 // 16x16x32 MFMA, 32 tokens per key tile.
 // K/V tiles pass through registers into two LDS buffers per matrix, one barrier per tile; LDS rows are
 // padded by 32 bytes, which keeps the 16-byte K reads and the transposed V reads free of bank conflicts.
@@ -985,7 +985,10 @@ static void plan_prefill(const td_paged_kv* kv, int32_t kv_len, int32_t n_q, int
   p.n_rows = n_q * p.q_per_kv;
   p.n_q = n_q;
   p.causal = causal;
-  p.staged = D == 256 || ((uintptr_t)kv->data & 15) != 0;
+  // Up to one key tile of the eight-wave kernel there is nothing to overlap, and its rings and phases cost more
+  // than they give: 32 heads of 128, 16 tokens 6.5 us against 4.4 (64 dimensions 5.5 against 4.0), 33 6.6 against
+  // 4.9, 64 6.5 against 5.4.
+  p.staged = D == 256 || kv_len <= 64 || ((uintptr_t)kv->data & 15) != 0;
   const int bn = p.staged ? 32 : 64, max_tiles = (kv_len + bn - 1) / bn;
   const int64_t cus = td_num_cus();
   double best = 0.0;

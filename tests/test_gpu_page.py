@@ -503,3 +503,35 @@ def test_rope_append_prompt_refuses_a_page_list_it_cannot_read(cuda):
         _kernels.rope_append_prompt(qkv, 1, 0, pool, table, ends, 4, 0)
     with pytest.raises(RuntimeError, match="ends of the page list"):
         _kernels.rope_append_prompt(qkv, 1, 0, pool, table, ends[:1].to(cuda), 4, 0)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("d", [64, 128, 256])
+def test_rope_kernels_agree_to_the_last_place(cuda, dtype, d):
+    """Aligned rows, unaligned rows, and the decode launch with one sequence per token: one unit in the last place, and
+    what the fp32 roundings of two products and of sin and cos leave of a sum that cancels (values up to 5).  The
+    prompt launch that appends equals the aligned one bit by bit, see above."""
+    from tidaldecode_amd import _kernels
+
+    n, hq, hkv, past = 37, 3, 2, 5000
+    q, k = (randn((n, h, d), h, dtype).to(dtype).to(cuda) for h in (hq, hkv))
+    outs = []
+    for off in (0, 1):
+        pair = []
+        for x in (q, k):
+            buf = torch.zeros(x.numel() + 8, dtype=dtype, device=cuda)
+            pair.append(buf[off: off + x.numel()].view(x.shape).copy_(x))
+        _kernels.apply_rope_in_place(*pair, past, 1.0, 1e4)
+        outs.append(pair)
+    ulp = 2.0 ** -10 if dtype == torch.float16 else 2.0 ** -7
+
+    def close(a, b):
+        a, b = a.double(), b.double()
+        return bool(((a - b).abs() <= ulp * a.abs() + 8 * 5 * 2.0 ** -24).all())
+
+    assert close(outs[0][0], outs[1][0]) and close(outs[0][1], outs[1][1])
+    pool = torch.zeros((n, 2, 1, hkv, d), dtype=dtype, device=cuda)
+    slots = torch.arange(n, dtype=torch.int32, device=cuda)
+    q_step = q.clone()
+    _kernels.rope_append_decode(q_step, k, k, pool, slots + past, slots, 0)
+    assert close(q_step, outs[0][0]) and close(pool[:, 0, 0], outs[0][1])

@@ -57,7 +57,10 @@ __device__ __forceinline__ void rope_sincos(double pos_over_scale, double log2_t
   sincospif((float)(2.0 * turns), &sn, &cs);
 }
 
-// one pair turned; every kernel rounds the same two products, so their results agree bit by bit
+// one pair turned, with the same product rounded in every kernel of this file; with and without APPEND
+// rope_prompt_kernel agrees bit by bit.  Other kernels may differ from it, and from each other, in the last
+// place: the compiler contracts the angle's products, and in the attention kernels that turn a token
+// themselves the pair's, as it finds best in each.
 __device__ __forceinline__ void turn(float lo, float hi, float sn, float cs, float& out_lo, float& out_hi) {
   out_lo = fmaf(lo, cs, -(hi * sn));
   out_hi = fmaf(lo, sn, hi * cs);
@@ -77,9 +80,10 @@ __device__ __forceinline__ void rotate_pair(uint16_t* row, int j, int half, floa
 // in flight while it turns the present ones; the angles, which need double precision, are formed once
 // per token and shared through LDS.  TOK tokens per workgroup: as many as 256 threads form angles for
 // at once when the tokens fill the chip anyway, one otherwise.
-// In place, bf16, D = 128, against 2-byte accesses (rope_kernel): 300 tokens x 32 / 8 heads 4.6 -> 3.1 us,
-// 2900 x 32 / 32 20.2 -> 14.8, 32768 x 32 / 32 244 -> 204 (5.3 TB/s).  APPEND against a split of the
-// projection, RoPE and append, 2900 x 32 / 32: 60-66 -> 22.3 us (6.4 TB/s).
+// In place, bf16, D = 128, against 2-byte accesses (rope_kernel), replayed on the same tensors: 300 tokens x
+// 32 / 8 heads 4.6 -> 3.1 us, 2900 x 32 / 32 20.2 -> 14.8, 32768 x 32 / 32 244 -> 204 (5.3 TB/s).  APPEND
+// against a split of the projection, RoPE and append, 2900 x 32 / 32: 60-66 -> 22.3 us (6.4 TB/s) in the same
+// way; inside a decoder's prefill, where other kernels have used the caches in between, 24.7.
 struct RopePrompt {
   const uint16_t *q, *k, *v;  // token rows, heads adjacent; v with APPEND only
   int64_t q_stride, k_stride, v_stride;
@@ -375,7 +379,8 @@ __device__ __forceinline__ float rms_block_sum(float ss) {
 // Threads past the end of the row reload the row's last chunk (an unconditional load keeps all
 // loads in flight together; a predicated one is waited for inside its branch) and drop it.
 // ADD: x + delta, rounded to the storage type, goes back to x and is what the norm is taken of; the
-// residual addition of a layer so costs no pass of its own (2900 x 4096 bf16: 20.0 -> 14.9 us for both).
+// residual addition of a layer so costs no pass of its own (2900 x 4096 bf16: 20.0 -> 14.9 us for both replayed
+// on the same tensors, 16.2 inside a decoder's prefill).
 template <typename T, int CH, bool ADD>
 __global__ __launch_bounds__(256) void rms_norm_vec_kernel(uint16_t* x, const uint16_t* delta, const uint16_t* w,
                                                            uint16_t* out, int cols, float eps) {
@@ -474,8 +479,8 @@ static void launch_rms_norm(void* x, const void* delta, const void* weight, void
 
 // The gated MLP's activation over a prompt: out = silu(gate) * up, silu rounded to the storage type
 // first as the model does it.  Bound by memory: [gate | up] is read once and the product written once,
-// where element-wise operators write silu(gate) and read it again (2900 x 11008 bf16: 78 -> 32 us,
-// 5.9 TB/s).  VEC: eight elements per thread; other widths and alignments take one.
+// where element-wise operators write silu(gate) and read it again (2900 x 11008 bf16: 78 -> 32 us replayed
+// on the same tensors; 41.8 us, 4.6 TB/s, inside a decoder's prefill).  VEC: eight elements per thread; other widths and alignments take one.
 template <typename T, bool VEC>
 __global__ __launch_bounds__(256) void silu_mul_kernel(const uint16_t* gate_up, uint16_t* out, int cols) {
   const uint16_t* gate = gate_up + (int64_t)blockIdx.x * 2 * cols;

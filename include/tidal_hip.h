@@ -459,8 +459,8 @@ int td_prefill_attn(const td_paged_kv* kv, const int32_t* page_table, int32_t n_
  * td_prefill_attn with scratch: where a few query rows leave the chip idle (a further turn on a long
  * cache, a short prompt) their keys are cut into pieces that several workgroups walk side by side and
  * a second launch adds up.  workspace: td_prefill_workspace_bytes(...) bytes of device memory (16-byte
- * aligned, any contents; 0 bytes: the call does not split), to be used by one call at a time.  With less
- * or NULL it runs as td_prefill_attn does.  Interface replaced: bsk_ops.h:80-88; the reference's kernel
+ * aligned, any contents, at most 256 MB; 0 bytes: the call does not split; asked for with the same kv as
+ * the call), to be used by one call at a time.  With less or NULL it runs as td_prefill_attn does.  Interface replaced: bsk_ops.h:80-88; the reference's kernel
  * splits the keys through its handler's workspace (kernels/include/prefill/prefill.cuh:674-870).
  */
 int64_t td_prefill_workspace_bytes(const td_paged_kv* kv, int32_t kv_len, int32_t n_q,

@@ -60,7 +60,7 @@ def _check_i32(x: torch.Tensor, name: str) -> None:
 
 
 def _stream() -> int:
-    # torch.cuda.current_stream().cuda_stream without building the Stream object (1.5 us a call)
+    # torch.cuda.current_stream().cuda_stream without building the Stream object (2.8 us a call against 0.2)
     return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 

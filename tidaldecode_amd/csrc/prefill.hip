@@ -3,9 +3,10 @@
 // (kernels/include/prefill/prefill.cuh:674-870, bound in tidal/ops/csrc/batch_prefill.cu:27-117).
 //
 // What bounds it.  A long prompt is a contraction (4 n^2 / 2 flops per head dimension and head), so the
-// matrix cores; but per 64 keys and 32 query rows the softmax costs a wave about as long as the two
-// products (1000 cycles of exp2, fma and pack against 1030 of MFMA), so the two have to run at the same
-// time.  A short prompt or a further turn on a long cache has few query rows and is bound by how many
+// matrix cores; but per 64 keys and 32 query rows the softmax costs a wave nearly as much as the two
+// products (some 130 instructions of exp2, fma and pack, exp2 at a quarter of the rate, against 1024 cycles of
+// MFMA), so the two have to run at the same time: 1567 cycles pass per wave and tile, the matrix cores being
+// busy for 65 % of them.  A short prompt or a further turn on a long cache has few query rows and is bound by how many
 // CUs have work at all.  Hence:
 //   - The query rows of all heads of a KV head are packed into one list of rows (token * group + head),
 //     cut into workgroup tiles of up to 256: grouped heads share every staged key, and 16 new tokens of four
@@ -22,11 +23,11 @@
 // (measured), so those 16 lanes must hit 16 different bank groups.  head_dim 128: four rows form a block
 // of 1024 + 16 bytes and piece p of row r lies at p ^ 4 (r % 4); head_dim 64: rows of 128 bytes, pieces
 // of K at p ^ ((r / 2) % 8), of V (read transposed, eight bytes a lane) at p ^ 4 ((r / 2) % 2).
-// Measured (bf16, pages of 16, us, before with one 128- or 256-row tile per query head and 16x16x32
-// MFMA -> now): prompt of 32768 x 32 heads 9168 -> 7059 (1246 TFLOP/s; the largest library GEMM reaches
-// 1560 here), 8192 x 32 over 8 KV heads 586 -> 462, 1000 x 32 38 -> 23, 300 x 32 14.7 -> 10.2 (bound by
-// the latency of its five key tiles and cold code); 500 new tokens on 32768 cached ones, 32 heads
-// 992 -> 254, over 8 KV heads 992 -> 242; 16 tokens, 8 KV heads 794 -> 32.
+// Measured in turn on one card (bf16, pages of 16, us, before with one 128- or 256-row tile per query head and
+// 16x16x32 MFMA -> now): prompt of 32768 x 32 heads 8633 -> 7592 (1159 TFLOP/s; a 16384^3 library GEMM reached
+// 1332 in the same run, and cards differ by 7 %), 8192 x 32 over 8 KV heads 588 -> 495, 1000 x 32 36.6 -> 24.0,
+// 300 x 32 14.1 -> 10.6 (bound by the latency of its five key tiles and cold code); 500 new tokens on 32768
+// cached ones, 32 heads 991 -> 285, over 8 KV heads 993 -> 252; 16 tokens, 8 KV heads 792 -> 33.
 // Rows past the end of the sequence are clamped (never out of the pool) and masked.
 
 #include <type_traits>
@@ -159,7 +160,7 @@ __device__ __forceinline__ bool prefill_piece(const PrefillParams& p, PrefillPie
 // head_dim 64 and 128: eight waves, 32 query rows each, key tiles of 64 tokens.
 // OCT: pages hold a multiple of eight tokens, so eight aligned tokens share a page: one page lookup per
 // wave and tile, made 64 tiles at a time.  Other page sizes look up a page per row (8192 x 28 heads
-// over 4: 480 us at pages of 1 and 454 at 4 against 403 at 16).
+// over 4: 477 us at pages of 1 and 476 at 4 against 441 at 16).
 template <typename T, int D, bool OCT>
 __global__ __launch_bounds__(512, 2) void prefill_attn_kernel(const PrefillParams p) {
   constexpr int BN = 64, NS = D / 16, DB = D / 32;
@@ -864,15 +865,19 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(const PrefillParams 
 // few query rows on a long cache (a further turn of a conversation) leave most of the chip idle however
 // many keys there are, and so do a short prompt and a prompt of few heads.  Pieces shorten the walk for the
 // price of a merge; smaller row tiles (waves without rows compute nothing) give more workgroups, each with a
-// SIMD per wave, and so a shorter step.  The estimate, in steps of a full workgroup (64 keys, 1.2 us): the
-// chip runs `slots` workgroups at a time (one of eight waves per CU, two of four); a workgroup of 256, 128
-// or 64 rows costs 1, 0.87 or 0.83 per key tile and 6.5 or 4.5 to start (page table, queries, first tiles,
-// cold code, diagonal), all measured; causal tiles start longest first, which leaves a tail of about a
-// quarter of the longest; pieces cost the merge launch (two) and their fp32 round trip through memory.
-// Measured at head_dim 128, pages of 16, us for tiles of 256 / 128 / 64 rows, whole: prompts of 32 heads
-// over 8 KV heads, 100 tokens 9.6 / 8.7 / 7.5, 300 14.0 / 11.7 / 10.5, 640 21 / 17.0 / 15.5, 1000 27 / 23 / 27,
-// 2000 48 / 47 / 80, 2900 75 / 92 / 152.  Pieces against whole tiles of 256: 500 rows of 32 heads on 32768
-// keys 254 against 600.
+// SIMD per wave, and so a shorter step.  The estimate, in steps of a full workgroup (at head_dim 128 64 keys and
+// 1.2 us, at 256 32 keys and 1.3 us): the chip runs `slots` workgroups at a time (one of eight waves per CU,
+// two of four); a workgroup of 256, 128 or 64 rows costs 1, 0.87 or 0.83 per key tile and 6.5 or 4.5 to start
+// (page table, queries, first tiles, cold code, diagonal), all measured at head_dim 128; causal tiles start
+// longest first, which leaves a tail of about a quarter of the longest; pieces cost the merge launch (two) and
+// their fp32 round trip through memory.
+// Measured with pages of 16, us for tiles of 256 / 128 / 64 rows, whole: prompts of 32 heads over 8 KV heads of
+// 128, 150 tokens 11.9 / 9.8 / 9.3, 300 14.8 / 12.7 / 11.4, 640 22.7 / 18.5 / 17.4, 1000 30 / 25 / 28, 2000
+// 54 / 50 / 83, 2900 81 / 96 / 157; of 64, 300 10.6 / 9.5 / 9.0, 1000 21 / 18 / 21, 2000 38 / 35 / 60, 2900
+// 54 / 68 / 112.  Pieces against whole tiles of 256: 500 rows of 32 heads of 128 on 32768 keys 272 against 670.
+// Against the best of the tile sizes and eight piece counts, the choice took 1.03 times as long at 64 and at 128
+// dimensions (51 and 34 shapes of 16 to 6000 rows, no keys to 32768 before them) and 1.01 at 256 (68 shapes),
+// at worst 1.19, 1.12 and 1.12.
 static double prefill_cost(const PrefillParams& p, double tile, int64_t tiles, int64_t jobs, int64_t c) {
   const int64_t slots = (int64_t)td_num_cus() * (p.staged ? 2 : 1);
   const double start = p.bm == 256 ? 6.5 : 4.5;

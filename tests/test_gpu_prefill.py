@@ -180,6 +180,11 @@ def test_row_packing_rings_and_pieces(cuda, dtype, hq, hkv, d, page, kv_len, n_q
         q = (q * torch.linspace(0.5, rise, n_q)[:, None, None]).to(dtype).float()
     planned = lib.td_prefill_workspace_bytes(_kernels._pool(case.pool.to(cuda), case.layout), kv_len, n_q, hq, 1)
     assert (planned > 0) == pieces
+    if rise:   # some row's weights of its second to fourth key tile do exceed its first tile's by 2^8
+        logit = torch.einsum("qhd,khd->hqk", q, case.k[:256].repeat_interleave(hq // hkv, 1)) / math.sqrt(d)
+        logit = logit.masked_fill(torch.arange(logit.size(2)) > torch.arange(kv_len - n_q, kv_len)[:, None], -1e30)
+        late = logit[..., 64:].amax(-1) - logit[..., :64].amax(-1)
+        assert late.max().item() * math.log2(math.e) > 8.0
     got = _run(cuda, case, q, True, dtype).float().cpu()
     want = _dense(q, case.k, case.v, True)
     assert ((got - want).abs() <= ATOL[dtype] * want.abs().clamp(min=1.0)).all()

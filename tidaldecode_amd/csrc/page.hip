@@ -195,8 +195,8 @@ static void launch_rope_prompt(const PoolGeom& g, const RopePrompt& p, int D, in
 #undef TD_ROPE
 }
 
-// Rows that are not 16-byte aligned (rope_prompt_kernel cannot read them).  grid: n_tokens; block: 256 threads = (D/2 pair columns) x
-// (512/D head slots)
+// Rows that are not 16-byte aligned (rope_prompt_kernel cannot read them).  grid: n_tokens; block: 256
+// threads = (D/2 pair columns) x (512/D head slots)
 template <typename T>
 __global__ __launch_bounds__(256) void rope_kernel(uint16_t* q, uint16_t* k, int n_tokens, int Hq,
                                                    int Hkv, int D, double past_len,
@@ -480,7 +480,8 @@ static void launch_rms_norm(void* x, const void* delta, const void* weight, void
 // The gated MLP's activation over a prompt: out = silu(gate) * up, silu rounded to the storage type
 // first as the model does it.  Bound by memory: [gate | up] is read once and the product written once,
 // where element-wise operators write silu(gate) and read it again (2900 x 11008 bf16: 78 -> 32 us replayed
-// on the same tensors; 41.8 us, 4.6 TB/s, inside a decoder's prefill).  VEC: eight elements per thread; other widths and alignments take one.
+// on the same tensors; 41.8 us, 4.6 TB/s, inside a decoder's prefill).  VEC: eight elements
+// per thread; other widths and alignments take one.
 template <typename T, bool VEC>
 __global__ __launch_bounds__(256) void silu_mul_kernel(const uint16_t* gate_up, uint16_t* out, int cols) {
   const uint16_t* gate = gate_up + (int64_t)blockIdx.x * 2 * cols;

@@ -567,8 +567,8 @@ __global__ __launch_bounds__(512, 2) void prefill_attn_kernel(const PrefillParam
 }
 
 // head_dim 256, whose output alone would take 128 registers of a wave in the kernel above; caches of up to 64
-// tokens; and pools that are not 16-byte aligned, which direct loads to LDS are not specified for: four waves of 16 query rows and
-// 16x16x32 MFMA, 32 tokens per key tile.
+// tokens; and pools that are not 16-byte aligned, which direct loads to LDS are not specified for: four waves of
+// 16 query rows and 16x16x32 MFMA, 32 tokens per key tile.
 // K/V tiles pass through registers into two LDS buffers per matrix, one barrier per tile; LDS rows are
 // padded by 32 bytes, which keeps the 16-byte K reads and the transposed V reads free of bank conflicts.
 // A step is a serial chain (scores, weights, values, barrier), so two workgroups share a compute unit: within

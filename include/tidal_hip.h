@@ -387,10 +387,11 @@ int td_topk_bounded(const void* values, int32_t values_dtype, int64_t values_str
                     int64_t workspace_bytes, void* stream);
 
 /*
- * Bytes of device scratch for td_topk.  Rows of up to 65536 elements never touch it (one launch,
- * every workgroup of a row selects on the whole row and emits a slice).  A few longer rows are
- * shared between workgroups through it (three launches; about 56 KiB per row); without it (NULL),
- * or with many long rows, the one-launch kernel re-reads such rows from L2 in every pass.  The
+ * Bytes of device scratch for td_topk.  Rows of up to 65536 elements never touch it, nor do rows of
+ * up to 262144 whose selection fits the list of the one-pass kernel (k up to about 5800).  Larger
+ * selections from a few long rows are shared between workgroups through it (three launches; about
+ * 56 KiB per row); without it (NULL), or with many long rows, every workgroup goes through the whole
+ * row, read again from L2 in every pass.  The
  * scratch must be zero-filled once before its first use; every call leaves it ready for the next.
  * Plays the part of the `buf` argument of topk_filtering (tidal/utils/controller.py:164-168).
  */

@@ -1,0 +1,87 @@
+"""GPU parity of the one-pass top-k (csrc/topk_filter.cuh): rows of up to 262144 scores whose
+selection fits its list.  Everything is bit-exact against the oracle's stable rule."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _run(cuda, v, k, *, bound=None, in_idx=None, table=None, page=1, lengths=None, vals=True, pad=0, skew=0):
+    """v on the host; `pad` extra columns between rows and `skew` elements in front of the first row move
+    the rows' addresses."""
+    from tidaldecode_amd import _kernels
+
+    rows, n = v.shape
+    flat = torch.full((skew + rows * (n + pad) + 1,), float("nan"), dtype=v.dtype, device=cuda)
+    dev = flat[skew: skew + rows * (n + pad)].view(rows, n + pad)[:, :n]
+    dev.copy_(v)
+    out = torch.full((rows, k), -1, dtype=torch.int32, device=cuda)
+    out_v = torch.zeros((rows, k), dtype=v.dtype, device=cuda) if vals else None
+    to = lambda t: None if t is None else t.to(cuda)
+    _kernels.topk_filtering(dev, to(in_idx), out_v, out, None, k, page_table=to(table), page_size=page,
+                            lengths=to(lengths), upper_bound=to(bound))
+    torch.cuda.synchronize()
+    return out.cpu().long(), None if out_v is None else out_v.cpu()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("n,k", [(1, 1), (3, 2), (255, 17), (1019, 300), (1020, 1020), (1021, 1), (2047, 2000),
+                                 (2049, 511), (4099, 64), (8191, 8191), (8192, 700), (8193, 4096), (16383, 5),
+                                 (32771, 2048), (65535, 1024), (65537, 4096), (131073, 3), (262143, 4096)])
+def test_edges_of_the_sizes(cuda, dtype, n, k):
+    from oracle import tidal_oracle as orc
+
+    g = torch.Generator().manual_seed(n * 7 + k)
+    v = torch.randn((3, n), generator=g).to(dtype)
+    want = orc.stable_topk(v.float(), k)
+    lse = torch.logsumexp(v.float(), 1)
+    for bound, pad, skew in ((None, 0, 0), (lse, 1, 0), (lse, 2, 1), (None, 3, 3)):
+        got, vals = _run(cuda, v, k, bound=bound, pad=pad, skew=skew)
+        assert torch.equal(got, want), (pad, skew)
+        assert torch.equal(vals, torch.gather(v, 1, want))
+
+
+@pytest.mark.parametrize("n,k,page", [(700, 90, 16), (700, 90, 7), (5001, 600, 1), (5001, 600, 48), (40003, 2000, 5),
+                                      (70001, 1500, 16)])
+def test_payloads_and_lengths(cuda, n, k, page):
+    from oracle import tidal_oracle as orc
+
+    g = torch.Generator().manual_seed(n + page)
+    groups, per = 3, 2
+    v = torch.randn((groups * per, n), generator=g)
+    lens = [n, max(1, n // 3), max(1, k // 2)]
+    n_pages = -(-n // page)
+    tables = torch.stack([torch.randperm(n_pages + 5, generator=g)[:n_pages] for _ in range(groups)]).int()
+    got, _ = _run(cuda, v, k, table=tables, page=page, lengths=torch.tensor(lens, dtype=torch.int32), vals=False)
+    for r in range(groups * per):
+        ln = lens[r // per]
+        pos = orc.stable_topk(v[r: r + 1, :ln], min(k, ln))[0]
+        want = tables[r // per].long()[pos // page] * page + pos % page
+        assert torch.equal(got[r, : len(want)], want) and (got[r, len(want):] == -1).all(), r
+    payload = torch.randint(0, 1 << 30, v.shape, generator=g, dtype=torch.int32)
+    got, _ = _run(cuda, v, k, in_idx=payload)
+    assert torch.equal(got, torch.gather(payload.long(), 1, orc.stable_topk(v, k)))
+
+
+@pytest.mark.parametrize("n,k", [(20000, 2048), (6000, 700), (100001, 4000)])
+def test_samples_that_mislead(cuda, n, k):
+    """The sampled elements all larger than the rest (the first threshold keeps too few), all smaller
+    (it keeps everything: more than the list holds), and rows of a few values only."""
+    from oracle import tidal_oracle as orc
+
+    g = torch.Generator().manual_seed(n)
+    threads = 512 if n <= 8192 else 1024
+    quads, lines = threads // 4, (-(-n // 4)) >> 2
+    at = (torch.arange(quads) * lines // quads)[:, None] * 16 + torch.arange(16)[None]
+    at = at.flatten()
+    high, low = torch.randn((2, n), generator=g), torch.randn((2, n), generator=g)
+    high[:, at] += 50.0
+    low[:, at] -= 50.0
+    few = torch.randint(0, 3, (2, n), generator=g).float()
+    one = torch.full((1, n), -2.5)
+    nan = torch.randn((2, n), generator=g)
+    nan[:, at[::3]] = float("nan")
+    nan[1, ::5] = float("inf")
+    for v in (high, low, few, one, nan):
+        got, _ = _run(cuda, v, k, vals=False)
+        assert torch.equal(got, orc.stable_topk(v, k))

@@ -6,12 +6,15 @@
 // equal to T.  Ties go to the lower position and each output row is sorted by position: the
 // result is a pure function of the input row.  -0 equals +0, every NaN ranks above +inf.
 //
-// Two routes:
+// Three routes:
+//   * topk_filter_kernel (topk_filter.cuh), one launch, one workgroup per row, every element touched
+//     once: rows of up to 262144 elements whose selection fits its list (k up to about 5800, any k up
+//     to 8192 elements);
 //   * topk_slice_kernel, one launch: every workgroup (1024 threads) of a row runs the selection on
-//     the whole row -- up to 64K elements from registers -- and emits its own slice of it.  All
-//     rows of up to 65536 elements, and longer ones when there are many rows or no scratch.
+//     the whole row -- up to 64K elements from registers -- and emits its own slice of it.  Larger
+//     selections, and longer rows when there are many of them or no scratch;
 //   * topk_coop_{hist,select,emit}_kernel, three launches over a zeroed scratch: the workgroups of
-//     a row share the row.  A few rows of more than 65536 elements.
+//     a row share the row.  Larger selections from a few rows of 65537 to 262144 elements.
 //
 // Replaces decode_select_k (kernels/include/topk/decode_select_k.cuh:25-62 of the reference),
 // which launches RAFT's radix_topk_one_block_kernel, one 512-thread block per head.
@@ -38,6 +41,7 @@ struct TopkParams {
   const int32_t* len_arr;     // per row group: elements that take part (clamped to 1..len), or null
   int32_t page_size;
   int32_t page_shift;  // log2(page_size) when it is a power of two, else -1
+  uint32_t page_magic; // (2^32 - 1) / page_size
   void* out_values;
   int32_t* out_idx;
   int64_t out_stride;
@@ -48,6 +52,11 @@ struct TopkParams {
 __device__ __forceinline__ const int32_t* table_of(const TopkParams& p, int row) {
   if (p.page_table == nullptr || p.page_table_stride == 0) return p.page_table;
   return p.page_table + (int64_t)(row / p.rows_per_table) * p.page_table_stride;
+}
+// where the row's output starts
+template <typename E>
+__device__ __forceinline__ E* out_row(const TopkParams& p, E* base, int row) {
+  return base + (int64_t)row * p.out_stride;
 }
 // elements of this row that take part, and how many of them are selected
 __device__ __forceinline__ int row_len(const TopkParams& p, int row) {
@@ -548,9 +557,8 @@ __global__ __launch_bounds__(kTopkThreads) void topk_coop_emit_kernel(const Topk
     const uint32_t kv = coop_key<T>(vals, i < len ? i : len - 1);
     key[j] = i < len ? kv : 0u;  // 0 lies below every real key
   }
-  int32_t* out_idx = p.out_idx + (int64_t)row * p.out_stride;
-  elem_t* out_val =
-      p.out_values ? reinterpret_cast<elem_t*>(p.out_values) + (int64_t)row * p.out_stride : nullptr;
+  int32_t* out_idx = out_row(p, p.out_idx, row);
+  elem_t* out_val = p.out_values ? out_row(p, reinterpret_cast<elem_t*>(p.out_values), row) : nullptr;
   // Payloads and values of every element are fetched right away, unconditionally (they sit in
   // L2): together with the keys they are one round trip, and no load follows a store (vector
   // loads and stores complete in order on one counter).
@@ -770,19 +778,16 @@ constexpr int kStream = 16;               // loads in flight per thread where a 
 constexpr int kOwn = 8;                   // runs of a slice that stay in registers for the emission
 constexpr uint32_t kNoElement = ~0u;      // d of the slots past the end of the row: beyond every window
 
+// The runs j_lo .. j_lo + rps - 1 of a row's output, by a workgroup that selects from the whole row.
 template <typename T, int IPT>
-__global__ __launch_bounds__(kTopkThreads) void topk_slice_kernel(const TopkParams p, int n_slices,
-                                                                  int rps, int rows) {
+__device__ __forceinline__ void select_slice(const TopkParams& p, int row, int j_lo, int rps, SliceLds& L) {
   typedef typename ElemOf<T>::type elem_t;
-  int slice, row;
-  if (!coop_decode(n_slices, rows, slice, row)) return;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int len = row_len(p, row);
   const int k = row_k(p, len);
   const elem_t* vals = reinterpret_cast<const elem_t*>(p.values) + (int64_t)row * p.values_stride;
   const int nruns = (len + kTopkThreads - 1) / kTopkThreads;
-  const int j_lo = slice * rps;
   if (j_lo >= nruns) return;  // a slice past the end of a short row (lengths on the device)
   const int j_hi = j_lo + rps < nruns ? j_lo + rps : nruns;
   const int n_own = j_hi - j_lo;
@@ -792,8 +797,6 @@ __global__ __launch_bounds__(kTopkThreads) void topk_slice_kernel(const TopkPara
     if (p.page_table) return slot_of(p, table, i);
     return i;
   };
-
-  __shared__ SliceLds L;
 
   // ---- 1. the row's scores as raw fp32 bits; the reference point that fixes the mapping to d -------
   // d: 0 for the reference point, growing as the scores fall, equal for equal scores (-0 == +0).
@@ -1111,9 +1114,8 @@ __global__ __launch_bounds__(kTopkThreads) void topk_slice_kernel(const TopkPara
     L.wa[wave] = bgt;
     L.wb[wave] = beq;
   }
-  int32_t* out_idx = p.out_idx + (int64_t)row * p.out_stride;
-  elem_t* out_val =
-      p.out_values ? reinterpret_cast<elem_t*>(p.out_values) + (int64_t)row * p.out_stride : nullptr;
+  int32_t* out_idx = out_row(p, p.out_idx, row);
+  elem_t* out_val = p.out_values ? out_row(p, reinterpret_cast<elem_t*>(p.out_values), row) : nullptr;
   if (n_own <= kOwn) {
     // the slice's runs from registers; every wave turns the (run, wave) counts into the offsets of
     // its own 64-element pieces by itself: run jj, wave w is entry 16 jj + w, two entries per lane
@@ -1211,6 +1213,14 @@ __global__ __launch_bounds__(kTopkThreads) void topk_slice_kernel(const TopkPara
   });
 }
 
+template <typename T, int IPT>
+__global__ __launch_bounds__(kTopkThreads) void topk_slice_kernel(const TopkParams p, int n_slices,
+                                                                  int rps, int rows) {
+  __shared__ SliceLds L;
+  int slice, row;
+  if (coop_decode(n_slices, rows, slice, row)) select_slice<T, IPT>(p, row, slice * rps, rps, L);
+}
+
 // Slices of a row for the sliced variant: enough workgroups to fill the chip when there are few
 // rows, one workgroup per row when there are many (every workgroup of a row repeats the selection
 // work on the whole row), whole 1024-element runs per slice.
@@ -1230,9 +1240,7 @@ static void launch_topk_sliced(const TopkParams& p, int rows, hipStream_t st) {
   int n_slices, rps;
   slice_shape(p.len, rows, n_slices, rps);
   const dim3 grid((rows + kXcds - 1) / kXcds * n_slices * kXcds), block(kTopkThreads);
-  if (p.len <= 8 * kTopkThreads)
-    hipLaunchKernelGGL((topk_slice_kernel<T, 8>), grid, block, 0, st, p, n_slices, rps, rows);
-  else if (p.len <= 16 * kTopkThreads)
+  if (p.len <= 16 * kTopkThreads)
     hipLaunchKernelGGL((topk_slice_kernel<T, 16>), grid, block, 0, st, p, n_slices, rps, rows);
   else if (p.len <= 24 * kTopkThreads)
     hipLaunchKernelGGL((topk_slice_kernel<T, 24>), grid, block, 0, st, p, n_slices, rps, rows);
@@ -1249,6 +1257,12 @@ static void launch_topk_sliced(const TopkParams& p, int rows, hipStream_t st) {
   else  // longer rows would not fit the registers of a 1024-thread workgroup: re-read per pass
     hipLaunchKernelGGL((topk_slice_kernel<T, 0>), grid, block, 0, st, p, n_slices, rps, rows);
 }
+
+}  // namespace tidal
+
+#include "topk_filter.cuh"
+
+namespace tidal {
 
 // workgroups per row for the cooperative path, 0 if it does not apply
 static int coop_slices(int len, int rows) {
@@ -1328,6 +1342,7 @@ extern "C" int td_topk_bounded(const void* values, int32_t values_dtype, int64_t
   p.len_arr = len_arr;
   p.page_size = page_size;
   p.page_shift = -1;
+  p.page_magic = 0xffffffffu / (uint32_t)(page_size >= 1 ? page_size : 1);
   if (page_size >= 1 && (page_size & (page_size - 1)) == 0) p.page_shift = __builtin_ctz(page_size);
   p.out_values = out_values;
   p.out_idx = out_idx;
@@ -1336,9 +1351,18 @@ extern "C" int td_topk_bounded(const void* values, int32_t values_dtype, int64_t
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   TD_REQUIRE(values_dtype == TD_F32 || values_dtype == TD_F16 || values_dtype == TD_BF16,
              "Top-k filtering failed to dispatch with dtype %d", values_dtype);
-  // A few long rows: the three cooperative launches split each row over workgroups that share the
-  // work through the scratch.  Everything else: one launch in which every workgroup of a row goes
-  // through the whole row (rows up to 64K elements from registers) and emits its slice.
+  bool done;
+  if (values_dtype == TD_F32) done = launch_topk_filter<F32>(p, rows, st);
+  else if (values_dtype == TD_F16) done = launch_topk_filter<F16>(p, rows, st);
+  else done = launch_topk_filter<BF16>(p, rows, st);
+  if (done) {
+    TD_HIP_CHECK(hipGetLastError());
+    return TD_OK;
+  }
+  // Selections beyond the list.  A few long rows: the three cooperative launches split each row over
+  // workgroups that share the work through the scratch.  Everything else: one launch in which every
+  // workgroup of a row goes through the whole row (rows up to 64K elements from registers) and emits
+  // its slice.
   const int slices = coop_slices(len, rows);
   if (len > 64 * kTopkThreads && slices && rows * slices <= 1024 && workspace &&
       workspace_bytes >= (int64_t)rows * kCoopRowWords * 4) {

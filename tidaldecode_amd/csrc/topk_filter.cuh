@@ -1,0 +1,497 @@
+// Top-k of a row by one workgroup that touches every element once (included by topk.hip).
+//
+// What bounds a selection out of 10^4 .. 10^5 scores is not their 40 .. 400 KB but the instructions
+// spent per score on the one compute unit that holds the row: an instruction per element costs a
+// 1024-thread workgroup 16 cycles, 0.5 us per row of 64K.  So the radix work is done on few elements:
+//
+//   1. a sample of 4 elements per thread, spread evenly over the row, gives a threshold that the k-th
+//      largest element exceeds almost surely (5 standard deviations of the sample's count);
+//   2. one pass over the row (loads in flight from the start) keeps the positions of what is not below
+//      it, about 1.1 .. 1.4 k elements, in LDS: two instructions per element, some more per survivor;
+//   3. the radix select of the k-th largest runs on the survivors (exact: fewer survivors than k start
+//      again with a lower threshold; more than the list holds -- rows of few distinct values -- leave
+//      the row to select_slice);
+//   4. the selected positions go into a bitmap in LDS, whose prefix counts give every one its place
+//      in position order, whatever order the survivors were listed in.
+//
+// Rows of up to 4 elements per thread are their own sample: the radix select on it is the result.
+//
+// Measured on one MI355X (fp32, bound and page table given, launches of a graph, us; in brackets the
+// kernel that had these rows before: every workgroup histograms the whole row, its scores in registers
+// up to 64K of them, and up to eight workgroups share the emission):
+//   32 x 777 -> 256     4.6 (7.3)     256 x 14000 -> 1024  11.1 (15.8)
+//   32 x 4096 -> 256    6.7 (8.3)     256 x 63000 -> 1024  23.3 (58.6)
+//   512 x 8192 -> 512   10.7 (19.5)   256 x 65537 -> 1024  24.4 (120)
+//   32 x 32769 -> 2048  12.6 (15.9)   8 x 102392 -> 4096   19.5 (28.6: three launches that share a row)
+// What is left is a chain: two trips to memory (sample, survivors' values), two radix levels of about
+// 1 us and the bitmap's 0.8; 256 rows of 63000 also read 64 MB at 2.8 TB/s.
+// The results are those of every other variant: the k largest, ties to the lower position, in
+// position order.
+#pragma once
+
+namespace tidal {
+
+constexpr uint32_t kKeyNegInf = 0x007fffffu, kKeyPosInf = 0xff800000u;
+constexpr uint32_t kMaxSpan = 0xff800000u;  // no two keys of scores lie further apart
+__device__ __forceinline__ float key_to_float(uint32_t key) {
+  return __builtin_bit_cast(float, (key & 0x80000000u) ? key & 0x7fffffffu : ~key);
+}
+__device__ __forceinline__ int bit_count(uint32_t x) { return x ? 32 - __builtin_clz(x) : 0; }
+
+// A row read four elements at a time.  The descriptor starts at the dword that holds element 0, so
+// that every load is dword aligned; `shift` elements (16-bit types: 0 or 1) lie in front of the row.
+// Vector i holds the elements 4 i - shift .. 4 i + 3 - shift; dwords past the end read as 0.
+template <typename T>
+struct RowVectors {
+  typedef typename std::conditional<std::is_same<T, F32>::value, u32x4, u32x2>::type vec;
+  __amdgpu_buffer_rsrc_t rsrc;
+  int shift;
+  __device__ __forceinline__ RowVectors(const void* row, int len) {
+    if constexpr (std::is_same<T, F32>::value) {
+      shift = 0;
+      rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(row), 0, len * 4, 0x00020000);
+    } else {
+      const uint64_t at = reinterpret_cast<uint64_t>(row);
+      shift = (int)((at >> 1) & 1);
+      rsrc = __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(at & ~3ull), 0,
+                                               ((len + shift) * 2 + 3) & ~3, 0x00020000);
+    }
+  }
+  // vector lane_vec + uniform_vec
+  __device__ __forceinline__ vec load(int lane_vec, int uniform_vec) const {
+    if constexpr (std::is_same<T, F32>::value)
+      return __builtin_bit_cast(vec, __builtin_amdgcn_raw_buffer_load_b128(rsrc, lane_vec * 16, uniform_vec * 16, 0));
+    else
+      return __builtin_bit_cast(vec, __builtin_amdgcn_raw_buffer_load_b64(rsrc, lane_vec * 8, uniform_vec * 8, 0));
+  }
+  __device__ static __forceinline__ float element(const vec& v, int c) {
+    if constexpr (std::is_same<T, F32>::value)
+      return __builtin_bit_cast(float, (uint32_t)v[c]);
+    else
+      return to_float<T>((uint16_t)((uint32_t)v[c >> 1] >> (16 * (c & 1))));
+  }
+};
+
+// bit i of the result: element i of the 16 in v[0 .. 3] is not below `floor` (a NaN is not below
+// anything).  Two instructions per element: the comparison's mask is shifted in as a carry.
+template <typename T>
+__device__ __forceinline__ uint32_t reach16(const typename RowVectors<T>::vec* v, float floor) {
+  uint32_t mask = 0;
+#pragma unroll
+  for (int i = 15; i >= 0; --i)
+    asm("v_cmp_nlt_f32 vcc, %1, %2\n\tv_addc_co_u32 %0, vcc, %0, %0, vcc"
+        : "+v"(mask)
+        : "v"(RowVectors<T>::element(v[i >> 2], i & 3)), "v"(floor)
+        : "vcc");
+  return mask;
+}
+
+constexpr int kFilterRank = 64;  // members of the threshold bin that are ranked in the lanes of a wave
+
+template <int NT, int CAP, int MAXLEN>
+struct FilterLds {
+  typedef typename std::conditional<(MAXLEN <= 65536), uint16_t, uint32_t>::type pos_t;
+  uint32_t hist[4 * NT];         // zero between the radix levels
+  pos_t pos[CAP];                // survivors
+  uint32_t bits[MAXLEN / 32];    // selected positions
+  uint16_t before[MAXLEN / 32];  // set bits in front of the word
+  uint32_t mem[kFilterRank];
+  uint32_t wa[16], wb[16];
+  uint32_t sh[4];
+  uint32_t n_cand, n_mem;
+};
+
+// page of position i for pages of any size: the quotient from a multiplication is at most one short
+__device__ __forceinline__ int page_of(const TopkParams& p, int i) {
+  int page = (int)__umulhi((uint32_t)i, p.page_magic);
+  if (i - page * p.page_size >= p.page_size) ++page;
+  return page;
+}
+
+// sums of the first `wave` and of all NW entries of arr
+template <int NW>
+__device__ __forceinline__ void sums_before(const uint32_t* arr, int wave, int lane, uint32_t& before, uint32_t& all) {
+  const uint32_t v = row_prefix_sum((lane & 15) < NW ? arr[lane & (NW - 1)] : 0u);
+  all = __builtin_amdgcn_readlane(v, NW - 1);
+  before = wave ? __builtin_amdgcn_readlane(v, wave - 1) : 0u;
+}
+
+// CAP: survivors the list holds; CAP >= MAXLEN: any row fits.
+template <typename T, int NT, int VPT, int CAP, int MAXLEN>
+__global__ __launch_bounds__(NT) void topk_filter_kernel(const TopkParams p) {
+  typedef typename ElemOf<T>::type elem_t;
+  typedef typename RowVectors<T>::vec vec;
+  typedef FilterLds<NT, CAP, MAXLEN> Lds;
+  constexpr int NW = NT / 64, CPT = CAP / NT, CHUNK = 4 * NT * VPT;
+  constexpr int kBits = NT == 1024 ? 12 : (NT == 512 ? 11 : 10);  // log2 of the bins
+  constexpr bool kFits = MAXLEN <= CAP;                 // the list holds any row: no way out needed
+  constexpr bool kSampled = MAXLEN > 4 * NT;            // rows may be longer than the sample
+  static_assert(CPT >= 4 && 4 * NT == 1 << kBits && (VPT == 4 || VPT == 8), "shapes");
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int row = blockIdx.x;
+  const int len = row_len(p, row), k = row_k(p, len);
+  const elem_t* vals = reinterpret_cast<const elem_t*>(p.values) + (int64_t)row * p.values_stride;
+  const RowVectors<T> rv(vals, len);
+  const int shift = rv.shift;
+
+  __shared__ union {
+    Lds f;
+    typename std::conditional<kFits, uint32_t, SliceLds>::type slice;
+  } lds;
+  Lds& L = lds.f;
+
+  // ---- the sample, then the row: everything in flight ------------------------------------------
+  const int nvec = (len + shift + 3) >> 2;
+  const bool whole = !kSampled || nvec <= NT;  // the sample is the row
+  // four threads share 16 consecutive elements: single vectors would pull a 128-byte line each
+  const int svec = whole ? tid : (int)((uint32_t)(tid >> 2) * (uint32_t)(nvec >> 2) / (uint32_t)(NT / 4)) * 4 + (tid & 3);
+  const vec sample = rv.load(svec, 0);
+  vec v[kSampled ? VPT : 4];
+  auto load_group = [&](int chunk, int g) {
+#pragma unroll
+    for (int j = 4 * g; j < 4 * g + 4; ++j) v[j] = rv.load(tid, (chunk * VPT + j) * NT);
+  };
+  if (!whole) {
+#pragma unroll
+    for (int g = 0; g < VPT / 4; ++g) load_group(0, g);
+  }
+
+  float bound = __builtin_nanf("");
+  if (p.row_bound) bound = p.row_bound[row];
+  const bool bounded = __builtin_fabsf(bound) < __builtin_inff();
+  reinterpret_cast<uint4*>(L.hist)[tid] = make_uint4(0, 0, 0, 0);
+  const int n_words = (len + 31) >> 5;
+  for (int i = tid; i < n_words; i += NT) L.bits[i] = 0;
+  if (tid == 0) L.n_cand = L.n_mem = 0;
+
+  // ---- 1. the sample's distances below a reference: the caller's bound or the sample's maximum ----
+  uint32_t sx[4], kmax = 0u;
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    sx[c] = KeyTraits<F32>::key(RowVectors<T>::element(sample, c));
+    if ((uint32_t)(4 * svec + c - shift) < (uint32_t)len) kmax = sx[c] > kmax ? sx[c] : kmax;
+  }
+  if (bounded) {
+    kmax = KeyTraits<F32>::key(bound);
+    // 16-bit scores may have been rounded up past a bound formed in fp32: one bf16 step of room
+    if constexpr (!std::is_same<T, F32>::value) kmax += 0x10000u;
+  } else {
+    kmax = (uint32_t)wave_max_i32((int32_t)(kmax ^ 0x80000000u));
+    if (lane == 0) L.wb[wave] = kmax;
+    __syncthreads();
+    kmax = (uint32_t)wave_max_i32((int32_t)L.wb[lane & (NW - 1)]) ^ 0x80000000u;
+  }
+  kmax = __builtin_amdgcn_readfirstlane(kmax);
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    const uint32_t d = sx[c] < kmax ? kmax - sx[c] : 0u;
+    sx[c] = (uint32_t)(4 * svec + c - shift) < (uint32_t)len ? d : kNoElement;
+  }
+  uint32_t rank = (uint32_t)k;
+  if (!whole) {
+    const float mu = (float)k * (float)(4 * NT) / (float)len;
+    rank = (uint32_t)(mu + 5.f * __builtin_sqrtf(mu) + 5.f);
+  }
+  __syncthreads();  // hist, bits and the counters are zero
+
+  // ---- radix select: the krem-th smallest of what each() hands out, as the krem-th smallest of the
+  // n_in ones in [lo, lo + 2^s): at most kFilterRank, or all equal (s == 0).  The window [lo, lo + last]
+  // comes first, what lies beyond it only if fewer than krem lie inside.  False: fewer than krem in all.
+  uint32_t lo, s, krem, n_in;
+  auto narrow = [&](uint32_t last, auto each) -> bool {
+    auto shift_of = [](uint32_t span) {
+      const int b = bit_count(span) - kBits;
+      return b > 0 ? (uint32_t)b : 0u;
+    };
+    lo = 0u;
+    s = shift_of(last);
+    for (;;) {
+      each([&](uint32_t x) {
+        const uint32_t d = x - lo;
+        if (d <= last) atomicAdd(&L.hist[d >> s], 1u);
+      });
+      __syncthreads();
+      uint4* h4 = reinterpret_cast<uint4*>(L.hist) + tid;
+      const uint4 a = *h4;
+      *h4 = make_uint4(0, 0, 0, 0);
+      const uint32_t local = (a.x + a.y) + (a.z + a.w);
+      const uint32_t incl = wave_prefix_sum_dpp(local, lane);
+      if (lane == 63) L.wa[wave] = incl;
+      __syncthreads();
+      uint32_t first, total;
+      sums_before<NW>(L.wa, wave, lane, first, total);
+      first += incl - local;
+      if (first < krem && krem <= first + local) {  // one thread of the workgroup, if any
+        const uint32_t b1 = first + a.x, b2 = b1 + a.y, b3 = b2 + a.z;
+        const int i = (krem > b1 ? 1 : 0) + (krem > b2 ? 1 : 0) + (krem > b3 ? 1 : 0);
+        L.sh[0] = (uint32_t)(4 * tid + i);
+        L.sh[1] = krem - (i == 0 ? first : (i == 1 ? b1 : (i == 2 ? b2 : b3)));
+        L.sh[2] = i == 0 ? a.x : (i == 1 ? a.y : (i == 2 ? a.z : a.w));
+      }
+      __syncthreads();
+      if (krem <= total) {
+        lo += __builtin_amdgcn_readfirstlane(L.sh[0]) << s;
+        krem = __builtin_amdgcn_readfirstlane(L.sh[1]);
+        n_in = __builtin_amdgcn_readfirstlane(L.sh[2]);
+        if (s == 0u || n_in <= (uint32_t)kFilterRank) return true;
+        last = (1u << s) - 1u;
+      } else {
+        if (last >= kMaxSpan - lo) return false;
+        krem -= total;
+        lo += last + 1u;
+        last = kMaxSpan - lo;
+      }
+      s = shift_of(last);
+    }
+  };
+  auto each_sample = [&](auto f) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c) f(sx[c]);
+  };
+  constexpr uint32_t kFirst = (1u << 29) - 1u;  // 64 binades below the reference first
+
+  // What is selected from, n slots: x (kNoElement: empty) and position.  The row itself if it is its
+  // own sample, else the survivors.
+  uint32_t x[CPT], krem0;
+  int32_t pos[CPT];
+  int n;
+  uint32_t C = 0;
+  auto each_slot = [&](auto f) {  // f(slot)
+#pragma unroll
+    for (int u4 = 0; u4 < CPT; u4 += 4) {
+      if (u4 * NT < n) {  // uniform
+#pragma unroll
+        for (int u = u4; u < u4 + 4; ++u) f(u);
+      }
+    }
+  };
+  if (whole) {
+#pragma unroll
+    for (int u = 0; u < CPT; ++u) {
+      x[u] = u < 4 ? sx[u & 3] : kNoElement;
+      const int at = 4 * svec + (u & 3) - shift;
+      pos[u] = at < 0 ? 0 : (at < len ? at : len - 1);
+    }
+    n = 4 * NT;
+    krem = krem0 = (uint32_t)k;
+    narrow(kFirst, each_sample);
+  } else if constexpr (kSampled) {
+    // ---- 2. the survivors: what is not below the far edge of the bin that holds rank `rank` ---------
+    uint32_t kbase;
+    for (;;) {
+      kbase = 0u;
+      krem = rank;
+      if (narrow(kFirst, each_sample)) {
+        const uint32_t edge = lo + ((1u << s) - 1u);
+        kbase = kmax > edge ? kmax - edge : 0u;
+      }
+      kbase = kbase < kKeyNegInf ? kKeyNegInf : (kbase > kKeyPosInf ? kKeyPosInf : kbase);
+      const float floor_f = key_to_float(kbase);
+      for (int chunk = 0; chunk * CHUNK < len + shift; ++chunk) {
+#pragma unroll
+        for (int g = 0; g < VPT / 4; ++g) {
+          const int first = 4 * ((chunk * VPT + 4 * g) * NT) - shift;  // position of the group's first element
+          if (first < len) {
+            uint32_t mask = reach16<T>(v + 4 * g, floor_f);
+            if (first < 0 || first + 16 * NT > len) {  // elements outside the row
+#pragma unroll
+              for (int j = 0; j < 4; ++j) {
+                const int at = first + 4 * (j * NT + tid), room = len - at;
+                const uint32_t ok = room >= 4 ? 15u : (room > 0 ? (1u << room) - 1u : 0u);
+                mask &= ~(15u << (4 * j)) | ((at < 0 ? ok & 14u : ok) << (4 * j));
+              }
+            }
+            if (__ballot(mask != 0u)) {
+              const uint32_t mine = __popc(mask);
+              const uint32_t incl = wave_prefix_sum_dpp(mine, lane);
+              const uint32_t all = __builtin_amdgcn_readlane(incl, 63);
+              uint32_t at = 0;
+              if (lane == 0) at = atomicAdd(&L.n_cand, all);
+              at = __builtin_amdgcn_readfirstlane(at);
+              if (kFits || at + all <= (uint32_t)CAP) {  // else counted, not listed
+                at += incl - mine;
+                while (mask) {
+                  const int i = __builtin_ctz(mask);
+                  mask &= mask - 1u;
+                  L.pos[at++] = (typename Lds::pos_t)(first + 4 * tid + (i & 12) * NT + (i & 3));
+                }
+              }
+            }
+          }
+          if ((chunk + 1) * CHUNK < len + shift) load_group(chunk + 1, g);
+        }
+      }
+      __syncthreads();
+      C = __builtin_amdgcn_readfirstlane(L.n_cand);
+      if (C >= (uint32_t)k) break;
+      rank = 2u * rank + 64u;  // an unlucky sample: the k-th largest lies below the floor
+#pragma unroll
+      for (int g = 0; g < VPT / 4; ++g) load_group(0, g);
+      __syncthreads();
+      if (tid == 0) L.n_cand = 0;  // (added to again behind the barriers of the next level)
+    }
+    if constexpr (!kFits) {
+      if (C > (uint32_t)CAP) {
+        const int n_runs = (len + kTopkThreads - 1) / kTopkThreads;
+        for (int j_lo = 0; j_lo < n_runs; j_lo += kSliceMaxRuns) {
+          __syncthreads();
+          select_slice<T, 0>(p, row, j_lo, kSliceMaxRuns, lds.slice);
+        }
+        return;
+      }
+    }
+    // ---- 3. the k-th largest of them: the (C - k + 1)-th smallest distance above the floor -----------
+    n = (int)C;
+#pragma unroll
+    for (int u = 0; u < CPT; ++u) x[u] = kNoElement;
+    each_slot([&](int u) {
+      const int i = u * NT + tid;
+      pos[u] = (int32_t)L.pos[i < n ? i : 0];
+    });
+    elem_t raw[CPT];
+    each_slot([&](int u) { raw[u] = vals[pos[u]]; });
+    each_slot([&](int u) {
+      float f;
+      if constexpr (std::is_same<T, F32>::value) f = raw[u];
+      else f = to_float<T>(raw[u]);
+      x[u] = u * NT + tid < n ? KeyTraits<F32>::key(f) - kbase : kNoElement;
+    });
+    krem = krem0 = C - (uint32_t)k + 1u;
+    narrow(kmax > kbase ? kmax - kbase : 0u, [&](auto f) { each_slot([&](int u) { f(x[u]); }); });
+  }
+  uint32_t below = krem0 - krem;  // smaller than the bin's members
+
+  // ---- the payloads (in flight from here on), and the members of the bin against each other --------
+  const int32_t* table = table_of(p, row);
+  int32_t pay[CPT];
+  if (p.in_idx) {
+    const int32_t* in = p.in_idx + (int64_t)row * p.in_idx_stride;
+    each_slot([&](int u) { pay[u] = in[pos[u]]; });
+  } else if (p.page_table) {
+    int32_t entry[CPT];
+    each_slot([&](int u) {
+      const int page = p.page_shift >= 0 ? pos[u] >> p.page_shift : page_of(p, pos[u]);
+      entry[u] = pos[u] - page * p.page_size;
+      pay[u] = table[page];
+    });
+    each_slot([&](int u) { pay[u] = pay[u] * p.page_size + entry[u]; });
+  } else {
+    each_slot([&](int u) { pay[u] = pos[u]; });
+  }
+  uint32_t thr = lo, ties = n_in;  // s == 0: the members are equal
+  if (s > 0u) {
+    each_slot([&](int u) {
+      if (x[u] - lo < (1u << s)) L.mem[atomicAdd(&L.n_mem, 1u)] = x[u];
+    });
+    __syncthreads();
+    const uint32_t mine = lane < (int)n_in ? L.mem[lane] : kNoElement;
+    uint32_t lt = 0, le = 0;
+    for (int i = 0; i < (int)n_in; ++i) {
+      const uint32_t other = __builtin_amdgcn_readlane(mine, i);
+      lt += other < mine ? 1u : 0u;
+      le += other <= mine ? 1u : 0u;
+    }
+    // krem <= n_in: some member has that rank
+    const int src = __builtin_ctzll(__ballot(lane < (int)n_in && lt < krem && krem <= le));
+    thr = __builtin_amdgcn_readlane(mine, src);
+    lt = __builtin_amdgcn_readlane(lt, src);
+    ties = __builtin_amdgcn_readlane(le, src) - lt;
+    below += lt;
+  }
+  // how many of the ties are taken; the sample counts down from the reference, the survivors up from
+  // the floor
+  const uint32_t r = whole ? (uint32_t)k - below : (uint32_t)k - (C - below - ties);
+
+  // ---- 4. places in position order ---------------------------------------------------------------
+  const int wpt = (n_words + NT - 1) / NT;
+  auto count_words = [&]() {  // before[w] = set bits in front of word w
+    __syncthreads();
+    uint32_t local = 0;
+    for (int i = 0; i < wpt; ++i) {
+      const int w = tid * wpt + i;
+      local += w < n_words ? __popc(L.bits[w]) : 0u;
+    }
+    const uint32_t incl = wave_prefix_sum_dpp(local, lane);
+    if (lane == 63) L.wa[wave] = incl;
+    __syncthreads();
+    uint32_t run, total;
+    sums_before<NW>(L.wa, wave, lane, run, total);
+    run += incl - local;
+    for (int i = 0; i < wpt; ++i) {
+      const int w = tid * wpt + i;
+      if (w < n_words) {
+        L.before[w] = (uint16_t)run;
+        run += __popc(L.bits[w]);
+      }
+    }
+    __syncthreads();
+  };
+  auto place_of = [&](int32_t at) -> uint32_t {
+    return (uint32_t)L.before[at >> 5] + __popc(L.bits[at >> 5] & ((1u << (at & 31)) - 1u));
+  };
+  const uint32_t flip = whole ? ~0u : 0u;  // selected: (x ^ flip) above (thr ^ flip)
+  uint32_t take = 0;                       // bit u: slot u of this thread
+  each_slot([&](int u) {
+    if (x[u] != kNoElement && ((x[u] ^ flip) > (thr ^ flip) || (x[u] == thr && r == ties))) take |= 1u << u;
+  });
+  if (r != ties) {  // the first r of the ties
+    each_slot([&](int u) {
+      if (x[u] == thr) atomicOr(&L.bits[pos[u] >> 5], 1u << (pos[u] & 31));
+    });
+    count_words();
+    each_slot([&](int u) {
+      if (x[u] == thr && place_of(pos[u]) < r) take |= 1u << u;
+    });
+    __syncthreads();
+    for (int i = tid; i < n_words; i += NT) L.bits[i] = 0;
+    __syncthreads();
+  }
+  each_slot([&](int u) {
+    if ((take >> u) & 1u) atomicOr(&L.bits[pos[u] >> 5], 1u << (pos[u] & 31));
+  });
+  count_words();
+  int32_t* out_idx = out_row(p, p.out_idx, row);
+  elem_t* out_val = p.out_values ? out_row(p, reinterpret_cast<elem_t*>(p.out_values), row) : nullptr;
+  each_slot([&](int u) {
+    if ((take >> u) & 1u) {
+      const uint32_t at = place_of(pos[u]);
+      out_idx[at] = pay[u];
+      if (out_val) out_val[at] = vals[pos[u]];
+    }
+  });
+}
+
+constexpr int kFilterCap = 8192;
+
+// Whether the survivors of a row of `len` elements fit the list with room to spare: the sample's
+// count, five standard deviations of the margin put on it and five of its own spread, scaled to the row.
+static bool filter_fits(int len, int k, int threads) {
+  const double m = 4.0 * threads;
+  if (len <= kFilterCap) return true;
+  const double mu = (double)k * m / len, want = mu + 5.0 * __builtin_sqrt(mu) + 5.0;
+  return (want + 5.0 * __builtin_sqrt(want)) * len / m <= 0.95 * kFilterCap;
+}
+
+// True: launched.  Threads by row length: the fewer, the cheaper the barriers and scans that make up
+// most of a short row's time; 1024 are needed where the row's elements are (32 x 8192 -> 512: 7.1 us
+// with 512, 9.3 at 10000 with 1024).  The limits of 65536 and 262144 are the LDS of the bitmap.
+template <typename T>
+static bool launch_topk_filter(const TopkParams& p, int rows, hipStream_t st) {
+  const dim3 grid(rows);
+  if (p.len <= 1024 - 4)
+    hipLaunchKernelGGL((topk_filter_kernel<T, 256, 4, 1024, 1024>), grid, dim3(256), 0, st, p);
+  else if (p.len <= 8192)
+    hipLaunchKernelGGL((topk_filter_kernel<T, 512, 4, 8192, 8192>), grid, dim3(512), 0, st, p);
+  else if (!filter_fits(p.len, p.k, 1024))
+    return false;
+  else if (p.len <= 65536)
+    hipLaunchKernelGGL((topk_filter_kernel<T, 1024, 8, kFilterCap, 65536>), grid, dim3(1024), 0, st, p);
+  else if (p.len <= 262144)
+    hipLaunchKernelGGL((topk_filter_kernel<T, 1024, 8, kFilterCap, 262144>), grid, dim3(1024), 0, st, p);
+  else
+    return false;
+  return true;
+}
+
+}  // namespace tidal

@@ -387,12 +387,26 @@ int td_topk_bounded(const void* values, int32_t values_dtype, int64_t values_str
                     int64_t workspace_bytes, void* stream);
 
 /*
+ * td_topk_bounded with the outputs of a group's rows apart: row r of the scores is row
+ * r % rows_per_table of group r / rows_per_table, and its output starts at
+ * (r / rows_per_table) * out_group_stride + (r % rows_per_table) * out_stride (0: groups follow each
+ * other, as in td_topk).  With out_group_stride < out_stride the sequences of a batch get one segment
+ * each of a list row per head, the layout td_decode_attn reads.  No counterpart in the reference.
+ */
+int td_topk_segments(const void* values, int32_t values_dtype, int64_t values_stride, int32_t rows,
+                     int32_t len, int32_t k, const int32_t* in_idx, int64_t in_idx_stride,
+                     const int32_t* page_table, int64_t page_table_stride, int32_t rows_per_table,
+                     const int32_t* len_arr, int32_t page_size, const float* row_bound,
+                     void* out_values, int32_t* out_idx, int64_t out_stride, int64_t out_group_stride,
+                     void* workspace, int64_t workspace_bytes, void* stream);
+
+/*
  * Bytes of device scratch for td_topk.  Rows of up to 65536 elements never touch it, nor do rows of
  * up to 262144 whose selection fits the list of the one-pass kernel (k up to about 5800).  Larger
  * selections from a few long rows are shared between workgroups through it (three launches; about
  * 56 KiB per row); without it (NULL), or with many long rows, every workgroup goes through the whole
- * row, read again from L2 in every pass.  The
- * scratch must be zero-filled once before its first use; every call leaves it ready for the next.
+ * row, read again from L2 in every pass.  The scratch must be
+ * zero-filled once before its first use; every call leaves it ready for the next.
  * Plays the part of the `buf` argument of topk_filtering (tidal/utils/controller.py:164-168).
  */
 int64_t td_topk_workspace_bytes(int32_t rows);

@@ -215,13 +215,15 @@ def topk_filtering(estimated_value: torch.Tensor, estimated_indices: Optional[to
                    buf: Optional[torch.Tensor], page_budget: int, *,
                    page_table: Optional[torch.Tensor] = None, page_size: int = 1,
                    lengths: Optional[torch.Tensor] = None,
-                   upper_bound: Optional[torch.Tensor] = None) -> None:
+                   upper_bound: Optional[torch.Tensor] = None,
+                   segment: Optional[int] = None) -> None:
     """bsk_ops.h:34-39 / topk.cu:7-44.  Row-wise top-``page_budget`` of ``estimated_value``
     ``[H, len]``; ``indices_out[h, j]`` is ``estimated_indices[h, p]`` of the selected position
     ``p``.  ``buf`` is scratch, as in the reference (there: RAFT's): a zero-initialised uint8 /
     any-dtype device tensor of at least ``topk_workspace_bytes(H)`` bytes through which the
-    workgroups of a row of more than 65536 elements share the work; shorter rows never touch it,
-    and without it (smaller or ``None``) every workgroup of a long row goes through the whole row.
+    workgroups of a row of more than 65536 elements share a large selection (``page_budget`` beyond
+    about 5800); other rows never touch it, and without it (smaller or ``None``) every workgroup of
+    such a row goes through the whole row.
     The call leaves ``buf`` zeroed where it must be for the next call.
 
     Deterministic where the reference is not: ties at the threshold go to the lower position
@@ -236,7 +238,9 @@ def topk_filtering(estimated_value: torch.Tensor, estimated_indices: Optional[to
     ``min(page_budget, lengths[g])`` of them, leaving the rest of their output row untouched.
     ``upper_bound`` (fp32 device ``[H]``): a value per row that no score of the row exceeds (a
     selection layer's log-sum-exp, the head count for summed probabilities); same result, without
-    the pass that finds the row maximum.  NaN entries mean "no bound".
+    the pass that finds the row maximum.  NaN entries mean "no bound".  ``segment``: the rows of a
+    group are spread over the rows of ``indices_out`` ``[H / groups, >= groups * segment]``, each
+    group in its own columns: row r of group g goes to ``indices_out[r, g * segment:]``.
     """
     _check_rows(estimated_value, "estimated_value")
     rows, length = estimated_value.shape
@@ -252,7 +256,7 @@ def topk_filtering(estimated_value: torch.Tensor, estimated_indices: Optional[to
     _check_rows(indices_out, "indices_out")
     _check_i32(indices_out, "indices_out")
     k = int(page_budget)
-    if indices_out.dim() != 2 or indices_out.size(0) != rows or indices_out.size(1) != k:
+    if segment is None and (indices_out.size(0) != rows or indices_out.size(1) != k):
         raise RuntimeError(f"indices_out must be [{rows}, {k}]")
     out_vals = None
     if d_out is not None and d_out.numel() > 0:
@@ -286,6 +290,14 @@ def topk_filtering(estimated_value: torch.Tensor, estimated_indices: Optional[to
             raise RuntimeError(f"lengths has {groups} entries for {rows} rows")
         rows_per_table = rows // groups
         len_ptr = lengths.data_ptr()
+    out_stride, out_group_stride = indices_out.stride(0), 0
+    if segment is not None:
+        per = rows_per_table or rows
+        if indices_out.size(0) != per or segment < max(k, 1) or indices_out.size(1) < rows // per * segment \
+                or out_vals is not None:
+            raise RuntimeError(f"segment {segment} of {k} selected: indices_out must be "
+                               f"[{per}, >= {rows // per} * segment], without d_out")
+        out_group_stride = int(segment)
     ws_ptr, ws_bytes = None, 0
     if buf is not None and buf.is_cuda and buf.is_contiguous():
         ws_bytes = buf.numel() * buf.element_size()
@@ -297,12 +309,12 @@ def topk_filtering(estimated_value: torch.Tensor, estimated_indices: Optional[to
         if upper_bound.dtype != torch.float32 or upper_bound.numel() != rows:
             raise RuntimeError(f"upper_bound must hold {rows} float32 values")
         bound_ptr = upper_bound.data_ptr()
-    check(lib.td_topk_bounded(estimated_value.data_ptr(),
-                              _dtype_code(estimated_value.dtype, "Top-k filtering"),
-                              estimated_value.stride(0), rows, length, k, in_ptr, in_stride,
-                              pt_ptr, pt_stride, rows_per_table, len_ptr, int(page_size),
-                              bound_ptr, out_vals, indices_out.data_ptr(), indices_out.stride(0),
-                              ws_ptr, ws_bytes if ws_ptr else 0, _stream()))
+    check(lib.td_topk_segments(estimated_value.data_ptr(),
+                               _dtype_code(estimated_value.dtype, "Top-k filtering"),
+                               estimated_value.stride(0), rows, length, k, in_ptr, in_stride,
+                               pt_ptr, pt_stride, rows_per_table, len_ptr, int(page_size),
+                               bound_ptr, out_vals, indices_out.data_ptr(), out_stride, out_group_stride,
+                               ws_ptr, ws_bytes if ws_ptr else 0, _stream()))
 
 
 def topk_workspace_bytes(rows: int) -> int:

@@ -45,6 +45,7 @@ struct TopkParams {
   void* out_values;
   int32_t* out_idx;
   int64_t out_stride;
+  int64_t out_group_stride;  // elements between the outputs of consecutive row groups
   const float* row_bound;  // per row: a value no score of the row exceeds (NaN: none known), or null
 };
 
@@ -56,7 +57,8 @@ __device__ __forceinline__ const int32_t* table_of(const TopkParams& p, int row)
 // where the row's output starts
 template <typename E>
 __device__ __forceinline__ E* out_row(const TopkParams& p, E* base, int row) {
-  return base + (int64_t)row * p.out_stride;
+  const int group = row / p.rows_per_table;
+  return base + (int64_t)group * p.out_group_stride + (int64_t)(row - group * p.rows_per_table) * p.out_stride;
 }
 // elements of this row that take part, and how many of them are selected
 __device__ __forceinline__ int row_len(const TopkParams& p, int row) {
@@ -1309,13 +1311,14 @@ __global__ __launch_bounds__(256) void score_reduce_kernel(const float* __restri
 
 using namespace tidal;
 
-extern "C" int td_topk_bounded(const void* values, int32_t values_dtype, int64_t values_stride,
-                               int32_t rows, int32_t len, int32_t k, const int32_t* in_idx,
-                               int64_t in_idx_stride, const int32_t* page_table,
-                               int64_t page_table_stride, int32_t rows_per_table,
-                               const int32_t* len_arr, int32_t page_size, const float* row_bound,
-                               void* out_values, int32_t* out_idx, int64_t out_stride,
-                               void* workspace, int64_t workspace_bytes, void* stream) {
+extern "C" int td_topk_segments(const void* values, int32_t values_dtype, int64_t values_stride,
+                                int32_t rows, int32_t len, int32_t k, const int32_t* in_idx,
+                                int64_t in_idx_stride, const int32_t* page_table,
+                                int64_t page_table_stride, int32_t rows_per_table,
+                                const int32_t* len_arr, int32_t page_size, const float* row_bound,
+                                void* out_values, int32_t* out_idx, int64_t out_stride,
+                                int64_t out_group_stride, void* workspace, int64_t workspace_bytes,
+                                void* stream) {
   TD_REQUIRE(values && out_idx, "td_topk: NULL values or out_idx");
   TD_REQUIRE(rows >= 1, "td_topk: rows %d < 1", rows);
   TD_REQUIRE(len >= 0 && k >= 0, "td_topk: len %d / k %d", len, k);
@@ -1323,6 +1326,7 @@ extern "C" int td_topk_bounded(const void* values, int32_t values_dtype, int64_t
              len);
   if (k > len) k = len;
   TD_REQUIRE(out_stride >= k, "td_topk: out_stride %lld < k %d", (long long)out_stride, k);
+  TD_REQUIRE(out_group_stride >= 0, "td_topk: out_group_stride %lld", (long long)out_group_stride);
   TD_REQUIRE(!in_idx || in_idx_stride >= 0, "td_topk: in_idx_stride %lld", (long long)in_idx_stride);
   TD_REQUIRE(!page_table || page_size >= 1, "td_topk: page_size %d", page_size);
   TD_REQUIRE((!page_table && !len_arr) || (rows_per_table >= 0 && page_table_stride >= 0),
@@ -1347,6 +1351,7 @@ extern "C" int td_topk_bounded(const void* values, int32_t values_dtype, int64_t
   p.out_values = out_values;
   p.out_idx = out_idx;
   p.out_stride = out_stride;
+  p.out_group_stride = out_group_stride ? out_group_stride : p.rows_per_table * out_stride;
   p.row_bound = row_bound;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   TD_REQUIRE(values_dtype == TD_F32 || values_dtype == TD_F16 || values_dtype == TD_BF16,
@@ -1390,6 +1395,18 @@ extern "C" int td_topk_bounded(const void* values, int32_t values_dtype, int64_t
   }
   TD_HIP_CHECK(hipGetLastError());
   return TD_OK;
+}
+
+extern "C" int td_topk_bounded(const void* values, int32_t values_dtype, int64_t values_stride,
+                               int32_t rows, int32_t len, int32_t k, const int32_t* in_idx,
+                               int64_t in_idx_stride, const int32_t* page_table,
+                               int64_t page_table_stride, int32_t rows_per_table,
+                               const int32_t* len_arr, int32_t page_size, const float* row_bound,
+                               void* out_values, int32_t* out_idx, int64_t out_stride,
+                               void* workspace, int64_t workspace_bytes, void* stream) {
+  return td_topk_segments(values, values_dtype, values_stride, rows, len, k, in_idx, in_idx_stride,
+                          page_table, page_table_stride, rows_per_table, len_arr, page_size, row_bound,
+                          out_values, out_idx, out_stride, 0, workspace, workspace_bytes, stream);
 }
 
 extern "C" int td_topk(const void* values, int32_t values_dtype, int64_t values_stride,

@@ -94,7 +94,6 @@ class BatchInferenceController:
                                           dtype=torch.float32, device=device)
         # lists: row r of sequence b lives in columns [b * budget, b * budget + selected[b])
         self.topk_dindices_buffer = torch.zeros((self.index_rows, max_batch * self.budget), **i32)
-        self._slots = torch.zeros((max_batch * self.index_rows, self.budget), **i32)
         self._list_starts = torch.arange(max_batch + 1, **i32) * self.budget
         self.topk_buf = torch.zeros(_kernels.topk_workspace_bytes(max_batch * self.index_rows),
                                     dtype=torch.uint8, device=device)
@@ -327,12 +326,10 @@ class BatchInferenceController:
         k_eff = min(k, n)
         # one call: row b * rows + r is row r of sequence b, ranks that sequence's tokens only
         # (its length is read on the device) and goes through that sequence's page table
-        out = self._slots[: B * rows, :k_eff]
-        _kernels.topk_filtering(scores[:, :n], None, None, out, self.topk_buf, k_eff,
+        # and lands in that sequence's segment of list row r
+        _kernels.topk_filtering(scores[:, :n], None, None, self.topk_dindices_buffer, self.topk_buf, k_eff,
                                 page_table=self.page_table[:B], page_size=P,
-                                lengths=self._row(_SEQ_LEN), upper_bound=bound)
-        self.topk_dindices_buffer.view(rows, self.max_batch, k)[:, :B, :k_eff] = \
-            out.view(B, rows, k_eff).permute(1, 0, 2)
+                                lengths=self._row(_SEQ_LEN), upper_bound=bound, segment=k)
 
     def attend_sparse(self, q: torch.Tensor, layer_idx: int, fresh=None) -> torch.Tensor:
         """Attention over the persisted token lists (``fresh`` as in ``attend_full``)."""

@@ -303,4 +303,37 @@ __host__ __device__ __forceinline__ int64_t ceil_div64(int64_t a, int64_t b) {
   return (a + b - 1) / b;
 }
 
+// Integer prefix sums and maxima over a wavefront by DPP
+template <int CTRL>
+__device__ __forceinline__ uint32_t dpp_u32(uint32_t x) {  // 0 where the source lane does not exist
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, 0xf, 0xf, true);
+}
+// inclusive prefix sum inside every row of 16 lanes (row_shr:1,2,4,8)
+__device__ __forceinline__ uint32_t row_prefix_sum(uint32_t x) {
+  x += dpp_u32<0x111>(x);
+  x += dpp_u32<0x112>(x);
+  x += dpp_u32<0x114>(x);
+  x += dpp_u32<0x118>(x);
+  return x;
+}
+// inclusive prefix sum over the wavefront
+__device__ __forceinline__ uint32_t wave_prefix_sum_dpp(uint32_t x, int lane) {
+  x = row_prefix_sum(x);
+  const uint32_t t0 = __builtin_amdgcn_readlane(x, 15), t1 = __builtin_amdgcn_readlane(x, 31),
+                 t2 = __builtin_amdgcn_readlane(x, 47);
+  return x + (lane >= 16 ? t0 : 0u) + (lane >= 32 ? t1 : 0u) + (lane >= 48 ? t2 : 0u);
+}
+// maximum over the wavefront (rows of 16 lanes by DPP, then the four rows); result in a scalar
+__device__ __forceinline__ int32_t wave_max_i32(int32_t x) {
+  int32_t y;
+  y = (int32_t)dpp_u32<0xB1>((uint32_t)x), x = x > y ? x : y;   // quad_perm [1,0,3,2]
+  y = (int32_t)dpp_u32<0x4E>((uint32_t)x), x = x > y ? x : y;   // quad_perm [2,3,0,1]
+  y = (int32_t)dpp_u32<0x141>((uint32_t)x), x = x > y ? x : y;  // row_half_mirror
+  y = (int32_t)dpp_u32<0x140>((uint32_t)x), x = x > y ? x : y;  // row_mirror
+  const int32_t a = __builtin_amdgcn_readlane(x, 0), b = __builtin_amdgcn_readlane(x, 16),
+                c = __builtin_amdgcn_readlane(x, 32), d = __builtin_amdgcn_readlane(x, 48);
+  const int32_t ab = a > b ? a : b, cd = c > d ? c : d;
+  return ab > cd ? ab : cd;
+}
+
 }  // namespace tidal

@@ -78,6 +78,7 @@ struct DecodeParams {
   float* ws_ml;     // [batch * H_q * max_splits, 2]
   int32_t* ws_cnt;  // [batch * head rows] ticket counters, ticket_stride words apart
   int32_t ticket_stride;
+  int32_t batch, slots;  // balanced launches: sequences, and workgroups per head row
   // the token being decoded (FRESH kernels): un-rotated k, v, its rotary cos/sin and its slot
   const void* fresh_k;
   const void* fresh_v;
@@ -126,9 +127,10 @@ __device__ __forceinline__ void load_coherent(const float* src, float& a, float&
 // Reduce the n_splits partial results of the QPG query heads of one head row and write o (and
 // lse).  Runs in one workgroup of NT threads: NT / (QPG * D / 2) "slots" of threads each own a
 // float2 column and a subset of the splits; slots are combined through LDS.
+// part_first: the partial of head slot 0 and split 0; part_heads: partials from one head slot to the next.
 template <typename T, int D, int QPG, int NT>
-__device__ __forceinline__ void merge_splits(const DecodeParams& p, int b, int qh0, int rq0, int gsz,
-                                             int n_splits) {
+__device__ __forceinline__ void merge_splits(const DecodeParams& p, int b, int64_t part_first, int part_heads,
+                                             int rq0, int gsz, int n_splits) {
   constexpr int COLS = QPG * D / 2;
   constexpr int SLOTS = NT / COLS;
   constexpr int PRE = SLOTS >= 8 ? 4 : (SLOTS >= 4 ? 8 : 16);  // partial loads in flight per thread
@@ -138,7 +140,7 @@ __device__ __forceinline__ void merge_splits(const DecodeParams& p, int b, int q
   const int tid = threadIdx.x;
   const int c = tid % COLS, slot = tid / COLS;
   const int j = c / (D / 2), d2 = c % (D / 2);
-  const int64_t part0 = ((int64_t)b * p.vheads + qh0 + j) * p.max_splits;
+  const int64_t part0 = part_first + (int64_t)j * part_heads;
 
   // (m, l) of every split and head: one pair per thread; the load is unconditional (clamped
   // thread index) so that it is in flight together with the partial loads below
@@ -147,8 +149,7 @@ __device__ __forceinline__ void merge_splits(const DecodeParams& p, int b, int q
   {
     const int tc = has_ml ? tid : 0;
     const int jj = tc / n_splits, ss = tc % n_splits;
-    load_coherent(p.ws_ml + (((int64_t)b * p.vheads + qh0 + jj) * p.max_splits + ss) * 2,
-                  ml_m, ml_l);
+    load_coherent(p.ws_ml + (part_first + (int64_t)jj * part_heads + ss) * 2, ml_m, ml_l);
   }
   // Loads are unconditional (index clamped, contribution zeroed) so that a batch of PRE of them
   // is in flight per thread; a branch around a load makes the compiler wait for each one.
@@ -258,8 +259,14 @@ __device__ __forceinline__ int seq_items(const DecodeParams& p, int b, SeqList& 
   return n_splits < 1 ? 1 : n_splits;
 }
 
-template <typename T, int D, int QPG, int U, int NW, bool PAGE_MODE, bool EMIT, bool LEAN, bool FRESH>
-__global__ __launch_bounds__(NW * 64) void decode_attn_kernel(const DecodeParams p) {
+// One of the n splits of a sequence; PLANNED: n is what the plan's chunk size gives, and the partials are
+// where the plan has them, else part_first is the first partial of the sequence in those of a head slot.
+struct Share {
+  int split, n_splits, part_first;
+};
+
+template <typename T, int D, int QPG, int U, int NW, bool PAGE_MODE, bool EMIT, bool LEAN, bool FRESH, bool PLANNED>
+__device__ __forceinline__ void attend_share(const DecodeParams& p, const int hrow, const int b, const Share& share) {
   static_assert(!FRESH || LEAN, "the fused decode step exists for the lean addressing only");
   constexpr int LPR = D / 8;     // lanes per K/V row
   constexpr int TPI = 64 / LPR;  // tokens one wave instruction covers
@@ -271,21 +278,19 @@ __global__ __launch_bounds__(NW * 64) void decode_attn_kernel(const DecodeParams
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane / LPR;   // lane group = token slot inside the instruction
   const int li = lane % LPR;  // 16-byte column of the row
-  // Splits are the slowest grid dimension: a sequence shorter than the planned maximum leaves its
-  // last splits without work, and those workgroups then reach the dispatcher after all the others
-  // instead of between them (where each one that ends at once hands its place to a workgroup that
-  // should have gone to an empty compute unit).
-  const int hrow = blockIdx.x;
-  const int b = blockIdx.y;
-  const int split = blockIdx.z;
+  const int split = share.split;
   const int qh0 = hrow * QPG;  // first head slot of this head row in the split workspace
   int kv_head, rq0, gsz;       // KV head, first query head, query heads that really exist in the row
   head_row_geom<QPG>(p, hrow, kv_head, rq0, gsz);
 
   SeqList s;
   int list_beg;
-  const int n_splits = seq_items(p, b, s, list_beg);
+  const int planned = seq_items(p, b, s, list_beg);
+  const int n_splits = PLANNED ? planned : share.n_splits;
   if (split >= n_splits) return;  // uniform for the whole workgroup
+  const int64_t part_first = PLANNED ? ((int64_t)b * p.vheads + qh0) * p.max_splits
+                                     : (int64_t)qh0 * p.slots + share.part_first;
+  const int part_heads = PLANNED ? p.max_splits : p.slots;
   const int idx_row = (QPG > 1 || p.idx_per_kv) ? kv_head : hrow;
   s.row = p.idx + (int64_t)idx_row * p.idx_row_stride + list_beg;
 
@@ -505,7 +510,7 @@ __global__ __launch_bounds__(NW * 64) void decode_attn_kernel(const DecodeParams
   __shared__ float emit_buf[EMIT ? NW * EMIT_FLOATS : 1];
   int emit_n = 0;       // tiles waiting in the strip
   int emit_first = 0;   // first token of the oldest waiting tile
-  const int emit_step = n_splits * NW * TILE;  // tokens between two tiles of this wave
+  const int STEP = n_splits * NW * TILE;  // tokens between two tiles of this wave
   auto emit_flush = [&]() {
     if constexpr (EMIT) {
       // The strip was written by other lanes of this wave than the ones that now read it.  LDS
@@ -519,7 +524,7 @@ __global__ __launch_bounds__(NW * 64) void decode_attn_kernel(const DecodeParams
       const int lt = lane / TILE, ltok = lane % TILE;
       for (int n0 = 0; n0 < emit_n; n0 += TPS) {
         const int n = n0 + lt;
-        const int i = emit_first + n * emit_step + ltok;
+        const int i = emit_first + n * STEP + ltok;
 #pragma unroll
         for (int j = 0; j < QPG; ++j) {
           if (n < emit_n && i < c1 && j < gsz) {
@@ -722,8 +727,7 @@ __global__ __launch_bounds__(NW * 64) void decode_attn_kernel(const DecodeParams
     }
   };
 
-  const int STEP = n_splits * NW * TILE;  // tokens between two tiles of one wave
-  int t = (split * NW + wave) * TILE;     // first token of this wave's current tile
+  int t = (split * NW + wave) * TILE;  // first token of this wave's current tile
   if (t < c1) {
     fetch_list(t, rawA);
     if (t + STEP < c1) fetch_list(t + STEP, rawB);
@@ -830,7 +834,7 @@ __global__ __launch_bounds__(NW * 64) void decode_attn_kernel(const DecodeParams
         if (p.lse && lane == 0)
           p.lse[(int64_t)b * p.num_qo_heads + qh] = L > 0.f ? (M + fast_log2(L)) * kLn2 : -INFINITY;
       } else {
-        const int64_t part = ((int64_t)b * p.vheads + qh0 + j) * p.max_splits + split;
+        const int64_t part = part_first + (int64_t)j * part_heads + split;
         float* dst = p.ws_o + part * D + lane * 8;
         store_coherent(dst + 0, r[0], r[1]);
         store_coherent(dst + 2, r[2], r[3]);
@@ -856,13 +860,69 @@ __global__ __launch_bounds__(NW * 64) void decode_attn_kernel(const DecodeParams
   // clobber), or dropping the barrier between the waves' waits and the ticket.
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
-  int32_t* ticket = p.ws_cnt + ((int64_t)b * gridDim.x + hrow) * p.ticket_stride;
+  int32_t* ticket = p.ws_cnt + ((int64_t)b * p.n_hrows + hrow) * p.ticket_stride;
   if (tid == 0)
     sm_ticket = __hip_atomic_fetch_add(ticket, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   __syncthreads();
   if (sm_ticket != n_splits - 1) return;
-  merge_splits<T, D, QPG, NW * 64>(p, b, qh0, rq0, gsz, n_splits);
+  merge_splits<T, D, QPG, NW * 64>(p, b, part_first, part_heads, rq0, gsz, n_splits);
   if (tid == 0) __hip_atomic_store(ticket, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Splits are the slowest grid dimension: a sequence shorter than the planned maximum leaves its
+// last splits without work, and those workgroups then reach the dispatcher after all the others
+// instead of between them (where each one that ends at once hands its place to a workgroup that
+// should have gone to an empty compute unit).
+template <typename T, int D, int QPG, int U, int NW, bool PAGE_MODE, bool EMIT, bool LEAN, bool FRESH>
+__global__ __launch_bounds__(NW * 64) void decode_attn_kernel(const DecodeParams p) {
+  attend_share<T, D, QPG, U, NW, PAGE_MODE, EMIT, LEAN, FRESH, true>(p, blockIdx.x, blockIdx.y,
+                                                                     Share{(int)blockIdx.z, 0, 0});
+}
+
+// A ragged batch on the shared-row kernels, of which a compute unit holds one: the workgroups of whole
+// rounds (p.slots per head row) are dealt to the sequences by their lengths, read on the device, so that
+// the longest piece is as short as that number allows.  With chunks planned from the longest sequence the
+// launch lasts as long as the largest remainder of one, and a batch of short sequences leaves most of the
+// chip idle.  One MI355X, bf16, logits out, even chunks -> dealt (us): 16 sequences of 500 .. 8192 tokens,
+// 32/8 heads x 128, 77 -> 69.7 (4.7 TB/s); 8 of 8000 .. 60000, 295 -> 261; 4 of 2000, 36.7 -> 15.8; 12 of
+// 400 .. 9000, 28/4 heads, 59.7 -> 51.  The lengths and the search cost 1.5 us, which is what equal lengths
+// lose (16 x 8192: 98.9 -> 100.7).  Runs of equal length laid over the ends of the sequences balance better
+// still but pay the start and the merge of every further sequence, 5 us: 72 for the first batch, 110 for
+// 16 x 8192.
+constexpr int kBalancedMaxBatch = 64;  // one lane per sequence
+
+template <typename T, int D, int QPG, int U, int NW, bool EMIT, bool LEAN, bool FRESH>
+__global__ __launch_bounds__(NW * 64) void decode_attn_balanced_kernel(const DecodeParams p) {
+  constexpr int WTILE = NW * U * (64 / (D / 8));  // tokens of a workgroup-wide tile
+  const int lane = threadIdx.x & 63, slot = blockIdx.y;
+  SeqList mine;
+  int beg;
+  seq_items(p, lane < p.batch ? lane : p.batch - 1, mine, beg);
+  int tiles = (mine.n_items + WTILE - 1) / WTILE;
+  tiles = lane < p.batch ? (tiles < 1 ? 1 : tiles) : 0;
+  // the shortest piece, in tiles, for which all sequences together have no more pieces than slots: lane l
+  // tries the l-th of 64 lengths between the mean and the longest sequence, which always fits
+  const int sum = (int)__builtin_amdgcn_readlane(wave_prefix_sum_dpp((uint32_t)tiles, lane), 63);
+  const int most = wave_max_i32(tiles);
+  const int least = (sum + p.slots - 1) / p.slots;  // <= most: slots >= batch
+  const int piece = least + (most - least) * lane / 63;
+  const float inv = 1.f / (float)piece;
+  int pieces = 0;
+  for (int b = 0; b < p.batch; ++b) {
+    const int n = __builtin_amdgcn_readlane(tiles, b);
+    int q = (int)((float)n * inv);  // within one of the quotient
+    q += (q + 1) * piece <= n ? 1 : 0;
+    q -= q * piece > n ? 1 : 0;
+    pieces += q + (q * piece < n ? 1 : 0);
+  }
+  const uint64_t fits = __ballot(pieces <= p.slots);
+  const int chosen = __builtin_amdgcn_readlane(piece, __builtin_ctzll(fits | (1ull << 63)));
+  const int n_splits = lane < p.batch ? (tiles + chosen - 1) / chosen : 0;
+  const int upto = (int)wave_prefix_sum_dpp((uint32_t)n_splits, lane);  // pieces of the sequences up to this lane's
+  const int b = __popcll(__ballot(lane < p.batch && upto <= slot));
+  if (b >= p.batch) return;
+  const int n = __builtin_amdgcn_readlane(n_splits, b), first = __builtin_amdgcn_readlane(upto, b) - n;
+  attend_share<T, D, QPG, U, NW, true, EMIT, LEAN, FRESH, false>(p, blockIdx.x, b, Share{slot - first, n, first});
 }
 
 // Second-kernel merge (plan.fused_merge == 0): one workgroup per (head row, sequence).
@@ -876,7 +936,8 @@ __global__ __launch_bounds__(NT) void merge_partials_kernel(const DecodeParams p
   if (n_splits <= 1) return;  // the attention kernel already wrote the final result
   int kv_head, rq0, gsz;
   head_row_geom<QPG>(p, hrow, kv_head, rq0, gsz);
-  merge_splits<T, D, QPG, NT>(p, b, hrow * QPG, rq0, gsz, n_splits);
+  merge_splits<T, D, QPG, NT>(p, b, ((int64_t)b * p.vheads + hrow * QPG) * p.max_splits, p.max_splits, rq0, gsz,
+                              n_splits);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -910,6 +971,17 @@ static int qpg_for(int num_qo_heads, int num_kv_heads, int idx_rows, int head_di
   return shape_supported(head_dim, padded, 8) ? padded : 1;
 }
 
+template <typename T, int D, int QPG, int NW, int U, bool EMIT>
+static void launch_balanced(const DecodeParams& p, dim3 grid, hipStream_t st) {
+  const dim3 even(grid.x, p.slots);
+  if (p.lean && p.fresh_k)
+    hipLaunchKernelGGL((decode_attn_balanced_kernel<T, D, QPG, U, NW, EMIT, true, true>), even, dim3(NW * 64), 0, st, p);
+  else if (p.lean)
+    hipLaunchKernelGGL((decode_attn_balanced_kernel<T, D, QPG, U, NW, EMIT, true, false>), even, dim3(NW * 64), 0, st, p);
+  else
+    hipLaunchKernelGGL((decode_attn_balanced_kernel<T, D, QPG, U, NW, EMIT, false, false>), even, dim3(NW * 64), 0, st, p);
+}
+
 template <typename T, int D, int QPG, int NW, int U, bool PAGE_MODE, bool EMIT>
 static void launch_lean(const DecodeParams& p, dim3 grid, hipStream_t st) {
   if (p.lean && p.fresh_k)
@@ -926,6 +998,15 @@ static void launch_lean(const DecodeParams& p, dim3 grid, hipStream_t st) {
 template <typename T, int D, int QPG, int NW, int U>
 static void launch_variant(const DecodeParams& p, bool page_mode, bool emit, bool merge_kernel,
                            dim3 grid, hipStream_t st) {
+  if constexpr (QPG > 1) {
+    if (p.slots > 0) {
+      if (emit)
+        launch_balanced<T, D, QPG, NW, U, true>(p, grid, st);
+      else
+        launch_balanced<T, D, QPG, NW, U, false>(p, grid, st);
+      return;
+    }
+  }
   if (page_mode) {
     if (emit)
       launch_lean<T, D, QPG, NW, U, true, true>(p, grid, st);

@@ -33,6 +33,14 @@ constexpr int64_t kTicketBytes = (int64_t)16384 * kTicketStride * 4;
 // head; longer lists go to the streaming kernel, whose waves pipeline several tiles.
 constexpr int64_t kSparseMaxItems = 64 * 256;
 
+// Workgroups per head row of a balanced launch (decode_attn_balanced_kernel): as many rounds of one per
+// compute unit as give every sequence one; at most 64 pieces of a sequence are merged.
+static int balanced_slots(int n_hrows, int batch) {
+  const int round = num_cus() / n_hrows < 1 ? 1 : num_cus() / n_hrows;
+  const int64_t slots = ceil_div64(batch, round) * round;
+  return (int)(slots > 64 ? 64 : slots);
+}
+
 static bool is_pow2(int64_t x) { return x > 0 && (x & (x - 1)) == 0; }
 
 }  // namespace tidal
@@ -239,6 +247,13 @@ extern "C" int td_decode_make_plan(int32_t batch, int32_t num_qo_heads, int32_t 
     max_splits = ceil_div64(max_items, chunk);
   }
   if (max_splits < 1) max_splits = 1;
+  // room for the partials of a balanced launch (one per slot and head slot), unless that alone would take
+  // the plan beyond the built-in scratch
+  if (batch > 1 && batch <= kBalancedMaxBatch && qpg > 1 && plan->chunk_tokens == 0) {
+    const int64_t wanted = ceil_div64(balanced_slots(n_hrows, batch), batch);
+    const int64_t bytes = kTicketBytes + (int64_t)batch * n_hrows * qpg * wanted * (head_dim + 2) * 4 + 512;
+    if (wanted > max_splits && bytes <= (int64_t)TD_STATIC_SCRATCH_BYTES) max_splits = wanted;
+  }
 
   plan->chunk_tokens = (int32_t)chunk;
   plan->max_splits = (int32_t)max_splits;
@@ -402,6 +417,14 @@ static int build_params(const td_paged_kv* kv, const td_index_list* list, const 
   char* ws = reinterpret_cast<char*>(workspace);
   p.ws_cnt = reinterpret_cast<int32_t*>(ws);
   p.ticket_stride = kTicketStride;
+  p.batch = batch;
+  // Balanced: the full attention of a batch on the shared-row kernels, merged in the launch, when the
+  // workspace holds its partials.
+  p.slots = 0;
+  if (qpg > 1 && batch > 1 && batch <= kBalancedMaxBatch && list->kind == TD_IDX_PAGES && plan->fused_merge) {
+    const int slots = balanced_slots(n_hrows, batch);
+    if ((int64_t)batch * plan->max_splits >= slots) p.slots = slots;
+  }
   p.ws_o = reinterpret_cast<float*>(ws ? ws + off_o : nullptr);
   p.ws_ml = reinterpret_cast<float*>(ws ? ws + off_ml : nullptr);
 

@@ -649,43 +649,11 @@ constexpr int kSliceCand = 1024;    // list entries in LDS; a fuller bin gets an
 constexpr int kSliceRank = 128;     // lists up to this size are ranked directly
 constexpr int kSliceMaxRuns = 64;   // 1024-element runs a slice may hold
 
-template <int CTRL>
-__device__ __forceinline__ uint32_t dpp_u32(uint32_t x) {  // 0 where the source lane does not exist
-  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, 0xf, 0xf, true);
-}
-// inclusive prefix sum inside every row of 16 lanes (row_shr:1,2,4,8)
-__device__ __forceinline__ uint32_t row_prefix_sum(uint32_t x) {
-  x += dpp_u32<0x111>(x);
-  x += dpp_u32<0x112>(x);
-  x += dpp_u32<0x114>(x);
-  x += dpp_u32<0x118>(x);
-  return x;
-}
-// inclusive prefix sum over the wavefront
-__device__ __forceinline__ uint32_t wave_prefix_sum_dpp(uint32_t x, int lane) {
-  x = row_prefix_sum(x);
-  const uint32_t t0 = __builtin_amdgcn_readlane(x, 15), t1 = __builtin_amdgcn_readlane(x, 31),
-                 t2 = __builtin_amdgcn_readlane(x, 47);
-  return x + (lane >= 16 ? t0 : 0u) + (lane >= 32 ? t1 : 0u) + (lane >= 48 ? t2 : 0u);
-}
 // arr[0] + ... + arr[n - 1], n <= 16 and the same in the whole wavefront; result in a scalar
 __device__ __forceinline__ uint32_t sum_first(const uint32_t* arr, int n, int lane) {
   const uint32_t v = row_prefix_sum(lane < n ? arr[lane & 15] : 0u);
   return __builtin_amdgcn_readlane(v, 15);
 }
-// maximum over the wavefront (rows of 16 lanes by DPP, then the four rows); result in a scalar
-__device__ __forceinline__ int32_t wave_max_i32(int32_t x) {
-  int32_t y;
-  y = (int32_t)dpp_u32<0xB1>((uint32_t)x), x = x > y ? x : y;   // quad_perm [1,0,3,2]
-  y = (int32_t)dpp_u32<0x4E>((uint32_t)x), x = x > y ? x : y;   // quad_perm [2,3,0,1]
-  y = (int32_t)dpp_u32<0x141>((uint32_t)x), x = x > y ? x : y;  // row_half_mirror
-  y = (int32_t)dpp_u32<0x140>((uint32_t)x), x = x > y ? x : y;  // row_mirror
-  const int32_t a = __builtin_amdgcn_readlane(x, 0), b = __builtin_amdgcn_readlane(x, 16),
-                c = __builtin_amdgcn_readlane(x, 32), d = __builtin_amdgcn_readlane(x, 48);
-  const int32_t ab = a > b ? a : b, cd = c > d ? c : d;
-  return ab > cd ? ab : cd;
-}
-
 struct SliceLds {
   uint32_t hist[kSliceBins];
   uint32_t cd[kSliceCand];   // list: d of the members of the threshold bin

@@ -1,0 +1,123 @@
+"""The native half of the entry points (csrc/host_calls.cpp): whatever it does not take as regular goes on in
+Python with the same result or the same error, and what it takes gives the bits that Python gives."""
+import numpy as np
+import pytest
+import torch
+
+from tidaldecode_amd import _kernels
+from tidaldecode_amd._lib import host_calls
+
+_NATIVE = ("forward", "attend", "topk", "rope_table", "rope_in_place", "append", "prefill", "gemv", "score_reduce",
+           "estimate")
+
+
+class _Off:
+    """host_calls with every function declining"""
+
+    def __getattr__(self, name):
+        assert name in _NATIVE
+        return lambda *a: False
+
+
+def test_wrong_argument_counts_are_type_errors():
+    for name in _NATIVE:
+        with pytest.raises(TypeError):
+            getattr(host_calls, name)(1, 2)
+
+
+def test_host_tensors_are_refused_as_before():
+    q = torch.zeros(1, 4, 64)
+    with pytest.raises(RuntimeError, match="q must be a CUDA tensor"):
+        _kernels.apply_rope_in_place(q, q, 0, 1.0, 1e4)
+    with pytest.raises(RuntimeError, match="must be a CUDA tensor"):
+        _kernels.topk_filtering(torch.zeros(2, 8), None, None, torch.zeros(2, 4, dtype=torch.int32), None, 4)
+    with pytest.raises(RuntimeError, match="must be a CUDA tensor"):
+        _kernels.gemv(torch.zeros(4, 8), torch.zeros(8))
+    assert host_calls.topk(q, None, None, q, None, 4, None, 1, None, None, None, 0, None) is False
+    assert host_calls.gemv(object(), None, None, 1e-5, False, None, False, None, 0) is False
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("heads,kv,d,page,layout,mode", [(8, 8, 128, 16, "NHD", "per_head"),
+                                                         (8, 2, 64, 4, "HND", "group_sum"),
+                                                         (4, 4, 256, 7, "NHD", "per_head")])
+def test_same_bits_as_the_python_path(cuda, monkeypatch, dtype, heads, kv, d, page, layout, mode):
+    from tidaldecode_amd import utils as ops
+    from tidaldecode_amd.utils import InferenceController
+
+    def run(native):
+        if not native:
+            monkeypatch.setattr(_kernels, "host_calls", _Off())
+            monkeypatch.setattr(ops, "host_calls", _Off())
+        g = torch.Generator(device=cuda).manual_seed(7)
+        randn = lambda *s: torch.randn(s, generator=g, device=cuda).to(dtype)
+        c = InferenceController(2, heads, d, page, 40, 400, dtype, cuda, num_kv_heads=kv, select_mode=mode,
+                                kv_layout=layout, page_order_seed=5)
+        c.kv_cache.pool.buf.zero_()
+        out = []
+        q, k, v = randn(300, heads, d), randn(300, kv, d), randn(300, kv, d)
+        c.prepare_metadata(300)
+        c.begin_forward(300)
+        ops.apply_rope_in_place(q, k, 0)
+        for layer in range(2):
+            ops.append_kv(k, v, c, layer)
+            out.append(ops.prefill_forward(q, c, layer))
+        for step in range(2):
+            c.prepare_metadata(1)
+            c.begin_forward(1)
+            q, k, v = randn(1, heads, d), randn(1, kv, d), randn(1, kv, d)
+            pos = torch.tensor([300 + step], dtype=torch.int32, device=cuda)
+            out += list(_kernels.rope_table(pos, d, 1.0, 5e5))
+            ops.apply_rope_in_place(q, k, 300 + step)
+            for layer in range(2):
+                ops.append_kv(k, v, c, layer)
+                if layer == 0:
+                    out.append(ops.decode_sparse_attn(q, c, layer, c.kv_indices_without_last, True))
+                    ops.decode_topk(c)
+                else:
+                    out.append(ops.decode_sparse_attn(q, c, layer, c.topk_dindices_buffer, False))
+            out += [c.qk_product.clone(), c.lse.clone(), c.topk_dindices_buffer.clone()]
+        w, x = randn(48, 64), randn(64)
+        out += [_kernels.gemv(w, x), _kernels.gemv(w, x, norm_weight=randn(64), pair_gated=True),
+                _kernels.gemv(w, x, residual=randn(48))]
+        torch.cuda.synchronize()
+        return out + [c.kv_cache.pool.buf]
+
+    a, b = run(True), run(False)
+    assert len(a) == len(b)
+    for x, y in zip(a, b):
+        assert x.dtype == y.dtype and x.shape == y.shape and torch.equal(x, y)
+
+
+@pytest.mark.gpu
+def test_irregular_forms_still_work(cuda):
+    """numpy integers, a value output, a workspace that is missing or too small, errors of the library."""
+    g = torch.Generator(device=cuda).manual_seed(1)
+    v = torch.randn((4, 500), generator=g, device=cuda)
+    out, vals = torch.zeros((4, 30), dtype=torch.int32, device=cuda), torch.zeros((4, 30), device=cuda)
+    _kernels.topk_filtering(v, None, vals, out, None, 30)
+    assert torch.equal(vals, torch.gather(v, 1, out.long()))
+    other = torch.zeros_like(out)
+    _kernels.topk_filtering(v, None, None, other, None, np.int64(30))
+    assert torch.equal(out, other)
+
+    h, d, page, pages = 4, 128, 16, 40
+    pool = torch.randn((pages, 2, page, h, d), generator=g, device=cuda).half()
+    q = torch.randn((1, h, d), generator=g, device=cuda).half()
+    table = torch.arange(pages - 1, dtype=torch.int32, device=cuda)[None]
+    w = _kernels.BatchDecodeWithPagedKVCachePyTorchWrapper(0)
+    o = torch.empty_like(q)
+    with pytest.raises(RuntimeError, match="BeginForward"):
+        w.forward(q, o, pool, table, None, 3, pages - 1, None)
+    w.begin_forward(None, h, h, d, page, torch.empty(0, dtype=torch.half))
+    first = None
+    for kw in ({}, dict(n_list=np.int64(pages - 1)), dict(n_list=pages - 1)):
+        w._workspace = None if first is None else torch.zeros(8, dtype=torch.uint8, device=cuda)
+        w.forward(q, o, pool, table, None, 3, pages - 1, None, **kw)
+        first = o.clone() if first is None else first
+        assert torch.equal(o, first) and w._workspace.numel() > 8
+    with pytest.raises(RuntimeError, match="o must have the shape of q"):
+        w.forward(q, o[:, :2].contiguous(), pool, table, None, 3, pages - 1, None)
+    with pytest.raises(RuntimeError, match="last_page_len"):
+        w.forward(q, o, pool, table, None, page + 1, pages - 1, None)

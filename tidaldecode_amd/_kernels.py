@@ -10,6 +10,9 @@ reference.  Differences, all additive:
 * ``forward`` writes ``qk_product`` when a non-empty tensor is passed (the reference's binding
   drops it, tidal/ops/csrc/approx_attn.cu:137) in list order, as natural-log-domain logits
   ``q.k/sqrt(D)``.
+* the regular case of the calls a decode step makes goes through one native call
+  (``csrc/host_calls.cpp``: same checks, same launch); what follows such a call in a function below
+  raises the errors and serves the irregular forms.
 * kernels run on torch's current stream (the reference always uses the null stream, which is
   torch's default current stream).
 """
@@ -20,7 +23,7 @@ import torch
 
 from . import _lib
 from ._lib import (DecodePlan, FreshToken, IndexList, PagedKV, TD_BF16, TD_F16, TD_F32, TD_HND, TD_IDX_PAGES,
-                   TD_IDX_SLOTS, TD_NHD, check, lib)
+                   TD_IDX_SLOTS, TD_NHD, check, host_calls, lib)
 
 _DTYPES = {torch.float16: TD_F16, torch.bfloat16: TD_BF16, torch.float32: TD_F32}
 
@@ -89,6 +92,8 @@ def _pool(kv_data: torch.Tensor, layout: int, name: str = "kv_data") -> PagedKV:
 def apply_rope_in_place(q: torch.Tensor, k: torch.Tensor, past_kv_len: int, rope_scale: float,
                         rope_theta: float) -> None:
     """bsk_ops.h:23-27 / page.cu:212-253.  q ``[N, H_q, D]``, k ``[N, H_kv, D]``."""
+    if q.is_cuda and host_calls.rope_in_place(q, k, past_kv_len, rope_scale, rope_theta, _stream()):
+        return
     _check_input(q, "q")
     _check_input(k, "k")
     _check_dim(3, q, "q")
@@ -178,6 +183,12 @@ def gemv(weight: torch.Tensor, x: torch.Tensor, *, norm_weight: Optional[torch.T
     ``residual`` (may be ``out``) is added to the product.  ``pair_gated``: ``weight`` stacks the
     gate and the up projection and ``out[i] = silu(weight[i] . f(x)) * (weight[i + rows/2] . f(x))``
     (``rows/2`` values).  Returns ``out``."""
+    if x.is_cuda and weight.dim() == 2:
+        if out is None:
+            n = weight.size(0)
+            out = torch.empty(n // 2 if pair_gated else n, dtype=x.dtype, device=x.device)
+        if host_calls.gemv(weight, x, norm_weight, eps, gated, residual, pair_gated, out, _stream()):
+            return out
     _check_input(x, "x")
     if not weight.is_cuda or weight.dim() != 2 or weight.stride(1) != 1:
         raise RuntimeError("gemv: weight must be a CUDA matrix with contiguous rows")
@@ -242,6 +253,10 @@ def topk_filtering(estimated_value: torch.Tensor, estimated_indices: Optional[to
     group are spread over the rows of ``indices_out`` ``[H / groups, >= groups * segment]``, each
     group in its own columns: row r of group g goes to ``indices_out[r, g * segment:]``.
     """
+    if d_out is None and estimated_value.is_cuda and host_calls.topk(
+            estimated_value, estimated_indices, d_out, indices_out, buf, page_budget, page_table, page_size, lengths,
+            upper_bound, segment, _stream(), None):
+        return
     _check_rows(estimated_value, "estimated_value")
     rows, length = estimated_value.shape
     in_ptr, in_stride = None, 0
@@ -331,6 +346,9 @@ def estimate_attn_score(q: torch.Tensor, o: torch.Tensor, metadata_data: torch.T
     metadata entries of ``metadata_indices`` except the newest one; ``q [1, H, D]``,
     ``o [H, entries]``.  ``metadata_indptr`` and ``metadata_last_page_idx`` are accepted for
     signature parity (all pages of ``metadata_indices`` are used, the last one is its last)."""
+    if q.is_cuda and host_calls.estimate(q, o, metadata_data, metadata_indices, metadata_last_page_len, layout,
+                                         _stream()):
+        return
     _check_input(q, "q")
     _check_dim(3, q, "q")
     _check_input(o, "o")
@@ -352,6 +370,10 @@ def estimate_attn_score(q: torch.Tensor, o: torch.Tensor, metadata_data: torch.T
 
 def _append(k, v, kv_data, kv_indices, kv_indptr, kv_last_page_len, metadata_data,
             metadata_indices, metadata_indptr, metadata_last_page_len, layout, decode: bool):
+    if k.is_cuda and host_calls.append(k, v, kv_data, kv_indices, kv_indptr, kv_last_page_len, metadata_data,
+                                       metadata_indices, metadata_indptr, metadata_last_page_len, layout, decode,
+                                       _stream()):
+        return
     # checks of tidal/ops/csrc/page.cu:19-55
     for t, n in ((k, "k"), (v, "v"), (kv_indices, "kv_indices")):
         _check_input(t, n)
@@ -504,6 +526,10 @@ def rope_table(positions: torch.Tensor, head_dim: int, rope_scale: float = 1.0,
                sin: Optional[torch.Tensor] = None):
     """Extension: cos / sin ``[B, D/2]`` float32 of the rotary angles of ``positions`` ``[B]``
     (int32); one call per decode step feeds every layer's fused ``forward(..., fresh=...)``."""
+    if cos is None and sin is None and positions.is_cuda:
+        made = host_calls.rope_table(positions, head_dim, rope_scale, rope_theta, _stream())
+        if made:
+            return made
     _check_input(positions, "positions")
     _check_i32(positions, "positions")
     b = positions.numel()
@@ -523,6 +549,10 @@ def prefill_with_paged_kv_cache(q, kv_data, kv_indices, kv_last_page_len, causal
     (``td_prefill_attn``; head_dim 64, 128 or 256).  ``allow_fp16_qk_reduction``, ``rope_scale``
     and ``rope_theta`` are accepted for signature parity: RoPE is applied before the cache is
     written (RotaryMode::kNone in the reference's call, batch_prefill.cu:95)."""
+    if q.is_cuda:
+        o = torch.empty_like(q)
+        if host_calls.prefill(q, o, kv_data, kv_indices, kv_last_page_len, causal, layout, _stream()):
+            return o
     _check_input(q, "q")
     _check_dim(3, q, "q")
     _check_input(kv_indices, "kv_indices")
@@ -633,6 +663,10 @@ class BatchDecodeWithPagedKVCachePyTorchWrapper:
         UN-rotated, cos/sin ``[B, D/2]`` float32 come from ``rope_table``; the kernel rotates q
         in registers, writes rotated k and v to ``dst_slot`` and attends to them from registers
         (power-of-two pages and pools below 4 GiB only)."""
+        if q.is_cuda and (index_kind == "slots" or index_kind == "pages") and host_calls.forward(
+                self, q, o, paged_kv_data, paged_kv_indices, paged_kv_indptr, paged_kv_last_page_len,
+                paged_kv_last_page_idx, qk_product, index_kind == "slots", lse, n_list, fresh, counts, _stream()):
+            return
         if not self._begun:
             raise RuntimeError("Please call BatchDecodeHandler's BeginForward() before calling "
                                "BatchDecodeWithPagedKVCacheWrapper()")
@@ -792,9 +826,10 @@ def score_reduce(logits: torch.Tensor, lse: torch.Tensor, num_kv_heads: int, n: 
     rows = 1 if mode == "head_sum" else int(num_kv_heads)
     if out is None:
         out = torch.empty((rows, n), dtype=torch.float32, device=logits.device)
+    reduce_mode = _lib.TD_REDUCE_HEAD_SUM if mode == "head_sum" else _lib.TD_REDUCE_GROUP_SUM
+    if host_calls.score_reduce(logits, lse, num_kv_heads, n, reduce_mode, out, _stream()):
+        return out
     check(lib.td_score_reduce(logits.data_ptr(), logits.stride(0), lse.data_ptr(), hq,
                               int(num_kv_heads), int(n),
-                              _lib.TD_REDUCE_HEAD_SUM if mode == "head_sum"
-                              else _lib.TD_REDUCE_GROUP_SUM,
-                              out.data_ptr(), out.stride(0), _stream()))
+                              reduce_mode, out.data_ptr(), out.stride(0), _stream()))
     return out

@@ -217,6 +217,21 @@ def _load():
 lib = _load()
 
 
+def _load_host_calls():
+    """The native half of the Python entry points (csrc/host_calls.cpp), bound to ``lib``."""
+    import torch  # noqa: F401  (its libraries are what the module links against)
+    try:
+        from . import _host_calls
+    except ImportError as e:
+        raise RuntimeError(f"{os.path.join(_HERE, '_host_calls.so')} is missing or stale ({e}): build it with "
+                           f"`make -C {os.path.join(_HERE, 'csrc')}`. tidaldecode_amd has no fallback path.") from e
+    _host_calls.bind({name: ctypes.cast(getattr(lib, name), c_void_p).value for name in SIGNATURES})
+    return _host_calls
+
+
+host_calls = _load_host_calls()
+
+
 def last_error() -> str:
     msg = lib.td_last_error()
     return msg.decode("utf-8", "replace") if msg else ""

@@ -10,6 +10,7 @@ from typing import Optional
 import torch
 
 from .. import _kernels
+from .._lib import host_calls
 from .batch_controller import BatchInferenceController
 from .controller import InferenceController
 from .paged import BatchDecodeWithPagedKVCacheWrapper, KvCache, KvPool, TensorLayout
@@ -111,6 +112,10 @@ def decode_topk(iController: InferenceController):
     if k == 0:
         return
     # no logit exceeds its head's log-sum-exp, no summed probability the head count
+    if c.select_mode == "per_head" and c.qk_product.is_cuda and host_calls.topk(
+            c.qk_product, None, None, c.topk_dindices_buffer, c.topk_buf, k, c.kv_indices_with_last, c.page_size, None,
+            c.lse, None, _kernels._stream(), n):
+        return
     scores, bound = c.qk_product, c.lse.view(-1)
     if c.select_mode != "per_head":
         _kernels.score_reduce(c.qk_product, c.lse.view(-1), c.num_kv_heads, n, c.select_mode,
@@ -135,8 +140,18 @@ def decode_sparse_attn(q: torch.Tensor, iController: InferenceController, layer_
     ``append_kv`` of the new token into this launch: q and k are then un-rotated.
     """
     c = iController
-    o = torch.empty_like(q)
     full = topk_indices is c.kv_indices_without_last
+    if q.is_cuda:
+        forced = full or c.select_scope == "exclude_last_page"
+        cache = c.kv_cache
+        o = host_calls.attend(c._decode_handler._wrapper, q, None, cache.pool.buf, topk_indices, None,
+                              cache.last_page_len if forced else 0, c.kv_last_page_idx if forced else 0,
+                              c.qk_product if output_qk_product else None, not full,
+                              c.lse if output_qk_product else None, None, fresh, None, _kernels._stream(),
+                              layer_idx % cache.pool.num_layers)
+        if o is not False:
+            return o
+    o = torch.empty_like(q)
     if full:
         c._decode_handler.forward(q, o, c.kv_cache.buf_layer(layer_idx), topk_indices, None,
                                   c.kv_cache.last_page_len, c.kv_last_page_idx,

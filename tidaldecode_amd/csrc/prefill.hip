@@ -26,7 +26,7 @@
 // Measured in turn on one card (bf16, pages of 16, us, before with one 128- or 256-row tile per query head and
 // 16x16x32 MFMA -> now): prompt of 32768 x 32 heads 8633 -> 7592 (1159 TFLOP/s; a 16384^3 library GEMM reached
 // 1332 in the same run, and cards differ by 7 %), 8192 x 32 over 8 KV heads 588 -> 495, 1000 x 32 36.6 -> 24.0,
-// 300 x 32 14.1 -> 10.6 (bound by the latency of its five key tiles and cold code); 500 new tokens on 32768
+// 300 x 32 14.1 -> 9.6 (staged kernel, two key groups: bound by the latency of five steps and cold code); 500 new tokens on 32768
 // cached ones, 32 heads 991 -> 285, over 8 KV heads 993 -> 252; 16 tokens, 8 KV heads 792 -> 33.
 // Rows past the end of the sequence are clamped (never out of the pool) and masked.
 
@@ -111,6 +111,7 @@ struct PrefillParams {
   // group), n_tiles workgroup tiles of bm of them, each cut into n_splits pieces of `chunk` keys.
   int32_t n_kv, n_rows, bm, n_tiles, n_splits, chunk, head_major;
   bool staged;     // prefill_attn_staged_kernel
+  int32_t key_groups;  // of it: 1 or 2
   float* part_o;   // [n_splits][n_kv * n_rows][D]: un-normalised partial results (n_splits > 1)
   float* part_ml;  // [n_splits][n_kv * n_rows][2]: running maximum (base 2) and denominator
 };
@@ -566,17 +567,18 @@ __global__ __launch_bounds__(512, 2) void prefill_attn_kernel(const PrefillParam
   }
 }
 
-// head_dim 256, whose output alone would take 128 registers of a wave in the kernel above; caches of up to 64
-// tokens; and pools that are not 16-byte aligned, which direct loads to LDS are not specified for: four waves of
-// 16 query rows and 16x16x32 MFMA, 32 tokens per key tile.
+// head_dim 256, whose output alone would take 128 registers of a wave in the kernel above; short caches (see
+// plan_prefill); and pools that are not 16-byte aligned, which direct loads to LDS are not specified for: four
+// waves of 16 query rows and 16x16x32 MFMA, 32 tokens per key tile.  KG = 2: four more waves with buffers of
+// their own take every other key tile of the same rows, and the two halves meet in LDS at the end.
 // K/V tiles pass through registers into two LDS buffers per matrix, one barrier per tile; LDS rows are
 // padded by 32 bytes, which keeps the 16-byte K reads and the transposed V reads free of bank conflicts.
 // A step is a serial chain (scores, weights, values, barrier), so two workgroups share a compute unit: within
 // 256 registers (186) instead of 328 with accumulators copied between register files, whole tiles of 16
 // heads, bf16, take 45.1 us instead of 47.1 for 1000 tokens, 142 instead of 202 for 2900, 497 instead of
 // 751 for 6000.
-template <typename T, int D>
-__global__ __launch_bounds__(256, 2) void prefill_attn_staged_kernel(const PrefillParams p) {
+template <typename T, int D, int KG>
+__device__ __forceinline__ void staged_attention(const PrefillParams& p) {
   constexpr int WR = 16;            // query rows per wavefront
   constexpr int NS = D / 32;        // 16-byte pieces of a Q/K row per lane (one MFMA each)
   constexpr int DC = D / 16;        // head dimensions per lane in the P.V product
@@ -587,14 +589,18 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_staged_kernel(const Prefi
   constexpr int CPT = CPR / 8;      // staging: chunks per thread, tile and matrix (row = tid / 8,
                                     // chunk = tid % 8 + 8 jc)
   static_assert(D % 64 == 0, "a thread stages whole pieces");
-  // two buffers per matrix: tile t + 1 is written while tile t is still being read
+  constexpr int STEP = BN * KG;     // tokens from one tile of a key group to its next
+  // two buffers per matrix and key group: tile t + 1 is written while tile t is still being read
   constexpr int TILE = BN * PITCH;
-  __shared__ __attribute__((aligned(16))) uint16_t ks[2 * TILE];
-  __shared__ __attribute__((aligned(16))) uint16_t vs[2 * TILE];
+  __shared__ __attribute__((aligned(16))) uint16_t sm[KG][4 * TILE];
 
   // the wave index is made scalar: the per-tile activity tests below must be real branches, because
   // matrix instructions do not honour the EXEC mask of a masked-off region
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tid = threadIdx.x & 255, lane = tid & 63;  // inside the key group
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6) & 3);
+  const int kg = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 8));
+  uint16_t* const ks = sm[kg];
+  uint16_t* const vs = sm[kg] + 2 * TILE;
   const int r = lane & 15, g = lane >> 4;
   PrefillPiece w;
   if (!prefill_piece(p, w)) return;  // uniform
@@ -654,7 +660,7 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_staged_kernel(const Prefi
   auto fetch_k = [&](int kt, u32x4 (&kreg)[CPT]) {  // needs lookup(kt) before it; fetch_v(kt) comes after it
     fetch(kt, pg, 0, kreg);
     pg_v = pg;
-    lookup(kt + BN);
+    lookup(kt + STEP);
   };
   auto stash = [&](int buf, const u32x4 (&kreg)[CPT]) {
 #pragma unroll
@@ -672,7 +678,7 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_staged_kernel(const Prefi
   auto compute = [&](int kt, int buf) {
     // A wave whose last query row lies before the key tile sees none of it (causal).  In an active wave a
     // row that lies wholly before the key tile is masked to zero weight below.
-    if (kt <= wave_last_pos) {
+    if (kt <= wave_last_pos && (KG == 1 || kt < kv_end)) {
       // ---- S^T = K Q^T ---------------------------------------------------------------------------
       // (the two matrix phases run at raised wave priority: while one wave of a SIMD is in its
       // softmax arithmetic, the other's matrix instructions are issued first and keep the matrix
@@ -760,34 +766,93 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_staged_kernel(const Prefi
     }
   };
 
-  // first tile into buffer 0, keys of the second into register set a
-  lookup(k_begin);
-  fetch_k(k_begin, kreg_a);
-  fetch_v(k_begin);
+  // first tile into buffer 0, keys of the second into register set a.  Key group kg takes the tiles kg,
+  // kg + KG, ...; the groups keep step (the barriers are shared), so a group may be handed a tile past the
+  // end: its rows are clamped, and compute leaves it alone.
+  const int k_first = k_begin + kg * BN;
+  lookup(k_first);
+  fetch_k(k_first, kreg_a);
+  fetch_v(k_first);
   stash(0, kreg_a);
-  if (k_begin + BN < kv_end) fetch_k(k_begin + BN, kreg_a);
+  if (k_begin + STEP < kv_end) fetch_k(k_first + STEP, kreg_a);
   // One barrier per tile: it makes tile kt visible in its buffer, and it tells that every wave has
-  // finished reading the other buffer, which the end of the step overwrites with tile kt + BN.
-  for (int kt = k_begin; kt < kv_end; kt += 2 * BN) {
+  // finished reading the other buffer, which the end of the step overwrites with the group's next tile.
+  for (int k0 = k_begin; k0 < kv_end; k0 += 2 * STEP) {  // of key group 0
+    const int kt = k0 + kg * BN;
     __syncthreads();
-    if (kt + BN < kv_end) fetch_v(kt + BN);
-    if (kt + 2 * BN < kv_end) fetch_k(kt + 2 * BN, kreg_b);
+    if (k0 + STEP < kv_end) fetch_v(kt + STEP);
+    if (k0 + 2 * STEP < kv_end) fetch_k(kt + 2 * STEP, kreg_b);
     compute(kt, 0);
-    if (kt + BN >= kv_end) break;
+    if (k0 + STEP >= kv_end) break;
     stash(1, kreg_a);
     __syncthreads();
-    if (kt + 2 * BN < kv_end) fetch_v(kt + 2 * BN);
-    if (kt + 3 * BN < kv_end) fetch_k(kt + 3 * BN, kreg_a);
-    compute(kt + BN, 1);
-    if (kt + 2 * BN < kv_end) stash(0, kreg_b);
+    if (k0 + 2 * STEP < kv_end) fetch_v(kt + 2 * STEP);
+    if (k0 + 3 * STEP < kv_end) fetch_k(kt + 3 * STEP, kreg_a);
+    compute(kt + STEP, 1);
+    if (k0 + 2 * STEP < kv_end) stash(0, kreg_b);
+  }
+
+  // ---- the key groups' results of a row meet in LDS: wave w of group 0 adds those of the waves w ------
+  // (a group in which a row sees no key has denominator 0 and is left out, whatever its values are)
+  const float l = rows_sum(l_run);
+  float m_row[4], l_row[4];  // of rows 4 g + i
+  if constexpr (KG > 1) {
+    static_assert((KG - 1) * 4 * 16 * D * 4 <= KG * 4 * TILE * 2, "the partial results fit the tiles' LDS");
+    __shared__ float sm_ml[KG][4][16][2];
+    f32x4* const part = reinterpret_cast<f32x4*>(&sm[0][0]);
+    __syncthreads();  // the last tiles have been read
+    if (g == 0) {
+      sm_ml[kg][wave][r][0] = m_run;
+      sm_ml[kg][wave][r][1] = l;
+    }
+    if (kg > 0) {
+#pragma unroll
+      for (int a = 0; a < DC; ++a) part[(((kg - 1) * 4 + wave) * DC + a) * 64 + lane] = oacc[a];
+    }
+    __syncthreads();
+    if (kg > 0) return;
+    float f[KG][4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      float m[KG], l_of[KG], top = kNegBig;
+#pragma unroll
+      for (int j = 0; j < KG; ++j) {
+        m[j] = sm_ml[j][wave][4 * g + i][0];
+        l_of[j] = sm_ml[j][wave][4 * g + i][1];
+        if (l_of[j] != 0.f) top = fmaxf(top, m[j]);
+      }
+      l_row[i] = 0.f;
+      m_row[i] = top;
+#pragma unroll
+      for (int j = 0; j < KG; ++j) {
+        f[j][i] = l_of[j] != 0.f ? fast_exp2(m[j] - top) : 0.f;
+        l_row[i] = fmaf(l_of[j], f[j][i], l_row[i]);
+      }
+    }
+#pragma unroll
+    for (int a = 0; a < DC; ++a) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) oacc[a][i] = f[0][i] != 0.f ? oacc[a][i] * f[0][i] : 0.f;
+#pragma unroll
+      for (int j = 1; j < KG; ++j) {
+        const f32x4 v = part[(((j - 1) * 4 + wave) * DC + a) * 64 + lane];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) oacc[a][i] = f[j][i] != 0.f ? fmaf(v[i], f[j][i], oacc[a][i]) : oacc[a][i];
+      }
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      m_row[i] = __shfl(m_run, 4 * g + i, 64);
+      l_row[i] = __shfl(l, 4 * g + i, 64);
+    }
   }
 
   // ---- normalise and store (or leave the piece's partial result): lane holds rows 4g + i,
   //      dimensions 16 a + r ------------------------------------------------------------------------
-  const float l = rows_sum(l_run);
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const float li = __shfl(l, 4 * g + i, 64);
+    const float li = l_row[i];
     const int row = wave_row0 + 4 * g + i;
     if (whole) {
       const float inv = li > 0.f ? 1.f / li : 0.f;
@@ -798,7 +863,7 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_staged_kernel(const Prefi
         for (int a = 0; a < DC; ++a) dst[16 * a] = from_float<T>(oacc[a][i] * inv);
       }
     } else {
-      const float mi = __shfl(m_run, 4 * g + i, 64);
+      const float mi = m_row[i];
       if (row < p.n_rows) {
         const int64_t part = ((int64_t)split * p.n_kv + kvh) * p.n_rows + row;
         float* dst = p.part_o + part * D + r;
@@ -811,6 +876,15 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_staged_kernel(const Prefi
       }
     }
   }
+}
+
+template <typename T, int D>
+__global__ __launch_bounds__(256, 2) void prefill_attn_staged_kernel(const PrefillParams p) {
+  staged_attention<T, D, 1>(p);
+}
+template <typename T, int D>
+__global__ __launch_bounds__(512, 2) void prefill_two_groups_kernel(const PrefillParams p) {
+  staged_attention<T, D, 2>(p);
 }
 
 // Adds up the pieces of every row whose keys were split: D / 4 adjacent threads own a row, four
@@ -917,9 +991,13 @@ static int64_t key_pieces(const PrefillParams& p, int kv_len, int bn, int64_t c)
 
 template <typename T>
 static int launch_prefill(const PrefillParams& p, int head_dim, bool oct, hipStream_t st) {
-  const dim3 grid(p.n_tiles * p.n_kv * p.n_splits), block(p.staged ? 256 : 512);
+  const dim3 grid(p.n_tiles * p.n_kv * p.n_splits), block(p.staged ? 256 * p.key_groups : 512);
   if (head_dim == 256)
     hipLaunchKernelGGL((prefill_attn_staged_kernel<T, 256>), grid, block, 0, st, p);
+  else if (head_dim == 128 && p.staged && p.key_groups == 2)
+    hipLaunchKernelGGL((prefill_two_groups_kernel<T, 128>), grid, block, 0, st, p);
+  else if (head_dim == 64 && p.staged && p.key_groups == 2)
+    hipLaunchKernelGGL((prefill_two_groups_kernel<T, 64>), grid, block, 0, st, p);
   else if (head_dim == 128 && p.staged)
     hipLaunchKernelGGL((prefill_attn_staged_kernel<T, 128>), grid, block, 0, st, p);
   else if (head_dim == 64 && p.staged)
@@ -981,19 +1059,18 @@ static int64_t prefill_ws_bytes(const PrefillParams& p, int head_dim) {
   return p.n_splits > 1 ? (int64_t)p.n_splits * p.n_kv * p.n_rows * (head_dim + 2) * 4 : 0;
 }
 
-// shape of the launch for a call that passed check_prefill
-static void plan_prefill(const td_paged_kv* kv, int32_t kv_len, int32_t n_q, int32_t num_qo_heads,
-                         int32_t causal, bool may_split, PrefillParams& p) {
+// Shape of the launch for a call that passed check_prefill: of the staged kernel or of the eight-wave kernel,
+// with pieces whose partial results take at most `limit` bytes.
+static void plan_shape(const td_paged_kv* kv, int32_t kv_len, int32_t n_q, int32_t num_qo_heads, int32_t causal,
+                       bool staged, int64_t limit, PrefillParams& p) {
   const int H = kv->num_kv_heads, D = kv->head_dim;
   p.n_kv = H;
   p.q_per_kv = num_qo_heads / H;
   p.n_rows = n_q * p.q_per_kv;
   p.n_q = n_q;
   p.causal = causal;
-  // Up to one key tile of the eight-wave kernel there is nothing to overlap, and its rings and phases cost more
-  // than they give: 32 heads of 128, 16 tokens 6.5 us against 4.4 (64 dimensions 5.5 against 4.0), 33 6.6 against
-  // 4.9, 64 6.5 against 5.4.
-  p.staged = D == 256 || kv_len <= 64 || ((uintptr_t)kv->data & 15) != 0;
+  p.staged = staged;
+  p.key_groups = 1;
   const int bn = p.staged ? 32 : 64, max_tiles = (kv_len + bn - 1) / bn;
   const int64_t cus = td_num_cus();
   double best = 0.0;
@@ -1004,10 +1081,10 @@ static void plan_prefill(const td_paged_kv* kv, int32_t kv_len, int32_t n_q, int
     const int64_t tiles = H * key_pieces(c, kv_len, bn, 1);
     for (int s = 1; s <= 64; s = s < 8 ? s + 1 : (s < 16 ? s + 2 : s * 2)) {
       const int chunk = (max_tiles + s - 1) / s;
-      if (s > 1 && (!may_split || chunk < 4 || (int64_t)c.n_tiles * H >= 8 * cus)) break;
+      if (s > 1 && (limit <= 0 || chunk < 4 || (int64_t)c.n_tiles * H >= 8 * cus)) break;
       c.chunk = chunk * bn;
       c.n_splits = 1 + (kv_len - 1) / c.chunk;
-      if (prefill_ws_bytes(c, D) > kMaxScratch) break;
+      if (prefill_ws_bytes(c, D) > limit) break;
       const double pieces = s > 1 ? 2.0 + (double)H * c.n_rows * D * 4e-6 * s / 4.0 : 0.0;
       // no cost is below that of the longest piece alone
       if (s > 1 && tile * chunk + pieces >= best) continue;
@@ -1024,6 +1101,34 @@ static void plan_prefill(const td_paged_kv* kv, int32_t kv_len, int32_t n_q, int
   }
   // one head after the other on its XCD once there are enough tiles for the last head to end evenly
   p.head_major = H % 8 == 0 && (int64_t)p.n_tiles * p.n_splits * H > 4 * (int64_t)td_num_cus();
+}
+
+// The plan that scratch is asked for: the staged kernel where the eight-wave one cannot run or has nothing to
+// overlap (up to one key tile).
+static void plan_prefill(const td_paged_kv* kv, int32_t kv_len, int32_t n_q, int32_t num_qo_heads, int32_t causal,
+                         bool may_split, PrefillParams& p) {
+  const bool staged = kv->head_dim == 256 || kv_len <= 64 || ((uintptr_t)kv->data & 15) != 0;
+  plan_shape(kv, kv_len, n_q, num_qo_heads, causal, staged, may_split ? kMaxScratch : 0, p);
+}
+
+// Short caches go to the staged kernel all the same, with no more scratch than was asked for: a step of either
+// kernel is a serial chain of about 1 us, the eight-wave kernel's rings and phases cost more to start than two
+// buffers, and two key groups halve the staged kernel's steps for 1 us of joining.  us, bf16, 32 / 8 heads of
+// 128 (32 / 32 within 0.4), eight waves | staged | staged with two key groups: 16 tokens 6.5 | 4.4 | 5.6, 96
+// 7.6 | 5.9 | 6.6, 128 7.8 | 6.7 | 6.7, 200 8.9 | 8.9 | 8.2, 300 10.6 | 11.5 | 9.8, 500 13.6 | 16.4 | 13.0; of
+// 64, 300 8.3 | 9.4 | 7.7.  A few rows on a cache of up to 1600 tokens, in pieces, eight waves | two key groups
+// with as much scratch: 16 on 500 12.4 | 11.9 (32 / 32 heads 11.6 | 10.9), 40 on 500 12.8 | 12.3, 16 on 1500
+// 12.8 | 12.0; 16 of 40 / 40 heads on 2000 15.1 | 15.5; twice as many row tiles gain nothing.
+static void plan_short(const td_paged_kv* kv, int32_t kv_len, int32_t n_q, int32_t num_qo_heads, int32_t causal,
+                       int64_t scratch, PrefillParams& p) {
+  if (p.staged || kv_len > 1600) return;
+  const int64_t cus = td_num_cus(), tiles64 = (int64_t)p.n_kv * ((p.n_rows + 63) / 64);
+  if (kv_len <= 96) {
+    plan_shape(kv, kv_len, n_q, num_qo_heads, causal, true, 0, p);
+  } else if (p.n_splits > 1 && kv_len > 256 ? tiles64 <= cus * 3 / 16 : kv_len <= 512 && tiles64 <= 2 * cus) {
+    plan_shape(kv, kv_len, n_q, num_qo_heads, causal, true, kv_len > 256 ? scratch : 0, p);
+    p.key_groups = 2;
+  }
 }
 
 extern "C" int64_t td_prefill_workspace_bytes(const td_paged_kv* kv, int32_t kv_len, int32_t n_q,
@@ -1051,6 +1156,7 @@ extern "C" int td_prefill_attn_split(const td_paged_kv* kv, const int32_t* page_
     plan_prefill(kv, kv_len, n_q, num_qo_heads, causal, false, p);
   TD_REQUIRE(p.n_splits == 1 || ((uintptr_t)workspace & 15) == 0,
              "td_prefill_attn: the workspace must be 16-byte aligned");
+  plan_short(kv, kv_len, n_q, num_qo_heads, causal, prefill_ws_bytes(p, D), p);
   p.part_o = reinterpret_cast<float*>(workspace);
   p.part_ml = p.part_o ? p.part_o + (int64_t)p.n_splits * p.n_kv * p.n_rows * D : nullptr;
   p.kv = reinterpret_cast<const uint16_t*>(kv->data);

@@ -215,8 +215,20 @@ extern "C" int td_decode_make_plan(int32_t batch, int32_t num_qo_heads, int32_t 
   int64_t chunk = max_items > 0 ? ceil_div64(max_items, splits) : tile;
   // A batch is planned from its longest sequence: chunks of that size leave the short sequences
   // with one long-running workgroup per head and the launch waits for the longest.  Finer chunks
-  // balance a ragged batch (8 sequences of 14K-63K tokens: 935 -> 769 us).
-  if (batch > 1 && qpg == 1 && chunk > 4096) chunk = 4096;
+  // balance a ragged batch (8 sequences of 14K-63K tokens: 935 -> 769 us at 4096 tokens) and end
+  // closer together; from 1024 tokens down the merges take back what that gives.  32 heads x 128,
+  // fp16, logits out, chunks of 4096 | 1024 tokens (or as near as the built-in scratch allows): 8
+  // sequences of 8192 .. 65536 1017 | 998 us, of 500 .. 8000 136 | 118; 16 heads, 8 of 2000 .. 30000
+  // 254 | 240; 40 heads, 3 of 2000 .. 40000 210 | 196.
+  if (batch > 1 && qpg == 1 && chunk > 1024) {
+    const int64_t per_split = (int64_t)batch * n_hrows * (head_dim + 2) * 4;
+    int64_t fit = ((int64_t)TD_STATIC_SCRATCH_BYTES - kTicketBytes - 512) / per_split;  // splits it holds
+    if (fit < ceil_div64(max_items, 4096)) fit = ceil_div64(max_items, 4096);
+    const int64_t finest = ceil_div64(max_items, fit < 64 ? fit : 64);
+    const int64_t wanted = finest > 1024 ? ceil_div64(finest, tile) * tile : 1024;
+    if (chunk > wanted) chunk = wanted;
+    if (chunk > 4096) chunk = 4096;
+  }
   // Shared rows in a batch: whole rounds of one workgroup per compute unit.  The split count with
   // the fewest rounds per split wins, chunks of 1024 tokens at least
   // (32/8 heads, 16 sequences x 8192 tokens: 2 splits = 256 workgroups 94 us, 3 splits 110, 1

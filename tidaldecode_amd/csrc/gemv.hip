@@ -6,9 +6,9 @@
 //   residual  y = residual + W x                      (the two residual additions of a layer)
 //   pair      y[i] = silu(W[i] x) * (W[i + rows/2] x) (gate and up projection in one launch: a
 //             wavefront owns row i and row i + rows/2, so the down projection gets a plain vector)
-// HBM-bound: every weight is read once (non-temporal 16-byte loads, 16 of them in flight per
-// lane), x is staged in LDS once per workgroup, a wavefront owns two rows at a time and reduces
-// with DPP.  Used by the decoder harness around the attention path (the reference runs torch
+// HBM-bound: every weight is read once (non-temporal 16-byte loads, 4 to 16 of them in flight per
+// lane), x is staged in LDS once per workgroup, a wavefront owns one or two rows and reduces with
+// DPP.  Used by the decoder harness around the attention path (the reference runs torch
 // nn.Linear there: tidal/models/SparseAttention.py:122,216, tidal/models/llama.py:108-122).
 
 #include "common.cuh"
@@ -209,11 +209,14 @@ __global__ __launch_bounds__(kGemvThreads) void gemv_kernel(
   }
 }
 
-template <typename T, int R, int UN, int XR>
-static void launch_gemv_x(const GemvParams& p, int mode, bool pair, hipStream_t st) {
-  const int units = pair ? (p.rows / 2 + R / 2 - 1) / (R / 2) : (p.rows + R - 1) / R;
+template <typename T, bool PAIR, int R, int UN, int XR>
+static void launch_gemv_x(const GemvParams& p, int mode, hipStream_t st) {
+  constexpr int HR = R > 1 ? R / 2 : 1;
+  constexpr bool pair = PAIR;
+  static_assert(!PAIR || R % 2 == 0, "a wavefront holds whole pairs");
+  const int units = pair ? (p.rows / 2 + HR - 1) / HR : (p.rows + R - 1) / R;
   const dim3 grid((units + kGemvWaves - 1) / kGemvWaves), block(kGemvThreads);
-  if (pair) {
+  if constexpr (PAIR) {
     if (mode == 0)
       hipLaunchKernelGGL((gemv_kernel<T, 0, true, R, UN, XR>), grid, block, 0, st, p.w, p.w_row_stride, p.rows, p.cols, p.x,
                        p.norm_weight, p.eps, p.residual, p.y);
@@ -232,30 +235,35 @@ static void launch_gemv_x(const GemvParams& p, int mode, bool pair, hipStream_t 
   }
 }
 
-template <typename T, int R, int UN>
-static void launch_gemv_shape(const GemvParams& p, int mode, bool pair, hipStream_t st) {
+template <typename T, bool PAIR, int R, int UN>
+static void launch_gemv_shape(const GemvParams& p, int mode, hipStream_t st) {
   const int per_thread = (p.cols / 8 + kGemvThreads - 1) / kGemvThreads;  // x chunks per thread
   if (per_thread <= 2)
-    launch_gemv_x<T, R, UN, 2>(p, mode, pair, st);
+    launch_gemv_x<T, PAIR, R, UN, 2>(p, mode, st);
   else if (per_thread <= 6)
-    launch_gemv_x<T, R, UN, 6>(p, mode, pair, st);
+    launch_gemv_x<T, PAIR, R, UN, 6>(p, mode, st);
   else if (per_thread <= 8)
-    launch_gemv_x<T, R, UN, 8>(p, mode, pair, st);
+    launch_gemv_x<T, PAIR, R, UN, 8>(p, mode, st);
   else
-    launch_gemv_x<T, R, UN, 15>(p, mode, pair, st);
+    launch_gemv_x<T, PAIR, R, UN, 15>(p, mode, st);
 }
 
-// Tall matrices: four rows per wavefront (fewer, longer-lived waves stream better); short ones:
-// two rows, so that the launch still has a few workgroups per compute unit (measured on
-// 4096..32000 x 4096 and 4096 x 11008: 4.4-6.0 TB/s).
+// One row per wavefront: waves that end one after the other keep the memory busier than fewer with more rows
+// each, whose last trips end together.  Long rows and row pairs take eight chunks per row and trip; short
+// matrices keep two rows, which halves what their few workgroups stage.  One MI355X, cold weights, launches of
+// a graph, us, before (four rows of four chunks; two of eight for the long rows) -> now: 12288 x 4096 17.7 ->
+// 16.9 (6.0 TB/s), 32000 x 4096 42.5 -> 40.6, 128256 x 4096 155.8 -> 151.4 (6.9 TB/s), 4096 x 11008 17.8 ->
+// 17.5, pairs 22016 x 4096 31.4 -> 29.2, 28672 x 4096 38.8 -> 37.0; 4096 x 4096 7.4 with either.
 template <typename T>
 static void launch_gemv(const GemvParams& p, int mode, bool pair, hipStream_t st) {
-  if (p.rows >= 8192)
-    launch_gemv_shape<T, 4, 4>(p, mode, pair, st);
-  else if (p.cols > 8192)  // few, long rows (the down projection): deeper batches, 19.0 -> 18.0 us
-    launch_gemv_shape<T, 2, 8>(p, mode, pair, st);
+  if (pair)
+    launch_gemv_shape<T, true, 2, 8>(p, mode, st);
+  else if (p.cols > 8192)
+    launch_gemv_shape<T, false, 1, 8>(p, mode, st);
+  else if (p.rows >= 8192)
+    launch_gemv_shape<T, false, 1, 4>(p, mode, st);
   else
-    launch_gemv_shape<T, 2, 4>(p, mode, pair, st);
+    launch_gemv_shape<T, false, 2, 4>(p, mode, st);
 }
 
 }  // namespace tidal

@@ -424,6 +424,21 @@ int td_estimate_score(const td_paged_kv* meta, const int32_t* meta_indices, int3
                       int64_t o_stride, void* stream);
 
 /*
+ * What a decode step of one sequence does in front of a page-estimate attention, in one launch: RoPE of
+ * q [num_qo_heads, head_dim] into q_out and of k [num_kv_heads, head_dim] from cos / sin [head_dim / 2]
+ * (td_rope_table), the append of k and v at entry last_page_len - 1 of page last_page_idx, the fold of k
+ * into that page's entry of the metadata (entry meta_last_page_len - 1 of the last of meta_indices), and,
+ * unless est is NULL, td_estimate_score of the rotated q over all entries in front of it.  q, k and v are
+ * read only; all tensors 16-byte aligned.  Replaces td_rope_in_place + td_append_kv + td_estimate_score
+ * of such a step.
+ */
+int td_rope_append_estimate(const td_paged_kv* kv, const td_paged_kv* meta, const void* q, const void* k,
+                            const void* v, void* q_out, int32_t num_qo_heads, const float* cos,
+                            const float* sin, int32_t last_page_idx, int32_t last_page_len,
+                            const int32_t* meta_indices, int32_t n_meta_pages, int32_t meta_last_page_len,
+                            void* est, int64_t est_stride, void* stream);
+
+/*
  * RMSNorm: out[r, :] = x[r, :] * rsqrt(mean(x[r, :]^2) + eps) * weight, fp32 math.
  * Replaces rms_norm_forward (bsk_ops.h:29-32, tidal/ops/csrc/rms_norm.cu:160-212).
  */

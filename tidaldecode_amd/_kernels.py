@@ -368,6 +368,42 @@ def estimate_attn_score(q: torch.Tensor, o: torch.Tensor, metadata_data: torch.T
                                 o.data_ptr(), o.stride(0), _stream()))
 
 
+def rope_append_estimate(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, kv_data: torch.Tensor,
+                         kv_last_page_len: int, kv_last_page_idx: int, metadata_data: torch.Tensor,
+                         metadata_indices: torch.Tensor, metadata_last_page_len: int, layout: int,
+                         cos: torch.Tensor, sin: torch.Tensor, estimate: bool = True
+                         ) -> Tuple[torch.Tensor, Optional[torch.Tensor]]:
+    """Extension: ``apply_rope_in_place``, ``append_kv_cache_decode`` with its metadata and (``estimate``)
+    ``estimate_attn_score`` of one decode step in one launch.  q ``[1, H_q, D]``, k, v ``[1, H_kv, D]`` are read
+    only; cos, sin from ``rope_table``; returns the rotated q and the bounds ``[H_q, entries - 1]`` (or None)."""
+    for t, n in ((q, "q"), (k, "k"), (v, "v"), (metadata_indices, "metadata_indices"), (cos, "cos"), (sin, "sin")):
+        _check_input(t, n)
+    for t, n in ((q, "q"), (k, "k"), (v, "v")):
+        _check_dim(3, t, n)
+    _check_i32(metadata_indices, "metadata_indices")
+    pool = _pool(kv_data, int(layout))
+    meta = _pool(metadata_data, int(layout), "metadata_data")
+    if q.size(0) != 1 or k.size(0) != 1 or k.shape != v.shape or k.size(1) != pool.num_kv_heads or \
+            q.size(2) != pool.head_dim or k.size(2) != pool.head_dim or \
+            not (q.dtype == k.dtype == v.dtype == kv_data.dtype == metadata_data.dtype):
+        raise RuntimeError("rope_append_estimate: q/k/v and the pools disagree in shape or dtype")
+    if cos.dtype != torch.float32 or sin.dtype != torch.float32 or cos.numel() != pool.head_dim // 2 or \
+            sin.numel() != pool.head_dim // 2:
+        raise RuntimeError("rope_append_estimate: cos and sin must be float32 [1, D/2]")
+    n_pages = metadata_indices.numel()
+    rotated = torch.empty_like(q)
+    est = None
+    if estimate:
+        entries = (n_pages - 1) * meta.page_size + int(metadata_last_page_len) - 1
+        est = torch.empty((q.size(1), entries), dtype=q.dtype, device=q.device)
+    check(lib.td_rope_append_estimate(pool, meta, q.data_ptr(), k.data_ptr(), v.data_ptr(), rotated.data_ptr(),
+                                      q.size(1), cos.data_ptr(), sin.data_ptr(), int(kv_last_page_idx),
+                                      int(kv_last_page_len), metadata_indices.data_ptr(), n_pages,
+                                      int(metadata_last_page_len), None if est is None else _ptr(est),
+                                      0 if est is None else est.stride(0), _stream()))
+    return rotated, est
+
+
 def _append(k, v, kv_data, kv_indices, kv_indptr, kv_last_page_len, metadata_data,
             metadata_indices, metadata_indptr, metadata_last_page_len, layout, decode: bool):
     if k.is_cuda and host_calls.append(k, v, kv_data, kv_indices, kv_indptr, kv_last_page_len, metadata_data,

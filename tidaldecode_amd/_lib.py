@@ -166,6 +166,11 @@ SIGNATURES = {
         [POINTER(PagedKV), c_void_p, c_int32, c_int32, c_void_p, c_int32, c_void_p, c_int64,
          c_void_p],
     ),
+    "td_rope_append_estimate": (
+        c_int32,
+        [POINTER(PagedKV), POINTER(PagedKV), c_void_p, c_void_p, c_void_p, c_void_p, c_int32, c_void_p, c_void_p,
+         c_int32, c_int32, c_void_p, c_int32, c_int32, c_void_p, c_int64, c_void_p],
+    ),
     "td_prefill_attn": (
         c_int32,
         [POINTER(PagedKV), c_void_p, c_int32, c_int32, c_void_p, c_void_p, c_int32, c_int32,

@@ -363,6 +363,124 @@ __global__ __launch_bounds__(256) void estimate_kernel(PoolGeom mg, const int32_
   if (li == 0 && e < n_entries) o[(int64_t)h * o_stride + e] = from_float<T>(acc);
 }
 
+// What a decode step of one sequence does in front of a page-estimate attention, in one launch: RoPE of q
+// (to q_out) and of the new k, the append of k and v, the fold of k into its page's bounds, and (est) the
+// upper bounds of q.k over every other page, as rope, append_copy_kernel, append_meta_kernel and
+// estimate_kernel do them.  Nothing here waits for anything else here: the bounds are those of full pages, and
+// every workgroup turns its head's q row itself, which costs it one look at the row and the step's cos / sin.
+// Bound by latency (32 heads x 640 pages: 5 MB of bounds, under 1 us at the memory's rate): four launches of
+// 2.1 + 2.5 + 3.1 + 4.6 us, each with a boundary of about 1 us, become one of 5.1 us (a step of 16 layers:
+// 1818 -> 1742 us).
+// grid: (1 + tiles of entries, query heads); the first tile of a head is its q row and, of the first query head
+// of a KV head, k and v.
+struct QuestFront {
+  const uint16_t *q, *k, *v;  // [heads, D]
+  uint16_t* q_out;
+  const float *cos, *sin;     // [D / 2]
+  int32_t q_per_kv, page, entry;  // the new token's slot
+  const int32_t* meta_indices;
+  int32_t meta_last, meta_entry;  // of meta_indices: the page, and in it the entry, of the new token's page
+  int32_t n_entries;              // entries estimated: those in front of it
+  uint16_t* est;
+  int64_t est_stride;
+  float type_max;
+};
+constexpr int kQuestEntries = 4;  // per lane group, in flight together
+
+template <typename T, int D>
+__global__ __launch_bounds__(256) void quest_front_kernel(PoolGeom kvg, PoolGeom mg, QuestFront p) {
+  constexpr int LPR = D / 8, GROUPS = 256 / LPR;
+  const int tid = threadIdx.x, li = tid % LPR, group = tid / LPR, h = blockIdx.y;
+  const bool upper = li >= LPR / 2;
+  const int c = (li % (LPR / 2)) * 8;  // first pair of this lane
+  const bool front = blockIdx.x == 0;
+  // group 1 of a head's first tile turns k instead of q
+  const int kvh = h / p.q_per_kv;
+  const bool with_k = front && h == kvh * p.q_per_kv;
+  const uint16_t* row = front && group == 1 ? p.k + (int64_t)kvh * D : p.q + (int64_t)h * D;
+  const u32x4 lo4 = *reinterpret_cast<const u32x4*>(row + c);
+  const u32x4 hi4 = *reinterpret_cast<const u32x4*>(row + c + D / 2);
+  f32x4 cs[2], sn[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    cs[i] = *reinterpret_cast<const f32x4*>(p.cos + c + 4 * i);
+    sn[i] = *reinterpret_cast<const f32x4*>(p.sin + c + 4 * i);
+  }
+  // the tile's bounds, in flight while the row is turned
+  u32x4 mx[kQuestEntries], mn[kQuestEntries];
+  const int first = ((int)blockIdx.x - 1) * GROUPS * kQuestEntries + group;
+  if (!front) {
+#pragma unroll
+    for (int u = 0; u < kQuestEntries; ++u) {
+      int e = first + u * GROUPS;
+      e = e < p.n_entries ? e : p.n_entries - 1;  // clamped: loads stay unconditional
+      const uint32_t page = (uint32_t)p.meta_indices[e / mg.page_size];
+      const uint16_t* at = reinterpret_cast<const uint16_t*>(mg.data) + k_offset(mg, page, e % mg.page_size, kvh) + li * 8;
+      mx[u] = *reinterpret_cast<const u32x4*>(at);
+      mn[u] = *reinterpret_cast<const u32x4*>(at + mg.v_offset);
+    }
+  }
+  const uint32_t lw[4] = {lo4.x, lo4.y, lo4.z, lo4.w}, hw[4] = {hi4.x, hi4.y, hi4.z, hi4.w};
+  uint32_t w[4];  // this lane's eight turned elements
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    float l0, l1, h0, h1, a0, a1, b0, b1;
+    unpack2<T>(lw[i], l0, l1);
+    unpack2<T>(hw[i], h0, h1);
+    turn(l0, h0, sn[i / 2][2 * (i & 1)], cs[i / 2][2 * (i & 1)], a0, b0);
+    turn(l1, h1, sn[i / 2][2 * (i & 1) + 1], cs[i / 2][2 * (i & 1) + 1], a1, b1);
+    w[i] = upper ? pack2<T>(b0, b1) : pack2<T>(a0, a1);
+  }
+  if (front) {
+    if (group == 0) *reinterpret_cast<u32x4*>(p.q_out + (int64_t)h * D + li * 8) = u32x4{w[0], w[1], w[2], w[3]};
+    if (!with_k || group != 1) return;
+    uint16_t* dst = reinterpret_cast<uint16_t*>(kvg.data) + k_offset(kvg, (uint32_t)p.page, p.entry, kvh) + li * 8;
+    *reinterpret_cast<u32x4*>(dst) = u32x4{w[0], w[1], w[2], w[3]};
+    *reinterpret_cast<u32x4*>(dst + kvg.v_offset) = *reinterpret_cast<const u32x4*>(p.v + (int64_t)kvh * D + li * 8);
+    uint16_t* at = reinterpret_cast<uint16_t*>(mg.data) +
+                   k_offset(mg, (uint32_t)p.meta_indices[p.meta_last], p.meta_entry, kvh) + li * 8;
+    uint32_t low[4], top[4];
+    {
+      const u32x4 t = *reinterpret_cast<const u32x4*>(at), b = *reinterpret_cast<const u32x4*>(at + mg.v_offset);
+      top[0] = t.x; top[1] = t.y; top[2] = t.z; top[3] = t.w;
+      low[0] = b.x; low[1] = b.y; low[2] = b.z; low[3] = b.w;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      float x0, x1, t0, t1, b0, b1;
+      unpack2<T>(w[i], x0, x1);
+      unpack2<T>(top[i], t0, t1);
+      unpack2<T>(low[i], b0, b1);
+      if (p.entry == 0) {  // the page's first token
+        t0 = t1 = -p.type_max;
+        b0 = b1 = p.type_max;
+      }
+      top[i] = pack2<T>(fmaxf(t0, x0), fmaxf(t1, x1));
+      low[i] = pack2<T>(fminf(b0, x0), fminf(b1, x1));
+    }
+    *reinterpret_cast<u32x4*>(at) = u32x4{top[0], top[1], top[2], top[3]};
+    *reinterpret_cast<u32x4*>(at + mg.v_offset) = u32x4{low[0], low[1], low[2], low[3]};
+    return;
+  }
+#pragma unroll
+  for (int u = 0; u < kQuestEntries; ++u) {
+    const uint32_t mxw[4] = {mx[u].x, mx[u].y, mx[u].z, mx[u].w}, mnw[4] = {mn[u].x, mn[u].y, mn[u].z, mn[u].w};
+    float acc = 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      float q0, q1, a0, a1, b0, b1;
+      unpack2<T>(w[i], q0, q1);
+      unpack2<T>(mxw[i], a0, a1);
+      unpack2<T>(mnw[i], b0, b1);
+      acc += fmaxf(q0 * a0, q0 * b0);
+      acc += fmaxf(q1 * a1, q1 * b1);
+    }
+    acc = group_sum<LPR>(acc);
+    const int e = first + u * GROUPS;
+    if (li == 0 && e < p.n_entries) p.est[(int64_t)h * p.est_stride + e] = from_float<T>(acc);
+  }
+}
+
 // RMSNorm, one 256-thread workgroup per row, fp32 accumulation.
 // Sum of squares over the workgroup: every wave reduces by butterfly, four partials through LDS.
 __device__ __forceinline__ float rms_block_sum(float ss) {
@@ -653,6 +771,68 @@ extern "C" int td_rope_append_decode(const td_paged_kv* kv, void* q, const void*
   else
     return fail(TD_ERR_UNSUPPORTED, "td_rope_append_decode failed to dispatch with dtype %d",
                 kv->dtype);
+  TD_HIP_CHECK(hipGetLastError());
+  return TD_OK;
+}
+
+extern "C" int td_rope_append_estimate(const td_paged_kv* kv, const td_paged_kv* meta, const void* q, const void* k,
+                                       const void* v, void* q_out, int32_t num_qo_heads, const float* cos,
+                                       const float* sin, int32_t last_page_idx, int32_t last_page_len,
+                                       const int32_t* meta_indices, int32_t n_meta_pages,
+                                       int32_t meta_last_page_len, void* est, int64_t est_stride, void* stream) {
+  int rc = check_pool(kv, "td_rope_append_estimate");
+  if (rc == TD_OK) rc = check_pool(meta, "td_rope_append_estimate (metadata)");
+  if (rc != TD_OK) return rc;
+  TD_REQUIRE(q && k && v && q_out && cos && sin && meta_indices, "td_rope_append_estimate: NULL argument");
+  const int H = kv->num_kv_heads, D = kv->head_dim;
+  TD_REQUIRE(meta->num_kv_heads == H && meta->head_dim == D && meta->dtype == kv->dtype && meta->layout == kv->layout,
+             "td_rope_append_estimate: kv and metadata pools differ in heads, head_dim, dtype or layout");
+  TD_REQUIRE(num_qo_heads >= H && num_qo_heads % H == 0, "td_rope_append_estimate: heads %d / %d", num_qo_heads, H);
+  if (D != 64 && D != 128 && D != 256)
+    return fail(TD_ERR_UNSUPPORTED, "td_rope_append_estimate: head_dim %d (supported: 64, 128, 256)", D);
+  if (kv->dtype != TD_F16 && kv->dtype != TD_BF16)
+    return fail(TD_ERR_UNSUPPORTED, "td_rope_append_estimate failed to dispatch with dtype %d", kv->dtype);
+  TD_REQUIRE(last_page_len >= 1 && last_page_len <= kv->page_size && last_page_idx >= 0 &&
+                 last_page_idx < kv->max_pages,
+             "td_rope_append_estimate: last page %d with %d entries", last_page_idx, last_page_len);
+  TD_REQUIRE(n_meta_pages >= 1 && meta_last_page_len >= 1 && meta_last_page_len <= meta->page_size,
+             "td_rope_append_estimate: %d metadata pages, the last with %d entries", n_meta_pages, meta_last_page_len);
+  const int64_t entries = (int64_t)(n_meta_pages - 1) * meta->page_size + meta_last_page_len - 1;
+  TD_REQUIRE(entries < ((int64_t)1 << 30) && (!est || est_stride >= entries),
+             "td_rope_append_estimate: est_stride %lld, %lld entries", (long long)est_stride, (long long)entries);
+  TD_REQUIRE((((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)q_out | (uintptr_t)cos | (uintptr_t)sin |
+               (uintptr_t)kv->data | (uintptr_t)meta->data) & 15) == 0,
+             "td_rope_append_estimate: tensors must be 16-byte aligned");
+  QuestFront p;
+  p.q = (const uint16_t*)q;
+  p.k = (const uint16_t*)k;
+  p.v = (const uint16_t*)v;
+  p.q_out = (uint16_t*)q_out;
+  p.cos = cos;
+  p.sin = sin;
+  p.q_per_kv = num_qo_heads / H;
+  p.page = last_page_idx;
+  p.entry = last_page_len - 1;
+  p.meta_indices = meta_indices;
+  p.meta_last = n_meta_pages - 1;
+  p.meta_entry = meta_last_page_len - 1;
+  p.n_entries = est ? (int32_t)entries : 0;
+  p.est = (uint16_t*)est;
+  p.est_stride = est_stride;
+  p.type_max = kv->dtype == TD_F16 ? 65504.f : 3.3895313892515355e38f;
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+#define TD_QUEST(T, DD)                                                                                  \
+  {                                                                                                      \
+    constexpr int kTile = 256 / (DD / 8) * kQuestEntries;                                                \
+    hipLaunchKernelGGL((quest_front_kernel<T, DD>), dim3(1 + (p.n_entries + kTile - 1) / kTile, num_qo_heads), \
+                       dim3(256), 0, st, geom_of(kv), geom_of(meta), p);                                 \
+  }
+  if (kv->dtype == TD_F16) {
+    if (D == 64) TD_QUEST(F16, 64) else if (D == 128) TD_QUEST(F16, 128) else TD_QUEST(F16, 256)
+  } else {
+    if (D == 64) TD_QUEST(BF16, 64) else if (D == 128) TD_QUEST(BF16, 128) else TD_QUEST(BF16, 256)
+  }
+#undef TD_QUEST
   TD_HIP_CHECK(hipGetLastError());
   return TD_OK;
 }

@@ -214,26 +214,26 @@ class TidalLlama:
             n_pages = len(ctrl.kv_cache.indicies)
             budget = max(1, min(int(ctrl._token_budget) // ctrl.page_size, n_pages - 1))
             self._quest = dict(
-                pos=pos, budget=budget,
+                budget=budget,
                 page_ids=ctrl.kv_indices_without_last.expand(self.config.num_heads, -1).contiguous(),
                 chosen=torch.zeros((self.config.num_heads, budget), dtype=torch.int32, device=self.device))
 
     def _attention_quest(self, idx, q, k, v):
-        """One layer of a Quest-style step built from the library's pieces: RoPE and append as
-        launches of their own (the append also updates the page's key bounds), then in layers 0 and 1
-        full attention, later an upper bound of the logits per page (decode_estimate), the best
-        pages (top-k over the bounds) and attention over those pages plus the page being filled.
-        Query heads of a group choose their own pages (one list per query head)."""
-        c, ctrl, qs = self.config, self.iController, self._quest
-        tidal_utils.apply_rope_in_place(q, k, qs["pos"], c.rope_scale, c.rope_theta)
-        tidal_utils.append_kv(k, v, ctrl, idx)
-        kv = ctrl.kv_cache.buf_layer(idx)
+        """One layer of a Quest-style step built from the library's pieces: one launch for RoPE, the
+        append (which also updates the page's key bounds) and, from layer 2 on, an upper bound of the
+        logits per page; then in layers 0 and 1 full attention, later the best pages (top-k over the
+        bounds) and attention over those pages plus the page being filled.  Query heads of a group
+        choose their own pages (one list per query head)."""
+        ctrl, qs = self.iController, self._quest
+        kv, cache, meta = ctrl.kv_cache.buf_layer(idx), ctrl.kv_cache, ctrl.metadata_cache
+        q, est = _kernels.rope_append_estimate(q, k, v, kv, cache.last_page_len, ctrl.kv_last_page_idx,
+                                               meta.buf_layer(idx), ctrl.metadata_indices, meta.last_page_len,
+                                               ctrl.layout, self._cos, self._sin, estimate=idx >= 2)
         o = torch.empty_like(q)
         if idx < 2:
             ctrl._decode_handler.forward(q, o, kv, ctrl.kv_indices_without_last, None,
-                                         ctrl.kv_cache.last_page_len, ctrl.kv_last_page_idx, None)
+                                         cache.last_page_len, ctrl.kv_last_page_idx, None)
             return o
-        est = tidal_utils.decode_estimate(q, ctrl, idx)
         _kernels.topk_filtering(est, qs["page_ids"], None, qs["chosen"], ctrl.topk_buf, qs["budget"])
         ctrl._decode_handler.forward(q, o, kv, qs["chosen"], None, ctrl.kv_cache.last_page_len,
                                      ctrl.kv_last_page_idx, None, index_kind="pages")

@@ -462,6 +462,11 @@ int td_rope_append_prompt(const td_paged_kv* kv, const void* qkv, int64_t qkv_st
                           const int32_t* kv_indices, const int32_t* kv_indptr, int32_t last_page_len,
                           float rope_scale, float rope_theta, void* stream);
 
+/* out[m, n] = x[m, k] w[n, k]^T in fp32 sums, rounded once to dtype (TD_F16 or TD_BF16), for few columns n (a
+ * multiple of 4) and many rows; rows of out lie out_stride elements apart; k: a multiple of 64. */
+int td_gemm_strip(const void* x, const void* w, void* out, int32_t m, int32_t n, int32_t k, int64_t out_stride,
+                  int32_t dtype, void* stream);
+
 /*
  * Measurement aid without a counterpart in the reference: the memory side of a sparse layer
  * alone.  Same grid and the same list -> slot -> K / V row loads as td_decode_attn for

@@ -134,6 +134,34 @@ def add_rms_norm(x: torch.Tensor, delta: torch.Tensor, weight: torch.Tensor, eps
     return out
 
 
+def _cut_columns(m: int, n: int, k: int) -> int:
+    """How many of the last columns of a product [m, k] x [n, k]^T are multiplied by a kernel of their own: a strip
+    of 256 where the library's tiles of 256 x 256 fill whole rounds of the 256 compute units and at most one strip's
+    tiles are left over, which would cost a round.  Measured on one MI355X over 2 to 32 rows of tiles, 16 to 160
+    strips and inner dimensions of 2048 to 8192: 0.99 to 1.8 times as fast up to 16 rows of tiles, 0.94 to 1.25
+    above; columns that are whole in 768 stay one product (the library then has narrower tiles: 0.74 to 1.8)."""
+    rows, strips = -(-m // 256), n // 256
+    tiles = rows * strips
+    if n % 256 or n % 768 == 0 or k % 64 or k > 1 << 24 or rows > 16 or tiles <= 256 or not 0 < tiles % 256 <= rows:
+        return 0
+    return 256
+
+
+def prompt_product(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
+    """Extension: ``x @ weight.t()`` of a prompt's rows x ``[n, K]`` and a weight ``[N, K]`` (inference only)."""
+    cut = _cut_columns(x.size(0), weight.size(0), x.size(1)) if x.dim() == 2 else 0
+    if not (cut and x.is_cuda and x.dtype == weight.dtype and x.dtype in (torch.float16, torch.bfloat16) and
+            x.is_contiguous() and weight.is_contiguous() and (x.data_ptr() | weight.data_ptr()) % 16 == 0 and
+            not torch.is_grad_enabled()):
+        return x @ weight.t()
+    main = weight.size(0) - cut
+    out = torch.empty((x.size(0), weight.size(0)), dtype=x.dtype, device=x.device)
+    torch.mm(x, weight[:main].t(), out=out[:, :main])
+    check(lib.td_gemm_strip(x.data_ptr(), weight[main:].data_ptr(), out[:, main:].data_ptr(), x.size(0), cut,
+                            x.size(1), out.stride(0), _dtype_code(x.dtype, "prompt_product"), _stream()))
+    return out
+
+
 def silu_mul(gate_up: torch.Tensor) -> torch.Tensor:
     """Extension: ``silu(gate) * up`` of rows ``[gate | up]``, ``[..., 2 I]`` -> ``[..., I]``."""
     _check_input(gate_up, "gate_up")

@@ -129,7 +129,7 @@ class TidalLlama:
         return tidal_utils.rms_norm_forward(x, weight, self.config.rms_norm_eps)
 
     def _mlp(self, layer, x):
-        return _kernels.silu_mul(x @ layer["w_gate_up"].t()) @ layer["w_down"].t()
+        return _kernels.silu_mul(_kernels.prompt_product(x, layer["w_gate_up"])) @ layer["w_down"].t()
 
     def _qkv(self, layer, h):
         c = self.config

@@ -85,3 +85,28 @@ def test_samples_that_mislead(cuda, n, k):
     for v in (high, low, few, one, nan):
         got, _ = _run(cuda, v, k, vals=False)
         assert torch.equal(got, orc.stable_topk(v, k))
+
+
+@pytest.mark.parametrize("n", [8192, 20000, 65536, 131072])
+def test_scores_just_above_the_samples_maximum(cuda, n):
+    """Scores that the sample misses, a few units in the last place above the largest it has, share that one's
+    bin; the selection ends between them (no bound: the sample's maximum is the reference).  The others lie so
+    close together that the sample's threshold takes two levels: the survivors' window does not end with a bin."""
+    from oracle import tidal_oracle as orc
+
+    threads = 512 if n <= 8192 else 1024
+    quads, lines = threads // 4, (-(-n // 4)) >> 2
+    sampled = ((torch.arange(quads) * lines // quads)[:, None] * 16 + torch.arange(16)[None]).flatten()
+    g = torch.Generator().manual_seed(n)
+    v = 3.0 + torch.randn((8, n), generator=g) * 2e-3
+    free = torch.ones(n, dtype=torch.bool)
+    free[sampled] = False
+    missed = torch.arange(n)[free]
+    for r in range(8):
+        v[r, sampled[-3]] = 4.0
+        at = missed[torch.randperm(len(missed), generator=g)[: 3 + r]]
+        v[r, at] = 4.0 + (1 + torch.arange(3 + r)) * 2.0 ** -21  # the spacing of floats from 4 to 8
+    for k in range(2, 13):
+        got, vals = _run(cuda, v, k)
+        want = orc.stable_topk(v, k)
+        assert torch.equal(got, want) and torch.equal(vals, torch.gather(v, 1, want)), k

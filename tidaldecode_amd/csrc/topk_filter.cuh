@@ -207,6 +207,7 @@ __global__ __launch_bounds__(NT) void topk_filter_kernel(const TopkParams p) {
     lo = 0u;
     s = shift_of(last);
     for (;;) {
+      last |= (1u << s) - 1u;  // whole bins: what lies in the last one is counted with it, also beyond the window
       each([&](uint32_t x) {
         const uint32_t d = x - lo;
         if (d <= last) atomicAdd(&L.hist[d >> s], 1u);

@@ -73,16 +73,23 @@ struct RowVectors {
 };
 
 // bit i of the result: element i of the 16 in v[0 .. 3] is not below `floor` (a NaN is not below
-// anything).  Two instructions per element: the comparison's mask is shifted in as a carry.
+// anything).  Two instructions per element: the comparison's mask is shifted in as a carry.  Four comparisons
+// write four scalar pairs before the first is read: a mask needs two wait states between the vector
+// instruction that writes it and the one that takes it as carry, and the compiler inserts none inside asm.
 template <typename T>
 __device__ __forceinline__ uint32_t reach16(const typename RowVectors<T>::vec* v, float floor) {
   uint32_t mask = 0;
 #pragma unroll
-  for (int i = 15; i >= 0; --i)
-    asm("v_cmp_nlt_f32 vcc, %1, %2\n\tv_addc_co_u32 %0, vcc, %0, %0, vcc"
-        : "+v"(mask)
-        : "v"(RowVectors<T>::element(v[i >> 2], i & 3)), "v"(floor)
-        : "vcc");
+  for (int i = 3; i >= 0; --i) {
+    uint64_t m0, m1, m2, m3;
+    asm("v_cmp_nlt_f32 %4, %8, %9\n\tv_cmp_nlt_f32 %3, %7, %9\n\t"
+        "v_cmp_nlt_f32 %2, %6, %9\n\tv_cmp_nlt_f32 %1, %5, %9\n\t"
+        "v_addc_co_u32 %0, %4, %0, %0, %4\n\tv_addc_co_u32 %0, %3, %0, %0, %3\n\t"
+        "v_addc_co_u32 %0, %2, %0, %0, %2\n\tv_addc_co_u32 %0, %1, %0, %0, %1"
+        : "+v"(mask), "=&s"(m0), "=&s"(m1), "=&s"(m2), "=&s"(m3)
+        : "v"(RowVectors<T>::element(v[i], 0)), "v"(RowVectors<T>::element(v[i], 1)),
+          "v"(RowVectors<T>::element(v[i], 2)), "v"(RowVectors<T>::element(v[i], 3)), "v"(floor));
+  }
   return mask;
 }
 

@@ -60,3 +60,31 @@ def test_a_value_in_tiles_behind_a_row_does_not_reach_it(cuda, behind):
     # the rows of whole 64-row tiles in front of the key tile that holds the first of them
     seen = first_bad // 64 * 64
     assert torch.isfinite(got[:seen].float()).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("kv_len,n_q,top", [(96, 96, 90), (300, 128, 100), (300, 128, 200), (500, 100, 499),
+                                            (1500, 16, 1111)])
+def test_a_weight_just_above_an_earlier_tile_is_not_rounded(cuda, dtype, d, kv_len, n_q, top):
+    """One key outweighs all others by 2^2.1 to 2^8.4, which the tiles in front of it do not show: its weight is
+    the row's reference and so exactly 1.  What is left are the roundings (u) of the result and of the small
+    weights, and 1e-5 for the sums and exponentials in 32 bits."""
+    from tidaldecode_amd import _kernels
+
+    g = torch.Generator().manual_seed(d + top)
+    pages = -(-kv_len // 16)
+    pool = torch.zeros((pages, 2, 16, 1, d))
+    pool.view(pages, 2, 16, d)[top // 16, 0, top % 16] = 1.0
+    pool[:, 1] = torch.randn((pages, 16, 1, d), generator=g)
+    pool = pool.to(dtype)
+    q = (torch.linspace(2.1, 8.4, n_q) / (math.sqrt(d) * math.log2(math.e)))[:, None, None].expand(n_q, 1, d).to(dtype)
+    got = _kernels.prefill_with_paged_kv_cache(q.contiguous().to(cuda), pool.to(cuda),
+                                               torch.arange(pages, dtype=torch.int32, device=cuda),
+                                               (kv_len - 1) % 16 + 1, False, 0, False, 1.0, 1e4)[:, 0].double().cpu()
+    k, v = (pool[:, i].reshape(-1, d)[:kv_len].double() for i in (0, 1))
+    p = (q[:, 0].double() @ k.t() / math.sqrt(d)).softmax(-1)
+    want = p @ v
+    p[:, top] = 0.0
+    u = 2.0 ** -11 if dtype == torch.float16 else 2.0 ** -8
+    assert ((got - want).abs() <= 1.01 * u * (want.abs() + p @ v.abs()) + 1e-5).all()

@@ -26,7 +26,7 @@
 // Measured in turn on one card (bf16, pages of 16, us, before with one 128- or 256-row tile per query head and
 // 16x16x32 MFMA -> now): prompt of 32768 x 32 heads 8633 -> 7592 (1159 TFLOP/s; a 16384^3 library GEMM reached
 // 1332 in the same run, and cards differ by 7 %), 8192 x 32 over 8 KV heads 588 -> 495, 1000 x 32 36.6 -> 24.0,
-// 300 x 32 14.1 -> 9.6 (staged kernel, two key groups: bound by the latency of five steps and cold code); 500 new tokens on 32768
+// 300 x 32 14.1 -> 9.8 (staged kernel, two key groups: bound by the latency of five steps and cold code); 500 new tokens on 32768
 // cached ones, 32 heads 991 -> 285, over 8 KV heads 993 -> 252; 16 tokens, 8 KV heads 792 -> 33.
 // Rows past the end of the sequence are clamped (never out of the pool) and masked.
 
@@ -112,6 +112,7 @@ struct PrefillParams {
   int32_t n_kv, n_rows, bm, n_tiles, n_splits, chunk, head_major;
   bool staged;     // prefill_attn_staged_kernel
   int32_t key_groups;  // of it: 1 or 2
+  float lag;           // of it: log2 of the largest weight a row may have before its reference point moves
   float* part_o;   // [n_splits][n_kv * n_rows][D]: un-normalised partial results (n_splits > 1)
   float* part_ml;  // [n_splits][n_kv * n_rows][2]: running maximum (base 2) and denominator
 };
@@ -719,10 +720,12 @@ __device__ __forceinline__ void staged_attention(const PrefillParams& p) {
       // m_run is kept in the scaled base-2 domain.  A masked entry (kNegBig) gives exp2(-huge) = 0 by
       // itself, also in a tile that masks the whole row (a later piece of the keys may begin with
       // one): the reference point never falls to where kNegBig lies.
-      // The running maximum only moves when the tile's maximum exceeds it by more than 2^8: softmax
-      // does not depend on the reference point, and the accumulator rescale below becomes rare.
+      // Softmax does not depend on the reference point, but a weight of 1 is exact in 16 bits and a larger one
+      // is rounded.  So the reference lags a row's maximum by no more than 2^lag (p.lag), and the accumulator's
+      // rescale stays rare.  With key groups a step is half as long: one row's move moves all rows of the wave.
       const float m_tile = fmaxf(t_max, kRowFloor) * p.scale_log2;
-      const float m_new = m_tile > m_run + 8.f ? m_tile : m_run;
+      const bool moves = KG == 1 ? m_tile > m_run + (D == 256 ? 8.f : p.lag) : __ballot(m_tile > m_run + p.lag) != 0;
+      const float m_new = moves ? fmaxf(m_tile, m_run) : m_run;
       const float alpha = fast_exp2(m_run - m_new);
       m_run = m_new;
       uint32_t pa[NSUB][2];
@@ -1071,6 +1074,7 @@ static void plan_shape(const td_paged_kv* kv, int32_t kv_len, int32_t n_q, int32
   p.causal = causal;
   p.staged = staged;
   p.key_groups = 1;
+  p.lag = 8.f;
   const int bn = p.staged ? 32 : 64, max_tiles = (kv_len + bn - 1) / bn;
   const int64_t cus = td_num_cus();
   double best = 0.0;
@@ -1114,20 +1118,27 @@ static void plan_prefill(const td_paged_kv* kv, int32_t kv_len, int32_t n_q, int
 // Short caches go to the staged kernel all the same, with no more scratch than was asked for: a step of either
 // kernel is a serial chain of about 1 us, the eight-wave kernel's rings and phases cost more to start than two
 // buffers, and two key groups halve the staged kernel's steps for 1 us of joining.  us, bf16, 32 / 8 heads of
-// 128 (32 / 32 within 0.4), eight waves | staged | staged with two key groups: 16 tokens 6.5 | 4.4 | 5.6, 96
-// 7.6 | 5.9 | 6.6, 128 7.8 | 6.7 | 6.7, 200 8.9 | 8.9 | 8.2, 300 10.6 | 11.5 | 9.8, 500 13.6 | 16.4 | 13.0; of
-// 64, 300 8.3 | 9.4 | 7.7.  A few rows on a cache of up to 1600 tokens, in pieces, eight waves | two key groups
-// with as much scratch: 16 on 500 12.4 | 11.9 (32 / 32 heads 11.6 | 10.9), 40 on 500 12.8 | 12.3, 16 on 1500
-// 12.8 | 12.0; 16 of 40 / 40 heads on 2000 15.1 | 15.5; twice as many row tiles gain nothing.
+// 128 (32 / 32 within 0.4), eight waves | staged | staged with two key groups: 16 tokens 6.5 | 4.0 | 5.6, 96
+// 7.3 | 5.8 | 6.6, 128 7.3 | 6.7 | 6.4, 200 8.8 | 8.9 | 8.1, 300 10.5 | 11.5 | 9.8, 500 13.5 | 16.4 | 13.3; of
+// 64, 500 10.1 | - | 10.0.  A few rows on a cache of up to 1600 tokens, in pieces, eight waves | two key groups
+// with as much scratch: 16 on 484 11.4 | 10.9, 40 on 460 11.9 | 11.3, 16 on 1484 12.5 | 11.9; 16 of 40 / 40
+// heads on 2000 15.1 | 15.5; twice as many row tiles gain nothing.
+// The reference points lag so little that no call is less exact than on the eight-wave kernel, whose first tile
+// shows a row twice as many keys.  Error against 64 bits in bf16, 1e-3, eight waves | here with a lag of 2^8 | now,
+// for queries of a normalised model and of four times the size: 96 tokens 1.88 | 1.91 | 1.87 and 1.72 | 1.87 | 1.70,
+// 300 1.98 | 1.96 | 1.94 and 1.81 | 1.92 | 1.70, 16 on 1500 2.28 | 2.26 | 2.19 and 1.78 | 1.87 | 1.67.  That costs
+// 0.1 - 0.4 us; a lag of 0 in the two groups as much again, and 500 tokens would gain nothing.
 static void plan_short(const td_paged_kv* kv, int32_t kv_len, int32_t n_q, int32_t num_qo_heads, int32_t causal,
                        int64_t scratch, PrefillParams& p) {
   if (p.staged || kv_len > 1600) return;
   const int64_t cus = td_num_cus(), tiles64 = (int64_t)p.n_kv * ((p.n_rows + 63) / 64);
   if (kv_len <= 96) {
     plan_shape(kv, kv_len, n_q, num_qo_heads, causal, true, 0, p);
+    p.lag = 0.f;
   } else if (p.n_splits > 1 && kv_len > 256 ? tiles64 <= cus * 3 / 16 : kv_len <= 512 && tiles64 <= 2 * cus) {
     plan_shape(kv, kv_len, n_q, num_qo_heads, causal, true, kv_len > 256 ? scratch : 0, p);
     p.key_groups = 2;
+    p.lag = 2.f;
   }
 }
 

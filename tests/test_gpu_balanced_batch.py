@@ -76,3 +76,47 @@ def test_fused_step_of_a_batch(cuda, batch, hi):
     assert (p0 - p1).abs().max() <= 2 ** -8 * 8 and (o0 - o1).abs().max() <= 1e-2
     fin = torch.isfinite(l0)
     assert torch.equal(fin, torch.isfinite(l1)) and (l0[fin] - l1[fin]).abs().max() <= 0.1
+
+
+def _pieces(cuda, heads, kv, d, lens, page=16, chunk=0):
+    """Attention of sequences of these lengths over lists of their pages; how many partial results a head has."""
+    from tidaldecode_amd import _kernels
+
+    batch, pages = len(lens), [-(-n // page) for n in lens]
+    w = _kernels.BatchDecodeWithPagedKVCachePyTorchWrapper(0)
+    w.chunk_tokens = chunk
+    w.begin_forward(None, heads, kv, d, page, torch.empty(0, dtype=torch.bfloat16))
+    g = torch.Generator(device=cuda).manual_seed(batch)
+    pool = torch.randn((sum(pages), 2, page, kv, d), generator=g, device=cuda).bfloat16()
+    first = [sum(pages[:b]) for b in range(batch)]
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=cuda)
+    table = torch.arange(sum(pages), dtype=torch.int32, device=cuda)[None]
+    q = torch.randn((batch, heads, d), generator=g, device=cuda).bfloat16()
+    o = torch.empty_like(q)
+    args = (q, o, pool, table, i32(first + [sum(pages)]), i32([(n - 1) % page + 1 for n in lens]),
+            i32([f + n - 1 for f, n in zip(first, pages)]), None)
+    w.forward(*args, n_list=max(pages) - 1, counts=i32([n - 1 for n in pages]))
+    for b in range(batch):
+        k, v = (pool[first[b]: first[b] + pages[b], i].reshape(-1, kv, d)[: lens[b]].float()
+                .repeat_interleave(heads // kv, 1).transpose(0, 1) for i in (0, 1))
+        want = torch.softmax((k @ q[b].float()[..., None])[..., 0] / math.sqrt(d), 1)[:, None] @ v
+        assert (o[b].float() - want[:, 0]).abs().max() <= 1e-2, b
+    plan = w._plan(batch, 1, (max(pages) - 1) * page + page, False)
+    partials = (w._workspace.numel() - (1 << 20)) // (4 * (d + 2) * plan.max_splits * batch) * plan.max_splits * batch
+    ml = (1 << 20) + (partials * d * 4 + 255) // 256 * 256
+    return int((w._workspace[ml: ml + partials * 8].view(torch.float32).view(-1, 2)[:, 1] > 0).sum()), partials // (
+        plan.max_splits * batch)
+
+
+@pytest.mark.parametrize("heads,kv,d,lens", [(8, 1, 128, [8192] * 16), (8, 1, 128, [40000, 50]),
+                                             (16, 2, 128, [20000, 36000, 1200, 36000]), (12, 2, 128, [4096] * 16),
+                                             (6, 2, 64, [6000] * 3 + [1000] * 5)])
+def test_few_head_rows_fill_the_chip(cuda, heads, kv, d, lens):
+    """Head rows times pieces take at least three quarters of the compute units, as far as 64 pieces of a
+    sequence (what a merge takes) and tiles of 128 tokens (256 of 64 dimensions) go."""
+    done, head_slots = _pieces(cuda, heads, kv, d, lens)
+    hrows = kv * -(-(heads // kv) // 8)
+    tile = 8 * 4 * (64 // (d // 8))
+    room = hrows * sum(min(64, -(-n // tile)) for n in lens)
+    assert done % head_slots == 0
+    assert done // head_slots * hrows >= 0.75 * min(256, room)

@@ -885,11 +885,13 @@ __global__ __launch_bounds__(NW * 64) void decode_attn_kernel(const DecodeParams
 // launch lasts as long as the largest remainder of one, and a batch of short sequences leaves most of the
 // chip idle.  One MI355X, bf16, logits out, even chunks -> dealt (us): 16 sequences of 500 .. 8192 tokens,
 // 32/8 heads x 128, 77 -> 69.7 (4.7 TB/s); 8 of 8000 .. 60000, 295 -> 261; 4 of 2000, 36.7 -> 15.8; 12 of
-// 400 .. 9000, 28/4 heads, 59.7 -> 51.  The lengths and the search cost 1.5 us, which is what equal lengths
-// lose (16 x 8192: 98.9 -> 100.7).  Runs of equal length laid over the ends of the sequences balance better
+// 400 .. 9000, 28/4 heads, 59.7 -> 51; few head rows: 8/1 heads, 16 of 2000 .. 32768, 55 -> 47, 40 of 300 .. 4000,
+// 4/1 heads, 26.3 -> 18.8, 16/2 heads, 8 of 8000 .. 65536, 99 -> 87.  The lengths and the search cost 1.5 - 2 us,
+// which is what equal lengths lose (16 x 8192: 98.9 -> 100.7; 8/1 heads, 16 x 32768: 69.1 -> 71.1).  Runs of equal length laid over the ends of the sequences balance better
 // still but pay the start and the merge of every further sequence, 5 us: 72 for the first batch, 110 for
 // 16 x 8192.
 constexpr int kBalancedMaxBatch = 64;  // one lane per sequence
+constexpr int kMergedPieces = 64;      // pieces of a sequence that merge_splits takes
 
 template <typename T, int D, int QPG, int U, int NW, bool EMIT, bool LEAN, bool FRESH>
 __global__ __launch_bounds__(NW * 64) void decode_attn_balanced_kernel(const DecodeParams p) {
@@ -901,10 +903,12 @@ __global__ __launch_bounds__(NW * 64) void decode_attn_balanced_kernel(const Dec
   int tiles = (mine.n_items + WTILE - 1) / WTILE;
   tiles = lane < p.batch ? (tiles < 1 ? 1 : tiles) : 0;
   // the shortest piece, in tiles, for which all sequences together have no more pieces than slots: lane l
-  // tries the l-th of 64 lengths between the mean and the longest sequence, which always fits
+  // tries the l-th of 64 lengths between the mean (or what cuts the longest sequence into as many pieces as
+  // are merged) and the longest sequence, which always fits
   const int sum = (int)__builtin_amdgcn_readlane(wave_prefix_sum_dpp((uint32_t)tiles, lane), 63);
   const int most = wave_max_i32(tiles);
-  const int least = (sum + p.slots - 1) / p.slots;  // <= most: slots >= batch
+  const int mean = (sum + p.slots - 1) / p.slots, fewest = (most + kMergedPieces - 1) / kMergedPieces;
+  const int least = mean > fewest ? mean : fewest;  // <= most: slots >= batch
   const int piece = least + (most - least) * lane / 63;
   const float inv = 1.f / (float)piece;
   int pieces = 0;

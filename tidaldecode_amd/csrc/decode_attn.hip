@@ -34,11 +34,11 @@ constexpr int64_t kTicketBytes = (int64_t)16384 * kTicketStride * 4;
 constexpr int64_t kSparseMaxItems = 64 * 256;
 
 // Workgroups per head row of a balanced launch (decode_attn_balanced_kernel): as many rounds of one per
-// compute unit as give every sequence one; at most 64 pieces of a sequence are merged.
+// compute unit as give every sequence one; at most kMergedPieces of a sequence are merged.
 static int balanced_slots(int n_hrows, int batch) {
   const int round = num_cus() / n_hrows < 1 ? 1 : num_cus() / n_hrows;
-  const int64_t slots = ceil_div64(batch, round) * round;
-  return (int)(slots > 64 ? 64 : slots);
+  const int64_t slots = ceil_div64(batch, round) * round, merged = (int64_t)batch * kMergedPieces;
+  return (int)(slots < merged ? slots : merged);
 }
 
 static bool is_pow2(int64_t x) { return x > 0 && (x & (x - 1)) == 0; }

@@ -120,6 +120,8 @@ typedef struct {
    * every call of this plan. */
   int32_t sparse_waves;
   int32_t sparse_rows;
+  int32_t balanced;        /* output: 1 if page lists of a batch on shared KV rows are dealt to the workgroups by
+                            * the sequences' lengths instead of in chunks; 0 where chunk_tokens was preset */
   int64_t workspace_bytes; /* device scratch the call needs (partials + tickets) */
 } td_decode_plan;
 

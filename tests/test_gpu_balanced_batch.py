@@ -120,3 +120,9 @@ def test_few_head_rows_fill_the_chip(cuda, heads, kv, d, lens):
     room = hrows * sum(min(64, -(-n // tile)) for n in lens)
     assert done % head_slots == 0
     assert done // head_slots * hrows >= 0.75 * min(256, room)
+
+
+def test_preset_chunks_are_kept(cuda):
+    """A chunk size set by the caller cuts every sequence, however long the others are."""
+    done, head_slots = _pieces(cuda, 8, 2, 128, [16384, 4096, 700], chunk=256)
+    assert done // head_slots == 64 + 16 + 3

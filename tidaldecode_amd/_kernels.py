@@ -662,7 +662,7 @@ class BatchDecodeWithPagedKVCachePyTorchWrapper:
         self._workspace = None
         self.waves_per_block = 0  # 0 = library default; tuning knob
         self.fused_merge = -1     # -1 = library default
-        self.chunk_tokens = 0     # 0 = library default
+        self.chunk_tokens = 0     # 0 = library default (ragged batches on shared KV rows: dealt by length)
         self.tile_rows = 0        # 0 = library default
         self.sparse_waves = 0     # short-list kernel: 0 = library default, -1 = never
         self.sparse_rows = 0

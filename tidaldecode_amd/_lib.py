@@ -77,6 +77,7 @@ class DecodePlan(Structure):
         ("fused_merge", c_int32),
         ("sparse_waves", c_int32),
         ("sparse_rows", c_int32),
+        ("balanced", c_int32),
         ("workspace_bytes", c_int64),
     ]
 

@@ -116,6 +116,7 @@ extern "C" int td_decode_make_plan(int32_t batch, int32_t num_qo_heads, int32_t 
   // tile; the streaming kernel at 8 waves x 4 rows (tile 128) can run the same plan when a call
   // turns out not to fit the short-list kernel (page lists, score output, large pools).
   int sw = plan->sparse_waves, sr = plan->sparse_rows;
+  plan->balanced = 0;
   // one query head per list walk with a power-of-two group size, or exactly 2, 4 or 8 query heads
   // sharing their KV head's list (no padding heads)
   const int group = num_qo_heads / num_kv_heads;
@@ -261,7 +262,8 @@ extern "C" int td_decode_make_plan(int32_t batch, int32_t num_qo_heads, int32_t 
   if (max_splits < 1) max_splits = 1;
   // room for the partials of a balanced launch (one per slot and head slot), unless that alone would take
   // the plan beyond the built-in scratch
-  if (batch > 1 && batch <= kBalancedMaxBatch && qpg > 1 && plan->chunk_tokens == 0) {
+  plan->balanced = batch > 1 && batch <= kBalancedMaxBatch && qpg > 1 && plan->chunk_tokens == 0;
+  if (plan->balanced) {
     const int64_t wanted = ceil_div64(balanced_slots(n_hrows, batch), batch);
     const int64_t bytes = kTicketBytes + (int64_t)batch * n_hrows * qpg * wanted * (head_dim + 2) * 4 + 512;
     if (wanted > max_splits && bytes <= (int64_t)TD_STATIC_SCRATCH_BYTES) max_splits = wanted;
@@ -431,9 +433,10 @@ static int build_params(const td_paged_kv* kv, const td_index_list* list, const 
   p.ticket_stride = kTicketStride;
   p.batch = batch;
   // Balanced: the full attention of a batch on the shared-row kernels, merged in the launch, when the
-  // workspace holds its partials.
+  // workspace holds its partials and the caller has not set the chunks.
   p.slots = 0;
-  if (qpg > 1 && batch > 1 && batch <= kBalancedMaxBatch && list->kind == TD_IDX_PAGES && plan->fused_merge) {
+  if (plan->balanced && qpg > 1 && batch > 1 && batch <= kBalancedMaxBatch && list->kind == TD_IDX_PAGES &&
+      plan->fused_merge) {
     const int slots = balanced_slots(n_hrows, batch);
     if ((int64_t)batch * plan->max_splits >= slots) p.slots = slots;
   }

@@ -1,10 +1,12 @@
 """The native half of the entry points (csrc/host_calls.cpp): whatever it does not take as regular goes on in
 Python with the same result or the same error, and what it takes gives the bits that Python gives."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
 
-from tidaldecode_amd import _kernels
+from tidaldecode_amd import _kernels, _lib
 from tidaldecode_amd._lib import host_calls
 
 _NATIVE = ("forward", "attend", "topk", "rope_table", "rope_in_place", "append", "prefill", "gemv", "score_reduce",
@@ -37,57 +39,110 @@ def test_host_tensors_are_refused_as_before():
     assert host_calls.gemv(object(), None, None, 1e-5, False, None, False, None, 0) is False
 
 
-@pytest.mark.gpu
-@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("heads,kv,d,page,layout,mode", [(8, 8, 128, 16, "NHD", "per_head"),
-                                                         (8, 2, 64, 4, "HND", "group_sum"),
-                                                         (4, 4, 256, 7, "NHD", "per_head")])
-def test_same_bits_as_the_python_path(cuda, monkeypatch, dtype, heads, kv, d, page, layout, mode):
+class _Recorder:
+    """host_calls, with what was called and did not decline"""
+
+    def __init__(self):
+        self.served = []
+
+    def __getattr__(self, name):
+        def call(*a):
+            made = getattr(host_calls, name)(*a)
+            if made is not False:
+                self.served.append((name, a))
+            return made
+        return call
+
+
+def _workload(cuda, dtype, heads, kv, d, page, layout, mode):
+    """A prompt and two decode steps through the public entry points; every tensor they make."""
     from tidaldecode_amd import utils as ops
     from tidaldecode_amd.utils import InferenceController
 
-    def run(native):
-        if not native:
-            monkeypatch.setattr(_kernels, "host_calls", _Off())
-            monkeypatch.setattr(ops, "host_calls", _Off())
-        g = torch.Generator(device=cuda).manual_seed(7)
-        randn = lambda *s: torch.randn(s, generator=g, device=cuda).to(dtype)
-        c = InferenceController(2, heads, d, page, 40, 400, dtype, cuda, num_kv_heads=kv, select_mode=mode,
-                                kv_layout=layout, page_order_seed=5)
-        c.kv_cache.pool.buf.zero_()
-        out = []
-        q, k, v = randn(300, heads, d), randn(300, kv, d), randn(300, kv, d)
-        c.prepare_metadata(300)
-        c.begin_forward(300)
-        ops.apply_rope_in_place(q, k, 0)
+    g = torch.Generator(device=cuda).manual_seed(7)
+    randn = lambda *s: torch.randn(s, generator=g, device=cuda).to(dtype)
+    c = InferenceController(2, heads, d, page, 40, 400, dtype, cuda, num_kv_heads=kv, select_mode=mode,
+                            kv_layout=layout, page_order_seed=5, with_metadata=True)
+    c.kv_cache.pool.buf.zero_()
+    c.metadata_cache.pool.buf.zero_()
+    out = []
+    q, k, v = randn(300, heads, d), randn(300, kv, d), randn(300, kv, d)
+    c.prepare_metadata(300)
+    c.begin_forward(300)
+    ops.apply_rope_in_place(q, k, 0)
+    for layer in range(2):
+        ops.append_kv(k, v, c, layer)
+        out.append(ops.prefill_forward(q, c, layer))
+    for step in range(2):
+        c.prepare_metadata(1)
+        c.begin_forward(1)
+        q, k, v = randn(1, heads, d), randn(1, kv, d), randn(1, kv, d)
+        pos = torch.tensor([300 + step], dtype=torch.int32, device=cuda)
+        out += list(_kernels.rope_table(pos, d, 1.0, 5e5))
+        ops.apply_rope_in_place(q, k, 300 + step)
         for layer in range(2):
             ops.append_kv(k, v, c, layer)
-            out.append(ops.prefill_forward(q, c, layer))
-        for step in range(2):
-            c.prepare_metadata(1)
-            c.begin_forward(1)
-            q, k, v = randn(1, heads, d), randn(1, kv, d), randn(1, kv, d)
-            pos = torch.tensor([300 + step], dtype=torch.int32, device=cuda)
-            out += list(_kernels.rope_table(pos, d, 1.0, 5e5))
-            ops.apply_rope_in_place(q, k, 300 + step)
-            for layer in range(2):
-                ops.append_kv(k, v, c, layer)
-                if layer == 0:
-                    out.append(ops.decode_sparse_attn(q, c, layer, c.kv_indices_without_last, True))
-                    ops.decode_topk(c)
-                else:
-                    out.append(ops.decode_sparse_attn(q, c, layer, c.topk_dindices_buffer, False))
-            out += [c.qk_product.clone(), c.lse.clone(), c.topk_dindices_buffer.clone()]
-        w, x = randn(48, 64), randn(64)
-        out += [_kernels.gemv(w, x), _kernels.gemv(w, x, norm_weight=randn(64), pair_gated=True),
-                _kernels.gemv(w, x, residual=randn(48))]
-        torch.cuda.synchronize()
-        return out + [c.kv_cache.pool.buf]
+            if layer == 0:
+                out.append(ops.decode_sparse_attn(q, c, layer, c.kv_indices_without_last, True))
+                ops.decode_topk(c)
+                out.append(ops.decode_estimate(q, c, layer))
+            else:
+                out.append(ops.decode_sparse_attn(q, c, layer, c.topk_dindices_buffer, False))
+        o = torch.empty_like(q)
+        c._decode_handler.forward(q, o, c.kv_cache.buf_layer(0), c.kv_indices_without_last, None,
+                                  c.kv_cache.last_page_len, c.kv_last_page_idx, None)
+        out += [o, c.qk_product.clone(), c.lse.clone(), c.topk_dindices_buffer.clone()]
+    w, x = randn(48, 64), randn(64)
+    out += [_kernels.gemv(w, x), _kernels.gemv(w, x, norm_weight=randn(64), pair_gated=True),
+            _kernels.gemv(w, x, residual=randn(48))]
+    torch.cuda.synchronize()
+    return out + [c.kv_cache.pool.buf, c.metadata_cache.pool.buf], c
 
-    a, b = run(True), run(False)
+
+_SHAPES = [(8, 8, 128, 16, "NHD", "per_head"), (8, 2, 64, 4, "HND", "group_sum"), (4, 4, 256, 7, "NHD", "per_head")]
+
+
+def _use(monkeypatch, calls):
+    from tidaldecode_amd import utils as ops
+
+    monkeypatch.setattr(_kernels, "host_calls", calls)
+    monkeypatch.setattr(ops, "host_calls", calls)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("shape", _SHAPES)
+def test_same_bits_as_the_python_path(cuda, monkeypatch, dtype, shape):
+    a, _ = _workload(cuda, dtype, *shape)
+    _use(monkeypatch, _Off())
+    b, _ = _workload(cuda, dtype, *shape)
     assert len(a) == len(b)
     for x, y in zip(a, b):
         assert x.dtype == y.dtype and x.shape == y.shape and torch.equal(x, y)
+
+
+@pytest.mark.gpu
+def test_launches_leave_the_interpreters_lock(cuda, monkeypatch):
+    """Every call that was served, once more with PyGILState_Check (1 where its thread holds the lock, which
+    reads as an error status) in place of the functions that launch."""
+    calls, keep = _Recorder(), []
+    _use(monkeypatch, calls)
+    for shape in _SHAPES:
+        keep.append(_workload(cuda, torch.bfloat16, *shape))
+    real = {name: ctypes.cast(getattr(_lib.lib, name), ctypes.c_void_p).value for name in _lib.SIGNATURES}
+    check = ctypes.cast(ctypes.pythonapi.PyGILState_Check, ctypes.c_void_p).value
+    on_host = ("td_last_error", "td_decode_make_plan", "td_topk_workspace_bytes", "td_prefill_workspace_bytes")
+    host_calls.bind({name: at if name in on_host else check for name, at in real.items()})
+    held = set()
+    try:
+        for name, args in calls.served:
+            try:
+                assert getattr(host_calls, name)(*args) is not False, name
+            except RuntimeError:
+                held.add(name)
+    finally:
+        host_calls.bind(real)
+    assert held == set()
 
 
 @pytest.mark.gpu

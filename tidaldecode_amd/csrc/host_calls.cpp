@@ -463,9 +463,9 @@ bool prefill_regular(PyObject* const* a, int& rc) {
   const int causal = a[5] == Py_True;
   if (q->size(2) != pool.head_dim || q->scalar_type() != kv->scalar_type() || kv_len < 0 || kv_len > INT32_MAX) return false;
   if (lib.prefill_workspace_bytes(&pool, (int32_t)kv_len, (int32_t)q->size(0), (int32_t)q->size(1), causal) != 0) return false;
-  rc = lib.prefill_attn_split(&pool, ptr_as<int32_t>(*idx), (int32_t)n_pages, (int32_t)kv_len, ptr(*q), ptr(*o),
-                              (int32_t)q->size(0), (int32_t)q->size(1), (float)(1.0 / std::sqrt((double)pool.head_dim)),
-                              causal, nullptr, 0, stream_of(a[7]));
+  rc = unlocked(lib.prefill_attn_split, &pool, ptr_as<int32_t>(*idx), (int32_t)n_pages, (int32_t)kv_len, ptr(*q),
+                ptr(*o), (int32_t)q->size(0), (int32_t)q->size(1), (float)(1.0 / std::sqrt((double)pool.head_dim)),
+                causal, nullptr, 0, stream_of(a[7]));
   return true;
 }
 

@@ -321,3 +321,18 @@ def test_caches_of_one_key_tile(cuda, hq, hkv, d, page, causal):
             got = _run(cuda, case, q, causal, dtype).float().cpu()
             want = _dense(q, case.k, case.v, causal)
             assert ((got - want).abs() <= ATOL[dtype] * want.abs().clamp(min=1.0)).all(), (kv_len, n_q)
+
+
+def test_a_call_with_scratch_makes_two_allocations(cuda):
+    """the result and the scratch"""
+    from tidaldecode_amd import _kernels
+
+    past, n_q, h, d = 8192, 1000, 32, 128
+    case = PagedCase(past + n_q, 8, d, 16, torch.bfloat16, seed=3)
+    q = randn((n_q, h, d), 4, torch.bfloat16)
+    assert _planned_bytes(case, q, True) > 0
+    q_d, pool, table = q.bfloat16().to(cuda), case.pool.to(cuda), case.page_table.int().to(cuda)
+    made = lambda: torch.cuda.memory_stats()["allocation.all.allocated"]
+    before = made()
+    _kernels.prefill_with_paged_kv_cache(q_d, pool, table, case.last_page_len, True, 0, False, 1.0, 1e4)
+    assert made() - before == 2

@@ -626,7 +626,6 @@ def prefill_with_paged_kv_cache(q, kv_data, kv_indices, kv_last_page_len, causal
     kv_len = (n_pages - 1) * pool.page_size + int(kv_last_page_len)
     if q.size(2) != pool.head_dim or q.dtype != kv_data.dtype:
         raise RuntimeError("prefill_with_paged_kv_cache: q does not fit the cache")
-    o = torch.empty_like(q)
     causal = int(bool(causal))
     # scratch of this call alone (torch's allocator hands it out again in stream order)
     ws_bytes = lib.td_prefill_workspace_bytes(pool, kv_len, q.size(0), q.size(1), causal)

@@ -26,3 +26,21 @@ def test_same_bits(cuda, hq, hkv, n):
         want = torch.exp(wide[:, :n].double() - lse[:, None].double()).view(rows, hq // rows, n).sum(1)
         # an exponential of 2^-20 relative error (arguments up to 2^5 in 32 bits), summed in 32 bits
         assert ((a.double() - want).abs() <= 2.0 ** -16 * want + 1e-12).all()
+
+
+@pytest.mark.parametrize("n", [2 ** 31 - 256, 2 ** 31 - 100, 2 ** 31 - 99])
+def test_as_many_tokens_as_a_row_may_have(cuda, n):
+    """More than one launch numbers; rows whose last workgroup of 256 tokens would end beyond 31 bits, and one
+    that is read a token at a time."""
+    from tidaldecode_amd import _kernels
+
+    logits = torch.zeros((1, n), device=cuda)
+    at = [0, 2 ** 30 - 65, 2 ** 30 - 64, 2 ** 30 + 1, n - 2, n - 1]
+    for j, i in enumerate(at):
+        logits[0, i] = j + 1.0
+    out = torch.full((1, n), -1.0, device=cuda)
+    _kernels.score_reduce(logits, torch.zeros(1, device=cuda), 1, n, "head_sum", out=out)
+    del logits
+    assert torch.allclose(out[0, at].cpu(), torch.arange(1.0, 7.0).exp(), rtol=1e-6)
+    out[0, at] = 1.0
+    assert out.amin() == 1.0 and out.amax() == 1.0

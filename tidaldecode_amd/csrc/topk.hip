@@ -1435,9 +1435,13 @@ extern "C" int td_score_reduce(const float* logits, int64_t logits_stride, const
   const bool wide = ((uintptr_t)logits & 15) == 0 && logits_stride % 4 == 0 &&
                     (int64_t)rows * n >= 1024 * 256;  // four workgroups a compute unit
   const int tokens = wide ? 256 : 64;
-  hipLaunchKernelGGL((wide ? score_reduce_kernel<4> : score_reduce_kernel<1>), dim3((n + tokens - 1) / tokens, rows),
-                     dim3(256), 0, reinterpret_cast<hipStream_t>(stream), logits, logits_stride, lse,
-                     num_qo_heads / rows, n, out, out_stride);
+  // a launch numbers its threads with 32 bits: 2^30 - 64 tokens at a time
+  for (int64_t first = 0; first < n; first += (1 << 30) - 64) {
+    const int part = (int)(n - first < (1 << 30) - 64 ? n - first : (1 << 30) - 64);
+    hipLaunchKernelGGL((wide ? score_reduce_kernel<4> : score_reduce_kernel<1>), dim3((part + tokens - 1) / tokens, rows),
+                       dim3(256), 0, reinterpret_cast<hipStream_t>(stream), logits + first, logits_stride, lse,
+                       num_qo_heads / rows, part, out + first, out_stride);
+  }
   TD_HIP_CHECK(hipGetLastError());
   return TD_OK;
 }

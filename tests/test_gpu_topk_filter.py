@@ -110,3 +110,59 @@ def test_scores_just_above_the_samples_maximum(cuda, n):
         got, vals = _run(cuda, v, k)
         want = orc.stable_topk(v, k)
         assert torch.equal(got, want) and torch.equal(vals, torch.gather(v, 1, want)), k
+
+
+def _crowded_rows(n, k, dtype, g):
+    """rows whose threshold lies in or next to many equal scores"""
+    pick = lambda share: torch.rand(n, generator=g) < share
+    mostly = lambda share, rest: torch.where(pick(share), 1.0 + torch.rand(n, generator=g), torch.tensor(rest))
+    inf = float("inf")
+    return torch.stack([
+        torch.full((n,), -3.5), torch.randint(0, 2, (n,), generator=g).float(), mostly(0.4 * k / n, 0.0),
+        mostly(1.08 * k / n, 0.0), mostly(0.4 * k / n, -inf), torch.full((n,), inf), torch.full((n,), float("nan")),
+        torch.where(pick(0.5), torch.tensor(0.0), torch.tensor(-0.0)), torch.where(pick(0.3 * k / n), inf, 2.0),
+        mostly(0.5 * k / n, 0.0) - mostly(0.3 * k / n, 0.0), torch.randint(-9, 9, (n,), generator=g).float(),
+    ]).to(dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("n,k", [(5000, 700), (8195, 3), (9001, 1500), (20000, 4000), (65536, 1024), (65537, 4000),
+                                 (262144, 2500)])
+def test_rows_of_few_values(cuda, dtype, n, k):
+    """More equal scores than the list holds: those above are listed, of the equal ones the first by position
+    are taken; a second crowd above or below the threshold's."""
+    from oracle import tidal_oracle as orc
+
+    g = torch.Generator().manual_seed(n + k)
+    v = _crowded_rows(n, k, dtype, g)
+    want = orc.stable_topk(v.float(), k)
+    payload = torch.randint(0, 1 << 30, v.shape, generator=g, dtype=torch.int32)
+    table = torch.randperm(-(-n // 48) + 3, generator=g).int()
+    for pad, skew in ((0, 0), (1, 1)):
+        got, vals = _run(cuda, v, k, pad=pad, skew=skew)
+        assert torch.equal(got, want), [r for r in range(len(v)) if not torch.equal(got[r], want[r])]
+        assert torch.equal(vals.nan_to_num(77.0), torch.gather(v, 1, want).nan_to_num(77.0))
+        got, _ = _run(cuda, v, k, in_idx=payload, pad=pad, skew=skew)
+        assert torch.equal(got, torch.gather(payload.long(), 1, want))
+        got, _ = _run(cuda, v, k, table=table, page=48, vals=False, pad=pad, skew=skew)
+        assert torch.equal(got, table.long()[want // 48] * 48 + want % 48)
+
+
+@pytest.mark.parametrize("n,k", [(4096, 256), (32768, 2048), (102392, 4096)])
+def test_rows_of_equal_scores_take_about_as_long_as_others(cuda, n, k):
+    """at most eight times as long (a selection by one workgroup that queues up at one address took 4 to 34 times)"""
+    from tidaldecode_amd import _kernels
+
+    out = torch.zeros((32, k), dtype=torch.int32, device=cuda)
+    took = {}
+    for kind, v in (("normal", torch.randn((32, n), device=cuda)), ("equal", torch.zeros((32, n), device=cuda))):
+        for _ in range(2):
+            _kernels.topk_filtering(v, None, None, out, None, k)
+        start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        start.record()
+        for _ in range(50):
+            _kernels.topk_filtering(v, None, None, out, None, k)
+        end.record()
+        torch.cuda.synchronize()
+        took[kind] = start.elapsed_time(end)
+    assert took["equal"] <= 8 * took["normal"], took

@@ -9,8 +9,9 @@
 //   2. one pass over the row (loads in flight from the start) keeps the positions of what is not below
 //      it, about 1.1 .. 1.4 k elements, in LDS: two instructions per element, some more per survivor;
 //   3. the radix select of the k-th largest runs on the survivors (exact: fewer survivors than k start
-//      again with a lower threshold; more than the list holds -- rows of few distinct values -- leave
-//      the row to select_slice);
+//      again with a lower threshold; more than the list holds -- rows of few distinct values -- once more
+//      with the sample's value at that rank as the threshold, equal scores being counted and not listed;
+//      should even what lies above it be too much, the row is left to select_slice);
 //   4. the selected positions go into a bitmap in LDS, whose prefix counts give every one its place
 //      in position order, whatever order the survivors were listed in.
 //
@@ -23,6 +24,11 @@
 //   32 x 4096 -> 256    6.7 (8.3)     256 x 63000 -> 1024  23.3 (58.6)
 //   512 x 8192 -> 512   10.7 (19.5)   256 x 65537 -> 1024  24.4 (120)
 //   32 x 32769 -> 2048  12.6 (15.9)   8 x 102392 -> 4096   19.5 (28.6: three launches that share a row)
+// Rows of equal scores, and of two values by halves, through the ties' threshold (before that kernel; a selection
+// by one workgroup out of the whole row, whose additions queue up at one address, took 130 and 630 for the second
+// and the last): 32 x 4096 -> 256 21.0, 17.2 (20.5, 14.2); 32 x 32769 -> 2048 27.4, 24.8 (98.8, 54.4); 256 x 63000
+// -> 1024 45.6, 42.5 (202, 120); 8 x 102392 -> 4096 40.9, 36.3 (211, 123).  Having that way out costs other rows
+// 0.1 - 0.3 us.
 // What is left is a chain: two trips to memory (sample, survivors' values), two radix levels of about
 // 1 us and the bitmap's 0.8; 256 rows of 63000 also read 64 MB at 2.8 TB/s.
 // The results are those of every other variant: the k largest, ties to the lower position, in
@@ -205,8 +211,10 @@ __global__ __launch_bounds__(NT) void topk_filter_kernel(const TopkParams p) {
   // ---- radix select: the krem-th smallest of what each() hands out, as the krem-th smallest of the
   // n_in ones in [lo, lo + 2^s): at most kFilterRank, or all equal (s == 0).  The window [lo, lo + last]
   // comes first, what lies beyond it only if fewer than krem lie inside.  False: fewer than krem in all.
+  // exact: until s == 0.  crowded: lanes with equal bins add together, for equal scores queue up at one
+  // address (from the second level on by itself: a bin of more than kFilterRank members was chosen).
   uint32_t lo, s, krem, n_in;
-  auto narrow = [&](uint32_t last, auto each) -> bool {
+  auto narrow = [&](uint32_t last, bool crowded, bool exact, auto each) -> bool {
     auto shift_of = [](uint32_t span) {
       const int b = bit_count(span) - kBits;
       return b > 0 ? (uint32_t)b : 0u;
@@ -215,10 +223,25 @@ __global__ __launch_bounds__(NT) void topk_filter_kernel(const TopkParams p) {
     s = shift_of(last);
     for (;;) {
       last |= (1u << s) - 1u;  // whole bins: what lies in the last one is counted with it, also beyond the window
-      each([&](uint32_t x) {
-        const uint32_t d = x - lo;
-        if (d <= last) atomicAdd(&L.hist[d >> s], 1u);
-      });
+      if (__builtin_expect(!crowded, 1)) {
+        each([&](uint32_t x) {
+          const uint32_t d = x - lo;
+          if (d <= last) atomicAdd(&L.hist[d >> s], 1u);
+        });
+      } else {
+        each([&](uint32_t x) {
+          const uint32_t d = x - lo, bin = d >> s;
+          uint64_t left = __ballot(d <= last);
+          while (left) {  // worth a turn for eight lanes and more
+            const int one = __builtin_ctzll(left);
+            const uint64_t same = __ballot(bin == (uint32_t)__builtin_amdgcn_readlane(bin, one)) & left;
+            if (__popcll(same) < 8) break;
+            if (lane == one) atomicAdd(&L.hist[bin], (uint32_t)__popcll(same));
+            left &= ~same;
+          }
+          if ((left >> lane) & 1u) atomicAdd(&L.hist[bin], 1u);
+        });
+      }
       __syncthreads();
       uint4* h4 = reinterpret_cast<uint4*>(L.hist) + tid;
       const uint4 a = *h4;
@@ -242,7 +265,8 @@ __global__ __launch_bounds__(NT) void topk_filter_kernel(const TopkParams p) {
         lo += __builtin_amdgcn_readfirstlane(L.sh[0]) << s;
         krem = __builtin_amdgcn_readfirstlane(L.sh[1]);
         n_in = __builtin_amdgcn_readfirstlane(L.sh[2]);
-        if (s == 0u || n_in <= (uint32_t)kFilterRank) return true;
+        if (s == 0u || (n_in <= (uint32_t)kFilterRank && !exact)) return true;
+        crowded = true;
         last = (1u << s) - 1u;
       } else {
         if (last >= kMaxSpan - lo) return false;
@@ -258,6 +282,8 @@ __global__ __launch_bounds__(NT) void topk_filter_kernel(const TopkParams p) {
     for (int c = 0; c < 4; ++c) f(sx[c]);
   };
   constexpr uint32_t kFirst = (1u << 29) - 1u;  // 64 binades below the reference first
+  // (a wave's own affair: eight lanes that sampled the same score)
+  const bool alike = __popcll(__ballot(sx[0] == (uint32_t)__builtin_amdgcn_readfirstlane(sx[0]))) >= 8;
 
   // What is selected from, n slots: x (kNoElement: empty) and position.  The row itself if it is its
   // own sample, else the survivors.
@@ -274,6 +300,31 @@ __global__ __launch_bounds__(NT) void topk_filter_kernel(const TopkParams p) {
       }
     }
   };
+  const int wpt = (n_words + NT - 1) / NT;
+  // before[w] = set bits in front of word w (of more than 16 bits hold: 65535); their number
+  auto count_words = [&]() -> uint32_t {
+    __syncthreads();
+    uint32_t local = 0;
+    for (int i = 0; i < wpt; ++i) {
+      const int w = tid * wpt + i;
+      local += w < n_words ? __popc(L.bits[w]) : 0u;
+    }
+    const uint32_t incl = wave_prefix_sum_dpp(local, lane);
+    if (lane == 63) L.wa[wave] = incl;
+    __syncthreads();
+    uint32_t run, total;
+    sums_before<NW>(L.wa, wave, lane, run, total);
+    run += incl - local;
+    for (int i = 0; i < wpt; ++i) {
+      const int w = tid * wpt + i;
+      if (w < n_words) {
+        L.before[w] = (uint16_t)(run < 65535u ? run : 65535u);
+        run += __popc(L.bits[w]);
+      }
+    }
+    __syncthreads();
+    return total;
+  };
   if (whole) {
 #pragma unroll
     for (int u = 0; u < CPT; ++u) {
@@ -283,16 +334,25 @@ __global__ __launch_bounds__(NT) void topk_filter_kernel(const TopkParams p) {
     }
     n = 4 * NT;
     krem = krem0 = (uint32_t)k;
-    narrow(kFirst, each_sample);
+    narrow(kFirst, alike, false, each_sample);
   } else if constexpr (kSampled) {
     // ---- 2. the survivors: what is not below the far edge of the bin that holds rank `rank` ---------
-    uint32_t kbase;
+    // above: a second time, what is above the sample's value at that rank
+    uint32_t kbase, tie = 0u;
+    bool above = false, equal = false;
     for (;;) {
       kbase = 0u;
       krem = rank;
-      if (narrow(kFirst, each_sample)) {
+      if (narrow(kFirst, above || alike, above, each_sample)) {
         const uint32_t edge = lo + ((1u << s) - 1u);
         kbase = kmax > edge ? kmax - edge : 0u;
+        equal = n_in > (uint32_t)kFilterRank;
+      }
+      if (__builtin_expect(above, 0)) {
+        tie = kbase;
+        C = CAP + 1u;
+        if (tie < kKeyNegInf || tie >= kKeyPosInf) break;
+        ++kbase;
       }
       kbase = kbase < kKeyNegInf ? kKeyNegInf : (kbase > kKeyPosInf ? kKeyPosInf : kbase);
       const float floor_f = key_to_float(kbase);
@@ -332,15 +392,80 @@ __global__ __launch_bounds__(NT) void topk_filter_kernel(const TopkParams p) {
       }
       __syncthreads();
       C = __builtin_amdgcn_readfirstlane(L.n_cand);
-      if (C >= (uint32_t)k) break;
-      rank = 2u * rank + 64u;  // an unlucky sample: the k-th largest lies below the floor
+      if (above || (C >= (uint32_t)k && (kFits || C <= (uint32_t)CAP))) break;
+      if (C >= (uint32_t)k)
+        above = true;
+      else
+        rank = 2u * rank + 64u;  // an unlucky sample: the k-th largest lies below the floor
 #pragma unroll
       for (int g = 0; g < VPT / 4; ++g) load_group(0, g);
       __syncthreads();
       if (tid == 0) L.n_cand = 0;  // (added to again behind the barriers of the next level)
     }
     if constexpr (!kFits) {
-      if (C > (uint32_t)CAP) {
+      if (__builtin_expect(above && C < (uint32_t)k, 0)) {
+        // The list holds what is above the ties, and the ties make up the rest: the first of them by position.
+        const float tie_f = key_to_float(tie);
+        for (int vec0 = 0; vec0 < nvec; vec0 += 4 * NT) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) v[j] = rv.load(tid, vec0 + j * NT);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const int at = 4 * (vec0 + j * NT + tid) - shift;
+            uint32_t four = 0;
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+              four |= RowVectors<T>::element(v[j], c) == tie_f && (uint32_t)(at + c) < (uint32_t)len ? 1u << c : 0u;
+            if (four) {
+              const int word = at < 0 ? 0 : at >> 5, bit = at & 31;
+              if (at < 0)
+                atomicOr(&L.bits[0], four >> 1);
+              else
+                atomicOr(&L.bits[word], four << bit);
+              if (bit > 28 && at >= 0 && (four >> (32 - bit))) atomicOr(&L.bits[word + 1], four >> (32 - bit));
+            }
+          }
+        }
+        const uint32_t wanted = (uint32_t)k - C;
+        if (count_words() >= wanted) {
+          for (int w = tid; w < n_words; w += NT) {
+            uint32_t word = L.bits[w];
+            const uint32_t first = L.before[w];
+            if (first + __popc(word) > wanted) {
+              const int keep = first < wanted ? (int)(wanted - first) : 0;
+              while (__popc(word) > keep) word &= 0x7fffffffu >> __builtin_clz(word);
+              L.bits[w] = word;
+            }
+          }
+          __syncthreads();
+          for (int i = tid; i < (int)C; i += NT) atomicOr(&L.bits[L.pos[i] >> 5], 1u << (L.pos[i] & 31));
+          count_words();
+          for (int w = tid; w < n_words; w += NT) {  // the list again, in order
+            uint32_t word = L.bits[w], at = L.before[w];
+            for (; word; word &= word - 1u) L.pos[at++] = (typename Lds::pos_t)(32 * w + __builtin_ctz(word));
+          }
+          __syncthreads();
+          int32_t* out_idx = out_row(p, p.out_idx, row);
+          elem_t* out_val = p.out_values ? out_row(p, reinterpret_cast<elem_t*>(p.out_values), row) : nullptr;
+          const int32_t* table = table_of(p, row);
+          const int32_t* in = p.in_idx ? p.in_idx + (int64_t)row * p.in_idx_stride : nullptr;
+          for (int i = tid; i < k; i += NT) {
+            const int at = (int)L.pos[i];
+            int32_t pay = at;
+            if (in) {
+              pay = in[at];
+            } else if (table) {
+              const int page = p.page_shift >= 0 ? at >> p.page_shift : page_of(p, at);
+              pay = table[page] * p.page_size + (at - page * p.page_size);
+            }
+            out_idx[i] = pay;
+            if (out_val) out_val[i] = vals[at];
+          }
+          return;
+        }
+        C = CAP + 1u;
+      }
+      if (__builtin_expect(C > (uint32_t)CAP, 0)) {
         const int n_runs = (len + kTopkThreads - 1) / kTopkThreads;
         for (int j_lo = 0; j_lo < n_runs; j_lo += kSliceMaxRuns) {
           __syncthreads();
@@ -366,7 +491,7 @@ __global__ __launch_bounds__(NT) void topk_filter_kernel(const TopkParams p) {
       x[u] = u * NT + tid < n ? KeyTraits<F32>::key(f) - kbase : kNoElement;
     });
     krem = krem0 = C - (uint32_t)k + 1u;
-    narrow(kmax > kbase ? kmax - kbase : 0u, [&](auto f) { each_slot([&](int u) { f(x[u]); }); });
+    narrow(kmax > kbase ? kmax - kbase : 0u, equal, false, [&](auto f) { each_slot([&](int u) { f(x[u]); }); });
   }
   uint32_t below = krem0 - krem;  // smaller than the bin's members
 
@@ -412,29 +537,6 @@ __global__ __launch_bounds__(NT) void topk_filter_kernel(const TopkParams p) {
   const uint32_t r = whole ? (uint32_t)k - below : (uint32_t)k - (C - below - ties);
 
   // ---- 4. places in position order ---------------------------------------------------------------
-  const int wpt = (n_words + NT - 1) / NT;
-  auto count_words = [&]() {  // before[w] = set bits in front of word w
-    __syncthreads();
-    uint32_t local = 0;
-    for (int i = 0; i < wpt; ++i) {
-      const int w = tid * wpt + i;
-      local += w < n_words ? __popc(L.bits[w]) : 0u;
-    }
-    const uint32_t incl = wave_prefix_sum_dpp(local, lane);
-    if (lane == 63) L.wa[wave] = incl;
-    __syncthreads();
-    uint32_t run, total;
-    sums_before<NW>(L.wa, wave, lane, run, total);
-    run += incl - local;
-    for (int i = 0; i < wpt; ++i) {
-      const int w = tid * wpt + i;
-      if (w < n_words) {
-        L.before[w] = (uint16_t)run;
-        run += __popc(L.bits[w]);
-      }
-    }
-    __syncthreads();
-  };
   auto place_of = [&](int32_t at) -> uint32_t {
     return (uint32_t)L.before[at >> 5] + __popc(L.bits[at >> 5] & ((1u << (at & 31)) - 1u));
   };

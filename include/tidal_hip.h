@@ -404,7 +404,8 @@ int td_topk_segments(const void* values, int32_t values_dtype, int64_t values_st
 
 /*
  * Bytes of device scratch for td_topk.  Rows of up to 65536 elements never touch it, nor do rows of
- * up to 262144 whose selection fits the list of the one-pass kernel (k up to about 5800).  Larger
+ * up to 262144 whose selection fits the list of the one-pass kernel (k up to about 4700 at 65536
+ * elements, 4100 at 102400, 3700 at 131072, 2600 at 262144).  Larger
  * selections from a few long rows are shared between workgroups through it (three launches; about
  * 56 KiB per row); without it (NULL), or with many long rows, every workgroup goes through the whole
  * row, read again from L2 in every pass.  The scratch must be
@@ -412,6 +413,13 @@ int td_topk_segments(const void* values, int32_t values_dtype, int64_t values_st
  * Plays the part of the `buf` argument of topk_filtering (tidal/utils/controller.py:164-168).
  */
 int64_t td_topk_workspace_bytes(int32_t rows);
+
+/*
+ * Which route this thread's last top-k took: "one pass" (one workgroup per row), "slices" (every
+ * workgroup of a row goes through the whole row) or "shared rows" (three launches over the scratch).
+ * A diagnostic for tests and benchmarks; the string is static.  No counterpart in the reference.
+ */
+const char* td_last_topk_route(void);
 
 /*
  * Page-level upper bound of the attention logits from the per-page key max / min metadata that

@@ -16,8 +16,8 @@ _scratch = {}
 
 def _shared_scratch(cuda, rows):
     """One scratch tensor for the whole module: zeroed at allocation only, so every cooperative
-    call after the first (rows of more than 65536 elements) relies on the previous call having
-    left it clean."""
+    call after the first (large selections from rows of more than 65536 elements) relies on the previous
+    call having left it clean."""
     from tidaldecode_amd import _kernels
 
     need = _kernels.topk_workspace_bytes(64)
@@ -53,7 +53,7 @@ def _check(values, k, cuda):
     assert np.array_equal(got.numpy(), want_c)
     expect = torch.gather(values, 1, want)  # values travel with their index (NaN == NaN here)
     assert torch.equal(torch.nan_to_num(vals.float(), nan=1e38), torch.nan_to_num(expect.float(), nan=1e38))
-    # with scratch: rows of more than 65536 elements take the three cooperative launches
+    # with scratch: large selections from rows of more than 65536 elements take the three cooperative launches
     got2, vals2 = _gpu_topk(values, k, cuda, scratch=True)
     assert torch.equal(got2, got), "cooperative path differs"
     assert torch.equal(torch.nan_to_num(vals2.float(), nan=1e38), torch.nan_to_num(vals.float(), nan=1e38))
@@ -142,7 +142,7 @@ def test_long_rows_with_crowded_threshold_bins(cuda, dtype):
 
 @pytest.mark.parametrize("n", [5000, 32768, 30000 + 77, 50000])
 def test_score_distributions_that_steer_the_radix_levels(cuda, n):
-    """The one-launch kernel maps scores to d = distance below the row maximum and starts its radix
+    """The one-launch kernels map scores to d = distance below the row maximum and start their radix
     select 64 binades below that maximum.  Rows that leave the usual road: all negative; fewer
     non-negative scores than k (threshold below zero); a threshold 100 binades below the maximum
     (second pass over the rest of the range); +0 / -0 ties at the threshold; denormals; a threshold
@@ -271,8 +271,8 @@ def test_payloads(cuda):
 
 
 def test_page_table_per_row_group(cuda):
-    """A batch of sequences in one call: rows of group g read page table g.  Short rows (one
-    workgroup per row) and long rows (several workgroups per row) against the oracle."""
+    """A batch of sequences in one call: rows of group g read page table g.  Rows of the one-pass kernel
+    (tests/test_gpu_topk_routes.py has the others) against the oracle."""
     from oracle import tidal_oracle as orc
 
     g = torch.Generator().manual_seed(17)

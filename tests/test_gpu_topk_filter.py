@@ -1,5 +1,6 @@
 """GPU parity of the one-pass top-k (csrc/topk_filter.cuh): rows of up to 262144 scores whose
-selection fits its list.  Everything is bit-exact against the oracle's stable rule."""
+selection fits its list.  Everything is bit-exact against the oracle's stable rule, and every call here takes
+that route."""
 import pytest
 import torch
 
@@ -20,6 +21,7 @@ def _run(cuda, v, k, *, bound=None, in_idx=None, table=None, page=1, lengths=Non
     to = lambda t: None if t is None else t.to(cuda)
     _kernels.topk_filtering(dev, to(in_idx), out_v, out, None, k, page_table=to(table), page_size=page,
                             lengths=to(lengths), upper_bound=to(bound))
+    assert _kernels.last_topk_route() == "one pass"
     torch.cuda.synchronize()
     return out.cpu().long(), None if out_v is None else out_v.cpu()
 
@@ -27,7 +29,8 @@ def _run(cuda, v, k, *, bound=None, in_idx=None, table=None, page=1, lengths=Non
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("n,k", [(1, 1), (3, 2), (255, 17), (1019, 300), (1020, 1020), (1021, 1), (2047, 2000),
                                  (2049, 511), (4099, 64), (8191, 8191), (8192, 700), (8193, 4096), (16383, 5),
-                                 (32771, 2048), (65535, 1024), (65537, 4096), (131073, 3), (262143, 4096)])
+                                 (32771, 2048), (65535, 1024), (65537, 4096), (131073, 3), (200000, 3000),
+                                 (262143, 2048), (262144, 2600)])
 def test_edges_of_the_sizes(cuda, dtype, n, k):
     from oracle import tidal_oracle as orc
 
@@ -63,7 +66,7 @@ def test_payloads_and_lengths(cuda, n, k, page):
     assert torch.equal(got, torch.gather(payload.long(), 1, orc.stable_topk(v, k)))
 
 
-@pytest.mark.parametrize("n,k", [(20000, 2048), (6000, 700), (100001, 4000)])
+@pytest.mark.parametrize("n,k", [(20000, 2048), (6000, 700), (100001, 4000), (262144, 2500)])
 def test_samples_that_mislead(cuda, n, k):
     """The sampled elements all larger than the rest (the first threshold keeps too few), all smaller
     (it keeps everything: more than the list holds), and rows of a few values only."""

@@ -261,8 +261,9 @@ def topk_filtering(estimated_value: torch.Tensor, estimated_indices: Optional[to
     ``p``.  ``buf`` is scratch, as in the reference (there: RAFT's): a zero-initialised uint8 /
     any-dtype device tensor of at least ``topk_workspace_bytes(H)`` bytes through which the
     workgroups of a row of more than 65536 elements share a large selection (``page_budget`` beyond
-    about 5800); other rows never touch it, and without it (smaller or ``None``) every workgroup of
-    such a row goes through the whole row.
+    about 4700 at 65536 elements, 4100 at 102400, 3700 at 131072, 2600 at 262144); other rows never
+    touch it, and without it (smaller or ``None``) every workgroup of such a row goes through the
+    whole row.
     The call leaves ``buf`` zeroed where it must be for the next call.
 
     Deterministic where the reference is not: ties at the threshold go to the lower position
@@ -358,6 +359,11 @@ def topk_filtering(estimated_value: torch.Tensor, estimated_indices: Optional[to
                                pt_ptr, pt_stride, rows_per_table, len_ptr, int(page_size),
                                bound_ptr, out_vals, indices_out.data_ptr(), out_stride, out_group_stride,
                                ws_ptr, ws_bytes if ws_ptr else 0, _stream()))
+
+
+def last_topk_route() -> str:
+    """Route this thread's last top-k took: "one pass", "slices" or "shared rows"."""
+    return lib.td_last_topk_route().decode()
 
 
 def topk_workspace_bytes(rows: int) -> int:

@@ -157,6 +157,7 @@ SIGNATURES = {
          c_int64, c_void_p],
     ),
     "td_topk_workspace_bytes": (c_int64, [c_int32]),
+    "td_last_topk_route": (c_char_p, []),
     "td_gather_probe": (
         c_int32,
         [POINTER(PagedKV), POINTER(IndexList), POINTER(DecodePlan), c_int32, c_int32, c_void_p,

@@ -8,8 +8,8 @@
 //
 // Three routes:
 //   * topk_filter_kernel (topk_filter.cuh), one launch, one workgroup per row, every element touched
-//     once: rows of up to 262144 elements whose selection fits its list (k up to about 5800, any k up
-//     to 8192 elements);
+//     once: rows of up to 262144 elements whose selection fits its list (any k up to 8192 elements, then
+//     k up to about 6600 that falls to 5900 at 16384, 4700 at 65536 and 2600 at 262144);
 //   * topk_slice_kernel, one launch: every workgroup (1024 threads) of a row runs the selection on
 //     the whole row -- up to 64K elements from registers -- and emits its own slice of it.  Larger
 //     selections, and longer rows when there are many of them or no scratch;
@@ -1305,6 +1305,10 @@ __global__ __launch_bounds__(256) void score_reduce_kernel(const float* __restri
 
 using namespace tidal;
 
+static thread_local const char* g_last_route = "none";
+
+extern "C" const char* td_last_topk_route(void) { return g_last_route; }
+
 extern "C" int td_topk_segments(const void* values, int32_t values_dtype, int64_t values_stride,
                                 int32_t rows, int32_t len, int32_t k, const int32_t* in_idx,
                                 int64_t in_idx_stride, const int32_t* page_table,
@@ -1356,6 +1360,7 @@ extern "C" int td_topk_segments(const void* values, int32_t values_dtype, int64_
   else done = launch_topk_filter<BF16>(p, rows, st);
   if (done) {
     TD_HIP_CHECK(hipGetLastError());
+    g_last_route = "one pass";
     return TD_OK;
   }
   // Selections beyond the list.  A few long rows: the three cooperative launches split each row over
@@ -1363,8 +1368,9 @@ extern "C" int td_topk_segments(const void* values, int32_t values_dtype, int64_
   // workgroup of a row goes through the whole row (rows up to 64K elements from registers) and emits
   // its slice.
   const int slices = coop_slices(len, rows);
-  if (len > 64 * kTopkThreads && slices && rows * slices <= 1024 && workspace &&
-      workspace_bytes >= (int64_t)rows * kCoopRowWords * 4) {
+  const bool shared = len > 64 * kTopkThreads && slices && rows * slices <= 1024 && workspace &&
+                      workspace_bytes >= (int64_t)rows * kCoopRowWords * 4;
+  if (shared) {
     uint32_t* ws = reinterpret_cast<uint32_t*>(workspace);
     const dim3 grid((rows + kXcds - 1) / kXcds * slices * kXcds), block(kTopkThreads);
     if (values_dtype == TD_F32) {
@@ -1388,6 +1394,7 @@ extern "C" int td_topk_segments(const void* values, int32_t values_dtype, int64_
     launch_topk_sliced<BF16>(p, rows, st);
   }
   TD_HIP_CHECK(hipGetLastError());
+  g_last_route = shared ? "shared rows" : "slices";
   return TD_OK;
 }
 

@@ -122,6 +122,25 @@ def test_same_bits_as_the_python_path(cuda, monkeypatch, dtype, shape):
 
 
 @pytest.mark.gpu
+def test_regular_calls_are_served_natively(cuda, monkeypatch):
+    """No entry declines the calls it is there for (Python would give the same results, only later)."""
+    calls = {}
+    for shape in _SHAPES:
+        recorder = _Recorder()
+        _use(monkeypatch, recorder)
+        _workload(cuda, torch.bfloat16, *shape)
+        names = [name for name, _ in recorder.served]
+        calls[shape] = {name: names.count(name) for name in _NATIVE}
+    for shape, served in calls.items():
+        # two steps of two layers: full attention through decode_sparse_attn needs its workspace once first
+        assert served["append"] == 6 and served["rope_in_place"] == 3 and served["rope_table"] == 2, (shape, served)
+        assert served["topk"] == 2 and served["estimate"] == 2 and served["gemv"] == 3, (shape, served)
+        assert served["attend"] >= 2 and served["forward"] == 2, (shape, served)
+        assert served["score_reduce"] == (2 if shape[-1] == "group_sum" else 0), (shape, served)
+    assert max(served["prefill"] for served in calls.values()) == 2, calls  # prompts whose plan wants no scratch
+
+
+@pytest.mark.gpu
 def test_launches_leave_the_interpreters_lock(cuda, monkeypatch):
     """Every call that was served, once more with PyGILState_Check (1 where its thread holds the lock, which
     reads as an error status) in place of the functions that launch."""

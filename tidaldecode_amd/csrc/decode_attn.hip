@@ -220,7 +220,8 @@ extern "C" int td_decode_make_plan(int32_t batch, int32_t num_qo_heads, int32_t 
   // closer together; from 1024 tokens down the merges take back what that gives.  32 heads x 128,
   // fp16, logits out, chunks of 4096 | 1024 tokens (or as near as the built-in scratch allows): 8
   // sequences of 8192 .. 65536 1017 | 998 us, of 500 .. 8000 136 | 118; 16 heads, 8 of 2000 .. 30000
-  // 254 | 240; 40 heads, 3 of 2000 .. 40000 210 | 196.
+  // 254 | 240; 40 heads, 3 of 2000 .. 40000 210 | 196.  Equal lengths, which need no balance, lose a
+  // little: 8 of 8192 180.7 | 183.3.
   if (batch > 1 && qpg == 1 && chunk > 1024) {
     const int64_t per_split = (int64_t)batch * n_hrows * (head_dim + 2) * 4;
     int64_t fit = ((int64_t)TD_STATIC_SCRATCH_BYTES - kTicketBytes - 512) / per_split;  // splits it holds

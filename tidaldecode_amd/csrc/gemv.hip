@@ -249,15 +249,18 @@ static void launch_gemv_shape(const GemvParams& p, int mode, hipStream_t st) {
 }
 
 // One row per wavefront: waves that end one after the other keep the memory busier than fewer with more rows
-// each, whose last trips end together.  Long rows and row pairs take eight chunks per row and trip; short
-// matrices keep two rows, which halves what their few workgroups stage.  One MI355X, cold weights, launches of
-// a graph, us, before (four rows of four chunks; two of eight for the long rows) -> now: 12288 x 4096 17.7 ->
-// 16.9 (6.0 TB/s), 32000 x 4096 42.5 -> 40.6, 128256 x 4096 155.8 -> 151.4 (6.9 TB/s), 4096 x 11008 17.8 ->
-// 17.5, pairs 22016 x 4096 31.4 -> 29.2, 28672 x 4096 38.8 -> 37.0; 4096 x 4096 7.4 with either.
+// each, whose last trips end together.  Long rows take eight chunks per trip, row pairs one pair of four chunks
+// (a trip of eight is 4096 columns: shorter rows load what they do not use); short matrices keep two rows, which
+// halves what their few workgroups stage.  One MI355X, cold weights, launches of a graph, us, before (four rows
+// of four chunks; two of eight for the long rows) -> now: 12288 x 4096 18.3 -> 17.0 (5.9 TB/s), 32000 x 4096 42.5
+// -> 40.5, 128256 x 4096 157 -> 151 (6.9 TB/s), 4096 x 11008 18.0 -> 17.8, 16384 x 16384 106 -> 83, 512 x 16384
+// 8.5 -> 6.6, 3584 x 18944 24.9 -> 25.5 (which loses); pairs 22016 x 4096 31.6 -> 29.6 (eight chunks 30.2), 28672 x
+// 4096 37.2 -> 36.5 (37.3), 22016 x 2048 16.3 -> 15.6 (20.4), 5632 x 2048 5.8 -> 5.8 (7.0), 22016 x 5120 38.6 -> 36.9
+// (40.9), 57344 x 8192 145 -> 141 (140); 4096 x 4096 7.4 with either.
 template <typename T>
 static void launch_gemv(const GemvParams& p, int mode, bool pair, hipStream_t st) {
   if (pair)
-    launch_gemv_shape<T, true, 2, 8>(p, mode, st);
+    launch_gemv_shape<T, true, 2, 4>(p, mode, st);
   else if (p.cols > 8192)
     launch_gemv_shape<T, false, 1, 8>(p, mode, st);
   else if (p.rows >= 8192)

@@ -27,16 +27,16 @@ def _run(cuda, v, k, route, *, scratch=False, segment=None, vals=False, **kw):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("n", [8200, 16000, 24000, 24576, 32768, 40960, 48000, 56000, 57344, 65536, 65537, 100003])
+@pytest.mark.parametrize("n", [3001, 4096, 8192, 8200, 16000, 24000, 24576, 32768, 40960, 48000, 56000, 57344, 65536, 65537, 100003])
 def test_every_register_size_of_the_slices(cuda, dtype, n):
-    """16 to 64 elements a thread, and rows that are read again in every pass."""
+    """8 to 64 elements a thread, and rows that are read again in every pass."""
     from oracle import tidal_oracle as orc
 
     g = torch.Generator().manual_seed(n)
     v = torch.randn((3, n), generator=g).to(dtype)
     v[2] = torch.randint(0, 7, (n,), generator=g).to(dtype)
     lse = torch.logsumexp(v.float(), 1)
-    for k in (max(6700, n // 2), n - 1):
+    for k in (max(n // 2, min(6700, n - 2)), n - 1):
         want = orc.stable_topk(v.float(), k)
         for bound in (None, lse):
             got, vals = _run(cuda, v, k, "slices", vals=True, upper_bound=bound)
@@ -74,3 +74,20 @@ def test_payloads_tables_lengths_and_segments(cuda, route, n, k, page, scratch):
         for got in (plain[r], row):
             assert torch.equal(got[: len(slots)], slots) and (got[len(slots):] == -1).all(), r
     assert (apart[:, groups * segment:] == -1).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows,n,most32,most16", [(3, 2048, 2048, 2048), (3, 2049, 1300, 600), (256, 8192, 1300, 600),
+                                                  (64, 8193, 1600, 0), (64, 32768, 3640, 1365), (65, 16384, 3276, 1024),
+                                                  (256, 16384, 4096, 3036), (2, 65536, 4748, 4096), (2, 65537, 4748, 4748)])
+def test_where_the_one_pass_ends(cuda, dtype, rows, n, most32, most16):
+    """The largest selection that one workgroup a row takes, and the next, which goes to the slices."""
+    from oracle import tidal_oracle as orc
+
+    g = torch.Generator().manual_seed(n + rows)
+    v = torch.randn((1, n), generator=g).to(dtype)
+    most = most32 if dtype == torch.float32 else most16
+    for k, route in ((most, "one pass"), (most + 1, "slices")):
+        if 1 <= k <= n:
+            got, _ = _run(cuda, v.repeat(rows, 1), k, route)
+            assert torch.equal(got, orc.stable_topk(v.float(), k).expand(rows, -1)), k

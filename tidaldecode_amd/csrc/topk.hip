@@ -8,8 +8,9 @@
 //
 // Three routes:
 //   * topk_filter_kernel (topk_filter.cuh), one launch, one workgroup per row, every element touched
-//     once: rows of up to 262144 elements whose selection fits its list (any k up to 8192 elements, then
-//     k up to about 6600 that falls to 5900 at 16384, 4700 at 65536 and 2600 at 262144);
+//     once: rows of up to 2048 elements, of up to 65536 where the selection is small enough for one
+//     workgroup to be faster (filter_pays: 32 rows of fp32 about 1300 .. 1600 and len / 9), of up to
+//     262144 where it fits the list (k up to about 4700 at 65536, 2600 at 262144);
 //   * topk_slice_kernel, one launch: every workgroup (1024 threads) of a row runs the selection on
 //     the whole row -- up to 64K elements from registers -- and emits its own slice of it.  Larger
 //     selections, and longer rows when there are many of them or no scratch;
@@ -1211,7 +1212,9 @@ static void launch_topk_sliced(const TopkParams& p, int rows, hipStream_t st) {
   int n_slices, rps;
   slice_shape(p.len, rows, n_slices, rps);
   const dim3 grid((rows + kXcds - 1) / kXcds * n_slices * kXcds), block(kTopkThreads);
-  if (p.len <= 16 * kTopkThreads)
+  if (p.len <= 8 * kTopkThreads)
+    hipLaunchKernelGGL((topk_slice_kernel<T, 8>), grid, block, 0, st, p, n_slices, rps, rows);
+  else if (p.len <= 16 * kTopkThreads)
     hipLaunchKernelGGL((topk_slice_kernel<T, 16>), grid, block, 0, st, p, n_slices, rps, rows);
   else if (p.len <= 24 * kTopkThreads)
     hipLaunchKernelGGL((topk_slice_kernel<T, 24>), grid, block, 0, st, p, n_slices, rps, rows);

@@ -583,12 +583,36 @@ static bool filter_fits(int len, int k, int threads) {
   return (want + 5.0 * __builtin_sqrt(want)) * len / m <= 0.95 * kFilterCap;
 }
 
+// Whether a row's only workgroup here is faster than the slices, whose workgroups (up to eight a row, 256 in all)
+// each go through the whole row: what grows with k is done by one workgroup here, and 16-bit scores nearly always
+// tie at the threshold, which costs another bitmap (3 us).  One MI355X, rows of N(0, 1) with a bound and a page
+// table, slices | one pass, us: fp32, 32 rows 8192 -> 1024 9.3 | 8.8, -> 2048 9.0 | 10.7, 12288 -> 1536 10.7 | 10.6,
+// -> 4096 10.2 | 14.3, 16384 -> 2048 10.5 | 10.7, 32768 -> 3072 14.9 | 13.9, 65536 -> 4096 27 | 18; 128 rows 16384
+// -> 2048 1.09 times, -> 3072 0.97 times as fast; 256 rows 12288 -> 3072 1.11, -> 4096 0.93; bf16, 32 rows 8192 ->
+// 512 1.00, 16384 -> 512 0.97, 24576 -> 512 0.99, 32768 -> 1536 1.01, 49152 -> 3072 0.98; 256 rows 12288 -> 2048 1.01.
+// Rows of up to 2048 elements gain at any k (bf16 1500 -> 1024, a tie and as many survivors as there can be, 0.96),
+// rows of more than 65536, which the slices read again in every pass, too.
+static bool filter_pays(int len, int k, int rows, bool half) {
+  if (len <= 2048 || len > 65536) return true;
+  int most;
+  if (len <= 8192)
+    most = half ? 600 : 1300;
+  else if (rows <= 64)
+    most = half ? (len - 16384) / 12 : (len < 14400 ? 1600 : len / 9);
+  else if (rows < 256)
+    most = half ? (len - 8192) / 8 : (len < 10000 ? 2000 : len / 5);
+  else
+    most = half ? 1500 + (len - 10240) / 4 : (len < 13200 ? 3300 : len / 4);
+  return k <= most;
+}
+
 // True: launched.  Threads by row length: the fewer, the cheaper the barriers and scans that make up
 // most of a short row's time; 1024 are needed where the row's elements are (32 x 8192 -> 512: 7.1 us
 // with 512, 9.3 at 10000 with 1024).  The limits of 65536 and 262144 are the LDS of the bitmap.
 template <typename T>
 static bool launch_topk_filter(const TopkParams& p, int rows, hipStream_t st) {
   const dim3 grid(rows);
+  if (!filter_pays(p.len, p.k, rows, !std::is_same<T, F32>::value)) return false;
   if (p.len <= 1024 - 4)
     hipLaunchKernelGGL((topk_filter_kernel<T, 256, 4, 1024, 1024>), grid, dim3(256), 0, st, p);
   else if (p.len <= 8192)

@@ -18,12 +18,42 @@ def _lens(kind, batch, hi):
     return torch.randint(1, hi + 1, (batch,), generator=g).tolist()
 
 
+@pytest.fixture(params=["planned", "balanced"])
+def launch(request, monkeypatch):
+    """As the planner decides, and balanced also where it takes even chunks (up to 64 sequences)."""
+    from tidaldecode_amd import _kernels
+
+    if request.param == "planned":
+        return
+    wrapper = _kernels.BatchDecodeWithPagedKVCachePyTorchWrapper
+    planned = wrapper._plan
+
+    def plan_of(self, batch, rows, items, short_list=True):
+        plan = planned(self, batch, rows, items, short_list)
+        heads, kv, d = self._geom[:3]
+        group = next(g for g in (2, 4, 8) if heads // kv <= g or g == 8)
+        hrows = kv * -(-(heads // kv) // group)
+        slots = -(-batch // max(1, 256 // hrows)) * max(1, 256 // hrows)
+        need = max(plan.max_splits, -(-min(slots, 64 * batch) // batch))
+        part = batch * hrows * group * need
+        plan.balanced, plan.max_splits = 1, need
+        plan.workspace_bytes = (1 << 20) + sum(-(-part * x // 256) * 256 for x in (d * 4, 8))
+        return plan
+
+    class Declines:
+        def __getattr__(self, name):
+            return lambda *a: False
+
+    monkeypatch.setattr(wrapper, "_plan", plan_of)
+    monkeypatch.setattr(_kernels, "host_calls", Declines())
+
+
 @pytest.mark.parametrize("heads,kv,d,page,dtype", [(32, 8, 128, 16, torch.bfloat16), (28, 4, 128, 16, torch.float16),
                                                    (6, 2, 64, 1, torch.float16), (16, 4, 256, 7, torch.bfloat16),
                                                    (40, 2, 128, 32, torch.bfloat16)])
 @pytest.mark.parametrize("kind,batch,hi", [("mixed", 2, 700), ("mixed", 16, 3000), ("one long", 9, 5000),
                                            ("equal", 5, 129), ("mixed", 64, 300), ("mixed", 65, 300)])
-def test_batches(cuda, heads, kv, d, page, dtype, kind, batch, hi):
+def test_batches(cuda, launch, heads, kv, d, page, dtype, kind, batch, hi):
     from tidaldecode_amd.utils import BatchInferenceController
 
     lens = _lens(kind, batch, hi)
@@ -50,7 +80,7 @@ def test_batches(cuda, heads, kv, d, page, dtype, kind, batch, hi):
 
 
 @pytest.mark.parametrize("batch,hi", [(3, 900), (16, 2000)])
-def test_fused_step_of_a_batch(cuda, batch, hi):
+def test_fused_step_of_a_batch(cuda, launch, batch, hi):
     """With the new tokens folded into the launch: the same outputs, logits and cache as the separate calls."""
     from tidaldecode_amd.utils import BatchInferenceController
 

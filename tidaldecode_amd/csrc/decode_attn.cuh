@@ -910,16 +910,20 @@ __global__ __launch_bounds__(NW * 64) void decode_attn_balanced_kernel(const Dec
   const int mean = (sum + p.slots - 1) / p.slots, fewest = (most + kMergedPieces - 1) / kMergedPieces;
   const int least = mean > fewest ? mean : fewest;  // <= most: slots >= batch
   const int piece = least + (most - least) * lane / 63;
-  const float inv = 1.f / (float)piece;
-  int pieces = 0;
-  for (int b = 0; b < p.batch; ++b) {
-    const int n = __builtin_amdgcn_readlane(tiles, b);
-    int q = (int)((float)n * inv);  // within one of the quotient
-    q += (q + 1) * piece <= n ? 1 : 0;
-    q -= q * piece > n ? 1 : 0;
-    pieces += q + (q * piece < n ? 1 : 0);
+  // pieces of a sequence: its tiles over the piece, rounded up.  In floats, exact here (fewer than 2^24 tiles):
+  // the quotient is taken a little large, so that its whole part is the floor or one more, and the remainder
+  // says whether another piece follows
+  const float length = (float)piece, inv = (1.f + 0x1p-21f) / length, tiles_f = (float)tiles;
+  float pieces = 0.f;
+  for (int b = 0; b < p.batch; b += 4) {  // (lanes past the last sequence hold none)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float n = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, tiles_f), b + i));
+      const float q = __builtin_truncf(n * inv);
+      pieces += q + (fmaf(-q, length, n) > 0.f ? 1.f : 0.f);
+    }
   }
-  const uint64_t fits = __ballot(pieces <= p.slots);
+  const uint64_t fits = __ballot(pieces <= (float)p.slots);
   const int chosen = __builtin_amdgcn_readlane(piece, __builtin_ctzll(fits | (1ull << 63)));
   const int n_splits = lane < p.batch ? (tiles + chosen - 1) / chosen : 0;
   const int upto = (int)wave_prefix_sum_dpp((uint32_t)n_splits, lane);  // pieces of the sequences up to this lane's

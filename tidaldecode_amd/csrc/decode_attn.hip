@@ -41,6 +41,31 @@ static int balanced_slots(int n_hrows, int batch) {
   return (int)(slots < merged ? slots : merged);
 }
 
+// Whether the balanced launch is worth its search and the merges it adds, from the longest sequence that the plan
+// is for; chunk: that of the even plan.  Its workgroups of one tile (`tile` tokens) take `per_tile` us; the lengths
+// and the search 1 - 2 us; where the even plan cuts no sequence, starting to merge at all 3 - 6 us, and partials of
+// eight heads queue up at the memory.  It pays where equal lengths would gain by more than that, and where the
+// even plan's workgroups last so long that their differences are worth more than the search (equal lengths then
+// lose 1 - 5 %).  One MI355X, bf16, logits out, even | balanced (with a search of 0.06 us a sequence, now 0.02),
+// us: 8/1 heads x 128, 2 x 400 12.4 | 12.7, 2 x 800 18.6 | 13.4, 24 x 800 20.8 | 23.6, 24 x 1600 35.0 | 26.3; 28/4
+// heads, 8 x 800 21.9 | 25.8, 24 x 1600 41.3 | 37.7; 32/8 heads, 8 x 400 9.9 | 10.8, 8 x 800 16.3 | 13.0, 24 of 1 ..
+// 1600 29.0 | 27.3 and 24 x 1600 31.5 | 33.1, 24 of 1 .. 4000 62.9 | 51.4, 64 x 800 (as many sequences as slots: none
+// is cut) 42.9 | 50.2; 32/8 heads x 64, 8 x 400 10.6 | 12.2, 8 x 800 13.8 | 12.8; 16/4 heads x 256, 8 x 100 10.2 |
+// 12.0, 8 x 200 13.7 | 12.6.
+static bool balancing_pays(int head_dim, int qpg, int n_hrows, int batch, int64_t max_items, int tile, int64_t chunk,
+                           int slots) {
+  const int64_t tiles = ceil_div64(max_items, tile), even = ceil_div64(max_items, chunk);
+  int64_t piece = ceil_div64(tiles * batch, slots);
+  if (piece < ceil_div64(tiles, kMergedPieces)) piece = ceil_div64(tiles, kMergedPieces);
+  const int64_t longest = tiles < chunk / tile ? tiles : chunk / tile;
+  if (slots <= batch || tiles < 1 || piece > longest) return false;
+  const double per_tile = head_dim == 256 ? 2.35 : (head_dim == 64 ? 1.35 : (qpg == 8 ? 1.75 : 1.25));
+  const double merge = even > 1 ? 1.5 : (head_dim == 256 ? 6.0 : (head_dim == 64 ? 3.0 : (qpg == 8 ? 5.4 : 4.8)));
+  const double more = (double)n_hrows * batch * (ceil_div64(tiles, piece) - even);
+  const double cost = merge + (qpg == 8 ? more * head_dim * (0.036 / 128) : 0.0);
+  return (double)(longest - piece) * per_tile > cost || (double)longest * per_tile >= (even > 1 ? 8.0 : 20.0);
+}
+
 static bool is_pow2(int64_t x) { return x > 0 && (x & (x - 1)) == 0; }
 
 }  // namespace tidal
@@ -263,7 +288,8 @@ extern "C" int td_decode_make_plan(int32_t batch, int32_t num_qo_heads, int32_t 
   if (max_splits < 1) max_splits = 1;
   // room for the partials of a balanced launch (one per slot and head slot), unless that alone would take
   // the plan beyond the built-in scratch
-  plan->balanced = batch > 1 && batch <= kBalancedMaxBatch && qpg > 1 && plan->chunk_tokens == 0;
+  plan->balanced = batch > 1 && batch <= kBalancedMaxBatch && qpg > 1 && plan->chunk_tokens == 0 &&
+                   balancing_pays(head_dim, qpg, n_hrows, batch, max_items, tile, chunk, balanced_slots(n_hrows, batch));
   if (plan->balanced) {
     const int64_t wanted = ceil_div64(balanced_slots(n_hrows, batch), batch);
     const int64_t bytes = kTicketBytes + (int64_t)batch * n_hrows * qpg * wanted * (head_dim + 2) * 4 + 512;

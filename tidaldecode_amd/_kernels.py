@@ -138,11 +138,13 @@ def _cut_columns(m: int, n: int, k: int) -> int:
     """How many of the last columns of a product [m, k] x [n, k]^T are multiplied by a kernel of their own: a strip
     of 256 where the library's tiles of 256 x 256 fill whole rounds of the 256 compute units and at most one strip's
     tiles are left over, which would cost a round.  Measured on one MI355X over 2 to 32 rows of tiles, 16 to 160
-    strips and inner dimensions of 2048 to 8192: 0.99 to 1.8 times as fast up to 16 rows of tiles, 0.94 to 1.25
-    above; columns that are whole in 768 stay one product (the library then has narrower tiles: 0.74 to 1.8)."""
+    strips and inner dimensions of 2048 to 8192: 0.94 (2900 x 5632 of 2048) to 2.1 times as fast up to 16 rows of
+    tiles, 0.94 to 1.25 above; columns that are whole in 768 stay one product (the library then has narrower tiles:
+    0.74 to 1.8), and so do 577 to 640 rows, which it takes in two tiles of 320 (0.95 to 0.98)."""
     rows, strips = -(-m // 256), n // 256
     tiles = rows * strips
-    if n % 256 or n % 768 == 0 or k % 64 or k > 1 << 24 or rows > 16 or tiles <= 256 or not 0 < tiles % 256 <= rows:
+    if n % 256 or n % 768 == 0 or k < 64 or k % 64 or k > 1 << 24 or rows > 16 or tiles <= 256 \
+            or not 0 < tiles % 256 <= rows or 576 < m <= 640:
         return 0
     return 256
 

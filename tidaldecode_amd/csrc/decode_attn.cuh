@@ -886,8 +886,9 @@ __global__ __launch_bounds__(NW * 64) void decode_attn_kernel(const DecodeParams
 // chip idle.  One MI355X, bf16, logits out, even chunks -> dealt (us): 16 sequences of 500 .. 8192 tokens,
 // 32/8 heads x 128, 77 -> 69.7 (4.7 TB/s); 8 of 8000 .. 60000, 295 -> 261; 4 of 2000, 36.7 -> 15.8; 12 of
 // 400 .. 9000, 28/4 heads, 59.7 -> 51; few head rows: 8/1 heads, 16 of 2000 .. 32768, 55 -> 47, 40 of 300 .. 4000,
-// 4/1 heads, 26.3 -> 18.8, 16/2 heads, 8 of 8000 .. 65536, 99 -> 87.  The lengths and the search cost 1.5 - 2 us,
-// which is what equal lengths lose (16 x 8192: 98.9 -> 100.7; 8/1 heads, 16 x 32768: 69.1 -> 71.1).  Runs of equal length laid over the ends of the sequences balance better
+// 4/1 heads, 26.1 -> 17.1, 16/2 heads, 8 of 8000 .. 65536, 98 -> 88.  The lengths and the search cost 1 us and more
+// with many sequences, which is what equal lengths lose (16 x 8192: 95.1 -> 96.2; 8/1 heads, 16 x 32768: 69.7 ->
+// 71.0); balancing_pays keeps short ones away.  Runs of equal length laid over the ends of the sequences balance better
 // still but pay the start and the merge of every further sequence, 5 us: 72 for the first batch, 110 for
 // 16 x 8192.
 constexpr int kBalancedMaxBatch = 64;  // one lane per sequence

@@ -299,19 +299,38 @@ __device__ __forceinline__ void attend_share(const DecodeParams& p, const int hr
   // (DRAM row locality of a streaming read) instead of as n_splits distant streams.
   const int c1 = s.n_items;
 
-  // query: QPG heads x 8 elements per lane, kept packed in the KV dtype
-  uint32_t qp[QPG][4];
+  // MMA: shared rows (QPG > 1) of head_dim 64 and 128, weighted values on the matrix cores.
+  constexpr bool MMA = QPG > 1 && LPR <= 16;
+  static_assert(!MMA || U == 4, "shared-row tiles: four rows per lane group");
+  // The scores: rows of 16 lanes with 2 or 4 heads stay on dot products (see `reduce`).
+  constexpr bool MMA_SCORES = MMA && (QPG == 8 || LPR == 8);
+  constexpr int NS = MMA ? D / 32 : 1;     // matrix instructions of a score
+  constexpr int NB = MMA ? TILE / 16 : 1;  // blocks of 16 tokens in a tile
+  const int g4 = lane >> 4, c16 = lane & 15;
+
+  // query, packed in the KV dtype.  MMA_SCORES: column c16 of the operand is head c16 % QPG, elements
+  // [32 s + 8 g4, +8); otherwise QPG heads x 8 elements per lane.
+  uint32_t qp[MMA_SCORES ? 1 : QPG][4];
+  u32x4 qm[NS];
   {
-    const u32x4* qptr =
-        reinterpret_cast<const u32x4*>(p.q) + ((int64_t)b * p.num_qo_heads + rq0) * LPR + li;
+    const u32x4* qptr = reinterpret_cast<const u32x4*>(p.q) + ((int64_t)b * p.num_qo_heads + rq0) * LPR;
+    if constexpr (MMA_SCORES) {
+      const int j = c16 % QPG;
 #pragma unroll
-    for (int j = 0; j < QPG; ++j) {
-      const u32x4 v = qptr[(j < gsz ? j : gsz - 1) * LPR];  // unconditional load, clamped row
-      const bool real = j < gsz;                            // padding heads score with q = 0
-      qp[j][0] = real ? v.x : 0u;
-      qp[j][1] = real ? v.y : 0u;
-      qp[j][2] = real ? v.z : 0u;
-      qp[j][3] = real ? v.w : 0u;
+      for (int x = 0; x < NS; ++x) {
+        const u32x4 v = qptr[(j < gsz ? j : gsz - 1) * LPR + 4 * x + g4];  // unconditional load, clamped row
+        qm[x] = j < gsz ? v : u32x4{0u, 0u, 0u, 0u};                       // padding heads score with q = 0
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < QPG; ++j) {
+        const u32x4 v = qptr[(j < gsz ? j : gsz - 1) * LPR + li];
+        const bool real = j < gsz;
+        qp[j][0] = real ? v.x : 0u;
+        qp[j][1] = real ? v.y : 0u;
+        qp[j][2] = real ? v.z : 0u;
+        qp[j][3] = real ? v.w : 0u;
+      }
     }
   }
 
@@ -367,8 +386,26 @@ __device__ __forceinline__ void attend_share(const DecodeParams& p, const int hr
   // through the main loop and costs more registers than it saves instructions.)
   auto finish_fresh = [&]() {
     if constexpr (FRESH) {
+      if constexpr (MMA_SCORES) {
+        // element d of the operand piece s has its partner, d +- D/2, at the same place of piece s +- NS/2
+        const float* cs = p.fresh_cos + (int64_t)b * (D / 2) + 8 * g4;
+        const float* sn = p.fresh_sin + (int64_t)b * (D / 2) + 8 * g4;
 #pragma unroll
-      for (int j = 0; j < QPG; ++j) rotate(qp[j]);
+        for (int x = 0; x < NS / 2; ++x)
+#pragma unroll
+          for (int w = 0; w < 4; ++w) {
+            const f32x2 c2 = *reinterpret_cast<const f32x2*>(cs + 32 * x + 2 * w);
+            const f32x2 s2 = *reinterpret_cast<const f32x2*>(sn + 32 * x + 2 * w);
+            float a0, a1, b0, b1;
+            unpack2<T>(qm[x][w], a0, a1);
+            unpack2<T>(qm[x + NS / 2][w], b0, b1);
+            qm[x][w] = pack2<T>(a0 * c2.x + b0 * -s2.x, a1 * c2.y + b1 * -s2.y);
+            qm[x + NS / 2][w] = pack2<T>(b0 * c2.x + a0 * s2.x, b1 * c2.y + a1 * s2.y);
+          }
+      } else {
+#pragma unroll
+        for (int j = 0; j < QPG; ++j) rotate(qp[j]);
+      }
       rotate(knew);
       const bool writer_row = rq0 == kv_head * p.q_per_kv;  // the KV head's first head row
       if (split == 0 && wave == 0 && g == 0 && writer_row) {
@@ -383,22 +420,19 @@ __device__ __forceinline__ void attend_share(const DecodeParams& p, const int hr
     }
   };
 
-  // Shared-row path (QPG > 1): after the reduce-scatter of q.k a lane works on ONE query head,
-  // hsel = li % QPG; the running maximum mh of a head is kept equal in all lanes of the wave, lh
-  // is the lane group's share of the denominator, and p.V runs on the matrix cores with the 16
-  // tokens of a tile as the inner dimension: accm[dd][i] = o[head (4g + i) % QPG][li * 8 + dd].
-  // MMA: that path, for head_dim 128 (rows of 16 lanes, tiles of 16 tokens: 4 rows x 4 groups).
-  // Other head sizes score their QPG query heads per loaded KV row on the vector ALU throughout.
-  constexpr bool MMA = QPG > 1 && LPR == 16;
-  static_assert(!MMA || (U == 4 && TPI == 4), "shared-row tiles are 16 tokens: 4 rows x 4 groups");
+  // Shared-row state: a lane works on ONE query head, c16 % QPG; the running maximum mh of a head is kept
+  // equal in all lanes of the wave, lh is the lane's share of the denominator, and accm[dd][i] is
+  // o[head (4 g4 + i) % QPG] of dimension dd of the lane (head_dim 128: li * 8 + dd; 64: see `weigh` below).
+  constexpr int NACC = MMA ? D / 16 : 1;
   float mh = kNegBig, lh = 0.f;
-  f32x4 accm[8];
+  f32x4 accm[NACC];
 #pragma unroll
-  for (int d = 0; d < 8; ++d) accm[d] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int d = 0; d < NACC; ++d) accm[d] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  float m[QPG], l[QPG], acc[QPG][8];
+  constexpr int NV = MMA ? 1 : QPG;  // heads on the vector ALU
+  float m[NV], l[NV], acc[NV][8];
 #pragma unroll
-  for (int j = 0; j < QPG; ++j) {
+  for (int j = 0; j < NV; ++j) {
     m[j] = kNegBig;
     l[j] = 0.f;
 #pragma unroll
@@ -508,6 +542,10 @@ __device__ __forceinline__ void attend_share(const DecodeParams& p, const int hr
   constexpr int EMIT_TILES = EMIT ? EMIT_FLOATS / (QPG * TILE) : 1;
   static_assert(EMIT_TILES >= 1, "logit strip too small for one tile");
   __shared__ float emit_buf[EMIT ? NW * EMIT_FLOATS : 1];
+  // Wave states at the end of the launch; before that, in the shared-row kernels, the wave's key tile on its
+  // way to operand layout (a wave only ever uses its own part before the barrier).
+  constexpr int STATE_F = QPG * D > NB * 16 * D / 2 || !MMA ? QPG * D : NB * 16 * D / 2;  // floats per wave
+  __shared__ __attribute__((aligned(16))) float sm_state[NW][STATE_F];
   int emit_n = 0;       // tiles waiting in the strip
   int emit_first = 0;   // first token of the oldest waiting tile
   const int STEP = n_splits * NW * TILE;  // tokens between two tiles of this wave
@@ -558,65 +596,108 @@ __device__ __forceinline__ void attend_share(const DecodeParams& p, const int hr
       }
     }
     if constexpr (MMA) {
-      float sv[U], xe[U];
+      float xe[NB][4], sv[NB][4];
+      if constexpr (MMA_SCORES) {
+      // ---- S = K Q^T -------------------------------------------------------------------------------
+      // A lane group loads whole rows of K, the matrix operand wants 16 rows side by side: the tile goes
+      // through the wave's own LDS (LDS accesses of one wave complete in order).  Row r of block x is token
+      // TPI (r % 4) + NB (r / 4) + x of the tile, so that a lane's four scores of a block are the tokens whose
+      // values its group holds.  Piece c of row r lies at c ^ r (head_dim 64: c ^ (r / 2)): sixteen rows, read
+      // at one piece, fall on different banks.  Dot products, which this replaces, take 4 QPG instructions per
+      // row and lane and a reduction over the row; eight heads of 128 were bound by them, and so were rows of
+      // eight lanes, whose values were weighted on the vector ALU as well.  bf16, logits out, three layers
+      // (two of them full), us, before -> now: 28/4 heads x 128 at 4140 tokens 81.8 -> 65.6, at 60000 148 ->
+      // 120; x 64 81.3 -> 55.7 and 138 -> 91.6; 32/8 heads x 64 at 16000 75.6 -> 68.2.  Two and four heads of
+      // 128 are bound by the loads and lose 1 - 3 % to the detour; a third tile of loads in flight costs them 9 %
+      // and eight heads 17 % at 60000 tokens.
+      auto place = [](int r, int c) { return r * (D * 2) + 16 * (c ^ (LPR == 16 ? r : (r >> 1) & 7)); };
+      char* const kt = reinterpret_cast<char*>(sm_state[wave]);
+      {
+        const int x = LPR == 16 ? 0 : g & 1, r0 = 4 * (LPR == 16 ? g : g >> 1);
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        float a[QPG];
+        for (int u = 0; u < U; ++u)
+          *reinterpret_cast<u32x4*>(kt + 16 * x * (D * 2) + place(r0 + u, li)) = kb[u];
+      }
+      asm volatile("" ::: "memory");
 #pragma unroll
-        for (int j = 0; j < QPG; ++j) {
-          a[j] = dot2<T>(qp[j][0], kb[u].x, 0.f);
-          a[j] = dot2<T>(qp[j][1], kb[u].y, a[j]);
-          a[j] = dot2<T>(qp[j][2], kb[u].z, a[j]);
-          a[j] = dot2<T>(qp[j][3], kb[u].w, a[j]);
+      for (int x = 0; x < NB; ++x) {
+        f32x4 st = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int y = 0; y < NS; ++y)
+          st = mfma_16x16x32<T>(
+              *reinterpret_cast<const u32x4*>(kt + 16 * x * (D * 2) + place(c16, 4 * y + g4)), qm[y], st);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          xe[x][u] = st[u] * p.scale_log2;
+          sv[x][u] = base + u * TPI + NB * g4 + x < c1 ? xe[x][u] : kNegBig;
         }
-        const float x = reduce_scatter16<QPG>(a, li) * p.scale_log2;  // head li % QPG
-        xe[u] = x;
-        sv[u] = (base + u * TPI + g < c1) ? x : kNegBig;
+      }
+      asm volatile("" ::: "memory");
+      } else {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          float a[QPG];
+#pragma unroll
+          for (int j = 0; j < QPG; ++j) {
+            a[j] = dot2<T>(qp[j][0], kb[u].x, 0.f);
+            a[j] = dot2<T>(qp[j][1], kb[u].y, a[j]);
+            a[j] = dot2<T>(qp[j][2], kb[u].z, a[j]);
+            a[j] = dot2<T>(qp[j][3], kb[u].w, a[j]);
+          }
+          xe[0][u] = reduce_scatter16<QPG>(a, li) * p.scale_log2;  // head li % QPG
+          sv[0][u] = base + u * TPI + g < c1 ? xe[0][u] : kNegBig;
+        }
       }
       if constexpr (EMIT) {
-        // The 16 / QPG lanes of a row that hold the same head hold the same sums, so no value has
-        // to move between lanes: copy c = li / QPG of head li % QPG keeps the logit of the tile's
-        // row c (token base + c TPI + g).  The logits wait in the wave's LDS strip, laid out
-        // [tile][head][token], and leave in batches (see emit_flush).
+        // The 16 / QPG columns that stand for the same head hold the same sums, so no value has to move
+        // between lanes: copy c = c16 / QPG keeps the scores c, c + COPIES, ... of the lane's.  The logits
+        // wait in the wave's LDS strip, laid out [tile][head][token], and leave in batches (see emit_flush).
         constexpr int COPIES = 16 / QPG;
-        const int head = li % QPG, c = li / QPG;
+        const int head = c16 % QPG, c = c16 / QPG;
         float* strip = emit_buf + (wave * EMIT_TILES + emit_n) * (QPG * TILE);
 #pragma unroll
-        for (int u0 = 0; u0 < U; u0 += COPIES) {
-          float e = xe[u0];
+        for (int n0 = 0; n0 < 4 * NB; n0 += COPIES) {
+          float e = xe[n0 / 4][n0 % 4];
 #pragma unroll
           for (int x = 1; x < COPIES; ++x)
-            if (u0 + x < U) e = (c == x) ? xe[u0 + x] : e;
-          if (u0 + c < U) strip[head * TILE + (u0 + c) * TPI + g] = e * kLn2;
+            if (n0 + x < 4 * NB) e = (c == x) ? xe[(n0 + x) / 4][(n0 + x) % 4] : e;
+          const int n = n0 + c;
+          if (n < 4 * NB) strip[head * TILE + n % 4 * TPI + NB * g4 + n / 4] = e * kLn2;
         }
         emit_push(base);
       }
-      float mt = fmaxf(fmaxf(sv[0], sv[1]), fmaxf(sv[2], sv[3]));
+      float mt = kNegBig;
+#pragma unroll
+      for (int x = 0; x < NB; ++x) mt = fmaxf(mt, fmaxf(fmaxf(sv[x][0], sv[x][1]), fmaxf(sv[x][2], sv[x][3])));
       mt = rows_max(mt);  // the tile's maximum over all four lane groups
       const float m_new = fmaxf(mh, mt);
       const float alpha = fast_exp2(mh - m_new);
       mh = m_new;
-      float pr[U];
+      float pr[NB][4], sum = 0.f;
 #pragma unroll
-      for (int u = 0; u < U; ++u)
-        pr[u] = (base + u * TPI + g < c1) ? fast_exp2(sv[u] - m_new) : 0.f;
+      for (int x = 0; x < NB; ++x) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          pr[x][u] = (base + u * TPI + NB * g4 + x < c1) ? fast_exp2(sv[x][u] - m_new) : 0.f;
+        sum += (pr[x][0] + pr[x][1]) + (pr[x][2] + pr[x][3]);
+      }
       // The probabilities enter the matrix product in the KV type; the denominator, which also
       // gives the log-sum-exp, stays in fp32.  bf16 keeps 8 bits of a weight (fp16 11): against an
       // exact denominator that is an error of 2^-9 |v| (2^-12 |v|) in o, which with few selected
       // tokens and |v| of 3-4 reached the tolerance together with the rounding of o itself.  The
       // weights are therefore split into a rounded part and the (rounded) remainder, two products
       // instead of one: twice the bits, and the matrix pipeline has the room.
-      const uint32_t p01 = pack2<T>(pr[0], pr[1]), p23 = pack2<T>(pr[2], pr[3]);
-      constexpr bool kSplitP = true;
-      uint32_t e01 = 0, e23 = 0;
-      if constexpr (kSplitP) {
-        float r0, r1, r2, r3;
-        unpack2<T>(p01, r0, r1);
-        unpack2<T>(p23, r2, r3);
-        e01 = pack2<T>(pr[0] - r0, pr[1] - r1);
-        e23 = pack2<T>(pr[2] - r2, pr[3] - r3);
-      }
-      lh = fmaf(lh, alpha, (pr[0] + pr[1]) + (pr[2] + pr[3]));
+      uint32_t hi[NB][2], rest[NB][2];
+#pragma unroll
+      for (int x = 0; x < NB; ++x)
+#pragma unroll
+        for (int w = 0; w < 2; ++w) {
+          hi[x][w] = pack2<T>(pr[x][2 * w], pr[x][2 * w + 1]);
+          float r0, r1;
+          unpack2<T>(hi[x][w], r0, r1);
+          rest[x][w] = pack2<T>(pr[x][2 * w] - r0, pr[x][2 * w + 1] - r1);
+        }
+      lh = fmaf(lh, alpha, sum);
       // rescale the accumulators: row 4g + i belongs to head (4g + i) % QPG; the factors are
       // wave-uniform per head (lane x < QPG holds head x), so they travel through SGPRs
       float ah[QPG];
@@ -631,12 +712,15 @@ __device__ __forceinline__ void attend_share(const DecodeParams& p, const int hr
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           float f;
-          if constexpr (QPG == 8)
-            f = (g & 1) ? ah[4 + i] : ah[i];
-          else
+          if constexpr (QPG == 8) {
+            float low = ah[i], high = ah[4 + i];
+            asm volatile("" : "+v"(low), "+v"(high));  // a choice of registers (else an array in scratch memory)
+            f = (g4 & 1) ? high : low;
+          } else {
             f = ah[i % QPG];
+          }
 #pragma unroll
-          for (int d = 0; d < 8; ++d) accm[d][i] *= f;
+          for (int d = 0; d < NACC; ++d) accm[d][i] *= f;
         }
       }
       // B operand of dimension dd: the four rows of the tile held by this lane, one 16-bit value
@@ -645,21 +729,47 @@ __device__ __forceinline__ void attend_share(const DecodeParams& p, const int hr
                                  {vb[1].x, vb[1].y, vb[1].z, vb[1].w},
                                  {vb[2].x, vb[2].y, vb[2].z, vb[2].w},
                                  {vb[3].x, vb[3].y, vb[3].z, vb[3].w}};
+      if constexpr (LPR == 16) {
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        const uint32_t lo0 = __builtin_amdgcn_perm(vw[1][c], vw[0][c], 0x05040100u);
-        const uint32_t lo1 = __builtin_amdgcn_perm(vw[3][c], vw[2][c], 0x05040100u);
-        const uint32_t hi0 = __builtin_amdgcn_perm(vw[1][c], vw[0][c], 0x07060302u);
-        const uint32_t hi1 = __builtin_amdgcn_perm(vw[3][c], vw[2][c], 0x07060302u);
-        accm[2 * c] = mfma_16x16x16<T>(p01, p23, lo0, lo1, accm[2 * c]);
-        accm[2 * c + 1] = mfma_16x16x16<T>(p01, p23, hi0, hi1, accm[2 * c + 1]);
-        if constexpr (kSplitP) {
-          accm[2 * c] = mfma_16x16x16<T>(e01, e23, lo0, lo1, accm[2 * c]);
-          accm[2 * c + 1] = mfma_16x16x16<T>(e01, e23, hi0, hi1, accm[2 * c + 1]);
+        for (int c = 0; c < 4; ++c) {
+          const uint32_t lo0 = __builtin_amdgcn_perm(vw[1][c], vw[0][c], 0x05040100u);
+          const uint32_t lo1 = __builtin_amdgcn_perm(vw[3][c], vw[2][c], 0x05040100u);
+          const uint32_t hi0 = __builtin_amdgcn_perm(vw[1][c], vw[0][c], 0x07060302u);
+          const uint32_t hi1 = __builtin_amdgcn_perm(vw[3][c], vw[2][c], 0x07060302u);
+          accm[2 * c] = mfma_16x16x16<T>(hi[0][0], hi[0][1], lo0, lo1, accm[2 * c]);
+          accm[2 * c + 1] = mfma_16x16x16<T>(hi[0][0], hi[0][1], hi0, hi1, accm[2 * c + 1]);
+          accm[2 * c] = mfma_16x16x16<T>(rest[0][0], rest[0][1], lo0, lo1, accm[2 * c]);
+          accm[2 * c + 1] = mfma_16x16x16<T>(rest[0][0], rest[0][1], hi0, hi1, accm[2 * c + 1]);
         }
+      } else {
+        // Rows of eight lanes: the two halves of a 16-lane row hold different tokens, block 0 and block 1.
+        // They exchange half of their dimensions, after which a lane has four dimensions (8 li + 4 (half) +
+        // 0 .. 3) of all eight tokens of its group.
+        uint32_t t[2][U][2];  // block, row, two dimensions each
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+          for (int w = 0; w < 2; ++w) {
+            t[0][u][w] = (uint32_t)__builtin_amdgcn_update_dpp((int)vw[u][w], (int)vw[u][2 + w], 0x128, 0xf, 0xc, false);
+            t[1][u][w] = (uint32_t)__builtin_amdgcn_update_dpp((int)vw[u][2 + w], (int)vw[u][w], 0x128, 0xf, 0x3, false);
+          }
+        const u32x4 pa = {hi[0][0], hi[0][1], hi[NB - 1][0], hi[NB - 1][1]};
+        const u32x4 pb = {rest[0][0], rest[0][1], rest[NB - 1][0], rest[NB - 1][1]};
+#pragma unroll
+        for (int w = 0; w < 2; ++w)
+#pragma unroll
+          for (int half = 0; half < 2; ++half) {
+            const uint32_t sel = half ? 0x07060302u : 0x05040100u;
+            const u32x4 vv = {__builtin_amdgcn_perm(t[0][1][w], t[0][0][w], sel),
+                              __builtin_amdgcn_perm(t[0][3][w], t[0][2][w], sel),
+                              __builtin_amdgcn_perm(t[1][1][w], t[1][0][w], sel),
+                              __builtin_amdgcn_perm(t[1][3][w], t[1][2][w], sel)};
+            accm[2 * w + half] = mfma_16x16x32<T>(pa, vv, accm[2 * w + half]);
+            accm[2 * w + half] = mfma_16x16x32<T>(pb, vv, accm[2 * w + half]);
+          }
       }
       return;
-    }
+    } else {
     float sc[QPG][U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -725,6 +835,7 @@ __device__ __forceinline__ void attend_share(const DecodeParams& p, const int hr
         acc[j][7] = fmaf(pr[u], v7, acc[j][7]);
       }
     }
+    }
   };
 
   int t = (split * NW + wave) * TILE;  // first token of this wave's current tile
@@ -759,7 +870,7 @@ __device__ __forceinline__ void attend_share(const DecodeParams& p, const int hr
     lh += __shfl_xor(lh, 32, 64);
   }
 #pragma unroll
-  for (int j = 0; j < (MMA ? 0 : QPG); ++j) {
+  for (int j = 0; j < (MMA ? 0 : NV); ++j) {
     float mw = m[j];
 #pragma unroll
     for (int off = LPR; off < 64; off <<= 1) mw = fmaxf(mw, __shfl_xor(mw, off, 64));
@@ -779,15 +890,15 @@ __device__ __forceinline__ void attend_share(const DecodeParams& p, const int hr
   // ---- merge the NW wave states of the workgroup through LDS ------------------------------------
   // every wave publishes its QPG states, one barrier, then wave j reduces query head j
   // (QPG <= NW; heads beyond the waves are handled by the waves again in a second trip)
-  __shared__ float sm_o[QPG][NW][8][LPR];
+  auto state = [&](int j, int w, int d, int at) -> float& { return sm_state[w][(j * 8 + d) * LPR + at]; };
   __shared__ float sm_ml[QPG][NW][2];
   __shared__ int sm_ticket;
   if constexpr (MMA) {
 #pragma unroll
     for (int j = 0; j < QPG; ++j) {  // head j is row j of the accumulator tile: group j / 4, i = j % 4
-      if (g == j / 4) {
+      if (g4 == j / 4) {
 #pragma unroll
-        for (int d = 0; d < 8; ++d) sm_o[j][wave][d][li] = accm[d][j % 4];
+        for (int d = 0; d < NACC; ++d) state(j, wave, LPR == 16 ? d : 4 * (c16 >> 3) + d, li) = accm[d][j % 4];
       }
     }
     if (lane < QPG) {
@@ -798,7 +909,7 @@ __device__ __forceinline__ void attend_share(const DecodeParams& p, const int hr
 #pragma unroll
     for (int j = 0; j < QPG; ++j) {
 #pragma unroll
-      for (int d = 0; d < 8; ++d) sm_o[j][wave][d][lane] = acc[j][d];
+      for (int d = 0; d < 8; ++d) state(j, wave, d, lane) = acc[j][d];
       if (lane == 0) {
         sm_ml[j][wave][0] = m[j];
         sm_ml[j][wave][1] = l[j];
@@ -819,7 +930,7 @@ __device__ __forceinline__ void attend_share(const DecodeParams& p, const int hr
         const float f = fast_exp2(sm_ml[j][w][0] - M);
         L = fmaf(sm_ml[j][w][1], f, L);
 #pragma unroll
-        for (int d = 0; d < 8; ++d) r[d] = fmaf(sm_o[j][w][d][lane], f, r[d]);
+        for (int d = 0; d < 8; ++d) r[d] = fmaf(state(j, w, d, lane), f, r[d]);
       }
       const int qh = rq0 + j;
       if (n_splits == 1) {

@@ -1,0 +1,27 @@
+"""Plans of the short-list kernel: they cover the list, keep to 64 splits, no split is empty, and the partials stay
+within the built-in scratch wherever a single split does."""
+import pytest
+
+from tidaldecode_amd._lib import DecodePlan, lib
+
+SCRATCH = 4 << 20
+
+
+@pytest.mark.parametrize("hq,hkv,d", [(32, 32, 128), (32, 8, 128), (28, 4, 128), (40, 40, 64), (28, 4, 64), (8, 1, 64)])
+@pytest.mark.parametrize("batch", [1, 3, 16])
+def test_plans(hq, hkv, d, batch):
+    for rows in {hq, hkv, 1}:
+        for items in [1, 31, 32, 33, 128, 129, 255, 256, 257, 400, 777, 1300, 2048, 2500, 4096, 6001, 12000, 16384]:
+            p = DecodePlan(0, 0, 0, 0, -1, 0, 0, 0)
+            assert lib.td_decode_make_plan(batch, hq, hkv, d, rows, items, p) == 0
+            assert p.sparse_waves in (4, 8) and p.sparse_rows == 8
+            assert p.chunk_tokens % (p.sparse_waves * 4096 // d) == 0
+            assert 1 <= p.max_splits <= 64 and (p.max_splits - 1) * p.chunk_tokens < items <= p.max_splits * p.chunk_tokens
+            single = p.workspace_bytes - (1 << 20)  # what one split takes, within the rounding of the two arrays
+            assert p.workspace_bytes <= SCRATCH or single // p.max_splits + (1 << 20) > SCRATCH or p.max_splits == 1 or \
+                items > 16384 // 2, (rows, items, p.max_splits, p.workspace_bytes)
+            # quotients by the product with 2^32 / chunk, rounded up, which the kernel forms
+            magic = ((1 << 32) + p.chunk_tokens - 1) // p.chunk_tokens
+            for n in (1, items // 2 + 1, items):
+                x = n + p.chunk_tokens - 1
+                assert (x * magic) >> 32 == x // p.chunk_tokens

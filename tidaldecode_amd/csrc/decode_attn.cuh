@@ -64,8 +64,10 @@ struct DecodeParams {
   int32_t last_idx;
   // split
   int32_t chunk_tokens;
-  int32_t chunk_shift;  // log2(chunk_tokens) or -1
-  int32_t qpk_shift;    // log2(q_per_kv) or -1
+  uint32_t chunk_magic;  // 2^32 / chunk_tokens, rounded up: exact for the short-list kernel's up to 2^16 tokens
+  int32_t num_kv_heads;
+  uint32_t kv_magic;    // 2^24 / q_per_kv, rounded up
+  int32_t list_shift;   // short-list kernel: log2 of the tokens a list entry stands for
   int32_t max_splits;
   int32_t fused_merge;
   float scale_log2;  // sm_scale * log2(e)
@@ -259,6 +261,49 @@ __device__ __forceinline__ int seq_items(const DecodeParams& p, int b, SeqList& 
   return n_splits < 1 ? 1 : n_splits;
 }
 
+// o += P V for four rows of values per lane: hi and rest are the weights as value and remainder in the KV type
+// (operand row c16: a head; head_dim 64: of the tokens of both halves of the 16-lane row), acc[e] dimension e of
+// the lane (head_dim 128: li * 8 + e; 64: li * 8 + 4 (c16 / 8) + e) of the heads 4 g4 + 0 .. 3.
+template <typename T, int D, int NH = 128 / D, int NACC = D / 16>
+__device__ __forceinline__ void weigh_rows(const uint32_t (&hi)[NH][2], const uint32_t (&rest)[NH][2],
+                                           const u32x4 (&v)[4], f32x4 (&acc)[NACC]) {
+  constexpr uint32_t kLow = 0x05040100u, kHigh = 0x07060302u;  // v_perm: the low or the high halves of two dwords
+  if constexpr (D == 128) {
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      const uint32_t lo0 = __builtin_amdgcn_perm(v[1][w], v[0][w], kLow), lo1 = __builtin_amdgcn_perm(v[3][w], v[2][w], kLow);
+      const uint32_t hi0 = __builtin_amdgcn_perm(v[1][w], v[0][w], kHigh), hi1 = __builtin_amdgcn_perm(v[3][w], v[2][w], kHigh);
+      acc[2 * w] = mfma_16x16x16<T>(hi[0][0], hi[0][1], lo0, lo1, acc[2 * w]);
+      acc[2 * w + 1] = mfma_16x16x16<T>(hi[0][0], hi[0][1], hi0, hi1, acc[2 * w + 1]);
+      acc[2 * w] = mfma_16x16x16<T>(rest[0][0], rest[0][1], lo0, lo1, acc[2 * w]);
+      acc[2 * w + 1] = mfma_16x16x16<T>(rest[0][0], rest[0][1], hi0, hi1, acc[2 * w + 1]);
+    }
+  } else {
+    // Rows of eight lanes: the two halves of a 16-lane row hold different tokens.  They exchange half of their
+    // dimensions, after which a lane has four dimensions of the eight tokens of both.
+    uint32_t t[2][4][2];  // half, row, two dimensions each
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int w = 0; w < 2; ++w) {
+        t[0][u][w] = (uint32_t)__builtin_amdgcn_update_dpp((int)v[u][w], (int)v[u][2 + w], 0x128, 0xf, 0xc, false);
+        t[1][u][w] = (uint32_t)__builtin_amdgcn_update_dpp((int)v[u][2 + w], (int)v[u][w], 0x128, 0xf, 0x3, false);
+      }
+    const u32x4 pa = {hi[0][0], hi[0][1], hi[NH - 1][0], hi[NH - 1][1]};
+    const u32x4 pb = {rest[0][0], rest[0][1], rest[NH - 1][0], rest[NH - 1][1]};
+#pragma unroll
+    for (int w = 0; w < 2; ++w)
+#pragma unroll
+      for (int half = 0; half < 2; ++half) {
+        const uint32_t sel = half ? kHigh : kLow;
+        const u32x4 vv = {__builtin_amdgcn_perm(t[0][1][w], t[0][0][w], sel), __builtin_amdgcn_perm(t[0][3][w], t[0][2][w], sel),
+                          __builtin_amdgcn_perm(t[1][1][w], t[1][0][w], sel), __builtin_amdgcn_perm(t[1][3][w], t[1][2][w], sel)};
+        acc[2 * w + half] = mfma_16x16x32<T>(pa, vv, acc[2 * w + half]);
+        acc[2 * w + half] = mfma_16x16x32<T>(pb, vv, acc[2 * w + half]);
+      }
+  }
+}
+
 // One of the n splits of a sequence; PLANNED: n is what the plan's chunk size gives, and the partials are
 // where the plan has them, else part_first is the first partial of the sequence in those of a head slot.
 struct Share {
@@ -422,7 +467,7 @@ __device__ __forceinline__ void attend_share(const DecodeParams& p, const int hr
 
   // Shared-row state: a lane works on ONE query head, c16 % QPG; the running maximum mh of a head is kept
   // equal in all lanes of the wave, lh is the lane's share of the denominator, and accm[dd][i] is
-  // o[head (4 g4 + i) % QPG] of dimension dd of the lane (head_dim 128: li * 8 + dd; 64: see `weigh` below).
+  // o[head (4 g4 + i) % QPG] of dimension dd of the lane (see weigh_rows).
   constexpr int NACC = MMA ? D / 16 : 1;
   float mh = kNegBig, lh = 0.f;
   f32x4 accm[NACC];
@@ -723,51 +768,7 @@ __device__ __forceinline__ void attend_share(const DecodeParams& p, const int hr
           for (int d = 0; d < NACC; ++d) accm[d][i] *= f;
         }
       }
-      // B operand of dimension dd: the four rows of the tile held by this lane, one 16-bit value
-      // each (v_perm picks the low or the high halves of two dwords)
-      const uint32_t vw[U][4] = {{vb[0].x, vb[0].y, vb[0].z, vb[0].w},
-                                 {vb[1].x, vb[1].y, vb[1].z, vb[1].w},
-                                 {vb[2].x, vb[2].y, vb[2].z, vb[2].w},
-                                 {vb[3].x, vb[3].y, vb[3].z, vb[3].w}};
-      if constexpr (LPR == 16) {
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          const uint32_t lo0 = __builtin_amdgcn_perm(vw[1][c], vw[0][c], 0x05040100u);
-          const uint32_t lo1 = __builtin_amdgcn_perm(vw[3][c], vw[2][c], 0x05040100u);
-          const uint32_t hi0 = __builtin_amdgcn_perm(vw[1][c], vw[0][c], 0x07060302u);
-          const uint32_t hi1 = __builtin_amdgcn_perm(vw[3][c], vw[2][c], 0x07060302u);
-          accm[2 * c] = mfma_16x16x16<T>(hi[0][0], hi[0][1], lo0, lo1, accm[2 * c]);
-          accm[2 * c + 1] = mfma_16x16x16<T>(hi[0][0], hi[0][1], hi0, hi1, accm[2 * c + 1]);
-          accm[2 * c] = mfma_16x16x16<T>(rest[0][0], rest[0][1], lo0, lo1, accm[2 * c]);
-          accm[2 * c + 1] = mfma_16x16x16<T>(rest[0][0], rest[0][1], hi0, hi1, accm[2 * c + 1]);
-        }
-      } else {
-        // Rows of eight lanes: the two halves of a 16-lane row hold different tokens, block 0 and block 1.
-        // They exchange half of their dimensions, after which a lane has four dimensions (8 li + 4 (half) +
-        // 0 .. 3) of all eight tokens of its group.
-        uint32_t t[2][U][2];  // block, row, two dimensions each
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-#pragma unroll
-          for (int w = 0; w < 2; ++w) {
-            t[0][u][w] = (uint32_t)__builtin_amdgcn_update_dpp((int)vw[u][w], (int)vw[u][2 + w], 0x128, 0xf, 0xc, false);
-            t[1][u][w] = (uint32_t)__builtin_amdgcn_update_dpp((int)vw[u][2 + w], (int)vw[u][w], 0x128, 0xf, 0x3, false);
-          }
-        const u32x4 pa = {hi[0][0], hi[0][1], hi[NB - 1][0], hi[NB - 1][1]};
-        const u32x4 pb = {rest[0][0], rest[0][1], rest[NB - 1][0], rest[NB - 1][1]};
-#pragma unroll
-        for (int w = 0; w < 2; ++w)
-#pragma unroll
-          for (int half = 0; half < 2; ++half) {
-            const uint32_t sel = half ? 0x07060302u : 0x05040100u;
-            const u32x4 vv = {__builtin_amdgcn_perm(t[0][1][w], t[0][0][w], sel),
-                              __builtin_amdgcn_perm(t[0][3][w], t[0][2][w], sel),
-                              __builtin_amdgcn_perm(t[1][1][w], t[1][0][w], sel),
-                              __builtin_amdgcn_perm(t[1][3][w], t[1][2][w], sel)};
-            accm[2 * w + half] = mfma_16x16x32<T>(pa, vv, accm[2 * w + half]);
-            accm[2 * w + half] = mfma_16x16x32<T>(pb, vv, accm[2 * w + half]);
-          }
-      }
+      weigh_rows<T, D>(hi, rest, vb, accm);
       return;
     } else {
     float sc[QPG][U];

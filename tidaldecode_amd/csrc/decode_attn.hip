@@ -66,6 +66,28 @@ static bool balancing_pays(int head_dim, int qpg, int n_hrows, int batch, int64_
   return (double)(longest - piece) * per_tile > cost || (double)longest * per_tile >= (even > 1 ? 8.0 : 20.0);
 }
 
+// What a short-list launch takes beyond its fixed 3 us, in us: workgroups of nw waves, `tiles` tiles of a workgroup
+// each (but for the last), rows x splits of them, dealt evenly to the compute units.  A compute unit by itself
+// takes 11 ns a token of 128 dimensions and 0.8 for every further trip of a wave; all together read 8 TB/s at
+// most; splits are merged, 16 partials at a time.  The constants fit nine head shapes, lists of 64 to 6000 tokens and
+// six workgroup shapes each (us, lists of 200 | 400 | 1300 | 4096 tokens): 32 heads x 128, four waves x 128 tokens
+// 6.2 | 6.4 | 9.1 | 16.1, eight x 256 5.6 | 7.8 | 8.7 | 15.5, eight x 512 5.6 | 8.8 | 12.1 | 15.5; 28/4 heads 7.5 | 7.5 |
+// 7.7 | 9.4, 6.1 | 8.9 | 9.3 | 9.6, 6.2 | 9.3 | 12.7 | 13.1; 40 heads x 64, four waves x 256 4.8 | 6.6 | 7.5 | 13.5,
+// eight x 512 4.9 | 6.6 | 9.1 | 15.3.  Powers of two alone, which the chunks were, cost 32 heads 5 % at 6000 tokens.
+static float short_list_cost(int head_dim, int qpg, int rows, int items, int nw, int tiles, int splits) {
+  const int wave_tile = 4096 / head_dim, cus = num_cus();
+  const int wgs = rows * splits, active = wgs < cus ? wgs : cus;
+  const int tokens = splits > 1 ? tiles * nw * wave_tile : (items + wave_tile - 1) / wave_tile * wave_tile;
+  const float per_cu = (float)((wgs + cus - 1) / cus) * (float)tokens * (float)head_dim;
+  const float alone = per_cu * (qpg > 1 ? 0.0125f / 128.f : 0.0112f / 128.f) + 0.8f * (float)(tiles - 1);
+  const float together = per_cu * (float)active * (4.f / 8.0e6f);
+  float merge = splits == 1 && tiles == 1 ? 0.02f * (float)(nw - tokens / wave_tile) : 0.f;  // idle waves
+  if (splits > 1)
+    merge = (qpg == 8 ? 2.f : (qpg > 1 ? 1.75f : 1.4f)) + (float)((splits - 1) / 16) * (qpg == 8 ? 1.f : 0.7f) +
+            (qpg > 1 ? 0.02f : 0.01f) * (float)splits;
+  return (alone > together ? alone : together) + merge;
+}
+
 static bool is_pow2(int64_t x) { return x > 0 && (x & (x - 1)) == 0; }
 
 }  // namespace tidal
@@ -137,57 +159,55 @@ extern "C" int td_decode_make_plan(int32_t batch, int32_t num_qo_heads, int32_t 
   }
 
   // ---- short lists: the sparse-layer kernel -------------------------------------------------------
-  // Chunks are a power of two (the kernel divides by shifting) and a multiple of the workgroup
-  // tile; the streaming kernel at 8 waves x 4 rows (tile 128) can run the same plan when a call
-  // turns out not to fit the short-list kernel (page lists, score output, large pools).
+  // Chunks are a multiple of the workgroup tile; the streaming kernel at 8 waves x 4 rows (tile 128, 256 at
+  // head_dim 64) can run the same plan when a call turns out not to fit the short-list kernel.
   int sw = plan->sparse_waves, sr = plan->sparse_rows;
   plan->balanced = 0;
-  // one query head per list walk with a power-of-two group size, or exactly 2, 4 or 8 query heads
-  // sharing their KV head's list (no padding heads)
-  const int group = num_qo_heads / num_kv_heads;
-  const bool heads_fit = qpg == 1 ? is_pow2(group) : (qpg == group && subs == 1);
-  bool sparse = sw >= 0 && sr >= 0 && head_dim == 128 && heads_fit && max_items > 0 &&
+  // one query head per list walk, or a KV head's up to eight query heads sharing its list
+  bool sparse = sw >= 0 && sr >= 0 && head_dim <= 128 && subs == 1 && max_items > 0 &&
                 max_items <= kSparseMaxItems &&
                 (plan->chunk_tokens == 0 || is_pow2(plan->chunk_tokens));
-  if (qpg > 1 && sr == 16) sparse = false;  // shared rows: 8 rows per lane only
+  if ((qpg > 1 || head_dim == 64) && sr == 16) sparse = false;  // 8 rows per lane only
   if (sparse) {
-    // Chunk: the smallest power of two from 128 tokens up that leaves at most 9/8 workgroups per
-    // compute unit.  Where even 512 tokens leave more than that (batches), the chunk grows on for
-    // as long as a full round of workgroups remains: fewer, longer workgroups then beat more
-    // partials to merge (8 sequences x 32 heads, lists of 1024: 27.0 us at 512 tokens, 25.3 at
-    // 1024; lists of 2048: 50.3 -> 47.5 at 2048; lists of 4096: 94.2 -> 90.4 at 4096; 16 sequences
-    // x 1024: 51.0 -> 49.4; a round that is not full loses: 4 sequences x 1024 at 1024 tokens are
-    // 128 workgroups and 20.3 us against 16.7).  Workgroup shape: 4 waves for 128-token chunks, 8
-    // waves otherwise, 8 K rows per lane.
+    // Workgroup shape and chunk with the least cost; more tiles or fewer waves have to gain.  Splits whose partials
+    // do not fit the built-in scratch are left alone, as that would refuse callers who have no other.
     int64_t chunk = plan->chunk_tokens;
-    if (chunk == 0) {
-      chunk = 128;
-      const int64_t rows_all = (int64_t)n_hrows * batch;
-      while (chunk < 512 && rows_all * ceil_div64(max_items, chunk) > num_cus() * 9 / 8) chunk <<= 1;
-      while (rows_all * ceil_div64(max_items, chunk) > num_cus() * 9 / 8 && chunk < max_items &&
-             rows_all * ceil_div64(max_items, chunk * 2) >= num_cus())
-        chunk <<= 1;
-      // Between one and 1.75 eight-wave workgroups of 256 tokens per compute unit neither 256 nor
-      // 512 tokens fill the chip evenly (36 heads x 2048 tokens: 288 workgroups, 32 compute units
-      // get a second one; 40 and 48 heads at 512 tokens: 160 and 192 workgroups for 256 compute
-      // units).  Four-wave workgroups of 128 tokens spread better there (measured, 2048 tokens:
-      // 36 heads 13.4 -> 12.0 us, 40 heads 12.95 -> 12.4, 48 heads 13.8 -> 13.2; no gain at 24,
-      // 32, 56 and 64 heads, which keep their plan).
-      const int64_t w256 = (int64_t)n_hrows * batch * ceil_div64(max_items, 256);
-      if (sw == 0 && (sr == 0 || sr == 8) && w256 > num_cus() && w256 * 4 < (int64_t)num_cus() * 7 &&
-          ceil_div64(max_items, 128) <= 64)
-        chunk = 128;
+    if (chunk == 0 && sr != 16) {
+      const int rows_all = n_hrows * batch, items = (int)max_items;
+      float best = 0.f;
+      const int preset = sw;
+      for (int nw = 8; nw >= 4; nw -= 4) {
+        if (preset != 0 && preset != nw) continue;
+        const int stile = nw * (4096 / head_dim), most = (items + stile - 1) / stile;
+        for (int tiles = 1;; tiles += tiles < 4 ? 1 : (tiles < 16 ? tiles / 4 * 2 : tiles / 2)) {
+          if (tiles > most) tiles = most;
+          const int splits = (most + tiles - 1) / tiles;
+          const bool fits = splits <= 64 && (splits == 1 || kTicketBytes + (int64_t)rows_all * qpg * splits * (head_dim + 2) * 4 +
+                                                                    512 <= (int64_t)TD_STATIC_SCRATCH_BYTES);
+          if (fits) {
+            const float cost = short_list_cost(head_dim, qpg, rows_all, items, nw, tiles, splits);
+            if (best == 0.f || cost < best - 0.01f) {
+              best = cost;
+              sw = nw;
+              chunk = (int64_t)tiles * stile;
+            }
+          }
+          if (tiles == most) break;
+        }
+      }
+    } else if (chunk == 0) {
+      chunk = 256;
     }
     while (ceil_div64(max_items, chunk) > 64) chunk <<= 1;
     if (sr == 0) sr = 8;
-    if (sw == 0) sw = (chunk < 256 || sr == 16) ? 4 : 8;
+    if (sw == 0) sw = (chunk < 32768 / head_dim || sr == 16) ? 4 : 8;
     if (!sparse_shape_supported(sw, sr, qpg))
       return fail(TD_ERR_UNSUPPORTED,
                   "td_decode_make_plan: no short-list kernel with %d waves x %d rows (4 or 8 waves, 8 or "
                   "16 rows)", sw, sr);
-    const int stile = sw * 4 * sr;
+    const int stile = sw * (512 / head_dim) * sr;
     if (plan->chunk_tokens == 0 && chunk < stile) chunk = stile;  // a preset shape with a larger tile
-    if (chunk % stile != 0 || chunk % 128 != 0) {
+    if (chunk % stile != 0 || chunk % (16384 / head_dim) != 0) {
       sparse = false;
     } else {
       plan->chunk_tokens = (int32_t)chunk;
@@ -443,11 +463,10 @@ static int build_params(const td_paged_kv* kv, const td_index_list* list, const 
   p.last_len = list->last_page_len;
   p.last_idx = list->last_page_idx;
   p.chunk_tokens = plan->chunk_tokens;
-  p.chunk_shift = p.qpk_shift = -1;
-  for (int sft = 0; sft < 31; ++sft) {
-    if ((1 << sft) == plan->chunk_tokens) p.chunk_shift = sft;
-    if ((1 << sft) == p.q_per_kv) p.qpk_shift = sft;
-  }
+  p.chunk_magic = plan->chunk_tokens > 1 ? (uint32_t)((((uint64_t)1 << 32) + plan->chunk_tokens - 1) / plan->chunk_tokens) : 0;
+  p.num_kv_heads = Hkv;
+  p.kv_magic = ((1u << 24) + (uint32_t)p.q_per_kv - 1) / (uint32_t)p.q_per_kv;
+  p.list_shift = p.page_mode ? p.page_shift : 0;
   p.max_splits = plan->max_splits;
   p.fused_merge = plan->fused_merge;
   p.scale_log2 = sm_scale * kLog2e;
@@ -473,24 +492,26 @@ static int build_params(const td_paged_kv* kv, const td_index_list* list, const 
   return TD_OK;
 }
 
-// Whether a call can run on the short-list kernel of its plan: token-slot lists, head_dim 128, one
-// query head per list walk or a whole group per shared list, no score output, chunks that are a
-// power-of-two multiple of the kernel's workgroup tile.  Returns 0 (no), kSparseLean (power-of-two
-// pages, pool below 4 GiB, strides within the 24-bit multiplier: 32-bit row offsets) or kSparseWide
-// (any page size, 64-bit row offsets; 8 rows per lane only).
+// Whether a call can run on the short-list kernel of its plan: one query head per list walk or a whole group per
+// shared list, chunks that are a power-of-two multiple of the kernel's workgroup tile.  Returns 0 (no), kSparseLean
+// (power-of-two pages, pool below 4 GiB, strides within the 24-bit multiplier: 32-bit row offsets) or kSparseWide
+// (any page size, 64-bit row offsets; token-slot lists without score output at head_dim 128 only, 8 rows per
+// lane, groups of 1, 2, 4 or 8).
 enum { kSparseNo = 0, kSparseLean = 1, kSparseWide = 2 };
 static int sparse_kernel_fits(const DecodeParams& p, const td_decode_plan* plan,
                               const td_index_list* list, int qpg, int head_dim, bool emit) {
+  const int64_t max_items = (int64_t)list->n_list_host * (list->kind == TD_IDX_PAGES ? p.page_size : 1) + p.page_size;
   if (plan->sparse_waves <= 0 || !sparse_shape_supported(plan->sparse_waves, plan->sparse_rows, qpg))
     return kSparseNo;
-  const int stile = plan->sparse_waves * 4 * plan->sparse_rows;
-  const bool heads_fit = qpg == 1 ? p.qpk_shift >= 0 : (p.q_per_kv == qpg && p.subs == 1);
-  if (!(list->kind == TD_IDX_SLOTS && !emit && heads_fit && head_dim == 128 && p.chunk_shift >= 0 &&
-        plan->chunk_tokens % stile == 0))
+  const int stile = plan->sparse_waves * (512 / head_dim) * plan->sparse_rows;
+  if (!(head_dim <= 128 && p.subs == 1 && max_items <= 2 * kSparseMaxItems && plan->chunk_tokens % stile == 0 &&
+        (plan->sparse_rows == 8 || (head_dim == 128 && list->kind == TD_IDX_SLOTS && !emit))))
     return kSparseNo;
   if (p.lean && p.page_stride_b < (1u << 24) && p.entry_stride_b < (1u << 24)) return kSparseLean;
   // a page's bytes and an entry's offset inside it stay 32-bit; the page base is a 64-bit product
-  if (plan->sparse_rows == 8 && p.page_stride * 2 < ((int64_t)1 << 32)) return kSparseWide;
+  const bool plain = list->kind == TD_IDX_SLOTS && !emit && head_dim == 128 &&
+                     (qpg == 1 ? is_pow2(p.q_per_kv) : p.q_per_kv == qpg);
+  if (plain && plan->sparse_rows == 8 && p.page_stride * 2 < ((int64_t)1 << 32)) return kSparseWide;
   return kSparseNo;
 }
 
@@ -518,12 +539,12 @@ extern "C" int td_decode_attn(const td_paged_kv* kv, const td_index_list* list,
                "td_decode_attn: batch %d x %d heads exceeds the ticket counters", batch, n_hrows * qpg);
     if (qpg > 1)
       rc = kv->dtype == TD_F16
-               ? launch_sparse_shared_f16(p, plan->sparse_waves, qpg, wide, merge_kernel, grid, st)
-               : launch_sparse_shared_bf16(p, plan->sparse_waves, qpg, wide, merge_kernel, grid, st);
+               ? launch_sparse_shared_f16(p, D, plan->sparse_waves, qpg, wide, merge_kernel, grid, st)
+               : launch_sparse_shared_bf16(p, D, plan->sparse_waves, qpg, wide, merge_kernel, grid, st);
     else if (kv->dtype == TD_F16)
-      rc = launch_sparse_f16(p, plan->sparse_waves, plan->sparse_rows, false, wide, merge_kernel, grid, st);
+      rc = launch_sparse_f16(p, D, plan->sparse_waves, plan->sparse_rows, false, wide, merge_kernel, grid, st);
     else
-      rc = launch_sparse_bf16(p, plan->sparse_waves, plan->sparse_rows, false, wide, merge_kernel, grid, st);
+      rc = launch_sparse_bf16(p, D, plan->sparse_waves, plan->sparse_rows, false, wide, merge_kernel, grid, st);
     if (rc != TD_OK) return rc;
     TD_HIP_CHECK(hipGetLastError());
     g_last_kernel = wide ? "short-list, 64-bit offsets" : "short-list";
@@ -624,7 +645,9 @@ extern "C" int td_gather_probe(const td_paged_kv* kv, const td_index_list* list,
                                nullptr, nullptr, out, (int64_t)1 << 40, p, qpg, n_hrows);
   if (prc != TD_OK) return prc;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  const int fits = qpg == 1 ? sparse_kernel_fits(p, plan, list, qpg, kv->head_dim, false) : kSparseNo;
+  const int fits = qpg == 1 && kv->head_dim == 128 && list->kind == TD_IDX_SLOTS && is_pow2(p.q_per_kv)
+                       ? sparse_kernel_fits(p, plan, list, qpg, kv->head_dim, false)
+                       : kSparseNo;
   if (fits != kSparseNo && list->last_page_len == 0 && !list->last_page_len_arr) {
     // the short-list kernel's own loads-only form; it reads `out` as q and writes nothing
     TD_REQUIRE(out_bytes >= (int64_t)batch * num_qo_heads * kv->head_dim * 2,
@@ -634,8 +657,8 @@ extern "C" int td_gather_probe(const td_paged_kv* kv, const td_index_list* list,
     const bool wide = fits == kSparseWide;
     const int src =
         kv->dtype == TD_F16
-            ? launch_sparse_f16(p, plan->sparse_waves, plan->sparse_rows, true, wide, false, sgrid, st)
-            : launch_sparse_bf16(p, plan->sparse_waves, plan->sparse_rows, true, wide, false, sgrid, st);
+            ? launch_sparse_f16(p, 128, plan->sparse_waves, plan->sparse_rows, true, wide, false, sgrid, st)
+            : launch_sparse_bf16(p, 128, plan->sparse_waves, plan->sparse_rows, true, wide, false, sgrid, st);
     if (src != TD_OK) return src;
     TD_HIP_CHECK(hipGetLastError());
     return TD_OK;

@@ -29,19 +29,29 @@ template <int N>
 __device__ __forceinline__ uint32_t row_bcast_u32(uint32_t x) {
   return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x150 + N, 0xf, 0xf, true);
 }
-template <int N>
-__device__ __forceinline__ float row_bcast_f32(float x) {
-  return __builtin_bit_cast(float, row_bcast_u32<N>(__builtin_bit_cast(uint32_t, x)));
+// value of lane N of this lane's group of LPR = 8 or 16 lanes
+template <int N, int LPR>
+__device__ __forceinline__ uint32_t group_bcast_u32(uint32_t x) {
+  if constexpr (LPR == 16) {
+    return row_bcast_u32<N>(x);
+  } else {
+    const int low = (int)row_bcast_u32<N % 8>(x);  // the upper eight lanes take theirs
+    return (uint32_t)__builtin_amdgcn_update_dpp(low, (int)x, 0x150 + N % 8 + 8, 0xf, 0xc, false);
+  }
+}
+template <int N, int LPR>
+__device__ __forceinline__ float group_bcast_f32(float x) {
+  return __builtin_bit_cast(float, group_bcast_u32<N, LPR>(__builtin_bit_cast(uint32_t, x)));
 }
 
-// a[u] = this lane's partial sum for row u (U rows, U = 8 or 16) over its 8 of the 128 dimensions;
-// returns the sum over the 16 lanes of the row group for row (lane % U).  Each butterfly step
+// a[u] = this lane's partial sum for row u (U rows, U = 8 or 16) over its 8 dimensions; returns the sum over
+// the LPR = 8 or 16 lanes of the row group for row (lane % U).  Each butterfly step
 // halves the rows a lane keeps and hands the other half to a partner whose lane index differs in
 // the step's bit (any partner of the opposite class does, as long as every lane's contribution is
 // counted once: xor 1, xor 2, rotate by 4, rotate by 8).
-template <int U>
+template <int U, int LPR>
 __device__ __forceinline__ float reduce_scatter_rows(float (&a)[U], int li) {
-  static_assert(U == 8 || U == 16, "rows per lane group");
+  static_assert(U == 8 || (U == 16 && LPR == 16), "rows per lane group");
   float c1[U / 2], c2[U / 4], c3[U / 8];
   {
     const bool hi = li & 1;
@@ -67,7 +77,8 @@ __device__ __forceinline__ float reduce_scatter_rows(float (&a)[U], int li) {
     for (int i = 0; i < U / 8; ++i) {
       const float keep = hi ? c2[2 * i + 1] : c2[2 * i];
       const float send = hi ? c2[2 * i] : c2[2 * i + 1];
-      c3[i] = keep + dpp_move<0x124>(send);  // row_ror:4: the sender sits in the other quad class
+      // row_ror:4: the sender sits in the other quad class; rows of eight lanes exchange with lane ^ 4
+      c3[i] = keep + (LPR == 16 ? dpp_move<0x124>(send) : lane_xor16<4>(send));
     }
   }
   if constexpr (U == 16) {
@@ -75,8 +86,10 @@ __device__ __forceinline__ float reduce_scatter_rows(float (&a)[U], int li) {
     const float keep = hi ? c3[1] : c3[0];
     const float send = hi ? c3[0] : c3[1];
     return keep + dpp_move<0x128>(send);  // row_ror:8
-  } else {
+  } else if constexpr (LPR == 16) {
     return c3[0] + dpp_move<0x128>(c3[0]);  // lanes li and li ^ 8 hold the same row
+  } else {
+    return c3[0];
   }
 }
 
@@ -135,41 +148,37 @@ __device__ __forceinline__ void scalar_load4(const int32_t* a0, const int32_t* a
       : "memory");
 }
 
-// The tail of a head's computation, run by ONE wave that holds the workgroup's partial result of
-// that head (lane: dimensions 2 lane, 2 lane + 1; M, L uniform): write the result if the head was
-// not split, else publish the partial, take the head's ticket and, as the last of the splits to
-// arrive, merge all partials.
-template <typename T>
-__device__ __forceinline__ void finish_head(const DecodeParams& p, int lane, int n_splits, int split,
-                                            int64_t part0, int32_t* ticket, uint32_t* o32,
-                                            float* lse_out, float o0, float o1, float M, float L) {
-  constexpr int D = 128;
+// The tail of a head's computation, run by ONE wave that holds the workgroup's partial result of that head (lane:
+// dimensions 2 lane, 2 lane + 1; M, L uniform): publish_head writes the result if the head was not split, else the
+// partial; after the ticket merge_head, in the last of the splits to arrive, merges all partials.
+template <typename T, int D>
+__device__ __forceinline__ void publish_head(const DecodeParams& p, int lane, int n_splits, int64_t part, uint32_t* o32,
+                                             float* lse_out, float o0, float o1, float M, float L) {
+  const bool live = D == 128 || lane < D / 2;  // lanes that hold dimensions
   if (n_splits == 1) {
     const float inv = L > 0.f ? 1.f / L : 0.f;
-    *o32 = pack2<T>(o0 * inv, o1 * inv);
+    if (live) *o32 = pack2<T>(o0 * inv, o1 * inv);
     if (lse_out && lane == 0) *lse_out = L > 0.f ? (M + fast_log2(L)) * kLn2 : -INFINITY;
     return;
   }
-  store_coherent(p.ws_o + (part0 + split) * D + 2 * lane, o0, o1);
-  if (lane == 0) store_coherent(p.ws_ml + (part0 + split) * 2, M, L);
-  if (!p.fused_merge) return;  // a second launch (merge_partials_kernel) reduces the partials
+  if (live) store_coherent(p.ws_o + part * D + 2 * lane, o0, o1);
+  if (lane == 0) store_coherent(p.ws_ml + part * 2, M, L);
+}
 
-  // Ordering.  The partial was stored by this wave alone, with device-scope write-through stores
-  // (sc1): such a store is acknowledged -- vmcnt decremented -- only once it has reached memory, the
-  // point where all XCDs meet, so after s_waitcnt vmcnt(0) the partial is visible device-wide.
-  // Only then is the ticket taken; the increment is a device-scope atomic performed at memory,
-  // so a wave that draws the last ticket knows that every other partial of the head had been
-  // acknowledged before its own ticket was even issued.  It reads them with device-scope loads
-  // (sc1), which do not hit lines a non-coherent cache level may still hold from earlier
-  // launches.  What would break this: a plain (non-sc1) store or load on ws_o / ws_ml, a compiler
-  // that moved the ticket above the wait (hence asm volatile with a memory clobber), or partials
-  // stored by several waves without a barrier between their waits and the ticket.
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  int tk = 0;
-  if (lane == 0) tk = __hip_atomic_fetch_add(ticket, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  tk = __builtin_amdgcn_readfirstlane(tk);
-  if (tk != n_splits - 1) return;
-
+// Ordering.  A head's partial was stored by one wave alone, with device-scope write-through stores
+// (sc1): such a store is acknowledged -- vmcnt decremented -- only when it has reached memory, the
+// point where all XCDs meet, so after the caller's s_waitcnt vmcnt(0) the partial is visible device-wide.
+// Only then is the ticket taken; the increment is a device-scope atomic performed at memory,
+// so a wave that draws the last ticket knows that every other partial of the head had been
+// acknowledged before its own ticket was even issued.  It reads them with device-scope loads
+// (sc1), which do not hit lines a non-coherent cache level may still hold from earlier
+// launches.  What would break this: a plain (non-sc1) store or load on ws_o / ws_ml, a compiler
+// that moved the ticket above the wait (hence asm volatile with a memory clobber), or partials
+// stored by several waves without a barrier between their waits and the ticket.
+template <typename T, int D>
+__device__ __forceinline__ void merge_head(const DecodeParams& p, int lane, int n_splits, int64_t part0, int32_t* ticket,
+                                           uint32_t* o32, float* lse_out) {
+  const bool live = D == 128 || lane < D / 2;
   float pm = kNegBig, pl = 0.f;  // (m, l) of split `lane`
   {
     const int sidx = lane < n_splits ? lane : n_splits - 1;
@@ -179,12 +188,14 @@ __device__ __forceinline__ void finish_head(const DecodeParams& p, int lane, int
   }
   constexpr int PRE = 16;  // partial loads in flight
   float pa[PRE], pb[PRE];
+  // 32-bit offsets from one scalar base: the loads go out two instructions apart instead of five
+  const char* const partials = reinterpret_cast<const char*>(p.ws_o + part0 * D);
+  const uint32_t mine = 8u * (uint32_t)(lane & (D / 2 - 1)), last = (uint32_t)(n_splits - 1) * (D * 4);
   auto issue = [&](int base) {
 #pragma unroll
     for (int u = 0; u < PRE; ++u) {
-      int sidx = base + u;
-      sidx = sidx < n_splits ? sidx : n_splits - 1;
-      load_coherent(p.ws_o + (part0 + sidx) * D + 2 * lane, pa[u], pb[u]);
+      const uint32_t at = (uint32_t)(base + u) * (D * 4);
+      load_coherent(reinterpret_cast<const float*>(partials + ((at < last ? at : last) + mine)), pa[u], pb[u]);
     }
   };
   issue(0);
@@ -206,40 +217,46 @@ __device__ __forceinline__ void finish_head(const DecodeParams& p, int lane, int
     }
   }
   const float inv = Lx > 0.f ? 1.f / Lx : 0.f;
-  *o32 = pack2<T>(ra * inv, rb * inv);
+  if (live) *o32 = pack2<T>(ra * inv, rb * inv);
   if (lse_out && lane == 0) *lse_out = Lx > 0.f ? (Mx + fast_log2(Lx)) * kLn2 : -INFINITY;
   if (lane == 0) __hip_atomic_store(ticket, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // QPG query heads per loaded K/V row: 1 (every head row is a query head with its own walk of a
-// list) or the 2, 4 or 8 query heads of a KV head that share one list (a head row is a KV head).
-template <typename T, int NW, int U, bool FRESH, bool PROBE = false, int QPG = 1, bool WIDE = false>
+// list) or the up to 2, 4 or 8 query heads of a KV head that share one list (a head row is a KV head;
+// groups of 3, 5, 6 and 7 leave head slots empty).  ANY: page lists, score output (compiled apart: the branches
+// cost the plain walk of token slots 1 - 2 %).
+template <typename T, int NW, int U, bool FRESH, bool PROBE = false, int QPG = 1, bool WIDE = false, int D = 128, bool ANY = false>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(1, U == 16 ? 2 : 4))) void sparse_attn_kernel(const DecodeParams p) {
   static_assert(QPG == 1 || U == 8, "shared KV rows: 8 rows per lane");
-  constexpr int D = 128;
-  constexpr int LPR = 16;       // lanes per K/V row
-  constexpr int TILE = 4 * U;   // tokens of a wave tile: lane group g holds tokens g U .. g U + U - 1
+  constexpr int LPR = D / 8;            // lanes per K/V row
+  constexpr int TILE = 64 / LPR * U;    // tokens of a wave tile: lane group g holds tokens g U .. g U + U - 1
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int g = lane >> 4, li = lane & 15;
+  const int g = lane / LPR, li = lane % LPR;
+  const int g4 = lane >> 4, c16 = lane & 15;  // 16-lane row and place in it (operands of the matrix products)
   const int hrow = blockIdx.x, b = blockIdx.y, split = blockIdx.z;
   // One batch of scalar loads for every kernel argument the main path uses: the compiler would
   // otherwise fetch them where they are first needed, a dependent round trip each time.
 #define TD_TOUCH(x) asm volatile("" ::"s"(x))
   TD_TOUCH(p.q); TD_TOUCH(p.kv); TD_TOUCH(p.v_offset); TD_TOUCH(p.idx); TD_TOUCH(p.indptr);
   TD_TOUCH(p.count_arr); TD_TOUCH(p.last_len_arr); TD_TOUCH(p.last_idx_arr);
-  TD_TOUCH(p.idx_row_stride); TD_TOUCH(p.idx_cols); TD_TOUCH(p.n_list_host); TD_TOUCH(p.qpk_shift);
-  TD_TOUCH(p.chunk_shift); TD_TOUCH(p.max_splits); TD_TOUCH(p.page_shift); TD_TOUCH(p.max_slot);
+  TD_TOUCH(p.idx_row_stride); TD_TOUCH(p.idx_cols); TD_TOUCH(p.n_list_host); TD_TOUCH(p.kv_magic);
+  TD_TOUCH(p.chunk_magic); TD_TOUCH(p.max_splits); TD_TOUCH(p.page_shift); TD_TOUCH(p.max_slot);
   TD_TOUCH(p.page_stride_b); TD_TOUCH(p.entry_stride_b); TD_TOUCH(p.head_stride);
+  TD_TOUCH(p.ws_o); TD_TOUCH(p.ws_ml); TD_TOUCH(p.ws_cnt); TD_TOUCH(p.o); TD_TOUCH(p.lse); TD_TOUCH(p.vheads);
+  TD_TOUCH(p.ticket_stride); TD_TOUCH(p.fused_merge);
   TD_TOUCH(p.last_len); TD_TOUCH(p.last_idx); TD_TOUCH(p.scale_log2); TD_TOUCH(p.num_qo_heads);
   if constexpr (FRESH) {
     TD_TOUCH(p.fresh_k); TD_TOUCH(p.fresh_v); TD_TOUCH(p.fresh_cos); TD_TOUCH(p.fresh_sin);
     TD_TOUCH(p.fresh_slot);
   }
 #undef TD_TOUCH
-  // the host sends only power-of-two group sizes here
-  const int kv_head = QPG > 1 ? hrow : hrow >> p.qpk_shift;
-  const int rq0 = hrow * QPG;              // first query head of the head row
+  // hrow / q_per_kv: kv_magic is 2^24 / q_per_kv rounded up, exact for the head rows that tickets exist for
+  const int list_shift = ANY ? p.list_shift : 0;
+  const int kv_head = QPG > 1 ? hrow : (int)(((uint64_t)(uint32_t)hrow * p.kv_magic) >> 24);
+  const int rq0 = QPG > 1 ? hrow * p.q_per_kv : hrow;  // first query head of the head row
+  const int gsz = QPG > 1 ? p.q_per_kv : 1;            // its query heads: at most QPG
   const int own = g * U + (li & (U - 1));  // the token of the tile this lane owns
 
   // ---- everything that depends on the kernel arguments only is requested at once ---------------
@@ -255,7 +272,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(1, U ==
   const int32_t* row = p.idx + (int64_t)idx_row * p.idx_row_stride + list_beg;
   const int cap = list_capacity(p.n_list_host, p.indptr != nullptr, list_beg, list_end, p.idx_cols);
   auto fetch_entry = [&](int t) -> int32_t {
-    int pos = t + own;
+    int pos = (t + own) >> list_shift;
     pos = pos < cap ? pos : cap - 1;
     return cap > 0 ? row[pos] : 0;
   };
@@ -266,39 +283,40 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(1, U ==
   // the new token's k and v, rotates q and k once, and leaves rotated q, rotated k and v in LDS for
   // the other waves (which then issue no global load besides their list entry and K/V rows: eight
   // waves per workgroup asking the same few cache lines for cos / sin cost the launch 0.5 us).
-  uint32_t qp[QPG][4];
-  const bool prep = FRESH && wave == 0;  // scalar
-  if constexpr (!FRESH) {
+  // One head: 8 elements per lane.  Shared rows: operand of the matrix product, column c16 is head
+  // c16 % QPG (empty head slots repeat the last head), elements [32 x + 8 g4, +8).
+  constexpr int NQ = QPG > 1 ? D / 32 : 1;
+  u32x4 qp[NQ];
+  auto load_q = [&](auto piece) __attribute__((always_inline)) {  // piece(head, 16-byte piece)
+    const int j = c16 % QPG < gsz ? c16 % QPG : gsz - 1;
 #pragma unroll
-    for (int j = 0; j < QPG; ++j) {
-      const u32x4 v =
-          reinterpret_cast<const u32x4*>(p.q)[((int64_t)b * p.num_qo_heads + rq0 + j) * LPR + li];
-      qp[j][0] = v.x; qp[j][1] = v.y; qp[j][2] = v.z; qp[j][3] = v.w;
-    }
-  }
+    for (int x = 0; x < NQ; ++x) qp[x] = QPG > 1 ? piece(j, 4 * x + g4) : piece(0, li);
+  };
+  const bool prep = FRESH && wave == 0;  // scalar
+  const u32x4* const q_rows = reinterpret_cast<const u32x4*>(p.q) + ((int64_t)b * p.num_qo_heads + rq0) * LPR;
+  if constexpr (!FRESH) load_q([&](int j, int c) { return q_rows[j * LPR + c]; });
   // What wave 0 loads for the fused step.  Defined in that wave only and read in that wave only:
   // giving the other waves a value here would make them wait for their list entry first (the
   // registers are the destination of loads in flight on the other side of the branch).
-  u32x4 q_raw[QPG], kn_raw, vn_raw;
+  constexpr int GR = 64 / LPR, QX = (QPG + GR - 1) / GR;  // lane group g prepares the heads g, g + GR, ...
+  u32x4 q_raw[QX], kn_raw, vn_raw;
   f32x4 cos_lo, cos_hi, sin_lo, sin_hi;
   if constexpr (FRESH) {
     if (prep) {
 #pragma unroll
-      for (int j = 0; j < QPG; ++j)
-        q_raw[j] = reinterpret_cast<const u32x4*>(p.q)[((int64_t)b * p.num_qo_heads + rq0 + j) * LPR + li];
+      for (int x = 0; x < QX; ++x) q_raw[x] = q_rows[(g + x * GR < gsz ? g + x * GR : gsz - 1) * LPR + li];
       constexpr int HALF = LPR / 2;
       const f32x4* cp = reinterpret_cast<const f32x4*>(p.fresh_cos + (int64_t)b * (D / 2) + (li % HALF) * 8);
       const f32x4* sp = reinterpret_cast<const f32x4*>(p.fresh_sin + (int64_t)b * (D / 2) + (li % HALF) * 8);
       cos_lo = cp[0]; cos_hi = cp[1]; sin_lo = sp[0]; sin_hi = sp[1];
-      const int n_kv = QPG > 1 ? p.num_qo_heads / QPG : p.num_qo_heads >> p.qpk_shift;
-      const int64_t fresh_off = ((int64_t)b * n_kv + kv_head) * LPR + li;
+      const int64_t fresh_off = ((int64_t)b * p.num_kv_heads + kv_head) * LPR + li;
       kn_raw = reinterpret_cast<const u32x4*>(p.fresh_k)[fresh_off];
       vn_raw = reinterpret_cast<const u32x4*>(p.fresh_v)[fresh_off];
     }
   }
 
   // ---- the sequence: listed entries, forced last page, splits ------------------------------------
-  // (seq_items of decode_attn.cuh with the division by the chunk size as a shift)
+  // (seq_items of decode_attn.cuh with the division by the chunk size as a product)
   SeqList s;
   s.n_list = p.n_list_host;
   s.last_len = p.last_len;
@@ -324,8 +342,9 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(1, U ==
   // a count beyond what the first fetch was clamped to would pair tokens with the wrong entries
   s.n_list = s.n_list < 0 ? 0 : (s.n_list > cap ? cap : s.n_list);
   s.last_len = s.last_len < 0 ? 0 : (s.last_len > p.page_size ? p.page_size : s.last_len);
-  const int c1 = s.n_list + s.last_len;
-  int n_splits = (c1 + p.chunk_tokens - 1) >> p.chunk_shift;
+  const int n_listed = s.n_list << list_shift;  // tokens: an entry is a slot, or a page of 2^list_shift of them
+  const int c1 = n_listed + s.last_len;
+  int n_splits = (int)__umulhi((uint32_t)(c1 + p.chunk_tokens - 1), p.chunk_magic);
   n_splits = n_splits > p.max_splits ? p.max_splits : n_splits;
   n_splits = n_splits < 1 ? 1 : n_splits;
   if (split >= n_splits) return;  // uniform for the workgroup
@@ -360,19 +379,21 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(1, U ==
   float acc[8];
 #pragma unroll
   for (int d = 0; d < 8; ++d) acc[d] = 0.f;
-  // Shared KV rows (QPG > 1): per-head maxima and denominators, and p.V on the matrix cores:
-  // accm[e][r] = o[head 4 g + r][li 8 + e], already summed over the four lane groups.
-  float mh[QPG], lh[QPG];
+  // Shared KV rows (QPG > 1): the lane's head is c16 % QPG; its maximum is equal in all lanes of the wave, lh the
+  // lane's share of its denominator, and accm[e][r] = o[head (4 g4 + r) % QPG] of the lane's dimension e
+  // (head_dim 128: li 8 + e; 64: li 8 + 4 (c16 / 8) + e), already summed over the lane groups.
+  float mh = kNegBig, lh = 0.f;
+  constexpr int NACC = QPG > 1 ? D / 16 : 1;
+  f32x4 accm[NACC];
 #pragma unroll
-  for (int j = 0; j < QPG; ++j) { mh[j] = kNegBig; lh[j] = 0.f; }
-  f32x4 accm[8];
-#pragma unroll
-  for (int d = 0; d < 8; ++d) accm[d] = f32x4{0.f, 0.f, 0.f, 0.f};
-  __shared__ __attribute__((aligned(16))) float sm_p[QPG > 1 ? NW * QPG * TILE : 4];
-  // fused decode step: rotated q rows, the new token's rotated key and its value, 256 bytes each
-  __shared__ __attribute__((aligned(16))) uint32_t sm_fresh[FRESH ? (QPG + 2) * 64 : 4];
-  uint32_t* const sm_knew = sm_fresh + (FRESH ? QPG * 64 : 0);
-  uint32_t* const sm_vnew = sm_knew + (FRESH ? 64 : 0);
+  for (int d = 0; d < NACC; ++d) accm[d] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // a wave's key tile on its way to operand layout; the wave states at the end of the launch
+  constexpr int STATE_F = QPG > 1 && TILE * D / 2 > QPG * D ? TILE * D / 2 : QPG * D;  // floats per wave
+  __shared__ __attribute__((aligned(16))) float sm_state[NW][STATE_F];
+  // fused decode step: rotated q rows, the new token's rotated key and its value, D elements each
+  __shared__ __attribute__((aligned(16))) uint32_t sm_fresh[FRESH ? (QPG + 2) * D / 2 : 4];
+  uint32_t* const sm_knew = sm_fresh + (FRESH ? QPG * D / 2 : 0);
+  uint32_t* const sm_vnew = sm_knew + (FRESH ? D / 2 : 0);
 
   // ---- one tile of the wave: slot and row offset of the lane's own token, then every K and V row ----
   u32x4 kb[U], vb[U];
@@ -382,7 +403,8 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(1, U ==
     const int i = t + own;
     valid = i < c1;
     // entry_raw was read at min(i, capacity - 1), which is i for every listed token (n_list <= capacity)
-    slot = i < s.n_list ? (uint32_t)entry_raw : last_base + (uint32_t)(i - s.n_list);
+    slot = i < n_listed ? ((uint32_t)entry_raw << list_shift) + (uint32_t)(i & ((1 << list_shift) - 1))
+                        : last_base + (uint32_t)(i - n_listed);
     slot = slot > p.max_slot ? p.max_slot : slot;
     off_t off_own = slot_offset(slot);
     // lanes past the end of the list repeat the first token of the tile (which exists: t < c1)
@@ -395,7 +417,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(1, U ==
       const char* ka[U];
 #define TD_ROW_OFF(N)                                                                              \
   if constexpr (N < U)                                                                             \
-    ka[N] = kbase + ((((uint64_t)row_bcast_u32<N>(hi_own)) << 32) | (uint64_t)row_bcast_u32<N>(lo_own)) + \
+    ka[N] = kbase + ((((uint64_t)group_bcast_u32<N, LPR>(hi_own)) << 32) | (uint64_t)group_bcast_u32<N, LPR>(lo_own)) + \
             head_byte_off;
       TD_ROW_OFF(0) TD_ROW_OFF(1) TD_ROW_OFF(2) TD_ROW_OFF(3) TD_ROW_OFF(4) TD_ROW_OFF(5)
       TD_ROW_OFF(6) TD_ROW_OFF(7) TD_ROW_OFF(8) TD_ROW_OFF(9) TD_ROW_OFF(10) TD_ROW_OFF(11)
@@ -404,6 +426,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(1, U ==
 #pragma unroll
       for (int u = 0; u < U; ++u)
         kb[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(ka[u]));
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int u = 0; u < U; ++u)
         vb[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(ka[u] + p.v_offset * 2));
@@ -414,7 +437,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(1, U ==
       off_own = valid ? off_own : off_first;
       uint32_t offs[U];
 #define TD_ROW_OFF(N) \
-  if constexpr (N < U) offs[N] = row_bcast_u32<N>(off_own) + head_byte_off;
+  if constexpr (N < U) offs[N] = group_bcast_u32<N, LPR>(off_own) + head_byte_off;
       TD_ROW_OFF(0) TD_ROW_OFF(1) TD_ROW_OFF(2) TD_ROW_OFF(3) TD_ROW_OFF(4) TD_ROW_OFF(5)
       TD_ROW_OFF(6) TD_ROW_OFF(7) TD_ROW_OFF(8) TD_ROW_OFF(9) TD_ROW_OFF(10) TD_ROW_OFF(11)
       TD_ROW_OFF(12) TD_ROW_OFF(13) TD_ROW_OFF(14) TD_ROW_OFF(15)
@@ -422,13 +445,29 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(1, U ==
 #pragma unroll
       for (int u = 0; u < U; ++u)
         kb[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(kbase + offs[u]));
+      // (left to itself the compiler takes K and V by turns, and q.k waits for all but the last V row: 32 heads,
+      // lists of 3500, a card at low clocks, 464 -> 452 us for 16 layers)
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int u = 0; u < U; ++u)
         vb[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(vbase + offs[u]));
     }
   };
 
-  // ---- arithmetic of the tile whose rows `issue` asked for ----------------------------------------
+  // one logit (base 2 in, natural out) of a selection layer
+  auto emit = [&](bool mine, int head, int i, float logit2) __attribute__((always_inline)) {
+    if (mine && i < c1) {
+      const int64_t at = ((int64_t)b * p.num_qo_heads + head) * p.score_stride + i;
+      if (p.scores_f32)
+        reinterpret_cast<float*>(p.scores)[at] = logit2 * kLn2;
+      else
+        reinterpret_cast<uint16_t*>(p.scores)[at] = from_float<T>(logit2 * kLn2);
+    }
+  };
+
+  // ---- arithmetic of the tile (of tokens t ..) whose rows `issue` asked for -------------------------
+  const int STEP = n_splits * NW * TILE;
+  int t = t0;
   auto compute = [&](bool first_tile) {
     if constexpr (PROBE) {  // measurement: the loads alone, no arithmetic and no merge
       u32x4 fold = {0u, 0u, 0u, 0u};
@@ -450,7 +489,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(1, U ==
         const uint32_t hm = hit ? 1u : 0u;
 #define TD_ROW_FIX(N)                   \
   if constexpr (N < U) {                \
-    if (row_bcast_u32<N>(hm)) {         \
+    if (group_bcast_u32<N, LPR>(hm)) {         \
       kb[N] = kn;                       \
       vb[N] = vn;                       \
     }                                   \
@@ -463,101 +502,123 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(1, U ==
     }
 
     if constexpr (QPG > 1) {
-      // The lane ends with the logits of ITS token for all QPG heads; maxima per head are made
-      // wave-uniform.  The weights then go through a strip of LDS private to the wave into the
-      // A-operand layout of a 16x16x16 matrix product (row = head, inner index = the 16 tokens
-      // 4c..4c+3 of the four lane groups), B = the four V rows a lane holds, one 16-bit element each.
-      constexpr bool kSplit = std::is_same<T, BF16>::value;  // bf16 weights travel as value + remainder
-      float* sp = sm_p + wave * (QPG * TILE);
-      float alpha[QPG];
+      // S = K Q^T on the matrix cores: the rows pass through the wave's own LDS into operand layout (LDS accesses
+      // of one wave complete in order), in blocks of 16 tokens.  Block (c, h) holds the tokens g U + 4 c + i of
+      // the lane groups g = NH g4 + h at row 4 g4 + i, which makes a lane's four scores of a block the tokens
+      // whose values its group holds: the weights are the operand of the second product as they stand.
+      // Piece x of row r lies at x ^ r (head_dim 64: x ^ (r / 2)), so that 16 rows read at one piece fall on
+      // different banks.  (Dot products, a reduction over the row for every head and a strip of LDS for the
+      // weights before: with the
+      // loads ordered as below, lists of 4096 for 32/8 heads x 128 9.9 -> 9.7 us, of 200 6.9 -> 6.1.)
+      constexpr int NH = 16 / LPR, NC = U / 4;
+      auto place = [](int r, int x) { return r * (D * 2) + 16 * (x ^ (LPR == 16 ? r : (r >> 1) & 7)); };
+      char* const kt = reinterpret_cast<char*>(sm_state[wave]);
 #pragma unroll
-      for (int j = 0; j < QPG; ++j) {
-        float part[U];
+      for (int u = 0; u < U; ++u)
+        *reinterpret_cast<u32x4*>(kt + ((u >> 2) * NH + g % NH) * (32 * D) + place(4 * (g / NH) + (u & 3), li)) = kb[u];
+      asm volatile("" ::: "memory");
+      float sv[NC][NH][4];
+      float mt = kNegBig;
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-          float a = dot2<T>(qp[j][0], kb[u].x, 0.f);
-          a = dot2<T>(qp[j][1], kb[u].y, a);
-          a = dot2<T>(qp[j][2], kb[u].z, a);
-          part[u] = dot2<T>(qp[j][3], kb[u].w, a);
+      for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int h = 0; h < NH; ++h) {
+          f32x4 st = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int x = 0; x < NQ; ++x)
+            st = mfma_16x16x32<T>(
+                *reinterpret_cast<const u32x4*>(kt + (c * NH + h) * (32 * D) + place(c16, 4 * x + g4)), qp[x], st);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) sv[c][h][i] = st[i] * p.scale_log2;
         }
-        const float red = reduce_scatter_rows<U>(part, li);
-        const float sv = valid ? red * p.scale_log2 : kNegBig;
-        const float m_new = fmaxf(mh[j], rows_max(row16_max(sv)));
-        alpha[j] = fast_exp2(mh[j] - m_new);
-        mh[j] = m_new;
-        const float pr = valid ? fast_exp2(sv - m_new) : 0.f;
-        lh[j] = lh[j] * alpha[j] + (li < 8 ? pr : 0.f);  // lanes li and li ^ 8 hold the same token
-        if (li < 8) sp[j * TILE + own] = pr;
+      asm volatile("" ::: "memory");
+      if (ANY && p.scores) {  // copy c16 / QPG of a head writes the tokens copy, copy + COPIES, ... of the lane's
+        constexpr int COPIES = 16 / QPG, NV = NC * NH * 4;
+        const int copy = c16 / QPG, head = c16 % QPG;
+#pragma unroll
+        for (int n0 = 0; n0 < NV; n0 += COPIES) {
+          float e = sv[n0 / 4 / NH][n0 / 4 % NH][n0 % 4];
+#pragma unroll
+          for (int x = 1; x < COPIES; ++x)
+            if (n0 + x < NV) e = copy == x ? sv[(n0 + x) / 4 / NH][(n0 + x) / 4 % NH][(n0 + x) % 4] : e;
+          const int n = n0 + copy;
+          emit(n < NV && head < gsz, rq0 + head, t + (NH * g4 + n / 4 % NH) * U + 4 * (n / 4 / NH) + n % 4, e);
+        }
       }
-      if (!first_tile) {  // later tiles: rescale what the earlier ones left (row r of group g: head 4 g + r)
+#pragma unroll
+      for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int h = 0; h < NH; ++h)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const bool there = t + (NH * g4 + h) * U + 4 * c + i < c1;
+            sv[c][h][i] = there ? sv[c][h][i] : kNegBig;
+            mt = fmaxf(mt, sv[c][h][i]);
+          }
+      const float m_new = fmaxf(mh, rows_max(mt));
+      const float alpha = fast_exp2(mh - m_new);
+      mh = m_new;
+      float sum = 0.f;
+#pragma unroll
+      for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int h = 0; h < NH; ++h)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const float pr = sv[c][h][i] > 0.5f * kNegBig ? fast_exp2(sv[c][h][i] - m_new) : 0.f;
+            sv[c][h][i] = pr;
+            sum += pr;
+          }
+      lh = fmaf(lh, alpha, sum);
+      if (!first_tile) {  // later tiles: rescale what the earlier ones left (row r of group g4: head 4 g4 + r)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const float f = (QPG == 8 && g == 1) ? alpha[(4 + r) % QPG] : alpha[r % QPG];
+          const float f = __shfl(alpha, (4 * g4 + r) % QPG, 64);
 #pragma unroll
-          for (int e = 0; e < 8; ++e) accm[e][r] *= f;
+          for (int e = 0; e < NACC; ++e) accm[e][r] *= f;
         }
       }
-      // the strip was written by other lanes of this wave: LDS accesses of a wave complete in
-      // issue order; the wait and the wave barrier pin that order for the compiler too
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      __builtin_amdgcn_wave_barrier();
+      // the weights travel in the KV type as value and remainder (see decode_attn_kernel)
 #pragma unroll
-      for (int c = 0; c < U / 4; ++c) {
-        f32x4 pa = *reinterpret_cast<const f32x4*>(sp + (li < QPG ? li : 0) * TILE + g * U + 4 * c);
-        if (li >= QPG) pa = f32x4{0.f, 0.f, 0.f, 0.f};  // rows past the heads of the group
-        const uint32_t ah0 = pack2<T>(pa.x, pa.y), ah1 = pack2<T>(pa.z, pa.w);
-        uint32_t al0 = 0, al1 = 0;
-        if constexpr (kSplit) {
-          float r0, r1, r2, r3;
-          unpack2<T>(ah0, r0, r1);
-          unpack2<T>(ah1, r2, r3);
-          al0 = pack2<T>(pa.x - r0, pa.y - r1);
-          al1 = pack2<T>(pa.z - r2, pa.w - r3);
-        }
-        const uint32_t vw[4][4] = {
-            {vb[4 * c].x, vb[4 * c].y, vb[4 * c].z, vb[4 * c].w},
-            {vb[4 * c + 1].x, vb[4 * c + 1].y, vb[4 * c + 1].z, vb[4 * c + 1].w},
-            {vb[4 * c + 2].x, vb[4 * c + 2].y, vb[4 * c + 2].z, vb[4 * c + 2].w},
-            {vb[4 * c + 3].x, vb[4 * c + 3].y, vb[4 * c + 3].z, vb[4 * c + 3].w}};
+      for (int c = 0; c < NC; ++c) {
+        uint32_t hi[NH][2], rest[NH][2];
 #pragma unroll
-        for (int w2 = 0; w2 < 4; ++w2) {
-          const uint32_t lo0 = __builtin_amdgcn_perm(vw[1][w2], vw[0][w2], 0x05040100u);
-          const uint32_t lo1 = __builtin_amdgcn_perm(vw[3][w2], vw[2][w2], 0x05040100u);
-          const uint32_t hi0 = __builtin_amdgcn_perm(vw[1][w2], vw[0][w2], 0x07060302u);
-          const uint32_t hi1 = __builtin_amdgcn_perm(vw[3][w2], vw[2][w2], 0x07060302u);
-          accm[2 * w2] = mfma_16x16x16<T>(ah0, ah1, lo0, lo1, accm[2 * w2]);
-          accm[2 * w2 + 1] = mfma_16x16x16<T>(ah0, ah1, hi0, hi1, accm[2 * w2 + 1]);
-          if constexpr (kSplit) {
-            accm[2 * w2] = mfma_16x16x16<T>(al0, al1, lo0, lo1, accm[2 * w2]);
-            accm[2 * w2 + 1] = mfma_16x16x16<T>(al0, al1, hi0, hi1, accm[2 * w2 + 1]);
+        for (int h = 0; h < NH; ++h)
+#pragma unroll
+          for (int w = 0; w < 2; ++w) {
+            hi[h][w] = pack2<T>(sv[c][h][2 * w], sv[c][h][2 * w + 1]);
+            float r0, r1;
+            unpack2<T>(hi[h][w], r0, r1);
+            rest[h][w] = pack2<T>(sv[c][h][2 * w] - r0, sv[c][h][2 * w + 1] - r1);
           }
-        }
+        const u32x4(&v4)[4] = *reinterpret_cast<const u32x4(*)[4]>(&vb[4 * c]);
+        weigh_rows<T, D>(hi, rest, v4, accm);
       }
-      asm volatile("" ::: "memory");  // the strip is rewritten by the next tile only after these reads
       return;
     }
     // q.k: U partial sums per lane, reduce-scattered so that the lane ends with its own token
     float part[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      float a = dot2<T>(qp[0][0], kb[u].x, 0.f);
-      a = dot2<T>(qp[0][1], kb[u].y, a);
-      a = dot2<T>(qp[0][2], kb[u].z, a);
-      part[u] = dot2<T>(qp[0][3], kb[u].w, a);
+      float a = dot2<T>(qp[0].x, kb[u].x, 0.f);
+      a = dot2<T>(qp[0].y, kb[u].y, a);
+      a = dot2<T>(qp[0].z, kb[u].z, a);
+      part[u] = dot2<T>(qp[0].w, kb[u].w, a);
     }
-    const float red = reduce_scatter_rows<U>(part, li);  // every lane takes part: no branch around it
-    const float sv = valid ? red * p.scale_log2 : kNegBig;
+    const float red = reduce_scatter_rows<U, LPR>(part, li) * p.scale_log2;  // every lane takes part: no branch around it
+    if (ANY && p.scores) emit(U >= LPR || li < U, rq0, t + own, red);
+    const float sv = valid ? red : kNegBig;
     const float m_new = fmaxf(m_run, rows_max(row16_max(sv)));
     const float alpha = fast_exp2(m_run - m_new);
     m_run = m_new;
     const float pr = valid ? fast_exp2(sv - m_new) : 0.f;
-    // with U == 8 the lanes li and li ^ 8 hold the same token: it counts once
-    l_lane = l_lane * alpha + ((U == 16 || li < 8) ? pr : 0.f);
+    // with fewer rows than lanes in a group the lanes li and li ^ 8 hold the same token: it counts once
+    l_lane = l_lane * alpha + ((U >= LPR || li < U) ? pr : 0.f);
 #pragma unroll
     for (int d = 0; d < 8; ++d) acc[d] *= alpha;
 #define TD_ROW_PV(N)                                        \
   if constexpr (N < U) {                                    \
-    const float pu = row_bcast_f32<N>(pr);                  \
+    const float pu = group_bcast_f32<N, LPR>(pr);                  \
     float v0, v1, v2, v3, v4, v5, v6, v7;                   \
     unpack2<T>(vb[N].x, v0, v1);                            \
     unpack2<T>(vb[N].y, v2, v3);                            \
@@ -579,9 +640,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(1, U ==
   };
 
   // ---- the wave's tiles: rows of the first one are asked for before anything else happens --------
-  const int STEP = n_splits * NW * TILE;
-  int t = t0;
-  bool live = t < c1;  // wave-uniform
+  const bool live = t < c1;  // wave-uniform
   if (!prep && live) issue(t, ent);
 
   if constexpr (FRESH) {
@@ -594,13 +653,14 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(1, U ==
       const float sgn = li < LPR / 2 ? -1.f : 1.f;  // y_lo = x_lo c - x_hi s,  y_hi = x_hi c + x_lo s
       const float rsn[8] = {sgn * sin_lo.x, sgn * sin_lo.y, sgn * sin_lo.z, sgn * sin_lo.w,
                             sgn * sin_hi.x, sgn * sin_hi.y, sgn * sin_hi.z, sgn * sin_hi.w};
-      // rotate-half RoPE of 8 elements per lane; the partner dimension (+- 64) sits 8 lanes away
+      // rotate-half RoPE of 8 elements per lane; the partner dimension (+- D/2) sits LPR/2 lanes away
       auto rotate = [&](uint32_t(&w)[4]) {
         float x[8], y[8];
 #pragma unroll
         for (int c = 0; c < 4; ++c) unpack2<T>(w[c], x[2 * c], x[2 * c + 1]);
 #pragma unroll
-        for (int d = 0; d < 8; ++d) y[d] = x[d] * rcs[d] + dpp_move<0x128>(x[d]) * rsn[d];
+        for (int d = 0; d < 8; ++d)
+          y[d] = x[d] * rcs[d] + (LPR == 16 ? dpp_move<0x128>(x[d]) : lane_xor16<4>(x[d])) * rsn[d];
 #pragma unroll
         for (int c = 0; c < 4; ++c) w[c] = pack2<T>(y[2 * c], y[2 * c + 1]);
       };
@@ -611,10 +671,11 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(1, U ==
         *reinterpret_cast<u32x4*>(sm_vnew + li * 4) = vn_raw;
       }
 #pragma unroll
-      for (int j = 0; j < QPG; ++j) {
-        uint32_t qj[4] = {q_raw[j].x, q_raw[j].y, q_raw[j].z, q_raw[j].w};
+      for (int x = 0; x < QX; ++x) {
+        uint32_t qj[4] = {q_raw[x].x, q_raw[x].y, q_raw[x].z, q_raw[x].w};
         rotate(qj);
-        if (g == 0) *reinterpret_cast<u32x4*>(sm_fresh + j * 64 + li * 4) = u32x4{qj[0], qj[1], qj[2], qj[3]};
+        const int j = g + x * GR;
+        if (j < gsz) *reinterpret_cast<u32x4*>(sm_fresh + j * (D / 2) + li * 4) = u32x4{qj[0], qj[1], qj[2], qj[3]};
       }
       if (live) issue(t, ent);
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the LDS writes have landed
@@ -625,11 +686,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(1, U ==
     asm volatile("" ::: "memory");
     // every wave, the first included: registers that no global load of either branch is still
     // writing to, so that the wait the compiler puts in front of this read is for LDS only
-#pragma unroll
-    for (int j = 0; j < QPG; ++j) {
-      const u32x4 v = *reinterpret_cast<const u32x4*>(sm_fresh + j * 64 + li * 4);
-      qp[j][0] = v.x; qp[j][1] = v.y; qp[j][2] = v.z; qp[j][3] = v.w;
-    }
+    load_q([&](int j, int c) { return *reinterpret_cast<const u32x4*>(sm_fresh + j * (D / 2) + c * 4); });
   }
 
   // the first tile apart from the loop: its rows were asked for above, and the loop then keeps no
@@ -645,7 +702,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(1, U ==
     // One workgroup per KV head writes the new token into the cache, from the copy in LDS and after
     // the tiles: a store in front of them would have the tiles' first register writes wait for it.
     // Nobody in this launch reads that slot from memory.
-    if (prep && split == 0 && (QPG > 1 || hrow == (kv_head << p.qpk_shift)) && g == 0) {
+    if (prep && split == 0 && (QPG > 1 || hrow == kv_head * p.q_per_kv) && g == 0) {
       const uint32_t ns = new_slot > p.max_slot ? p.max_slot : new_slot;
       char* dst = reinterpret_cast<char*>(const_cast<void*>(p.kv)) + slot_offset(ns) + head_byte_off;
       *reinterpret_cast<u32x4*>(dst) = *reinterpret_cast<const u32x4*>(sm_knew + li * 4);
@@ -654,31 +711,29 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(1, U ==
   }
 
   if constexpr (PROBE) return;
-  __shared__ __attribute__((aligned(16))) float sm_o[NW][QPG][D];
+  auto state = [&](int w, int j, int d) -> float* { return &sm_state[w][j * D + d]; };
   __shared__ float sm_ml[NW][QPG][2];
   if constexpr (QPG > 1) {
-    // the matrix product already summed the lane groups: the lanes of group g hold heads 4g..4g+3
+    // the matrix product already summed the lane groups: the lanes of group g4 hold heads 4 g4 .. 4 g4 + 3
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const int head = 4 * g + r;
+      const int head = 4 * g4 + r;
       if (head < QPG) {
-        *reinterpret_cast<f32x4*>(&sm_o[wave][head][li * 8]) =
-            f32x4{accm[0][r], accm[1][r], accm[2][r], accm[3][r]};
-        *reinterpret_cast<f32x4*>(&sm_o[wave][head][li * 8 + 4]) =
-            f32x4{accm[4][r], accm[5][r], accm[6][r], accm[7][r]};
+#pragma unroll
+        for (int e = 0; e < NACC; e += 4)
+          *reinterpret_cast<f32x4*>(state(wave, head, li * 8 + (LPR == 16 ? e : 4 * (c16 >> 3)))) =
+              f32x4{accm[e][r], accm[e + 1][r], accm[e + 2][r], accm[e + 3][r]};
       }
     }
-#pragma unroll
-    for (int j = 0; j < QPG; ++j) {
-      const float lw = rows_sum(group_sum<16>(lh[j]));
-      if (lane == 0) {
-        sm_ml[wave][j][0] = mh[j];
-        sm_ml[wave][j][1] = lw;
-      }
+    const float lw = rows_sum(lh);
+    if (lane < QPG) {
+      sm_ml[wave][lane][0] = mh;
+      sm_ml[wave][lane][1] = lw;
     }
   } else {
-    // ---- the four lane groups of the wave: the maximum is shared, so the sums simply add --------
-    // reduce-scatter over the groups: lane (g, li) ends with dimensions li 8 + g 2 + {0, 1}
+    // ---- the lane groups of the wave: the maximum is shared, so the sums simply add --------------
+    // reduce-scatter over the groups: lane (g, li) ends with dimensions li 8 + g4 2 + {0, 1} (head_dim 128),
+    // or, the two halves of a 16-lane row being groups of their own, with the one of them that is c16 / 8
     float r0, r1;
     {
       float x, y, h[4];
@@ -693,15 +748,35 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(1, U ==
       r1 = x + y;
     }
     const float l_w = rows_sum(group_sum<16>(l_lane));
-    *reinterpret_cast<f32x2*>(&sm_o[wave][0][li * 8 + g * 2]) = f32x2{r0, r1};
+    if constexpr (LPR == 16) {
+      *reinterpret_cast<f32x2*>(state(wave, 0, li * 8 + g4 * 2)) = f32x2{r0, r1};
+    } else {
+      const bool odd = c16 >= 8;
+      *state(wave, 0, li * 8 + g4 * 2 + (c16 >> 3)) = (odd ? r1 : r0) + dpp_move<0x128>(odd ? r0 : r1);
+    }
     if (lane == 0) {
       sm_ml[wave][0][0] = m_run;
       sm_ml[wave][0][1] = l_w;
     }
   }
-  // ---- the waves of the workgroup meet in LDS; wave j carries on alone with head j --------------
+  // ---- the waves of the workgroup meet in LDS; wave j carries on alone with the heads j, j + NW ------
+  constexpr int HW = (QPG + NW - 1) / NW;  // heads of a wave
+  uint32_t* out[HW];                       // where they go, before the barrier
+  float* lse_out[HW];
+  int64_t part[HW];
+#pragma unroll
+  for (int x = 0; x < HW; ++x) {
+    const int j = wave + x * NW;
+    out[x] = reinterpret_cast<uint32_t*>(p.o) + ((int64_t)b * p.num_qo_heads + rq0 + j) * (D / 2) + lane;
+    lse_out[x] = p.lse ? p.lse + (int64_t)b * p.num_qo_heads + rq0 + j : nullptr;
+    part[x] = ((int64_t)b * p.vheads + hrow * QPG + j) * p.max_splits;
+  }
+  int32_t* const tickets = p.ws_cnt + (((int64_t)b * gridDim.x + hrow) * QPG + wave) * p.ticket_stride;
   __syncthreads();
-  for (int j = wave; j < QPG; j += NW) {
+#pragma unroll
+  for (int x = 0; x < HW; ++x) {
+    const int j = wave + x * NW;
+    if (j >= gsz) break;
     float M = kNegBig;
 #pragma unroll
     for (int w = 0; w < NW; ++w) M = fmaxf(M, sm_ml[w][j][0]);
@@ -710,16 +785,23 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(1, U ==
     for (int w = 0; w < NW; ++w) {
       const float f = fast_exp2(sm_ml[w][j][0] - M);
       L = fmaf(sm_ml[w][j][1], f, L);
-      const f32x2 v = *reinterpret_cast<const f32x2*>(&sm_o[w][j][2 * lane]);
+      const f32x2 v = *reinterpret_cast<const f32x2*>(state(w, j, 2 * (lane & (D / 2 - 1))));
       o0 = fmaf(v.x, f, o0);
       o1 = fmaf(v.y, f, o1);
     }
-    const int qh = rq0 + j;
-    uint32_t* o32 = reinterpret_cast<uint32_t*>(p.o) + ((int64_t)b * p.num_qo_heads + qh) * (D / 2) + lane;
-    float* lse_out = p.lse ? p.lse + (int64_t)b * p.num_qo_heads + qh : nullptr;
-    const int64_t part0 = ((int64_t)b * p.vheads + qh) * p.max_splits;
-    int32_t* ticket = p.ws_cnt + (((int64_t)b * gridDim.x + hrow) * QPG + j) * p.ticket_stride;
-    finish_head<T>(p, lane, n_splits, split, part0, ticket, o32, lse_out, o0, o1, M, L);
+    publish_head<T, D>(p, lane, n_splits, part[x] + split, out[x], lse_out[x], o0, o1, M, L);
+  }
+  // (without a merge here a second launch, merge_partials_kernel, reduces the partials)
+  if (n_splits == 1 || !p.fused_merge || wave >= gsz) return;
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  int tk = 0;  // lane x: the ticket of head wave + x NW (eight heads by four waves: 28/4 heads, lists of 1024 8.7 -> 7.6 us)
+  if (lane < HW && wave + lane * NW < gsz)
+    tk = __hip_atomic_fetch_add(tickets + (HW > 1 ? lane * NW * p.ticket_stride : 0), 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+  for (int x = 0; x < HW; ++x) {
+    const int j = wave + x * NW;
+    if (j < gsz && __builtin_amdgcn_readlane(tk, x) == n_splits - 1)
+      merge_head<T, D>(p, lane, n_splits, part[x], tickets + x * NW * p.ticket_stride, out[x], lse_out[x]);
   }
 }
 
@@ -732,8 +814,26 @@ static bool sparse_shape_supported(int nw, int rows, int qpg = 1) {
 
 // `wide`: 64-bit row offsets and pages of any size (8 rows per lane only)
 template <typename T>
-static int launch_sparse(const DecodeParams& p, int nw, int rows, bool probe, bool wide, dim3 grid,
+static int launch_sparse(const DecodeParams& p, int head_dim, int nw, int rows, bool probe, bool wide, dim3 grid,
                          hipStream_t st) {
+  const bool any = p.list_shift > 0 || p.scores;
+#define TD_SPARSE_CASE(N_, D_, ANY_)                                                                               \
+  if (nw == N_ && rows == 8 && head_dim == D_ && any == ANY_ && !wide && !probe && (D_ == 64 || ANY_)) {           \
+    if (p.fresh_k)                                                                                                 \
+      hipLaunchKernelGGL((sparse_attn_kernel<T, N_, 8, true, false, 1, false, D_, ANY_>), grid, dim3(N_ * 64), 0,  \
+                         st, p);                                                                                   \
+    else                                                                                                           \
+      hipLaunchKernelGGL((sparse_attn_kernel<T, N_, 8, false, false, 1, false, D_, ANY_>), grid, dim3(N_ * 64), 0, \
+                         st, p);                                                                                   \
+    return TD_OK;                                                                                                  \
+  }
+  TD_SPARSE_CASE(4, 64, false)
+  TD_SPARSE_CASE(8, 64, false)
+  TD_SPARSE_CASE(4, 64, true)
+  TD_SPARSE_CASE(8, 64, true)
+  TD_SPARSE_CASE(4, 128, true)
+  TD_SPARSE_CASE(8, 128, true)
+#undef TD_SPARSE_CASE
 #define TD_SPARSE_CASE(N_, U_)                                                                   \
   if (nw == N_ && rows == U_ && !wide) {                                                         \
     if (probe)                                                                                   \
@@ -772,29 +872,40 @@ static int launch_sparse(const DecodeParams& p, int nw, int rows, bool probe, bo
 
 // shared KV rows: QPG query heads per list walk
 template <typename T>
-static int launch_sparse_shared(const DecodeParams& p, int nw, int qpg, bool wide, dim3 grid, hipStream_t st) {
-#define TD_SPARSE_CASE(N_, Q_, W_)                                                                  \
-  if (nw == N_ && qpg == Q_ && wide == W_) {                                                        \
-    if (p.fresh_k)                                                                                  \
-      hipLaunchKernelGGL((sparse_attn_kernel<T, N_, 8, true, false, Q_, W_>), grid, dim3(N_ * 64),  \
-                         0, st, p);                                                                 \
-    else                                                                                            \
-      hipLaunchKernelGGL((sparse_attn_kernel<T, N_, 8, false, false, Q_, W_>), grid, dim3(N_ * 64), \
-                         0, st, p);                                                                 \
-    return TD_OK;                                                                                   \
+static int launch_sparse_shared(const DecodeParams& p, int head_dim, int nw, int qpg, bool wide, dim3 grid,
+                                hipStream_t st) {
+  const bool any = p.list_shift > 0 || p.scores;
+#define TD_SPARSE_CASE(Q_, W_, D_, ANY_)                                                                    \
+  if (qpg == Q_ && wide == W_ && head_dim == D_ && any == ANY_) {                                           \
+    if (nw == 4 && p.fresh_k)                                                                               \
+      hipLaunchKernelGGL((sparse_attn_kernel<T, 4, 8, true, false, Q_, W_, D_, ANY_>), grid, dim3(256), 0,  \
+                         st, p);                                                                            \
+    else if (nw == 4)                                                                                       \
+      hipLaunchKernelGGL((sparse_attn_kernel<T, 4, 8, false, false, Q_, W_, D_, ANY_>), grid, dim3(256), 0, \
+                         st, p);                                                                            \
+    else if (p.fresh_k)                                                                                     \
+      hipLaunchKernelGGL((sparse_attn_kernel<T, 8, 8, true, false, Q_, W_, D_, ANY_>), grid, dim3(512), 0,  \
+                         st, p);                                                                            \
+    else                                                                                                    \
+      hipLaunchKernelGGL((sparse_attn_kernel<T, 8, 8, false, false, Q_, W_, D_, ANY_>), grid, dim3(512), 0, \
+                         st, p);                                                                            \
+    return TD_OK;                                                                                           \
   }
-  TD_SPARSE_CASE(4, 2, false)
-  TD_SPARSE_CASE(4, 4, false)
-  TD_SPARSE_CASE(4, 8, false)
-  TD_SPARSE_CASE(8, 2, false)
-  TD_SPARSE_CASE(8, 4, false)
-  TD_SPARSE_CASE(8, 8, false)
-  TD_SPARSE_CASE(4, 2, true)
-  TD_SPARSE_CASE(4, 4, true)
-  TD_SPARSE_CASE(4, 8, true)
-  TD_SPARSE_CASE(8, 2, true)
-  TD_SPARSE_CASE(8, 4, true)
-  TD_SPARSE_CASE(8, 8, true)
+  TD_SPARSE_CASE(2, false, 128, false)
+  TD_SPARSE_CASE(4, false, 128, false)
+  TD_SPARSE_CASE(8, false, 128, false)
+  TD_SPARSE_CASE(2, true, 128, false)
+  TD_SPARSE_CASE(4, true, 128, false)
+  TD_SPARSE_CASE(8, true, 128, false)
+  TD_SPARSE_CASE(2, false, 64, false)
+  TD_SPARSE_CASE(4, false, 64, false)
+  TD_SPARSE_CASE(8, false, 64, false)
+  TD_SPARSE_CASE(2, false, 128, true)
+  TD_SPARSE_CASE(4, false, 128, true)
+  TD_SPARSE_CASE(8, false, 128, true)
+  TD_SPARSE_CASE(2, false, 64, true)
+  TD_SPARSE_CASE(4, false, 64, true)
+  TD_SPARSE_CASE(8, false, 64, true)
 #undef TD_SPARSE_CASE
   return fail(TD_ERR_UNSUPPORTED,
               "sparse decode attention: no kernel for %d waves with %d query heads per shared row", nw, qpg);
@@ -802,13 +913,13 @@ static int launch_sparse_shared(const DecodeParams& p, int nw, int qpg, bool wid
 
 // Launches the sparse-layer kernel (and, when the plan asks for it, the second-launch merge);
 // defined once per element type (and once more for shared KV rows) in sparse_attn_*.hip.
-int launch_sparse_f16(const DecodeParams& p, int nw, int rows, bool probe, bool wide, bool merge_kernel,
+int launch_sparse_f16(const DecodeParams& p, int head_dim, int nw, int rows, bool probe, bool wide, bool merge_kernel,
                       dim3 grid, hipStream_t st);
-int launch_sparse_bf16(const DecodeParams& p, int nw, int rows, bool probe, bool wide, bool merge_kernel,
+int launch_sparse_bf16(const DecodeParams& p, int head_dim, int nw, int rows, bool probe, bool wide, bool merge_kernel,
                        dim3 grid, hipStream_t st);
-int launch_sparse_shared_f16(const DecodeParams& p, int nw, int qpg, bool wide, bool merge_kernel, dim3 grid,
+int launch_sparse_shared_f16(const DecodeParams& p, int head_dim, int nw, int qpg, bool wide, bool merge_kernel, dim3 grid,
                              hipStream_t st);
-int launch_sparse_shared_bf16(const DecodeParams& p, int nw, int qpg, bool wide, bool merge_kernel, dim3 grid,
+int launch_sparse_shared_bf16(const DecodeParams& p, int head_dim, int nw, int qpg, bool wide, bool merge_kernel, dim3 grid,
                               hipStream_t st);
 
 }  // namespace tidal

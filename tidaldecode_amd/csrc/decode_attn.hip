@@ -190,6 +190,8 @@ extern "C" int td_decode_make_plan(int32_t batch, int32_t num_qo_heads, int32_t 
               best = cost;
               sw = nw;
               chunk = (int64_t)tiles * stile;
+            } else if (cost > best + 3.f && rows_all * splits <= num_cus()) {
+              break;  // longer walks on fewer compute units: no merge costs that much
             }
           }
           if (tiles == most) break;

@@ -148,6 +148,10 @@ __device__ __forceinline__ void scalar_load4(const int32_t* a0, const int32_t* a
       : "memory");
 }
 
+__device__ __forceinline__ const float* bytes_on(const float* base, uint32_t bytes) {
+  return reinterpret_cast<const float*>(reinterpret_cast<const char*>(base) + bytes);
+}
+
 // The tail of a head's computation, run by ONE wave that holds the workgroup's partial result of that head (lane:
 // dimensions 2 lane, 2 lane + 1; M, L uniform): publish_head writes the result if the head was not split, else the
 // partial; after the ticket merge_head, in the last of the splits to arrive, merges all partials.
@@ -188,14 +192,13 @@ __device__ __forceinline__ void merge_head(const DecodeParams& p, int lane, int 
   }
   constexpr int PRE = 16;  // partial loads in flight
   float pa[PRE], pb[PRE];
-  // 32-bit offsets from one scalar base: the loads go out two instructions apart instead of five
-  const char* const partials = reinterpret_cast<const char*>(p.ws_o + part0 * D);
+  // 32-bit byte offsets from one scalar base: the loads go out two instructions apart instead of five
   const uint32_t mine = 8u * (uint32_t)(lane & (D / 2 - 1)), last = (uint32_t)(n_splits - 1) * (D * 4);
   auto issue = [&](int base) {
 #pragma unroll
     for (int u = 0; u < PRE; ++u) {
       const uint32_t at = (uint32_t)(base + u) * (D * 4);
-      load_coherent(reinterpret_cast<const float*>(partials + ((at < last ? at : last) + mine)), pa[u], pb[u]);
+      load_coherent(bytes_on(p.ws_o + part0 * D, (at < last ? at : last) + mine), pa[u], pb[u]);
     }
   };
   issue(0);
@@ -244,7 +247,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(1, U ==
   TD_TOUCH(p.idx_row_stride); TD_TOUCH(p.idx_cols); TD_TOUCH(p.n_list_host); TD_TOUCH(p.kv_magic);
   TD_TOUCH(p.chunk_magic); TD_TOUCH(p.max_splits); TD_TOUCH(p.page_shift); TD_TOUCH(p.max_slot);
   TD_TOUCH(p.page_stride_b); TD_TOUCH(p.entry_stride_b); TD_TOUCH(p.head_stride);
-  TD_TOUCH(p.ws_o); TD_TOUCH(p.ws_ml); TD_TOUCH(p.ws_cnt); TD_TOUCH(p.o); TD_TOUCH(p.lse); TD_TOUCH(p.vheads);
+  TD_TOUCH(p.ws_cnt); TD_TOUCH(p.o); TD_TOUCH(p.lse); TD_TOUCH(p.vheads);
   TD_TOUCH(p.ticket_stride); TD_TOUCH(p.fused_merge);
   TD_TOUCH(p.last_len); TD_TOUCH(p.last_idx); TD_TOUCH(p.scale_log2); TD_TOUCH(p.num_qo_heads);
   if constexpr (FRESH) {

@@ -444,7 +444,7 @@ def _append(k, v, kv_data, kv_indices, kv_indptr, kv_last_page_len, metadata_dat
             metadata_indices, metadata_indptr, metadata_last_page_len, layout, decode: bool):
     if k.is_cuda and host_calls.append(k, v, kv_data, kv_indices, kv_indptr, kv_last_page_len, metadata_data,
                                        metadata_indices, metadata_indptr, metadata_last_page_len, layout, decode,
-                                       _stream()):
+                                       _stream(), -1):
         return
     # checks of tidal/ops/csrc/page.cu:19-55
     for t, n in ((k, "k"), (v, "v"), (kv_indices, "kv_indices")):
@@ -622,8 +622,8 @@ def prefill_with_paged_kv_cache(q, kv_data, kv_indices, kv_last_page_len, causal
     and ``rope_theta`` are accepted for signature parity: RoPE is applied before the cache is
     written (RotaryMode::kNone in the reference's call, batch_prefill.cu:95)."""
     if q.is_cuda:
-        o = torch.empty_like(q)
-        if host_calls.prefill(q, o, kv_data, kv_indices, kv_last_page_len, causal, layout, _stream()):
+        o = host_calls.prefill(q, kv_data, kv_indices, kv_last_page_len, causal, layout, _stream(), -1)
+        if o is not False:
             return o
     _check_input(q, "q")
     _check_dim(3, q, "q")
@@ -635,6 +635,7 @@ def prefill_with_paged_kv_cache(q, kv_data, kv_indices, kv_last_page_len, causal
     if q.size(2) != pool.head_dim or q.dtype != kv_data.dtype:
         raise RuntimeError("prefill_with_paged_kv_cache: q does not fit the cache")
     causal = int(bool(causal))
+    o = torch.empty_like(q)
     # scratch of this call alone (torch's allocator hands it out again in stream order)
     ws_bytes = lib.td_prefill_workspace_bytes(pool, kv_len, q.size(0), q.size(1), causal)
     ws = None

@@ -434,13 +434,14 @@ bool rope_in_place_regular(PyObject* const* a, int& rc) {
 }
 
 // _append: (k, v, kv_data, kv_indices, kv_indptr, kv_last_page_len, metadata_data, metadata_indices, metadata_indptr,
-// metadata_last_page_len, layout, decode, stream)
+// metadata_last_page_len, layout, decode, stream, layer: that of kv_data's pools of all layers, or -1)
 bool append_regular(PyObject* const* a, int& rc) {
   const at::Tensor *k = tensor(a[0]), *v = tensor(a[1]), *kv = tensor(a[2]), *idx = tensor(a[3]), *indptr = tensor(a[4]);
-  int64_t last, layout, meta_last = 0;
+  int64_t last, layout, layer, meta_last = 0;
   td_paged_kv pool, meta_pool, *meta = nullptr;
   if (!dense(k, 3) || !dense(v, 3) || !dense(idx, 1) || !i32(idx) || !indptr || !i32(indptr) ||
-      !integer(a[5], INT32_MIN, INT32_MAX, last) || !integer(a[10], 0, 1, layout) || !pool_of(kv, layout, pool))
+      !integer(a[5], INT32_MIN, INT32_MAX, last) || !integer(a[10], 0, 1, layout) ||
+      !integer(a[13], -1, INT32_MAX, layer) || !pool_of(kv, layout, pool, layer))
     return false;
   if ((a[11] == Py_True && k->size(0) != 1) || k->sizes() != v->sizes() || k->scalar_type() != v->scalar_type() ||
       pool.num_kv_heads != k->size(1) || pool.head_dim != k->size(2) || kv->scalar_type() != k->scalar_type())
@@ -461,22 +462,31 @@ bool append_regular(PyObject* const* a, int& rc) {
   return true;
 }
 
-// prefill_with_paged_kv_cache: (q, o, kv_data, kv_indices, kv_last_page_len, causal, layout, stream); a plan that
-// wants scratch is the caller's
-bool prefill_regular(PyObject* const* a, int& rc) {
-  const at::Tensor *q = tensor(a[0]), *o = tensor(a[1]), *kv = tensor(a[2]), *idx = tensor(a[3]);
-  int64_t last, layout;
+// prefill_with_paged_kv_cache: (q, kv_data, kv_indices, kv_last_page_len, causal, layout, stream, layer: that of
+// kv_data's pools of all layers, or -1); the output and the scratch of this call alone are allocated here
+bool prefill_regular(PyObject* const* a, at::Tensor& o, int& rc) {
+  const at::Tensor *q = tensor(a[0]), *kv = tensor(a[1]), *idx = tensor(a[2]);
+  int64_t last, layout, layer;
   td_paged_kv pool;
-  if (!dense(q, 3) || !dense(o, 3) || !dense(idx) || !i32(idx) || !integer(a[4], INT32_MIN, INT32_MAX, last) ||
-      !PyBool_Check(a[5]) || !integer(a[6], 0, 1, layout) || !pool_of(kv, layout, pool))
+  if (!dense(q, 3) || !dense(idx) || !i32(idx) || !integer(a[3], INT32_MIN, INT32_MAX, last) || !PyBool_Check(a[4]) ||
+      !integer(a[5], 0, 1, layout) || !integer(a[7], -1, INT32_MAX, layer) || !pool_of(kv, layout, pool, layer))
     return false;
   const int64_t n_pages = idx->numel(), kv_len = (n_pages - 1) * pool.page_size + last;
-  const int causal = a[5] == Py_True;
+  const int causal = a[4] == Py_True;
   if (q->size(2) != pool.head_dim || q->scalar_type() != kv->scalar_type() || kv_len < 0 || kv_len > INT32_MAX) return false;
-  if (lib.prefill_workspace_bytes(&pool, (int32_t)kv_len, (int32_t)q->size(0), (int32_t)q->size(1), causal) != 0) return false;
+  o = at::empty_like(*q);
+  int64_t bytes = lib.prefill_workspace_bytes(&pool, (int32_t)kv_len, (int32_t)q->size(0), (int32_t)q->size(1), causal);
+  at::Tensor scratch;  // (torch's allocator hands it out again in stream order)
+  if (bytes > 0) {
+    try {
+      scratch = at::empty({bytes}, q->options().dtype(at::kByte));
+    } catch (const c10::OutOfMemoryError&) {  // slower without, but a call needs none
+      bytes = 0;
+    }
+  }
   rc = unlocked(lib.prefill_attn_split, &pool, ptr_as<int32_t>(*idx), (int32_t)n_pages, (int32_t)kv_len, ptr(*q),
-                ptr(*o), (int32_t)q->size(0), (int32_t)q->size(1), (float)(1.0 / std::sqrt((double)pool.head_dim)),
-                causal, nullptr, 0, stream_of(a[7]));
+                ptr(o), (int32_t)q->size(0), (int32_t)q->size(1), (float)(1.0 / std::sqrt((double)pool.head_dim)),
+                causal, bytes > 0 ? ptr(scratch) : nullptr, bytes, stream_of(a[6]));
   return true;
 }
 
@@ -566,10 +576,11 @@ PyObject* entry(PyObject*, PyObject* const* args, Py_ssize_t n) {
   if (!takes(n, N)) return nullptr;
   return outcome([&](int& rc) { return F(args, rc); }, [] { Py_RETURN_TRUE; });
 }
-PyObject* attend(PyObject*, PyObject* const* args, Py_ssize_t n) {
-  if (!takes(n, 16)) return nullptr;
+template <bool (*F)(PyObject* const*, at::Tensor&, int&), int N>
+PyObject* maker(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  if (!takes(n, N)) return nullptr;
   at::Tensor o;
-  return outcome([&](int& rc) { return attend_regular(args, o, rc); }, [&] { return THPVariable_Wrap(std::move(o)); });
+  return outcome([&](int& rc) { return F(args, o, rc); }, [&] { return THPVariable_Wrap(std::move(o)); });
 }
 PyObject* rope_table(PyObject*, PyObject* const* args, Py_ssize_t n) {
   if (!takes(n, 5)) return nullptr;
@@ -585,15 +596,16 @@ PyObject* rope_table(PyObject*, PyObject* const* args, Py_ssize_t n) {
 }
 
 #define TD_ENTRY(name, fn, n) {name, (PyCFunction)(void (*)(void))(entry<fn, n>), METH_FASTCALL, nullptr}
+#define TD_MAKER(name, fn, n) {name, (PyCFunction)(void (*)(void))(maker<fn, n>), METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {
     {"bind", bind, METH_O, "addresses of libtidal_hip.so's entry points by name"},
     TD_ENTRY("forward", forward_regular, 15),
     TD_ENTRY("topk", topk_regular, 13),
-    {"attend", (PyCFunction)(void (*)(void))attend, METH_FASTCALL, nullptr},
+    TD_MAKER("attend", attend_regular, 16),
     {"rope_table", (PyCFunction)(void (*)(void))rope_table, METH_FASTCALL, nullptr},
     TD_ENTRY("rope_in_place", rope_in_place_regular, 6),
-    TD_ENTRY("append", append_regular, 13),
-    TD_ENTRY("prefill", prefill_regular, 8),
+    TD_ENTRY("append", append_regular, 14),
+    TD_MAKER("prefill", prefill_regular, 8),
     TD_ENTRY("gemv", gemv_regular, 9),
     TD_ENTRY("score_reduce", score_reduce_regular, 7),
     TD_ENTRY("estimate", estimate_regular, 7),

@@ -60,6 +60,11 @@ def _meta_args(iController: InferenceController, layer_idx: int):
 def append_kv(k: torch.Tensor, v: torch.Tensor, iController: InferenceController, layer_idx: int):
     """Append the new k/v ``[N, H_kv, D]`` to the paged cache of a layer (prefill for N > 1,
     decode for N == 1)."""
+    c, cache = iController, iController.kv_cache
+    if k.is_cuda and c.metadata_cache is None and host_calls.append(
+            k, v, cache.pool.buf, c.kv_indices_with_last, c.kv_indptr_for_append, cache.last_page_len, None, None, None,
+            0, c.layout, k.size(0) <= 1, _kernels._stream(), layer_idx % cache.pool.num_layers):
+        return
     fn = _kernels.append_kv_cache_prefill if k.size(0) > 1 else _kernels.append_kv_cache_decode
     fn(k, v, iController.kv_cache.buf_layer(layer_idx), iController.kv_indices_with_last,
        iController.kv_indptr_for_append, iController.kv_cache.last_page_len,
@@ -81,6 +86,12 @@ def prefill_forward(q: torch.Tensor, iController: InferenceController, layer_idx
                     rope_scale: Optional[float] = None, rope_theta: Optional[float] = None
                     ) -> torch.Tensor:
     """Causal attention of the new tokens over the cache (K/V already appended)."""
+    if q.is_cuda:
+        c, cache = iController, iController.kv_cache
+        o = host_calls.prefill(q, cache.pool.buf, c.kv_indices_with_last, cache.last_page_len, True, c.layout,
+                               _kernels._stream(), layer_idx % cache.pool.num_layers)
+        if o is not False:
+            return o
     return _kernels.prefill_with_paged_kv_cache(
         q, iController.kv_cache.buf_layer(layer_idx), iController.kv_indices_with_last,
         iController.kv_cache.last_page_len, True, iController.layout, False,

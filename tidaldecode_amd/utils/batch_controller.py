@@ -26,6 +26,7 @@ from typing import List, Optional, Sequence
 import torch
 
 from .. import _kernels, _lib
+from .._lib import TD_REDUCE_GROUP_SUM, host_calls
 from .controller import _logits_dtype
 from .paged import BatchDecodeWithPagedKVCacheWrapper, KvPool, TensorLayout
 
@@ -97,6 +98,7 @@ class BatchInferenceController:
         self._list_starts = torch.arange(max_batch + 1, **i32) * self.budget
         self.topk_buf = torch.zeros(_kernels.topk_workspace_bytes(max_batch * self.index_rows),
                                     dtype=torch.uint8, device=device)
+        self._view_base = self._view = self._view_batch = None
         self._handle = BatchDecodeWithPagedKVCacheWrapper(kv_layout=kv_layout)
         self._handle.begin_forward(None, num_heads, num_kv_heads, head_dim, page_size, dtype)
         layer_bytes = self.pool.buf[0].numel() * self.pool.buf.element_size()
@@ -255,6 +257,23 @@ class BatchInferenceController:
     def _row(self, r: int) -> torch.Tensor:
         return self._meta[r, : self.batch]
 
+    def _views(self) -> dict:
+        """The slices of the controller's tensors that every layer of a step takes, made once per batch size (a
+        slice costs the host 1 us, a layer took nine)."""
+        base, of = (self.qk_product, self.lse, self.page_table, self._meta, self.score_sum), self._view_base
+        if of is None or self._view_batch != self.batch or any(a is not b for a, b in zip(base, of)):
+            B, rows = self.batch, self.batch * self.index_rows
+            self._view = dict(
+                tables=self.page_table[:B], table_row=self.page_table.view(1, -1), starts=self._table_starts[: B + 1],
+                list_starts=self._list_starts[: B + 1], qk=self.qk_product[: B * self.num_heads], lse=self.lse[:B],
+                bound=self.lse[:B].view(-1), last_len=self._row(_LAST_LEN), last_idx=self._row(_LAST_IDX),
+                before=self._row(_PAGES_BEFORE_LAST), selected=self._row(_SELECTED), slots=self._row(_DST_SLOT),
+                seq_len=self._row(_SEQ_LEN), positions=self._row(_POSITION))
+            if self.score_sum is not None:
+                self._view.update(sums=self.score_sum[:rows], sum_bound=self.score_bound[:rows])
+            self._view_base, self._view_batch = base, self.batch
+        return self._view
+
     @property
     def positions(self) -> torch.Tensor:
         return self._row(_POSITION)
@@ -269,7 +288,7 @@ class BatchInferenceController:
 
     def rope_table(self, rope_scale: float = 1.0, rope_theta: float = 1e4):
         """cos, sin ``[B, D/2]`` of the new tokens' positions (once per step, all layers)."""
-        return _kernels.rope_table(self.positions, self.head_dim, rope_scale, rope_theta)
+        return _kernels.rope_table(self._views()["positions"], self.head_dim, rope_scale, rope_theta)
 
     # ---- cache writes -------------------------------------------------------------------------
     def append_prompt(self, b: int, k: torch.Tensor, v: torch.Tensor, layer_idx: int) -> None:
@@ -293,22 +312,25 @@ class BatchInferenceController:
         if fresh is None:
             return None
         k, v, cos, sin = fresh
-        return (k, v, cos, sin, self.dst_slots)
+        return (k, v, cos, sin, self._views()["slots"])
 
     def attend_full(self, q: torch.Tensor, layer_idx: int, output_qk_product: bool = False,
                     fresh=None) -> torch.Tensor:
         """Attention of every sequence's new token over its whole cache; with
         ``output_qk_product`` the logits and log-sum-exps are kept for ``select``.
         ``fresh=(k, v, cos, sin)`` folds RoPE and the append of the new tokens into the launch."""
-        B = self.batch
+        w, pool, fresh = self._views(), self.pool, self._fresh(fresh)
+        scores, lse = (w["qk"], w["lse"]) if output_qk_product else (None, None)
+        n_list = -(-max(self._cap) // self.page_size) - 1
+        if q.is_cuda:
+            o = host_calls.attend(self._handle._wrapper, q, None, pool.buf, w["table_row"], w["starts"], w["last_len"],
+                                  w["last_idx"], scores, False, lse, n_list, fresh, w["before"], _kernels._stream(),
+                                  layer_idx % pool.num_layers)
+            if o is not False:
+                return o
         o = torch.empty_like(q)
-        self._handle.forward(
-            q, o, self.buf_layer(layer_idx), self.page_table.view(1, -1),
-            self._table_starts[: B + 1], self._row(_LAST_LEN), self._row(_LAST_IDX),
-            self.qk_product[: B * self.num_heads] if output_qk_product else None,
-            lse=self.lse[:B] if output_qk_product else None,
-            n_list=-(-max(self._cap) // self.page_size) - 1, counts=self._row(_PAGES_BEFORE_LAST),
-            fresh=self._fresh(fresh))
+        self._handle.forward(q, o, self.buf_layer(layer_idx), w["table_row"], w["starts"], w["last_len"], w["last_idx"],
+                             scores, lse=lse, n_list=n_list, counts=w["before"], fresh=fresh)
         return o
 
     def select(self) -> None:
@@ -316,27 +338,36 @@ class BatchInferenceController:
         physical token slots, sorted by position, in its segment of ``topk_dindices_buffer``."""
         B, P, k = self.batch, self.page_size, self.budget
         n = max(self._cap)   # an upper bound; every sequence's own length is read on the device
-        rows = self.index_rows
-        scores, bound = self.qk_product[: B * self.num_heads], self.lse[:B].view(-1)
+        rows, w = self.index_rows, self._views()
+        scores, bound = w["qk"], w["bound"]
         if self.select_mode != "per_head":
             # the B * H_q logit rows form B * rows groups of consecutive heads: one grouped sum
-            _kernels.score_reduce(scores, self.lse[:B].view(-1), B * rows, n, "group_sum",
-                                  out=self.score_sum[: B * rows])
-            scores, bound = self.score_sum[: B * rows], self.score_bound[: B * rows]
+            if not (scores.is_cuda and host_calls.score_reduce(scores, bound, B * rows, n, TD_REDUCE_GROUP_SUM, w["sums"],
+                                                               _kernels._stream())):
+                _kernels.score_reduce(scores, bound, B * rows, n, "group_sum", out=w["sums"])
+            scores, bound = w["sums"], w["sum_bound"]
         k_eff = min(k, n)
         # one call: row b * rows + r is row r of sequence b, ranks that sequence's tokens only
         # (its length is read on the device) and goes through that sequence's page table
         # and lands in that sequence's segment of list row r
+        if scores.is_cuda and host_calls.topk(scores, None, None, self.topk_dindices_buffer, self.topk_buf, k_eff,
+                                              w["tables"], P, w["seq_len"], bound, k, _kernels._stream(), n):
+            return
         _kernels.topk_filtering(scores[:, :n], None, None, self.topk_dindices_buffer, self.topk_buf, k_eff,
-                                page_table=self.page_table[:B], page_size=P,
-                                lengths=self._row(_SEQ_LEN), upper_bound=bound, segment=k)
+                                page_table=w["tables"], page_size=P,
+                                lengths=w["seq_len"], upper_bound=bound, segment=k)
 
     def attend_sparse(self, q: torch.Tensor, layer_idx: int, fresh=None) -> torch.Tensor:
         """Attention over the persisted token lists (``fresh`` as in ``attend_full``)."""
-        B = self.batch
+        w, pool, fresh = self._views(), self.pool, self._fresh(fresh)
+        n_list = min(self.budget, max(self._cap))
+        if q.is_cuda:
+            o = host_calls.attend(self._handle._wrapper, q, None, pool.buf, self.topk_dindices_buffer, w["list_starts"], 0,
+                                  0, None, True, None, n_list, fresh, w["selected"], _kernels._stream(),
+                                  layer_idx % pool.num_layers)
+            if o is not False:
+                return o
         o = torch.empty_like(q)
-        self._handle.forward(q, o, self.buf_layer(layer_idx), self.topk_dindices_buffer,
-                             self._list_starts[: B + 1], 0, 0, None, index_kind="slots",
-                             n_list=min(self.budget, max(self._cap)), counts=self.selected,
-                             fresh=self._fresh(fresh))
+        self._handle.forward(q, o, self.buf_layer(layer_idx), self.topk_dindices_buffer, w["list_starts"], 0, 0, None,
+                             index_kind="slots", n_list=n_list, counts=w["selected"], fresh=fresh)
         return o

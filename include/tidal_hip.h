@@ -476,6 +476,10 @@ int td_rope_append_prompt(const td_paged_kv* kv, const void* qkv, int64_t qkv_st
  * multiple of 4) and many rows; rows of out lie out_stride elements apart; k: a multiple of 64. */
 int td_gemm_strip(const void* x, const void* w, void* out, int32_t m, int32_t n, int32_t k, int64_t out_stride,
                   int32_t dtype, void* stream);
+/* out [m, n] = x [m, k] w [n, k]^T for the few rows of a short prompt, n a multiple of 64, k of 128.  splits > 1 cuts
+ * k; parts then holds splits * m * n floats (16-byte aligned), free again when the call's work is done. */
+int td_gemm_rows(const void* x, const void* w, void* out, int32_t m, int32_t n, int32_t k, int32_t splits, void* parts,
+                 int64_t parts_bytes, int32_t dtype, void* stream);
 
 /*
  * Measurement aid without a counterpart in the reference: the memory side of a sparse layer

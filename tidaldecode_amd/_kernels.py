@@ -149,18 +149,37 @@ def _cut_columns(m: int, n: int, k: int) -> int:
     return 256
 
 
+def _row_splits(m: int, n: int, k: int) -> int:
+    """Cuts of the inner dimension with which td_gemm_rows takes a product [m, k] x [n, k]^T, 0: the library's.  One
+    tile of rows, few enough columns that the library leaves the chip idle, workgroups for all 256 compute units
+    with eight steps of 128 each (measured at the kernel; 80 rows of 6144 columns are where it draws level)."""
+    if not 17 <= m <= 144 or n > 8192 or n % 64 or k % 128 or k < 2048 or k > 1 << 20 or (n > 4096 and m <= 80):
+        return 0
+    splits = min(256 // (n // 64), k // 1024, 8)
+    return splits if splits > 1 else 0
+
+
 def prompt_product(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     """Extension: ``x @ weight.t()`` of a prompt's rows x ``[n, K]`` and a weight ``[N, K]`` (inference only)."""
-    cut = _cut_columns(x.size(0), weight.size(0), x.size(1)) if x.dim() == 2 else 0
-    if not (cut and x.is_cuda and x.dtype == weight.dtype and x.dtype in (torch.float16, torch.bfloat16) and
-            x.is_contiguous() and weight.is_contiguous() and (x.data_ptr() | weight.data_ptr()) % 16 == 0 and
-            not torch.is_grad_enabled()):
+    cut = splits = 0
+    if x.dim() == 2 and x.is_cuda and x.dtype == weight.dtype and x.dtype in (torch.float16, torch.bfloat16) and \
+            x.is_contiguous() and weight.is_contiguous() and (x.data_ptr() | weight.data_ptr()) % 16 == 0 and \
+            x.size(1) == weight.size(1) and not torch.is_grad_enabled():
+        splits = _row_splits(x.size(0), weight.size(0), x.size(1))
+        cut = 0 if splits else _cut_columns(x.size(0), weight.size(0), x.size(1))
+    if not (cut or splits):
         return x @ weight.t()
-    main = weight.size(0) - cut
     out = torch.empty((x.size(0), weight.size(0)), dtype=x.dtype, device=x.device)
+    code = _dtype_code(x.dtype, "prompt_product")
+    if splits:
+        parts = torch.empty((splits, *out.shape), dtype=torch.float32, device=x.device)
+        check(lib.td_gemm_rows(x.data_ptr(), weight.data_ptr(), out.data_ptr(), *out.shape, x.size(1), splits,
+                               parts.data_ptr(), parts.numel() * 4, code, _stream()))
+        return out
+    main = weight.size(0) - cut
     torch.mm(x, weight[:main].t(), out=out[:, :main])
     check(lib.td_gemm_strip(x.data_ptr(), weight[main:].data_ptr(), out[:, main:].data_ptr(), x.size(0), cut,
-                            x.size(1), out.stride(0), _dtype_code(x.dtype, "prompt_product"), _stream()))
+                            x.size(1), out.stride(0), code, _stream()))
     return out
 
 

@@ -129,7 +129,7 @@ class TidalLlama:
         return tidal_utils.rms_norm_forward(x, weight, self.config.rms_norm_eps)
 
     def _mlp(self, layer, x):
-        return _kernels.silu_mul(_kernels.prompt_product(x, layer["w_gate_up"])) @ layer["w_down"].t()
+        return _kernels.prompt_product(_kernels.silu_mul(_kernels.prompt_product(x, layer["w_gate_up"])), layer["w_down"])
 
     def _qkv(self, layer, h):
         c = self.config
@@ -147,7 +147,7 @@ class TidalLlama:
         c, ctrl = self.config, self.iController
         if ctrl.metadata_cache is None:
             return _kernels.rope_append_prompt(
-                h @ layer["wqkv"].t(), c.num_heads, past, ctrl.kv_cache.buf_layer(idx),
+                _kernels.prompt_product(h, layer["wqkv"]), c.num_heads, past, ctrl.kv_cache.buf_layer(idx),
                 ctrl.kv_indices_with_last, ctrl.kv_indptr_for_append, ctrl.kv_cache.last_page_len,
                 ctrl.layout, c.rope_scale, c.rope_theta)
         q, k, v = self._qkv(layer, h)  # the page bounds come from the append of its own
@@ -173,7 +173,8 @@ class TidalLlama:
                 _kernels.add_rms_norm(x, mlp, layer["ln1"], c.rms_norm_eps)
             q = self._qkv_to_cache(layer, h, idx, past)
             o = tidal_utils.prefill_forward(q, ctrl, idx)
-            h = _kernels.add_rms_norm(x, o.view(n, -1) @ layer["wo"].t(), layer["ln2"], c.rms_norm_eps)
+            h = _kernels.add_rms_norm(x, _kernels.prompt_product(o.view(n, -1), layer["wo"]), layer["ln2"],
+                                      c.rms_norm_eps)
             mlp = self._mlp(layer, h)
         ctrl.end_forward()
         h = self._rms(x[-1:], self.norm) if mlp is None else \

@@ -22,7 +22,7 @@
 // up to 64K of them, and up to eight workgroups share the emission):
 //   32 x 777 -> 256     4.6 (7.3)     256 x 14000 -> 1024  11.1 (15.8)
 //   32 x 4096 -> 256    6.7 (8.3)     256 x 63000 -> 1024  23.3 (58.6)
-//   512 x 8192 -> 512   10.7 (19.5)   256 x 65537 -> 1024  24.4 (120)
+//   512 x 8192 -> 512    9.7 (19.5)   256 x 65537 -> 1024  24.4 (120)
 //   32 x 32769 -> 2048  12.6 (15.9)   8 x 102392 -> 4096   19.5 (28.6: three launches that share a row)
 // Rows of equal scores, and of two values by halves, through the ties' threshold (before that kernel; a selection
 // by one workgroup out of the whole row, whose additions queue up at one address, took 130 and 630 for the second
@@ -99,6 +99,7 @@ __device__ __forceinline__ uint32_t reach16(const typename RowVectors<T>::vec* v
   return mask;
 }
 
+constexpr int kMidLen = 10240;   // longest rows of 512 threads
 constexpr int kFilterRank = 64;  // members of the threshold bin that are ranked in the lanes of a wave
 
 template <int NT, int CAP, int MAXLEN>
@@ -130,15 +131,20 @@ __device__ __forceinline__ void sums_before(const uint32_t* arr, int wave, int l
 }
 
 // CAP: survivors the list holds; CAP >= MAXLEN: any row fits.
+// kMidLen: two workgroups of a compute unit (four waves a SIMD) are worth the 20 bytes that the registers of the
+// ties' way spill: 512 fp32 rows of 8193 -> 512 10.4 us, with one workgroup 14.4.
 template <typename T, int NT, int VPT, int CAP, int MAXLEN>
-__global__ __launch_bounds__(NT) void topk_filter_kernel(const TopkParams p) {
+__global__ __launch_bounds__(NT, MAXLEN == kMidLen ? 4 : 1) void topk_filter_kernel(const TopkParams p) {
   typedef typename ElemOf<T>::type elem_t;
   typedef typename RowVectors<T>::vec vec;
   typedef FilterLds<NT, CAP, MAXLEN> Lds;
   constexpr int NW = NT / 64, CPT = CAP / NT, CHUNK = 4 * NT * VPT;
   constexpr int kBits = NT == 1024 ? 12 : (NT == 512 ? 11 : 10);  // log2 of the bins
   constexpr bool kFits = MAXLEN <= CAP;                 // the list holds any row: no way out needed
+  constexpr bool kTied = !kFits || MAXLEN > 8192;       // many survivors: the ties' threshold
+  constexpr uint32_t kMost = kFits ? 4096u : CAP;       // (a list that long is rows of few distinct values)
   constexpr bool kSampled = MAXLEN > 4 * NT;            // rows may be longer than the sample
+  constexpr bool kTieRank = !std::is_same<T, F32>::value;
   static_assert(CPT >= 4 && 4 * NT == 1 << kBits && (VPT == 4 || VPT == 8), "shapes");
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -392,7 +398,7 @@ __global__ __launch_bounds__(NT) void topk_filter_kernel(const TopkParams p) {
       }
       __syncthreads();
       C = __builtin_amdgcn_readfirstlane(L.n_cand);
-      if (above || (C >= (uint32_t)k && (kFits || C <= (uint32_t)CAP))) break;
+      if (above || (C >= (uint32_t)k && (!kTied || C <= kMost))) break;
       if (C >= (uint32_t)k)
         above = true;
       else
@@ -402,7 +408,7 @@ __global__ __launch_bounds__(NT) void topk_filter_kernel(const TopkParams p) {
       __syncthreads();
       if (tid == 0) L.n_cand = 0;  // (added to again behind the barriers of the next level)
     }
-    if constexpr (!kFits) {
+    if constexpr (kTied) {
       if (__builtin_expect(above && C < (uint32_t)k, 0)) {
         // The list holds what is above the ties, and the ties make up the rest: the first of them by position.
         const float tie_f = key_to_float(tie);
@@ -466,12 +472,20 @@ __global__ __launch_bounds__(NT) void topk_filter_kernel(const TopkParams p) {
         C = CAP + 1u;
       }
       if (__builtin_expect(C > (uint32_t)CAP, 0)) {
-        const int n_runs = (len + kTopkThreads - 1) / kTopkThreads;
-        for (int j_lo = 0; j_lo < n_runs; j_lo += kSliceMaxRuns) {
+        if constexpr (!kFits) {
+          const int n_runs = (len + kTopkThreads - 1) / kTopkThreads;
+          for (int j_lo = 0; j_lo < n_runs; j_lo += kSliceMaxRuns) {
+            __syncthreads();
+            select_slice<T, 0>(p, row, j_lo, kSliceMaxRuns, lds.slice);
+          }
+          return;
+        } else {  // the list holds the whole row
+          for (int i = tid; i < len; i += NT) L.pos[i] = (typename Lds::pos_t)i;
+          for (int i = tid; i < n_words; i += NT) L.bits[i] = 0;
+          C = (uint32_t)len;
+          kbase = kKeyNegInf;
           __syncthreads();
-          select_slice<T, 0>(p, row, j_lo, kSliceMaxRuns, lds.slice);
         }
-        return;
       }
     }
     // ---- 3. the k-th largest of them: the (C - k + 1)-th smallest distance above the floor -----------
@@ -545,7 +559,23 @@ __global__ __launch_bounds__(NT) void topk_filter_kernel(const TopkParams p) {
   each_slot([&](int u) {
     if (x[u] != kNoElement && ((x[u] ^ flip) > (thr ^ flip) || (x[u] == thr && r == ties))) take |= 1u << u;
   });
-  if (r != ties) {  // the first r of the ties
+  if (kTieRank && r != ties && ties <= (uint32_t)kFilterRank) {
+    // the first r of a few ties: their positions against each other in the lanes of every wave (the bitmap below
+    // takes three barriers and two scans more: bf16, 32 x 640 -> 128 5.5 -> 5.1 us; fp32 scores
+    // seldom tie, and the branch costs their rows 0.1)
+    each_slot([&](int u) {
+      if (x[u] == thr) L.hist[1u + atomicAdd(&L.hist[0], 1u)] = (uint32_t)pos[u];  // (zero since the last level)
+    });
+    __syncthreads();
+    const uint32_t mine = lane < (int)ties ? L.hist[1 + lane] : 0u;
+    uint32_t earlier = 0;
+    for (int i = 0; i < (int)ties; ++i) earlier += (uint32_t)__builtin_amdgcn_readlane(mine, i) < mine ? 1u : 0u;
+    const int last = __builtin_ctzll(__ballot(lane < (int)ties && earlier == r - 1u));  // 1 <= r < ties
+    const uint32_t until = __builtin_amdgcn_readlane(mine, last);
+    each_slot([&](int u) {
+      if (x[u] == thr && (uint32_t)pos[u] <= until) take |= 1u << u;
+    });
+  } else if (r != ties) {  // the first r of the ties
     each_slot([&](int u) {
       if (x[u] == thr) atomicOr(&L.bits[pos[u] >> 5], 1u << (pos[u] & 31));
     });
@@ -590,13 +620,19 @@ static bool filter_fits(int len, int k, int threads) {
 // -> 4096 10.2 | 14.3, 16384 -> 2048 10.5 | 10.7, 32768 -> 3072 14.9 | 13.9, 65536 -> 4096 27 | 18; 128 rows 16384
 // -> 2048 1.09 times, -> 3072 0.97 times as fast; 256 rows 12288 -> 3072 1.11, -> 4096 0.93; bf16, 32 rows 8192 ->
 // 512 1.00, 16384 -> 512 0.97, 24576 -> 512 0.99, 32768 -> 1536 1.01, 49152 -> 3072 0.98; 256 rows 12288 -> 2048 1.01.
+// More than 256 rows: a compute unit holds two of the 512-thread workgroups here and one of the slices' 1024: fp32 |
+// bf16, 512 rows 3000 -> 1024 | 15.1 | 10.7, 8192 -> 2048 18.2 | 12.8, 8192 -> 2500 18.3 | 14.1 and 18.6 | 16.2, 5000
+// -> 2500 18.7 | 16.5 and 18.9 | 17.2, 8192 -> 4096 20.9 | 20.7 and 21.3 | 21.7.  bf16 rows of up to kMidLen: 128 rows
+// 8193 -> 512 10.4 | 9.6, 10240 -> 800 10.7 | 10.4, -> 1000 10.7 | 10.8; 256 rows 9000 -> 1500 12.9 | 12.6.
 // Rows of up to 2048 elements gain at any k (bf16 1500 -> 1024, a tie and as many survivors as there can be, 0.96),
 // rows of more than 65536, which the slices read again in every pass, too.
 static bool filter_pays(int len, int k, int rows, bool half) {
   if (len <= 2048 || len > 65536) return true;
   int most;
   if (len <= 8192)
-    most = half ? 600 : 1300;
+    most = rows > 256 ? 2500 : (half ? 600 : 1300);
+  else if (half && len <= kMidLen && rows > 64)
+    most = rows < 256 ? 800 : 1500;
   else if (rows <= 64)
     most = half ? (len - 16384) / 12 : (len < 14400 ? 1600 : len / 9);
   else if (rows < 256)
@@ -608,7 +644,11 @@ static bool filter_pays(int len, int k, int rows, bool half) {
 
 // True: launched.  Threads by row length: the fewer, the cheaper the barriers and scans that make up
 // most of a short row's time; 1024 are needed where the row's elements are (32 x 8192 -> 512: 7.1 us
-// with 512, 9.3 at 10000 with 1024).  The limits of 65536 and 262144 are the LDS of the bitmap.
+// with 512, 9.3 at 10000 with 1024).  Up to kMidLen the registers of 512 hold a list of the whole row and still two
+// workgroups a compute unit: fp32, with 1024 | 512 threads: 32 x 8193 -> 512 8.7 | 7.6, 256 x 10240 -> 800 9.3 | 8.8,
+// 512 x 8193 -> 512 16.6 | 10.4, 1000 x 10240 -> 2000 41.3 | 30.2; where a row has a compute unit to itself the larger
+// selections gain nothing (256 x 9000 -> 1200 9.8 | 9.4, -> 1500 10.1 | 10.2).  Longer rows in 512 threads leave one
+// workgroup there (16384: 170 registers): 8% at k <= 1024, -12% at 3300, not taken.  The limits of 65536 and 262144 are the LDS of the bitmap.
 template <typename T>
 static bool launch_topk_filter(const TopkParams& p, int rows, hipStream_t st) {
   const dim3 grid(rows);
@@ -617,6 +657,8 @@ static bool launch_topk_filter(const TopkParams& p, int rows, hipStream_t st) {
     hipLaunchKernelGGL((topk_filter_kernel<T, 256, 4, 1024, 1024>), grid, dim3(256), 0, st, p);
   else if (p.len <= 8192)
     hipLaunchKernelGGL((topk_filter_kernel<T, 512, 4, 8192, 8192>), grid, dim3(512), 0, st, p);
+  else if (p.len <= kMidLen && (p.k <= 1200 || rows > 256))
+    hipLaunchKernelGGL((topk_filter_kernel<T, 512, 4, kMidLen, kMidLen>), grid, dim3(512), 0, st, p);
   else if (!filter_fits(p.len, p.k, 1024))
     return false;
   else if (p.len <= 65536)

@@ -39,6 +39,33 @@ _LAST_IDX, _DST_SLOT, _POSITION = (_lib.TD_STEP_LAST_PAGE_IDX, _lib.TD_STEP_DST_
 _SELECTED, _STEPS, _META_ROWS = _lib.TD_STEP_N_SELECTED, _lib.TD_STEP_COUNT, _lib.TD_STEP_WORDS
 
 
+class _Views(dict):
+    """Slices by name; holds the tensors that they are taken of, not the controller."""
+
+    _of = dict(
+        tables=lambda v: v.page_table[: v.batch], table_row=lambda v: v.page_table.view(1, -1),
+        starts=lambda v: v.table_starts[: v.batch + 1], list_starts=lambda v: v.list_starts[: v.batch + 1],
+        qk=lambda v: v.qk_product[: v.batch * v.heads], lse=lambda v: v.lse_all[: v.batch], bound=lambda v: v["lse"].view(-1),
+        last_len=lambda v: v.row(_LAST_LEN), last_idx=lambda v: v.row(_LAST_IDX), before=lambda v: v.row(_PAGES_BEFORE_LAST),
+        selected=lambda v: v.row(_SELECTED), slots=lambda v: v.row(_DST_SLOT), seq_len=lambda v: v.row(_SEQ_LEN),
+        positions=lambda v: v.row(_POSITION), sums=lambda v: v.score_sum[: v.batch * v.index_rows],
+        sum_bound=lambda v: v.score_bound[: v.batch * v.index_rows])
+
+    def __init__(self, c: "BatchInferenceController"):
+        self.batch, self.heads, self.index_rows = c.batch, c.num_heads, c.index_rows
+        self.page_table, self.table_starts, self.list_starts, self.meta = c.page_table, c._table_starts, c._list_starts, c._meta
+        self.qk_product, self.lse_all = c.qk_product, c.lse
+        if c.score_sum is not None:
+            self.score_sum, self.score_bound = c.score_sum, c.score_bound
+
+    def row(self, r: int) -> torch.Tensor:
+        return self.meta[r, : self.batch]
+
+    def __missing__(self, name: str) -> torch.Tensor:
+        self[name] = view = self._of[name](self)
+        return view
+
+
 class BatchInferenceController:
     def __init__(self, num_layers: int, num_heads: int, head_dim: int, page_size: int,
                  token_budget: int, max_seq_len: int, max_batch: int, dtype, device, *,
@@ -257,20 +284,12 @@ class BatchInferenceController:
     def _row(self, r: int) -> torch.Tensor:
         return self._meta[r, : self.batch]
 
-    def _views(self) -> dict:
-        """The slices of the controller's tensors that every layer of a step takes, made once per batch size (a
-        slice costs the host 1 us, a layer took nine)."""
+    def _views(self) -> "_Views":
+        """The slices of the controller's tensors that every layer of a step takes, each made when it is first asked
+        for and once per batch size (a slice costs the host 1 us, a layer took nine)."""
         base, of = (self.qk_product, self.lse, self.page_table, self._meta, self.score_sum), self._view_base
         if of is None or self._view_batch != self.batch or any(a is not b for a, b in zip(base, of)):
-            B, rows = self.batch, self.batch * self.index_rows
-            self._view = dict(
-                tables=self.page_table[:B], table_row=self.page_table.view(1, -1), starts=self._table_starts[: B + 1],
-                list_starts=self._list_starts[: B + 1], qk=self.qk_product[: B * self.num_heads], lse=self.lse[:B],
-                bound=self.lse[:B].view(-1), last_len=self._row(_LAST_LEN), last_idx=self._row(_LAST_IDX),
-                before=self._row(_PAGES_BEFORE_LAST), selected=self._row(_SELECTED), slots=self._row(_DST_SLOT),
-                seq_len=self._row(_SEQ_LEN), positions=self._row(_POSITION))
-            if self.score_sum is not None:
-                self._view.update(sums=self.score_sum[:rows], sum_bound=self.score_bound[:rows])
+            self._view = _Views(self)
             self._view_base, self._view_batch = base, self.batch
         return self._view
 

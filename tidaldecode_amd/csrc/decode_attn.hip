@@ -495,7 +495,7 @@ static int build_params(const td_paged_kv* kv, const td_index_list* list, const 
 }
 
 // Whether a call can run on the short-list kernel of its plan: one query head per list walk or a whole group per
-// shared list, chunks that are a power-of-two multiple of the kernel's workgroup tile.  Returns 0 (no), kSparseLean
+// shared list, chunks that are a multiple of the kernel's workgroup tile.  Returns 0 (no), kSparseLean
 // (power-of-two pages, pool below 4 GiB, strides within the 24-bit multiplier: 32-bit row offsets) or kSparseWide
 // (any page size, 64-bit row offsets; token-slot lists without score output at head_dim 128 only, 8 rows per
 // lane, groups of 1, 2, 4 or 8).

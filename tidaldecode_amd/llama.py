@@ -342,7 +342,7 @@ class TidalLlama:
         ctrl = self.iController
         t0 = time.perf_counter()
         self.begin_decode_step()
-        logits = self.decode_layers(self.embed.index_select(0, token.to(self.device).view(1)))
+        logits = self.decode_layers(self.embed[token.to(self.device).view(1)])
         ctrl.end_forward()
         torch.cuda.synchronize()
         ctrl.decode_latency.append(time.perf_counter() - t0)

@@ -118,7 +118,6 @@ class InferenceController:
         self.num_selected = 0
         self._indptr2 = torch.zeros(2, dtype=torch.int32, device=device)
         self._meta_indptr2 = torch.zeros(2, dtype=torch.int32, device=device)
-        self._indptr_pages = 0  # what _indptr2 holds
 
         self.prefill_latency = []
         self.decode_latency = []
@@ -142,8 +141,7 @@ class InferenceController:
         cache = self.kv_cache
         n_pages = len(cache.indicies)
         if updateTensor:
-            if self._indptr_pages != n_pages:  # (a launch, which most steps do without)
-                self._indptr2[1] = self._indptr_pages = n_pages
+            self._indptr2[1] = n_pages  # (every time: a captured call writes when it is replayed, not here)
             self.kv_indptr_for_append = self._indptr2
             self.kv_last_page_idx = cache.indicies[-1]
             self.kv_indices_with_last = cache.indices_device

@@ -187,6 +187,19 @@ def test_controller_budget_arithmetic(scope):
         InferenceController(2, 8, 64, 16, 100, 1000, torch.float16, dev, num_kv_heads=3)
 
 
+def test_page_count_is_written_by_every_forward():
+    """A call captured into a graph writes the count on replay only, so no later call may take it as written."""
+    from tidaldecode_amd.utils import InferenceController
+
+    c = InferenceController(2, 8, 64, 16, 100, 1000, torch.float16, torch.device("cpu"))
+    c.prepare_metadata(500)
+    c.begin_forward(500)
+    c.kv_indptr_for_append[1] = 7         # what a replay of an earlier capture leaves
+    c.prepare_metadata(1)
+    c.begin_forward(1)
+    assert c.kv_indptr_for_append.tolist() == [0, 32]
+
+
 def test_batch_controller_bookkeeping():
     """Page-table segments, per-step metadata and page accounting of the batched controller
     (host arithmetic only: no kernel runs)."""

@@ -39,31 +39,29 @@ _LAST_IDX, _DST_SLOT, _POSITION = (_lib.TD_STEP_LAST_PAGE_IDX, _lib.TD_STEP_DST_
 _SELECTED, _STEPS, _META_ROWS = _lib.TD_STEP_N_SELECTED, _lib.TD_STEP_COUNT, _lib.TD_STEP_WORDS
 
 
-class _Views(dict):
-    """Slices by name; holds the tensors that they are taken of, not the controller."""
+# What the steps of a layer take of the controller's tensors (`_kept`)
+def _positions_of(c):
+    return c._row(_POSITION)
 
-    _of = dict(
-        tables=lambda v: v.page_table[: v.batch], table_row=lambda v: v.page_table.view(1, -1),
-        starts=lambda v: v.table_starts[: v.batch + 1], list_starts=lambda v: v.list_starts[: v.batch + 1],
-        qk=lambda v: v.qk_product[: v.batch * v.heads], lse=lambda v: v.lse_all[: v.batch], bound=lambda v: v["lse"].view(-1),
-        last_len=lambda v: v.row(_LAST_LEN), last_idx=lambda v: v.row(_LAST_IDX), before=lambda v: v.row(_PAGES_BEFORE_LAST),
-        selected=lambda v: v.row(_SELECTED), slots=lambda v: v.row(_DST_SLOT), seq_len=lambda v: v.row(_SEQ_LEN),
-        positions=lambda v: v.row(_POSITION), sums=lambda v: v.score_sum[: v.batch * v.index_rows],
-        sum_bound=lambda v: v.score_bound[: v.batch * v.index_rows])
 
-    def __init__(self, c: "BatchInferenceController"):
-        self.batch, self.heads, self.index_rows = c.batch, c.num_heads, c.index_rows
-        self.page_table, self.table_starts, self.list_starts, self.meta = c.page_table, c._table_starts, c._list_starts, c._meta
-        self.qk_product, self.lse_all = c.qk_product, c.lse
-        if c.score_sum is not None:
-            self.score_sum, self.score_bound = c.score_sum, c.score_bound
+def _full_of(c):
+    b = c.batch
+    return (c.page_table.view(1, -1), c._table_starts[: b + 1], c._row(_LAST_LEN), c._row(_LAST_IDX),
+            c._row(_PAGES_BEFORE_LAST), c._row(_DST_SLOT), c.qk_product[: b * c.num_heads], c.lse[:b])
 
-    def row(self, r: int) -> torch.Tensor:
-        return self.meta[r, : self.batch]
 
-    def __missing__(self, name: str) -> torch.Tensor:
-        self[name] = view = self._of[name](self)
-        return view
+def _sparse_of(c):
+    return c._list_starts[: c.batch + 1], c._row(_SELECTED), c._row(_DST_SLOT)
+
+
+def _select_of(c):
+    b = c.batch
+    return c.qk_product[: b * c.num_heads], c.lse[:b].view(-1), c.page_table[:b], c._row(_SEQ_LEN)
+
+
+def _sums_of(c):
+    n = c.batch * c.index_rows
+    return c.score_sum[:n], c.score_bound[:n]
 
 
 class BatchInferenceController:
@@ -112,7 +110,7 @@ class BatchInferenceController:
                                      dtype=_logits_dtype(logits_dtype, dtype, select_mode),
                                      device=device)
         self.lse = torch.zeros((max_batch, num_heads), dtype=torch.float32, device=device)
-        self.score_sum = None
+        self.score_sum = self.score_bound = None
         if select_mode != "per_head":
             self.score_sum = torch.zeros((max_batch * self.index_rows, self.score_cols),
                                          dtype=torch.float32, device=device)
@@ -125,7 +123,7 @@ class BatchInferenceController:
         self._list_starts = torch.arange(max_batch + 1, **i32) * self.budget
         self.topk_buf = torch.zeros(_kernels.topk_workspace_bytes(max_batch * self.index_rows),
                                     dtype=torch.uint8, device=device)
-        self._view_base = self._view = self._view_batch = None
+        self._kept_of, self._kept_views = None, {}
         self._handle = BatchDecodeWithPagedKVCacheWrapper(kv_layout=kv_layout)
         self._handle.begin_forward(None, num_heads, num_kv_heads, head_dim, page_size, dtype)
         layer_bytes = self.pool.buf[0].numel() * self.pool.buf.element_size()
@@ -284,14 +282,20 @@ class BatchInferenceController:
     def _row(self, r: int) -> torch.Tensor:
         return self._meta[r, : self.batch]
 
-    def _views(self) -> "_Views":
-        """The slices of the controller's tensors that every layer of a step takes, each made when it is first asked
-        for and once per batch size (a slice costs the host 1 us, a layer took nine)."""
-        base, of = (self.qk_product, self.lse, self.page_table, self._meta, self.score_sum), self._view_base
-        if of is None or self._view_batch != self.batch or any(a is not b for a, b in zip(base, of)):
-            self._view = _Views(self)
-            self._view_base, self._view_batch = base, self.batch
-        return self._view
+    def _kept(self, of):
+        """The slices ``of(self)``, kept for as long as the batch size and the tensors stay (a slice costs the host
+        1 us, a layer took nine)."""
+        at = self._kept_of
+        if at is None or at[0] != self.batch or at[1] is not self.qk_product or at[2] is not self.lse or \
+                at[3] is not self.page_table or at[4] is not self._meta or at[5] is not self.score_sum or \
+                at[6] is not self.score_bound:
+            self._kept_of = (self.batch, self.qk_product, self.lse, self.page_table, self._meta, self.score_sum,
+                             self.score_bound)
+            self._kept_views = {}
+        views = self._kept_views.get(of)
+        if views is None:
+            views = self._kept_views[of] = of(self)
+        return views
 
     @property
     def positions(self) -> torch.Tensor:
@@ -307,7 +311,7 @@ class BatchInferenceController:
 
     def rope_table(self, rope_scale: float = 1.0, rope_theta: float = 1e4):
         """cos, sin ``[B, D/2]`` of the new tokens' positions (once per step, all layers)."""
-        return _kernels.rope_table(self._views()["positions"], self.head_dim, rope_scale, rope_theta)
+        return _kernels.rope_table(self._kept(_positions_of), self.head_dim, rope_scale, rope_theta)
 
     # ---- cache writes -------------------------------------------------------------------------
     def append_prompt(self, b: int, k: torch.Tensor, v: torch.Tensor, layer_idx: int) -> None:
@@ -327,29 +331,30 @@ class BatchInferenceController:
                                     self.dst_slots, int(self.layout), rope_scale, rope_theta)
 
     # ---- attention ----------------------------------------------------------------------------
-    def _fresh(self, fresh):
+    def _fresh(self, fresh, slots):
         if fresh is None:
             return None
         k, v, cos, sin = fresh
-        return (k, v, cos, sin, self._views()["slots"])
+        return (k, v, cos, sin, slots)
 
     def attend_full(self, q: torch.Tensor, layer_idx: int, output_qk_product: bool = False,
                     fresh=None) -> torch.Tensor:
         """Attention of every sequence's new token over its whole cache; with
         ``output_qk_product`` the logits and log-sum-exps are kept for ``select``.
         ``fresh=(k, v, cos, sin)`` folds RoPE and the append of the new tokens into the launch."""
-        w, pool, fresh = self._views(), self.pool, self._fresh(fresh)
-        scores, lse = (w["qk"], w["lse"]) if output_qk_product else (None, None)
+        table, starts, last_len, last_idx, before, slots, scores, lse = self._kept(_full_of)
+        pool, fresh = self.pool, self._fresh(fresh, slots)
+        if not output_qk_product:
+            scores = lse = None
         n_list = -(-max(self._cap) // self.page_size) - 1
         if q.is_cuda:
-            o = host_calls.attend(self._handle._wrapper, q, None, pool.buf, w["table_row"], w["starts"], w["last_len"],
-                                  w["last_idx"], scores, False, lse, n_list, fresh, w["before"], _kernels._stream(),
-                                  layer_idx % pool.num_layers)
+            o = host_calls.attend(self._handle._wrapper, q, None, pool.buf, table, starts, last_len, last_idx, scores,
+                                  False, lse, n_list, fresh, before, _kernels._stream(), layer_idx % pool.num_layers)
             if o is not False:
                 return o
         o = torch.empty_like(q)
-        self._handle.forward(q, o, self.buf_layer(layer_idx), w["table_row"], w["starts"], w["last_len"], w["last_idx"],
-                             scores, lse=lse, n_list=n_list, counts=w["before"], fresh=fresh)
+        self._handle.forward(q, o, self.buf_layer(layer_idx), table, starts, last_len, last_idx, scores, lse=lse,
+                             n_list=n_list, counts=before, fresh=fresh)
         return o
 
     def select(self) -> None:
@@ -357,36 +362,38 @@ class BatchInferenceController:
         physical token slots, sorted by position, in its segment of ``topk_dindices_buffer``."""
         B, P, k = self.batch, self.page_size, self.budget
         n = max(self._cap)   # an upper bound; every sequence's own length is read on the device
-        rows, w = self.index_rows, self._views()
-        scores, bound = w["qk"], w["bound"]
+        rows = self.index_rows
+        scores, bound, tables, lengths = self._kept(_select_of)
         if self.select_mode != "per_head":
             # the B * H_q logit rows form B * rows groups of consecutive heads: one grouped sum
-            if not (scores.is_cuda and host_calls.score_reduce(scores, bound, B * rows, n, TD_REDUCE_GROUP_SUM, w["sums"],
+            sums, sum_bound = self._kept(_sums_of)
+            if not (scores.is_cuda and host_calls.score_reduce(scores, bound, B * rows, n, TD_REDUCE_GROUP_SUM, sums,
                                                                _kernels._stream())):
-                _kernels.score_reduce(scores, bound, B * rows, n, "group_sum", out=w["sums"])
-            scores, bound = w["sums"], w["sum_bound"]
+                _kernels.score_reduce(scores, bound, B * rows, n, "group_sum", out=sums)
+            scores, bound = sums, sum_bound
         k_eff = min(k, n)
         # one call: row b * rows + r is row r of sequence b, ranks that sequence's tokens only
         # (its length is read on the device) and goes through that sequence's page table
         # and lands in that sequence's segment of list row r
         if scores.is_cuda and host_calls.topk(scores, None, None, self.topk_dindices_buffer, self.topk_buf, k_eff,
-                                              w["tables"], P, w["seq_len"], bound, k, _kernels._stream(), n):
+                                              tables, P, lengths, bound, k, _kernels._stream(), n):
             return
         _kernels.topk_filtering(scores[:, :n], None, None, self.topk_dindices_buffer, self.topk_buf, k_eff,
-                                page_table=w["tables"], page_size=P,
-                                lengths=w["seq_len"], upper_bound=bound, segment=k)
+                                page_table=tables, page_size=P,
+                                lengths=lengths, upper_bound=bound, segment=k)
 
     def attend_sparse(self, q: torch.Tensor, layer_idx: int, fresh=None) -> torch.Tensor:
         """Attention over the persisted token lists (``fresh`` as in ``attend_full``)."""
-        w, pool, fresh = self._views(), self.pool, self._fresh(fresh)
+        starts, selected, slots = self._kept(_sparse_of)
+        pool, fresh = self.pool, self._fresh(fresh, slots)
         n_list = min(self.budget, max(self._cap))
         if q.is_cuda:
-            o = host_calls.attend(self._handle._wrapper, q, None, pool.buf, self.topk_dindices_buffer, w["list_starts"], 0,
-                                  0, None, True, None, n_list, fresh, w["selected"], _kernels._stream(),
+            o = host_calls.attend(self._handle._wrapper, q, None, pool.buf, self.topk_dindices_buffer, starts, 0, 0,
+                                  None, True, None, n_list, fresh, selected, _kernels._stream(),
                                   layer_idx % pool.num_layers)
             if o is not False:
                 return o
         o = torch.empty_like(q)
-        self._handle.forward(q, o, self.buf_layer(layer_idx), self.topk_dindices_buffer, w["list_starts"], 0, 0, None,
-                             index_kind="slots", n_list=n_list, counts=w["selected"], fresh=fresh)
+        self._handle.forward(q, o, self.buf_layer(layer_idx), self.topk_dindices_buffer, starts, 0, 0, None,
+                             index_kind="slots", n_list=n_list, counts=selected, fresh=fresh)
         return o

@@ -548,14 +548,14 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(1, U ==
           emit(n < NV && head < gsz, rq0 + head, t + (NH * g4 + n / 4 % NH) * U + 4 * (n / 4 / NH) + n % 4, e);
         }
       }
+      const int left = c1 - t - NH * g4 * U;  // tokens from the lane's first on
 #pragma unroll
       for (int c = 0; c < NC; ++c)
 #pragma unroll
         for (int h = 0; h < NH; ++h)
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-            const bool there = t + (NH * g4 + h) * U + 4 * c + i < c1;
-            sv[c][h][i] = there ? sv[c][h][i] : kNegBig;
+            sv[c][h][i] = h * U + 4 * c + i < left ? sv[c][h][i] : kNegBig;
             mt = fmaxf(mt, sv[c][h][i]);
           }
       const float m_new = fmaxf(mh, rows_max(mt));
@@ -568,7 +568,8 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(1, U ==
         for (int h = 0; h < NH; ++h)
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-            const float pr = sv[c][h][i] > 0.5f * kNegBig ? fast_exp2(sv[c][h][i] - m_new) : 0.f;
+            // (by position, not by value: a NaN logit keeps its weight)
+            const float pr = h * U + 4 * c + i < left ? fast_exp2(sv[c][h][i] - m_new) : 0.f;
             sv[c][h][i] = pr;
             sum += pr;
           }

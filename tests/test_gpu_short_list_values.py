@@ -62,3 +62,64 @@ def test_nan_keys_and_queries_show(cuda, dtype, hq, hkv, d, n, pages, waves):
             if pages:
                 nans = torch.isnan(scores[:, :n].cpu())
                 assert torch.equal(nans, torch.isnan(orc.attn_logits(qq, kk)))
+
+
+@pytest.mark.parametrize("waves,pages,dtype,hq,hkv,d", [
+    (w, pages, dt, *shape) for shape in [(4, 4, 64), (4, 2, 64), (8, 2, 64), (14, 2, 64)] for w in (0, -1)
+    for pages in (False, True) for dt in (torch.float16, torch.bfloat16)] + [
+    (0, False, torch.float16, *shape) for shape in [(4, 4, 128), (4, 2, 128), (8, 2, 128), (16, 2, 128)]])
+def test_infinite_values_stay_infinite(cuda, waves, pages, dtype, hq, hkv, d):
+    """An infinite element of a value is infinite in the output of every head that reads it, not NaN, and nowhere else."""
+    for n in (40, 300, 2100):
+        k, v, q = randn((n, hkv, d), n, dtype), randn((n, hkv, d), n + 1, dtype), randn((hq, d), n + 2, dtype)
+        v[5, 0, 3], v[n - 7, hkv - 1, 9] = float("inf"), float("-inf")
+        case = PagedCase(n, hkv, d, 16, dtype, seed=n, kv=(k, v))
+        o = _attend(cuda, case, q, None if pages else torch.arange(n).repeat(hkv, 1), waves=waves).float().cpu()
+        want = torch.zeros_like(o)
+        want[: hq // hkv, 3], want[hq - hq // hkv:, 9] = float("inf"), float("-inf")
+        assert torch.equal(torch.where(torch.isfinite(o), torch.zeros_like(o), o), want), n
+
+
+@pytest.mark.parametrize("hq,hkv", [(4, 2), (8, 2), (14, 2)])
+@pytest.mark.parametrize("n,waves", [(4000, 0), (16000, -1)])
+def test_a_flat_tail_counts(cuda, hq, hkv, n, waves):
+    """One token of weight 1 and the rest of 2^-26 each, which fp16 does not hold: the sum of the rest is the output."""
+    d, dtype = 64, torch.float16
+    k, v, q = torch.zeros((n, hkv, d)), torch.ones((n, hkv, d)), torch.zeros((hq, d))
+    v[0], q[:, 0] = 0.0, 8.0
+    k[1:, :, 0] = torch.tensor(-18.02).to(dtype).float()
+    case = PagedCase(n, hkv, d, 16, dtype, kv=(k, v))
+    o = _attend(cuda, case, q, None if waves < 0 else torch.arange(n).repeat(hkv, 1), waves=waves).double().cpu()
+    rest = (n - 1) * torch.exp(k[1, 0, 0].double())
+    want = rest / (1 + rest)
+    assert ((o - want).abs() <= 2.0 ** -11 * want + 2.0 ** -20 * want).all()  # the output's rounding, and the sums'
+
+
+@pytest.mark.parametrize("hq,hkv", [(4, 2), (8, 2), (14, 2)])
+@pytest.mark.parametrize("waves", [0, -1])
+def test_weights_keep_their_bits(cuda, hq, hkv, waves):
+    """Four tokens of one weight w against values that cancel 4 w to 2^-24 of it: what is left shows the weight's error.
+    w is the one of bf16 logits that a bf16 value and its bf16 remainder hold worst (2^-17 of it)."""
+    d, dtype = 64, torch.bfloat16
+    x = torch.arange(1, 90).float() / 128  # exact in bf16
+    w = torch.exp(-x.double())
+    hi = w.bfloat16().double()
+    lost = (w - hi - (w - hi).bfloat16().double()).abs() / w
+    at = int(lost.argmax())
+    assert lost[at] >= 2.0 ** -17.5
+    w, values, left = w[at], [1.0] * 4, 4 * w[at]
+    for _ in range(3):
+        values.append(-float(left.bfloat16()))
+        left = left + values[-1]
+    n = len(values)
+    k, v, q = torch.zeros((n, hkv, d)), torch.zeros((n, hkv, d)), torch.zeros((hq, d))
+    q[:, 0] = 8.0
+    k[:4, :, 0] = -x[at]
+    v[:, :, :] = torch.tensor(values)[:, None, None]
+    case = PagedCase(n, hkv, d, 16, dtype, kv=(k, v))
+    o = _attend(cuda, case, q, torch.arange(n).repeat(hkv, 1) if waves == 0 else None, waves=waves).double().cpu()
+    total = 4 * w + 3
+    # the exponential and its argument, each within 2^-23, and the sums of 7 products of up to 4 in 32 bits
+    bound = (4 * w * 2.0 ** -22 + n * 2.0 ** -24 * 4) / total
+    assert bound < 0.5 * 4 * w * lost[at] / total
+    assert ((o - left / total).abs() <= bound + 2.0 ** -8 * (left / total).abs()).all()

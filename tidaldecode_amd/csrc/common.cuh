@@ -94,6 +94,18 @@ __device__ __forceinline__ uint32_t pack2<BF16>(float lo, float hi) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{lo, hi}, bf16x2));
 }
 
+// the same, truncated
+template <typename T>
+__device__ __forceinline__ uint32_t pack2_toward_zero(float lo, float hi);
+template <>
+__device__ __forceinline__ uint32_t pack2_toward_zero<F16>(float lo, float hi) {
+  return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(lo, hi));
+}
+template <>
+__device__ __forceinline__ uint32_t pack2_toward_zero<BF16>(float lo, float hi) {
+  return __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, hi), __builtin_bit_cast(uint32_t, lo), 0x07060302u);
+}
+
 // scalar conversions (used by the small kernels)
 template <typename T>
 __device__ __forceinline__ float to_float(uint16_t b);

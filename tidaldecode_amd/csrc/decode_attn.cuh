@@ -261,22 +261,62 @@ __device__ __forceinline__ int seq_items(const DecodeParams& p, int b, SeqList& 
   return n_splits < 1 ? 1 : n_splits;
 }
 
-// o += P V for four rows of values per lane: hi and rest are the weights as value and remainder in the KV type
-// (operand row c16: a head; head_dim 64: of the tokens of both halves of the 16-lane row), acc[e] dimension e of
-// the lane (head_dim 128: li * 8 + e; 64: li * 8 + 4 (c16 / 8) + e) of the heads 4 g4 + 0 .. 3.
-template <typename T, int D, int NH = 128 / D, int NACC = D / 16>
-__device__ __forceinline__ void weigh_rows(const uint32_t (&hi)[NH][2], const uint32_t (&rest)[NH][2],
-                                           const u32x4 (&v)[4], f32x4 (&acc)[NACC]) {
+// The matrix cores take the weights of shared rows in the KV type, as a sum of parts.
+// kRounded: a rounded value and the rounded remainder, 16 bits of a weight in bf16 and 22 in fp16.
+// kWhole: three truncated parts, which hold all 24 bits, so that nothing is lost against products in fp32.  Every part
+// of a weight above 0 is above 0 (fp16: of 2^-39 and more): an infinite value times a remainder of 0, or of the other
+// sign, would give NaN.  fp16 weights are taken times kWeightScale, or those below 2^-25 would vanish beside a
+// denominator that counts them.  Head_dim 64 takes kWhole, and short lists in fp16 do: their values met fp32 weights or
+// a single part before they came to the matrix cores in two.  The third product costs 1 - 3 %: one layer, rounded |
+// whole, us: 28/4 heads x 64, bf16, lists of 4096 7.20 | 7.31, 60000 tokens 24.9 | 25.3; 32/8 heads x 64, fp16, 60000
+// tokens 37.1 | 37.5; 32/8 heads x 128, fp16, lists of 4096 8.2 | 8.4.
+enum WeightParts { kRounded = 2, kWhole = 3 };
+template <typename T, WeightParts PARTS>
+constexpr float kWeightScale = PARTS == kWhole && std::is_same<T, F16>::value ? 32768.f : 1.f;
+
+template <typename T, WeightParts PARTS>
+__device__ __forceinline__ void split_weights(float w0, float w1, uint32_t (&part)[PARTS]) {
+  float r0, r1;
+  if constexpr (PARTS == kRounded) {
+    part[0] = pack2<T>(w0, w1);
+    unpack2<T>(part[0], r0, r1);
+    part[1] = pack2<T>(w0 - r0, w1 - r1);
+  } else {
+    constexpr float kLeast = std::is_same<T, F16>::value ? 0x1p-24f : 0x1p-120f;  // what a part holds at least
+    w0 *= kWeightScale<T, PARTS>;
+    w1 *= kWeightScale<T, PARTS>;
+    const float least0 = fminf(w0, kLeast), least1 = fminf(w1, kLeast);
+#pragma unroll
+    for (int x = 0; x < 3; ++x) {
+      part[x] = pack2_toward_zero<T>(w0, w1);
+      unpack2<T>(part[x], r0, r1);
+      w0 = fmaxf(w0 - r0, least0);
+      w1 = fmaxf(w1 - r1, least1);
+    }
+  }
+}
+
+// o += P V for four rows of values per lane: pr are the weights of one head (column c16; head_dim 64: of the tokens of
+// both halves of the 16-lane row), acc[e] dimension e of the lane (head_dim 128: li * 8 + e; 64: li * 8 + 4 (c16 / 8)
+// + e) of the heads 4 g4 + 0 .. 3, times kWeightScale.
+template <typename T, int D, WeightParts PARTS, int NH = 128 / D, int NACC = D / 16>
+__device__ __forceinline__ void weigh_rows(const float (&pr)[NH][4], const u32x4 (&v)[4], f32x4 (&acc)[NACC]) {
   constexpr uint32_t kLow = 0x05040100u, kHigh = 0x07060302u;  // v_perm: the low or the high halves of two dwords
+  uint32_t part[NH][2][PARTS];
+#pragma unroll
+  for (int h = 0; h < NH; ++h)
+#pragma unroll
+    for (int w = 0; w < 2; ++w) split_weights<T, PARTS>(pr[h][2 * w], pr[h][2 * w + 1], part[h][w]);
   if constexpr (D == 128) {
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
       const uint32_t lo0 = __builtin_amdgcn_perm(v[1][w], v[0][w], kLow), lo1 = __builtin_amdgcn_perm(v[3][w], v[2][w], kLow);
       const uint32_t hi0 = __builtin_amdgcn_perm(v[1][w], v[0][w], kHigh), hi1 = __builtin_amdgcn_perm(v[3][w], v[2][w], kHigh);
-      acc[2 * w] = mfma_16x16x16<T>(hi[0][0], hi[0][1], lo0, lo1, acc[2 * w]);
-      acc[2 * w + 1] = mfma_16x16x16<T>(hi[0][0], hi[0][1], hi0, hi1, acc[2 * w + 1]);
-      acc[2 * w] = mfma_16x16x16<T>(rest[0][0], rest[0][1], lo0, lo1, acc[2 * w]);
-      acc[2 * w + 1] = mfma_16x16x16<T>(rest[0][0], rest[0][1], hi0, hi1, acc[2 * w + 1]);
+#pragma unroll
+      for (int x = 0; x < PARTS; ++x) {
+        acc[2 * w] = mfma_16x16x16<T>(part[0][0][x], part[0][1][x], lo0, lo1, acc[2 * w]);
+        acc[2 * w + 1] = mfma_16x16x16<T>(part[0][0][x], part[0][1][x], hi0, hi1, acc[2 * w + 1]);
+      }
     }
   } else {
     // Rows of eight lanes: the two halves of a 16-lane row hold different tokens.  They exchange half of their
@@ -289,8 +329,6 @@ __device__ __forceinline__ void weigh_rows(const uint32_t (&hi)[NH][2], const ui
         t[0][u][w] = (uint32_t)__builtin_amdgcn_update_dpp((int)v[u][w], (int)v[u][2 + w], 0x128, 0xf, 0xc, false);
         t[1][u][w] = (uint32_t)__builtin_amdgcn_update_dpp((int)v[u][2 + w], (int)v[u][w], 0x128, 0xf, 0x3, false);
       }
-    const u32x4 pa = {hi[0][0], hi[0][1], hi[NH - 1][0], hi[NH - 1][1]};
-    const u32x4 pb = {rest[0][0], rest[0][1], rest[NH - 1][0], rest[NH - 1][1]};
 #pragma unroll
     for (int w = 0; w < 2; ++w)
 #pragma unroll
@@ -298,8 +336,10 @@ __device__ __forceinline__ void weigh_rows(const uint32_t (&hi)[NH][2], const ui
         const uint32_t sel = half ? kHigh : kLow;
         const u32x4 vv = {__builtin_amdgcn_perm(t[0][1][w], t[0][0][w], sel), __builtin_amdgcn_perm(t[0][3][w], t[0][2][w], sel),
                           __builtin_amdgcn_perm(t[1][1][w], t[1][0][w], sel), __builtin_amdgcn_perm(t[1][3][w], t[1][2][w], sel)};
-        acc[2 * w + half] = mfma_16x16x32<T>(pa, vv, acc[2 * w + half]);
-        acc[2 * w + half] = mfma_16x16x32<T>(pb, vv, acc[2 * w + half]);
+#pragma unroll
+        for (int x = 0; x < PARTS; ++x)
+          acc[2 * w + half] = mfma_16x16x32<T>(u32x4{part[0][0][x], part[0][1][x], part[NH - 1][0][x], part[NH - 1][1][x]}, vv,
+                                               acc[2 * w + half]);
       }
   }
 }
@@ -469,6 +509,7 @@ __device__ __forceinline__ void attend_share(const DecodeParams& p, const int hr
   // equal in all lanes of the wave, lh is the lane's share of the denominator, and accm[dd][i] is
   // o[head (4 g4 + i) % QPG] of dimension dd of the lane (see weigh_rows).
   constexpr int NACC = MMA ? D / 16 : 1;
+  constexpr WeightParts kParts = D == 64 ? kWhole : kRounded;
   float mh = kNegBig, lh = 0.f;
   f32x4 accm[NACC];
 #pragma unroll
@@ -730,18 +771,7 @@ __device__ __forceinline__ void attend_share(const DecodeParams& p, const int hr
       // gives the log-sum-exp, stays in fp32.  bf16 keeps 8 bits of a weight (fp16 11): against an
       // exact denominator that is an error of 2^-9 |v| (2^-12 |v|) in o, which with few selected
       // tokens and |v| of 3-4 reached the tolerance together with the rounding of o itself.  The
-      // weights are therefore split into a rounded part and the (rounded) remainder, two products
-      // instead of one: twice the bits, and the matrix pipeline has the room.
-      uint32_t hi[NB][2], rest[NB][2];
-#pragma unroll
-      for (int x = 0; x < NB; ++x)
-#pragma unroll
-        for (int w = 0; w < 2; ++w) {
-          hi[x][w] = pack2<T>(pr[x][2 * w], pr[x][2 * w + 1]);
-          float r0, r1;
-          unpack2<T>(hi[x][w], r0, r1);
-          rest[x][w] = pack2<T>(pr[x][2 * w] - r0, pr[x][2 * w + 1] - r1);
-        }
+      // weights are therefore split into parts (weigh_rows).
       lh = fmaf(lh, alpha, sum);
       // rescale the accumulators: row 4g + i belongs to head (4g + i) % QPG; the factors are
       // wave-uniform per head (lane x < QPG holds head x), so they travel through SGPRs
@@ -768,7 +798,7 @@ __device__ __forceinline__ void attend_share(const DecodeParams& p, const int hr
           for (int d = 0; d < NACC; ++d) accm[d][i] *= f;
         }
       }
-      weigh_rows<T, D>(hi, rest, vb, accm);
+      weigh_rows<T, D, kParts>(pr, vb, accm);
       return;
     } else {
     float sc[QPG][U];
@@ -899,7 +929,7 @@ __device__ __forceinline__ void attend_share(const DecodeParams& p, const int hr
     for (int j = 0; j < QPG; ++j) {  // head j is row j of the accumulator tile: group j / 4, i = j % 4
       if (g4 == j / 4) {
 #pragma unroll
-        for (int d = 0; d < NACC; ++d) state(j, wave, LPR == 16 ? d : 4 * (c16 >> 3) + d, li) = accm[d][j % 4];
+        for (int d = 0; d < NACC; ++d) state(j, wave, LPR == 16 ? d : 4 * (c16 >> 3) + d, li) = accm[d][j % 4] * (1.f / kWeightScale<T, kParts>);
       }
     }
     if (lane < QPG) {

@@ -387,6 +387,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(1, U ==
   // (head_dim 128: li 8 + e; 64: li 8 + 4 (c16 / 8) + e), already summed over the lane groups.
   float mh = kNegBig, lh = 0.f;
   constexpr int NACC = QPG > 1 ? D / 16 : 1;
+  constexpr WeightParts kParts = D == 64 || std::is_same<T, F16>::value ? kWhole : kRounded;
   f32x4 accm[NACC];
 #pragma unroll
   for (int d = 0; d < NACC; ++d) accm[d] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -582,21 +583,10 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(1, U ==
           for (int e = 0; e < NACC; ++e) accm[e][r] *= f;
         }
       }
-      // the weights travel in the KV type as value and remainder (see decode_attn_kernel)
 #pragma unroll
       for (int c = 0; c < NC; ++c) {
-        uint32_t hi[NH][2], rest[NH][2];
-#pragma unroll
-        for (int h = 0; h < NH; ++h)
-#pragma unroll
-          for (int w = 0; w < 2; ++w) {
-            hi[h][w] = pack2<T>(sv[c][h][2 * w], sv[c][h][2 * w + 1]);
-            float r0, r1;
-            unpack2<T>(hi[h][w], r0, r1);
-            rest[h][w] = pack2<T>(sv[c][h][2 * w] - r0, sv[c][h][2 * w + 1] - r1);
-          }
         const u32x4(&v4)[4] = *reinterpret_cast<const u32x4(*)[4]>(&vb[4 * c]);
-        weigh_rows<T, D>(hi, rest, v4, accm);
+        weigh_rows<T, D, kParts>(sv[c], v4, accm);
       }
       return;
     }
@@ -726,7 +716,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(1, U ==
 #pragma unroll
         for (int e = 0; e < NACC; e += 4)
           *reinterpret_cast<f32x4*>(state(wave, head, li * 8 + (LPR == 16 ? e : 4 * (c16 >> 3)))) =
-              f32x4{accm[e][r], accm[e + 1][r], accm[e + 2][r], accm[e + 3][r]};
+              f32x4{accm[e][r], accm[e + 1][r], accm[e + 2][r], accm[e + 3][r]} * (1.f / kWeightScale<T, kParts>);
       }
     }
     const float lw = rows_sum(lh);

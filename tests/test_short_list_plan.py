@@ -2,7 +2,8 @@
 within the built-in scratch wherever a single split does."""
 import pytest
 
-from tidaldecode_amd._lib import DecodePlan, lib
+from tidaldecode_amd._lib import TD_ERR_UNSUPPORTED, DecodePlan, lib
+
 
 SCRATCH = 4 << 20
 
@@ -25,3 +26,12 @@ def test_plans(hq, hkv, d, batch):
             for n in (1, items // 2 + 1, items):
                 x = n + p.chunk_tokens - 1
                 assert (x * magic) >> 32 == x // p.chunk_tokens
+
+
+@pytest.mark.parametrize("waves,rows", [(1, 0), (2, 0), (3, 8), (5, 0), (16, 0), (0, 4), (8, 12)])
+def test_preset_shapes_that_no_kernel_has(waves, rows):
+    """An error, not a division by the chunk that no shape gave."""
+    for hq, hkv, idx_rows in [(32, 32, 32), (32, 8, 8), (32, 8, 32)]:
+        p = DecodePlan(0, 0, 0, 0, -1, waves, rows, 0)
+        assert lib.td_decode_make_plan(1, hq, hkv, 128, idx_rows, 2048, p) == TD_ERR_UNSUPPORTED
+        assert b"no short-list kernel" in lib.td_last_error()

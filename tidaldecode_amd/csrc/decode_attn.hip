@@ -168,6 +168,10 @@ extern "C" int td_decode_make_plan(int32_t batch, int32_t num_qo_heads, int32_t 
                 max_items <= kSparseMaxItems &&
                 (plan->chunk_tokens == 0 || is_pow2(plan->chunk_tokens));
   if ((qpg > 1 || head_dim == 64) && sr == 16) sparse = false;  // 8 rows per lane only
+  if (sparse && !sparse_shape_supported(sw == 0 ? 8 : sw, sr == 0 ? 8 : sr, qpg))
+    return fail(TD_ERR_UNSUPPORTED,
+                "td_decode_make_plan: no short-list kernel with %d waves x %d rows (4 or 8 waves, 8 or "
+                "16 rows)", sw, sr);
   if (sparse) {
     // Workgroup shape and chunk with the least cost; more tiles or fewer waves have to gain.  Splits whose partials
     // do not fit the built-in scratch are left alone, as that would refuse callers who have no other.
@@ -203,10 +207,6 @@ extern "C" int td_decode_make_plan(int32_t batch, int32_t num_qo_heads, int32_t 
     while (ceil_div64(max_items, chunk) > 64) chunk <<= 1;
     if (sr == 0) sr = 8;
     if (sw == 0) sw = (chunk < 32768 / head_dim || sr == 16) ? 4 : 8;
-    if (!sparse_shape_supported(sw, sr, qpg))
-      return fail(TD_ERR_UNSUPPORTED,
-                  "td_decode_make_plan: no short-list kernel with %d waves x %d rows (4 or 8 waves, 8 or "
-                  "16 rows)", sw, sr);
     const int stile = sw * (512 / head_dim) * sr;
     if (plan->chunk_tokens == 0 && chunk < stile) chunk = stile;  // a preset shape with a larger tile
     if (chunk % stile != 0 || chunk % (16384 / head_dim) != 0) {

@@ -35,3 +35,6 @@ def test_preset_shapes_that_no_kernel_has(waves, rows):
         p = DecodePlan(0, 0, 0, 0, -1, waves, rows, 0)
         assert lib.td_decode_make_plan(1, hq, hkv, 128, idx_rows, 2048, p) == TD_ERR_UNSUPPORTED
         assert b"no short-list kernel" in lib.td_last_error()
+    for hq, hkv, d, idx_rows in [(32, 32, 64, 32), (32, 8, 64, 8), (28, 4, 128, 4), (28, 4, 128, 28)]:
+        p = DecodePlan(0, 0, 0, 0, -1, waves, rows, 0)  # shapes that the short-list kernel came to later: ignored
+        assert lib.td_decode_make_plan(1, hq, hkv, d, idx_rows, 2048, p) == 0 and p.sparse_waves == 0

@@ -168,10 +168,15 @@ extern "C" int td_decode_make_plan(int32_t batch, int32_t num_qo_heads, int32_t 
                 max_items <= kSparseMaxItems &&
                 (plan->chunk_tokens == 0 || is_pow2(plan->chunk_tokens));
   if ((qpg > 1 || head_dim == 64) && sr == 16) sparse = false;  // 8 rows per lane only
-  if (sparse && !sparse_shape_supported(sw == 0 ? 8 : sw, sr == 0 ? 8 : sr, qpg))
-    return fail(TD_ERR_UNSUPPORTED,
-                "td_decode_make_plan: no short-list kernel with %d waves x %d rows (4 or 8 waves, 8 or "
-                "16 rows)", sw, sr);
+  if (sparse && !sparse_shape_supported(sw == 0 ? 8 : sw, sr == 0 ? 8 : sr, qpg)) {
+    // head_dim 64 and other groups had no short-list kernel to preset once, and keep ignoring what it does not have
+    const int group = num_qo_heads / num_kv_heads;
+    if (head_dim == 128 && (qpg == 1 ? is_pow2(group) : qpg == group))
+      return fail(TD_ERR_UNSUPPORTED,
+                  "td_decode_make_plan: no short-list kernel with %d waves x %d rows (4 or 8 waves, 8 or "
+                  "16 rows)", sw, sr);
+    sparse = false;
+  }
   if (sparse) {
     // Workgroup shape and chunk with the least cost; more tiles or fewer waves have to gain.  Splits whose partials
     // do not fit the built-in scratch are left alone, as that would refuse callers who have no other.

@@ -38,3 +38,12 @@ def test_preset_shapes_that_no_kernel_has(waves, rows):
     for hq, hkv, d, idx_rows in [(32, 32, 64, 32), (32, 8, 64, 8), (28, 4, 128, 4), (28, 4, 128, 28)]:
         p = DecodePlan(0, 0, 0, 0, -1, waves, rows, 0)  # shapes that the short-list kernel came to later: ignored
         assert lib.td_decode_make_plan(1, hq, hkv, d, idx_rows, 2048, p) == 0 and p.sparse_waves == 0
+
+
+@pytest.mark.parametrize("waves", [0, 4, 8])
+@pytest.mark.parametrize("batch", [1, 4, 16, 64, 256])
+def test_sixteen_rows_a_lane_keep_to_the_scratch(waves, batch):
+    for items in (100, 777, 2048, 5000, 16384):
+        p = DecodePlan(0, 0, 0, 0, -1, waves, 16, 0)
+        assert lib.td_decode_make_plan(batch, 32, 32, 128, 32, items, p) == 0 and p.sparse_rows == 16
+        assert p.workspace_bytes <= SCRATCH or p.max_splits == 1

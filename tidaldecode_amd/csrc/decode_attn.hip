@@ -181,8 +181,13 @@ extern "C" int td_decode_make_plan(int32_t batch, int32_t num_qo_heads, int32_t 
     // Workgroup shape and chunk with the least cost; more tiles or fewer waves have to gain.  Splits whose partials
     // do not fit the built-in scratch are left alone, as that would refuse callers who have no other.
     int64_t chunk = plan->chunk_tokens;
+    const int rows_all = n_hrows * batch;
+    auto fits = [&](int64_t splits) {
+      return splits == 1 || kTicketBytes + (int64_t)rows_all * qpg * splits * (head_dim + 2) * 4 + 512 <=
+                                (int64_t)TD_STATIC_SCRATCH_BYTES;
+    };
     if (chunk == 0 && sr != 16) {
-      const int rows_all = n_hrows * batch, items = (int)max_items;
+      const int items = (int)max_items;
       float best = 0.f;
       const int preset = sw;
       for (int nw = 8; nw >= 4; nw -= 4) {
@@ -191,9 +196,7 @@ extern "C" int td_decode_make_plan(int32_t batch, int32_t num_qo_heads, int32_t 
         for (int tiles = 1;; tiles += tiles < 4 ? 1 : (tiles < 16 ? tiles / 4 * 2 : tiles / 2)) {
           if (tiles > most) tiles = most;
           const int splits = (most + tiles - 1) / tiles;
-          const bool fits = splits <= 64 && (splits == 1 || kTicketBytes + (int64_t)rows_all * qpg * splits * (head_dim + 2) * 4 +
-                                                                    512 <= (int64_t)TD_STATIC_SCRATCH_BYTES);
-          if (fits) {
+          if (splits <= 64 && fits(splits)) {
             const float cost = short_list_cost(head_dim, qpg, rows_all, items, nw, tiles, splits);
             if (best == 0.f || cost < best - 0.01f) {
               best = cost;
@@ -208,6 +211,7 @@ extern "C" int td_decode_make_plan(int32_t batch, int32_t num_qo_heads, int32_t 
       }
     } else if (chunk == 0) {
       chunk = 256;
+      while (!fits(ceil_div64(max_items, chunk))) chunk <<= 1;
     }
     while (ceil_div64(max_items, chunk) > 64) chunk <<= 1;
     if (sr == 0) sr = 8;

@@ -122,3 +122,27 @@ def test_page_lists_of_a_ragged_batch(cuda, hq, hkv, d):
     torch.cuda.synchronize()
     for i, c in enumerate(cases):
         assert tolerance_report(o[i], orc.sparse_layer_gather(q[i], c.k, c.v, chosen[i])) <= ATOL[dtype], i
+
+
+@pytest.mark.parametrize("batch,kernel", [(1024, "short-list"), (1025, "streaming")])
+def test_batches_of_more_head_slots_than_tickets(cuda, batch, kernel):
+    from tidaldecode_amd import _kernels
+
+    hq, hkv, d, page, n, k = 14, 2, 64, 16, 3000, 130   # eight head slots a KV head
+    dtype, g = torch.bfloat16, torch.Generator().manual_seed(batch)
+    case = PagedCase(n, hkv, d, page, dtype, seed=4)
+    pos = torch.randint(0, n, (hkv, batch * k), generator=g)
+    q = randn((batch, hq, d), 9, dtype)
+    qd = q.to(dtype).to(cuda)
+    o = torch.full_like(qd, float("nan"))
+    w = _wrapper(hq, hkv, d, page, dtype)
+    starts = (torch.arange(batch + 1) * k).to(torch.int32).to(cuda)
+    for _ in range(2):  # twice: tickets and partials are reused
+        w.forward(qd, o, case.pool.to(cuda), case.slots_of(pos).to(torch.int32).to(cuda), starts, 0, 0, None,
+                  index_kind="slots", n_list=k)
+    assert _kernels.last_decode_kernel() == kernel
+    for h in range(hkv):
+        at = pos[h].view(batch, k)
+        kk, vv, qh = case.k[at, h], case.v[at, h], q[:, h * 7:(h + 1) * 7]
+        want = torch.softmax(qh @ kk.transpose(1, 2) / d ** 0.5, -1) @ vv
+        assert tolerance_report(o[:, h * 7:(h + 1) * 7], want) <= ATOL[dtype]

@@ -2,7 +2,7 @@
 within the built-in scratch wherever a single split does."""
 import pytest
 
-from tidaldecode_amd._lib import TD_ERR_UNSUPPORTED, DecodePlan, lib
+from tidaldecode_amd._lib import TD_ERR_INVALID_ARG, TD_ERR_UNSUPPORTED, DecodePlan, lib
 
 
 SCRATCH = 4 << 20
@@ -47,3 +47,23 @@ def test_sixteen_rows_a_lane_keep_to_the_scratch(waves, batch):
         p = DecodePlan(0, 0, 0, 0, -1, waves, 16, 0)
         assert lib.td_decode_make_plan(batch, 32, 32, 128, 32, items, p) == 0 and p.sparse_rows == 16
         assert p.workspace_bytes <= SCRATCH or p.max_splits == 1
+
+
+@pytest.mark.parametrize("hq,hkv,d,slots", [(28, 4, 128, 32), (40, 8, 128, 64), (48, 8, 128, 64), (32, 8, 64, 32),
+                                            (14, 2, 64, 16), (32, 8, 128, 32), (32, 32, 128, 32)])
+def test_batches_beyond_a_ticket_per_head_slot_stream(hq, hkv, d, slots):
+    """The short-list kernel takes a ticket per head slot (padded groups have more of them than heads), the streaming
+    kernel one per head row: up to 16384 of either."""
+    most = 16384 // slots
+    for batch, waves in [(most, (4, 8)), (most + 1, (0,))]:
+        p = DecodePlan(0, 0, 0, 0, -1, 0, 0, 0)
+        rc = lib.td_decode_make_plan(batch, hq, hkv, d, hkv, 512, p)
+        if hq == hkv and batch > most:
+            assert rc == TD_ERR_INVALID_ARG  # a head row a head: no tickets for either
+        else:
+            assert rc == 0 and p.sparse_waves in waves
+    hrows = hkv if hq > hkv else hq
+    p = DecodePlan(0, 0, 0, 0, -1, 0, 0, 0)
+    assert lib.td_decode_make_plan(16384 // hrows, hq, hkv, d, hkv, 512, p) == 0
+    assert lib.td_decode_make_plan(16384 // hrows + 1, hq, hkv, d, hkv, 512, DecodePlan(0, 0, 0, 0, -1, 0, 0, 0)) == \
+        TD_ERR_INVALID_ARG

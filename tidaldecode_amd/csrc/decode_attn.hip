@@ -27,7 +27,8 @@ static int64_t align256(int64_t x) { return (x + 255) & ~(int64_t)255; }
 // tickets of a launch are all taken within a microsecond, and counters that share a line queue up
 // behind one another at the memory channel (measured: 0.4 us of a 9.7 us launch).
 constexpr int kTicketStride = 16;  // int32 words between counters
-constexpr int64_t kTicketBytes = (int64_t)16384 * kTicketStride * 4;
+constexpr int64_t kTickets = 16384;
+constexpr int64_t kTicketBytes = kTickets * kTicketStride * 4;
 
 // The short-list kernel (sparse_attn.cuh) covers a list in one pass of at most 64 workgroups per
 // head; longer lists go to the streaming kernel, whose waves pipeline several tiles.
@@ -163,9 +164,10 @@ extern "C" int td_decode_make_plan(int32_t batch, int32_t num_qo_heads, int32_t 
   // head_dim 64) can run the same plan when a call turns out not to fit the short-list kernel.
   int sw = plan->sparse_waves, sr = plan->sparse_rows;
   plan->balanced = 0;
-  // one query head per list walk, or a KV head's up to eight query heads sharing its list
+  // one query head per list walk, or a KV head's up to eight query heads sharing its list; the streaming kernel takes
+  // what has more head slots than there are tickets, as it needs but one a head row
   bool sparse = sw >= 0 && sr >= 0 && head_dim <= 128 && subs == 1 && max_items > 0 &&
-                max_items <= kSparseMaxItems &&
+                max_items <= kSparseMaxItems && (int64_t)batch * n_hrows * qpg <= kTickets &&
                 (plan->chunk_tokens == 0 || is_pow2(plan->chunk_tokens));
   if ((qpg > 1 || head_dim == 64) && sr == 16) sparse = false;  // 8 rows per lane only
   if (sparse && !sparse_shape_supported(sw == 0 ? 8 : sw, sr == 0 ? 8 : sr, qpg)) {
@@ -232,9 +234,6 @@ extern "C" int td_decode_make_plan(int32_t batch, int32_t num_qo_heads, int32_t 
   if (sparse) {
     if (plan->fused_merge < 0) plan->fused_merge = 1;
     plan->fused_merge = plan->fused_merge ? 1 : 0;
-    TD_REQUIRE((int64_t)batch * n_hrows * qpg * kTicketStride * 4 <= kTicketBytes,
-               "td_decode_make_plan: batch %d x %d heads exceeds the %lld ticket counters", batch,
-               n_hrows * qpg, (long long)(kTicketBytes / (kTicketStride * 4)));
     const int64_t n_part = (int64_t)batch * n_hrows * qpg * plan->max_splits;
     plan->workspace_bytes = kTicketBytes + align256(n_part * head_dim * 4) + align256(n_part * 2 * 4);
     return TD_OK;
@@ -333,9 +332,9 @@ extern "C" int td_decode_make_plan(int32_t batch, int32_t num_qo_heads, int32_t 
   plan->tile_rows = rows;
   if (plan->fused_merge < 0) plan->fused_merge = 1;
   plan->fused_merge = plan->fused_merge ? 1 : 0;
-  TD_REQUIRE((int64_t)batch * n_hrows * kTicketStride * 4 <= kTicketBytes,
+  TD_REQUIRE((int64_t)batch * n_hrows <= kTickets,
              "td_decode_make_plan: batch %d x %d head rows exceeds the %lld ticket counters", batch,
-             n_hrows, (long long)(kTicketBytes / (kTicketStride * 4)));
+             n_hrows, (long long)kTickets);
   const int64_t n_part = (int64_t)batch * n_hrows * qpg * max_splits;  // head slots incl. padding
   plan->workspace_bytes = kTicketBytes + align256(n_part * head_dim * 4) + align256(n_part * 2 * 4);
   return TD_OK;
@@ -411,7 +410,7 @@ static int build_params(const td_paged_kv* kv, const td_index_list* list, const 
   const int64_t off_o = kTicketBytes;
   const int64_t off_ml = off_o + align256(n_part * D * 4);
   const int64_t need = off_ml + align256(n_part * 2 * 4);
-  TD_REQUIRE((int64_t)batch * n_hrows * kTicketStride * 4 <= kTicketBytes,
+  TD_REQUIRE((int64_t)batch * n_hrows <= kTickets,
              "td_decode_attn: batch %d x %d head rows exceeds the ticket counters", batch, n_hrows);
   TD_REQUIRE(plan->max_splits <= 64, "td_decode_attn: plan has %d splits (limit 64)",
              plan->max_splits);
@@ -504,7 +503,7 @@ static int build_params(const td_paged_kv* kv, const td_index_list* list, const 
 }
 
 // Whether a call can run on the short-list kernel of its plan: one query head per list walk or a whole group per
-// shared list, chunks that are a multiple of the kernel's workgroup tile.  Returns 0 (no), kSparseLean
+// shared list, chunks that are a multiple of the kernel's workgroup tile, a ticket a head slot.  Returns 0 (no), kSparseLean
 // (power-of-two pages, pool below 4 GiB, strides within the 24-bit multiplier: 32-bit row offsets) or kSparseWide
 // (any page size, 64-bit row offsets; token-slot lists without score output at head_dim 128 only, 8 rows per
 // lane, groups of 1, 2, 4 or 8).
@@ -512,7 +511,8 @@ enum { kSparseNo = 0, kSparseLean = 1, kSparseWide = 2 };
 static int sparse_kernel_fits(const DecodeParams& p, const td_decode_plan* plan,
                               const td_index_list* list, int qpg, int head_dim, bool emit) {
   const int64_t max_items = (int64_t)list->n_list_host * (list->kind == TD_IDX_PAGES ? p.page_size : 1) + p.page_size;
-  if (plan->sparse_waves <= 0 || !sparse_shape_supported(plan->sparse_waves, plan->sparse_rows, qpg))
+  if (plan->sparse_waves <= 0 || !sparse_shape_supported(plan->sparse_waves, plan->sparse_rows, qpg) ||
+      (int64_t)p.batch * p.vheads > kTickets)
     return kSparseNo;
   const int stile = plan->sparse_waves * (512 / head_dim) * plan->sparse_rows;
   if (!(head_dim <= 128 && p.subs == 1 && max_items <= 2 * kSparseMaxItems && plan->chunk_tokens % stile == 0 &&
@@ -546,8 +546,6 @@ extern "C" int td_decode_attn(const td_paged_kv* kv, const td_index_list* list,
   const int fits = sparse_kernel_fits(p, plan, list, qpg, D, scores != nullptr);
   if (fits != kSparseNo) {
     const bool wide = fits == kSparseWide;
-    TD_REQUIRE((int64_t)batch * n_hrows * qpg * kTicketStride * 4 <= kTicketBytes,
-               "td_decode_attn: batch %d x %d heads exceeds the ticket counters", batch, n_hrows * qpg);
     if (qpg > 1)
       rc = kv->dtype == TD_F16
                ? launch_sparse_shared_f16(p, D, plan->sparse_waves, qpg, wide, merge_kernel, grid, st)

@@ -49,6 +49,37 @@ def test_rule(cuda, m, n, k, splits):
         assert got.shape == (m, n) and ((got.float() - want).abs() <= _bound(want, 2 * mag, k, torch.bfloat16)).all()
 
 
+@pytest.mark.parametrize("m", [64, 16])  # a row count the kernel takes, one that is the library's anyway
+def test_calls_that_are_the_librarys(cuda, m):
+    """What torch's own product does, or refuses, and the kernel could not: operands on two devices, a weight of one
+    dimension, vmap, tangents, traces, tensors of another class."""
+    from tidaldecode_amd._kernels import prompt_product
+
+    g = torch.Generator(device=cuda).manual_seed(m)
+    x = torch.randn((m, 4096), generator=g, device=cuda).bfloat16()
+    w = torch.randn((512, 4096), generator=g, device=cuda).bfloat16()
+    with torch.no_grad():
+        with pytest.raises(RuntimeError, match="device"):
+            prompt_product(x, w.cpu())
+        with pytest.raises(RuntimeError, match="device"):
+            prompt_product(x.cpu(), w)
+        with pytest.raises(RuntimeError, match="shape"):
+            prompt_product(x, w[:, :4032].contiguous())
+        assert torch.equal(prompt_product(x, w[0].contiguous()), x @ w[0])
+        rows = torch.stack([x, 2 * x])
+        assert torch.equal(torch.func.vmap(lambda a: prompt_product(a, w))(rows), torch.func.vmap(lambda a: a @ w.t())(rows))
+        with torch.autograd.forward_ad.dual_level():
+            dual = torch.autograd.forward_ad.make_dual(x, x)
+            assert torch.autograd.forward_ad.unpack_dual(prompt_product(dual, w)).tangent is not None
+        traced = torch.jit.trace(prompt_product, (x, w), check_trace=False)
+        assert torch.equal(traced(3 * x, w), (3 * x) @ w.t())
+
+        class Watched(torch.Tensor):
+            pass
+
+        assert type(prompt_product(x.as_subclass(Watched), w)) is Watched
+
+
 def test_arguments_are_checked(cuda):
     from tidaldecode_amd import _lib
 

@@ -159,15 +159,26 @@ def _row_splits(m: int, n: int, k: int) -> int:
     return splits if splits > 1 else 0
 
 
+def _served_directly(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    """Whether a kernel of this library may read a product's operands: on the current device both, and no wrapper,
+    tangent, trace or mode that has to see torch's own operation."""
+    return (x.is_cuda and weight.device == x.device and x.device.index == torch.cuda.current_device() and
+            not torch.is_grad_enabled() and torch.autograd.forward_ad._current_level < 0 and
+            all(type(t) in (torch.Tensor, torch.nn.Parameter) and not torch._C._functorch.is_functorch_wrapped_tensor(t)
+                for t in (x, weight)) and
+            torch._C._len_torch_dispatch_stack() == 0 and not torch.compiler.is_compiling() and
+            not torch.jit.is_tracing() and
+            x.dtype == weight.dtype and x.dtype in (torch.float16, torch.bfloat16) and
+            x.is_contiguous() and weight.is_contiguous() and (x.data_ptr() | weight.data_ptr()) % 16 == 0)
+
+
 def prompt_product(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     """Extension: ``x @ weight.t()`` of a prompt's rows x ``[n, K]`` and a weight ``[N, K]`` (inference only)."""
     cut = splits = 0
-    if x.dim() == 2 and x.is_cuda and x.dtype == weight.dtype and x.dtype in (torch.float16, torch.bfloat16) and \
-            x.is_contiguous() and weight.is_contiguous() and (x.data_ptr() | weight.data_ptr()) % 16 == 0 and \
-            x.size(1) == weight.size(1) and not torch.is_grad_enabled():
+    if x.dim() == 2 and weight.dim() == 2 and x.size(1) == weight.size(1):
         splits = _row_splits(x.size(0), weight.size(0), x.size(1))
         cut = 0 if splits else _cut_columns(x.size(0), weight.size(0), x.size(1))
-    if not (cut or splits):
+    if not (cut or splits) or not _served_directly(x, weight):
         return x @ weight.t()
     out = torch.empty((x.size(0), weight.size(0)), dtype=x.dtype, device=x.device)
     code = _dtype_code(x.dtype, "prompt_product")

@@ -206,6 +206,15 @@ int td_decode_make_plan(int32_t batch, int32_t num_qo_heads, int32_t num_kv_head
                    int32_t idx_rows, int64_t max_items, td_decode_plan* plan);
 
 /*
+ * 1 if a call of td_decode_attn is one for the short-list kernel by what it reads (the planner sees neither the kind of
+ * list, td_idx_kind, nor the score output), else 0: plan such a call with sparse_waves = -1, which cuts it for the
+ * streaming kernel.  td_decode_attn goes by the same rule, whatever the plan says.  The other arguments as in
+ * td_decode_make_plan.  Host arithmetic.  No counterpart in the reference (one kernel there).
+ */
+int td_short_list_pays(int32_t batch, int32_t num_qo_heads, int32_t num_kv_heads, int32_t head_dim, int32_t idx_rows,
+                       int64_t max_items, int32_t kind, int32_t has_scores);
+
+/*
  * Decode attention of one new token per sequence over the listed tokens of a paged KV pool:
  * o[b,h,:] = softmax(q[b,h,:] . K_sel^T / sqrt(D)) V_sel, online softmax in base 2, fp32
  * accumulation, split over tokens and merged by log-sum-exp.

@@ -146,3 +146,30 @@ def test_batches_of_more_head_slots_than_tickets(cuda, batch, kernel):
         kk, vv, qh = case.k[at, h], case.v[at, h], q[:, h * 7:(h + 1) * 7]
         want = torch.softmax(qh @ kk.transpose(1, 2) / d ** 0.5, -1) @ vv
         assert tolerance_report(o[:, h * 7:(h + 1) * 7], want) <= ATOL[dtype]
+
+
+@pytest.mark.parametrize("n,kernel", [(4608, "short-list"), (4624, "streaming")])  # either side of 72 MiB
+def test_the_library_goes_by_what_a_call_reads(cuda, n, kernel):
+    """Pages of a whole sequence with a plan made without the wrapper's knowledge of the call."""
+    from tidaldecode_amd import _kernels, _lib
+
+    h, d, page, dtype = 32, 128, 16, torch.float16
+    g = torch.Generator(device=cuda).manual_seed(n)
+    pool = torch.randn((n // page, 2, page, h, d), generator=g, device=cuda).to(dtype)
+    q = torch.randn((1, h, d), generator=g, device=cuda).to(dtype)
+    o = torch.full_like(q, float("nan"))
+    table = torch.arange(n // page - 1, dtype=torch.int32, device=cuda)
+    kv = _lib.PagedKV(pool.data_ptr(), n // page, h, d, page, _lib.TD_NHD, _lib.TD_F16)
+    lst = _lib.IndexList()
+    lst.idx, lst.idx_rows, lst.idx_row_stride, lst.kind = table.data_ptr(), 1, table.numel(), _lib.TD_IDX_PAGES
+    lst.n_list_host, lst.last_page_len, lst.last_page_idx = table.numel(), page, n // page - 1
+    plan = _lib.DecodePlan(0, 0, 0, 0, -1, 0, 0, 0)
+    _lib.check(_lib.lib.td_decode_make_plan(1, h, h, d, 1, n, plan))
+    assert plan.sparse_waves > 0
+    ws = torch.zeros(plan.workspace_bytes, dtype=torch.uint8, device=cuda)
+    _lib.check(_lib.lib.td_decode_attn(kv, lst, plan, q.data_ptr(), o.data_ptr(), 1, h, d ** -0.5, None, _lib.TD_F32, 0,
+                                       None, None, ws.data_ptr(), ws.numel(), torch.cuda.current_stream().cuda_stream))
+    assert _kernels.last_decode_kernel() == kernel
+    k, v = (pool[:, i].reshape(n, h, d).float().transpose(0, 1).contiguous() for i in (0, 1))
+    want = torch.softmax((k * q[0].float()[:, None]).sum(-1) / d ** 0.5, -1)[:, None] @ v
+    assert tolerance_report(o[0], want[:, 0]) <= ATOL[dtype]

@@ -150,7 +150,8 @@ def test_launches_leave_the_interpreters_lock(cuda, monkeypatch):
         keep.append(_workload(cuda, torch.bfloat16, *shape))
     real = {name: ctypes.cast(getattr(_lib.lib, name), ctypes.c_void_p).value for name in _lib.SIGNATURES}
     check = ctypes.cast(ctypes.pythonapi.PyGILState_Check, ctypes.c_void_p).value
-    on_host = ("td_last_error", "td_decode_make_plan", "td_topk_workspace_bytes", "td_prefill_workspace_bytes")
+    on_host = ("td_last_error", "td_decode_make_plan", "td_short_list_pays", "td_topk_workspace_bytes",
+               "td_prefill_workspace_bytes")
     host_calls.bind({name: at if name in on_host else check for name, at in real.items()})
     held = set()
     try:

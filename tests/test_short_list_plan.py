@@ -2,7 +2,7 @@
 within the built-in scratch wherever a single split does."""
 import pytest
 
-from tidaldecode_amd._lib import TD_ERR_INVALID_ARG, TD_ERR_UNSUPPORTED, DecodePlan, lib
+from tidaldecode_amd._lib import TD_ERR_INVALID_ARG, TD_ERR_UNSUPPORTED, TD_IDX_PAGES, TD_IDX_SLOTS, DecodePlan, lib
 
 
 SCRATCH = 4 << 20
@@ -67,3 +67,16 @@ def test_batches_beyond_a_ticket_per_head_slot_stream(hq, hkv, d, slots):
     assert lib.td_decode_make_plan(16384 // hrows, hq, hkv, d, hkv, 512, p) == 0
     assert lib.td_decode_make_plan(16384 // hrows + 1, hq, hkv, d, hkv, 512, DecodePlan(0, 0, 0, 0, -1, 0, 0, 0)) == \
         TD_ERR_INVALID_ARG
+
+
+@pytest.mark.parametrize("hq,hkv,d,rows", [(32, 32, 128, 32), (32, 8, 128, 8), (28, 4, 128, 4), (28, 4, 128, 28),
+                                           (32, 8, 64, 1)])
+def test_which_calls_are_for_the_short_list_kernel(hq, hkv, d, rows):
+    def pays(kind, items, scores, batch=1):
+        return lib.td_short_list_pays(batch, hq, hkv, d, rows, items, kind, scores)
+
+    most = (72 << 20) // 4 // ((hq if rows == hq else hkv) * d)  # tokens of 72 MiB
+    for kind, scores in [(TD_IDX_PAGES, 0), (TD_IDX_PAGES, 1), (TD_IDX_SLOTS, 1)]:
+        assert pays(kind, most, scores) and not pays(kind, most + 1, scores)
+        assert pays(kind, 500, scores, 4) and not pays(kind, 2049, scores, 2)
+    assert pays(TD_IDX_SLOTS, 1 << 20, 0) and pays(TD_IDX_SLOTS, 2049, 0, 64)

@@ -730,8 +730,8 @@ class BatchDecodeWithPagedKVCachePyTorchWrapper:
         self._plans.clear()
 
     def _plan(self, batch: int, idx_rows: int, max_items: int, short_list: bool = True) -> DecodePlan:
-        """``short_list``: the call has token-slot lists and no score output, or reads little (host_calls.cpp:
-        short_list), which the planner cannot see; other calls get a plan shaped for the streaming kernel."""
+        """``short_list``: td_short_list_pays for the call, which goes by what the planner cannot see; other calls
+        get a plan shaped for the streaming kernel."""
         sparse_waves = self.sparse_waves if short_list else -1
         key = (batch, idx_rows, max_items, self.waves_per_block, self.fused_merge,
                self.chunk_tokens, self.tile_rows, sparse_waves, self.sparse_rows)
@@ -826,9 +826,8 @@ class BatchDecodeWithPagedKVCachePyTorchWrapper:
 
         max_items = lst.n_list_host * (page if kind == TD_IDX_PAGES else 1) + max_last
         has_scores = qk_product is not None and qk_product.numel() > 0
-        width = (hq if rows == hq else hkv) * d
-        plan = self._plan(batch, rows, max_items, (kind == TD_IDX_SLOTS and not has_scores) or
-                          ((batch == 1 or max_items <= 2048) and batch * max_items * width <= (72 << 20) // 4))
+        plan = self._plan(batch, rows, max_items,
+                          bool(lib.td_short_list_pays(batch, hq, hkv, d, rows, max_items, kind, int(has_scores))))
         if not self.static_scratch and plan.workspace_bytes > 0 and (self._workspace is None or
                                          self._workspace.numel() < plan.workspace_bytes or
                                          self._workspace.device != q.device):

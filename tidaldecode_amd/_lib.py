@@ -107,6 +107,7 @@ SIGNATURES = {
         c_int32,
         [c_int32, c_int32, c_int32, c_int32, c_int32, c_int64, POINTER(DecodePlan)],
     ),
+    "td_short_list_pays": (c_int32, [c_int32, c_int32, c_int32, c_int32, c_int32, c_int64, c_int32, c_int32]),
     "td_decode_attn": (
         c_int32,
         [POINTER(PagedKV), POINTER(IndexList), POINTER(DecodePlan), c_void_p, c_void_p, c_int32,

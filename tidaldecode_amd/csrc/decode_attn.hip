@@ -91,6 +91,19 @@ static float short_list_cost(int head_dim, int qpg, int rows, int items, int nw,
 
 static bool is_pow2(int64_t x) { return x > 0 && (x & (x - 1)) == 0; }
 
+// Token-slot lists without score output go to the short-list kernel, and of the others the calls that read up to 72 MiB
+// (width: elements of K a token, and as many of V) and, in a batch, up to 2048 tokens a sequence.
+// Its one trip from list to rows saves the streaming kernel's pipeline where that never fills.  Two selection
+// layers, one sparse one and their top-k, us, streaming -> short-list: 32 heads x 128 at 300 tokens 35.5 -> 31.6,
+// 4000 59.3 -> 56.2, 6000 (98 MB) 68.7 -> 71.8; 16 heads 8000 58.5 -> 55.1; 32/8 heads 2500 46.0 -> 42.5, 8000 57.2 ->
+// 49.7; 28/4 heads 4000 52.2 -> 44.4; 4 sequences of 500 .. 2000, 32/8 heads, 54.7 -> 46.7; 6 of 1000 .. 4000 (101 MB)
+// 69.6 -> 74.6.  Where the pool then excludes the short-list kernel its chunks serve the streaming kernel no worse than
+// those planned for that: pages of 12 tokens, 8 sequences of 2000, 28/4 heads 13.4 | 14.5, one of 4000, 32/8 heads 10.4 |
+// 11.6, 16 of 1500, 32/8 heads 24.4 | 24.4.
+static bool short_list_pays(bool slots, bool scores, int64_t batch, int64_t max_items, int64_t width) {
+  return (slots && !scores) || ((batch == 1 || max_items <= 2048) && batch * max_items * width <= (72 << 20) / 4);
+}
+
 }  // namespace tidal
 
 // Scratch of td_decode_attn_noalloc: ticket counters and split partials in device memory that
@@ -502,28 +515,38 @@ static int build_params(const td_paged_kv* kv, const td_index_list* list, const 
   return TD_OK;
 }
 
-// Whether a call can run on the short-list kernel of its plan: one query head per list walk or a whole group per
-// shared list, chunks that are a multiple of the kernel's workgroup tile, a ticket a head slot.  Returns 0 (no), kSparseLean
-// (power-of-two pages, pool below 4 GiB, strides within the 24-bit multiplier: 32-bit row offsets) or kSparseWide
-// (any page size, 64-bit row offsets; token-slot lists without score output at head_dim 128 only, 8 rows per
-// lane, groups of 1, 2, 4 or 8).
+// Whether a call runs on the short-list kernel of its plan: one query head per list walk or a whole group per shared
+// list, chunks that are a multiple of the kernel's workgroup tile, a ticket a head slot, and little to read.  Returns 0
+// (no), kSparseLean (power-of-two pages, pool below 4 GiB, strides within the 24-bit multiplier: 32-bit row offsets) or
+// kSparseWide (any page size, 64-bit row offsets; token-slot lists without score output at head_dim 128 only, 8 rows per
+// lane, groups of 1, 2, 4 or 8, and a list per query head in groups of a power of two: the others stay with the streaming
+// kernel, as nobody measured them).
 enum { kSparseNo = 0, kSparseLean = 1, kSparseWide = 2 };
 static int sparse_kernel_fits(const DecodeParams& p, const td_decode_plan* plan,
                               const td_index_list* list, int qpg, int head_dim, bool emit) {
-  const int64_t max_items = (int64_t)list->n_list_host * (list->kind == TD_IDX_PAGES ? p.page_size : 1) + p.page_size;
+  const bool slots = list->kind == TD_IDX_SLOTS;
+  const int64_t listed = (int64_t)list->n_list_host * (slots ? 1 : p.page_size);
   if (plan->sparse_waves <= 0 || !sparse_shape_supported(plan->sparse_waves, plan->sparse_rows, qpg) ||
       (int64_t)p.batch * p.vheads > kTickets)
     return kSparseNo;
   const int stile = plan->sparse_waves * (512 / head_dim) * plan->sparse_rows;
-  if (!(head_dim <= 128 && p.subs == 1 && max_items <= 2 * kSparseMaxItems && plan->chunk_tokens % stile == 0 &&
-        (plan->sparse_rows == 8 || (head_dim == 128 && list->kind == TD_IDX_SLOTS && !emit))))
+  if (!(head_dim <= 128 && p.subs == 1 && listed + p.page_size <= 2 * kSparseMaxItems && plan->chunk_tokens % stile == 0 &&
+        (plan->sparse_rows == 8 || (head_dim == 128 && slots && !emit))))
+    return kSparseNo;
+  if (!short_list_pays(slots, emit, p.batch, listed + (list->last_page_len_arr ? p.page_size : list->last_page_len),
+                       (int64_t)(list->idx_rows == p.num_qo_heads ? p.num_qo_heads : p.num_kv_heads) * head_dim))
     return kSparseNo;
   if (p.lean && p.page_stride_b < (1u << 24) && p.entry_stride_b < (1u << 24)) return kSparseLean;
   // a page's bytes and an entry's offset inside it stay 32-bit; the page base is a 64-bit product
-  const bool plain = list->kind == TD_IDX_SLOTS && !emit && head_dim == 128 &&
-                     (qpg == 1 ? is_pow2(p.q_per_kv) : p.q_per_kv == qpg);
+  const bool plain = slots && !emit && head_dim == 128 && (qpg == 1 ? is_pow2(p.q_per_kv) : p.q_per_kv == qpg);
   if (plain && plan->sparse_rows == 8 && p.page_stride * 2 < ((int64_t)1 << 32)) return kSparseWide;
   return kSparseNo;
+}
+
+extern "C" int td_short_list_pays(int32_t batch, int32_t num_qo_heads, int32_t num_kv_heads, int32_t head_dim,
+                                  int32_t idx_rows, int64_t max_items, int32_t kind, int32_t has_scores) {
+  const int64_t width = (int64_t)(idx_rows == num_qo_heads ? num_qo_heads : num_kv_heads) * head_dim;
+  return short_list_pays(kind == TD_IDX_SLOTS, has_scores != 0, batch, max_items, width) ? 1 : 0;
 }
 
 extern "C" int td_decode_attn(const td_paged_kv* kv, const td_index_list* list,

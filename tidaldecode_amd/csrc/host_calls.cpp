@@ -20,6 +20,7 @@ namespace {
 struct Lib {
   decltype(&td_last_error) last_error;
   decltype(&td_decode_make_plan) make_plan;
+  decltype(&td_short_list_pays) short_list_pays;
   decltype(&td_decode_attn) decode_attn;
   decltype(&td_decode_attn_noalloc) decode_attn_noalloc;
   decltype(&td_topk_segments) topk_segments;
@@ -50,6 +51,7 @@ PyObject* bind(PyObject*, PyObject* table) {
 #define TD_TAKE(f) \
   if (!take(table, "td_" #f, lib.f)) return nullptr;
   TD_TAKE(last_error)
+  TD_TAKE(short_list_pays)
   TD_TAKE(decode_attn)
   TD_TAKE(decode_attn_noalloc)
   TD_TAKE(topk_segments)
@@ -163,17 +165,6 @@ bool attr_int(PyObject* self, PyObject* name, int32_t& out) {
   if (!v.o || !integer(v.o, INT32_MIN, INT32_MAX, x)) return false;
   out = (int32_t)x;
   return true;
-}
-
-// Whether a call is planned for the short-list kernel: token-slot lists without score output, and of the others those
-// that read up to 72 MiB (width: elements of K a token, and as many of V) and, in a batch, up to 2048 tokens a sequence.
-// Its one trip from list to rows saves the streaming kernel's pipeline where that never fills.  Two selection
-// layers, one sparse one and their top-k, us, streaming -> short-list: 32 heads x 128 at 300 tokens 35.5 -> 31.6,
-// 4000 59.3 -> 56.2, 6000 (98 MB) 68.7 -> 71.8; 16 heads 8000 58.5 -> 55.1; 32/8 heads 2500 46.0 -> 42.5, 8000 57.2 ->
-// 49.7; 28/4 heads 4000 52.2 -> 44.4; 4 sequences of 500 .. 2000, 32/8 heads, 54.7 -> 46.7; 6 of 1000 .. 4000 (101 MB)
-// 69.6 -> 74.6.
-bool short_list(bool slots, bool scores, int64_t batch, int64_t max_items, int64_t width) {
-  return (slots && !scores) || ((batch == 1 || max_items <= 2048) && batch * max_items * width <= (72 << 20) / 4);
 }
 
 // (self, q, o, paged_kv_data, paged_kv_indices, paged_kv_indptr, last_page_len, last_page_idx, qk_product, slots, lse,
@@ -293,7 +284,9 @@ bool forward_layer(PyObject* const* a, int64_t layer, at::Tensor* made, int& rc)
       !attr_int(self, names.tile_rows, plan.tile_rows) || !attr_int(self, names.fused_merge, plan.fused_merge) ||
       !attr_int(self, names.sparse_waves, plan.sparse_waves) || !attr_int(self, names.sparse_rows, plan.sparse_rows))
     return false;
-  if (!short_list(slots, scores != nullptr, batch, max_items, (rows == hq ? hq : hkv) * d)) plan.sparse_waves = -1;
+  if (!lib.short_list_pays((int32_t)batch, (int32_t)hq, (int32_t)hkv, (int32_t)d, (int32_t)rows, max_items, list.kind,
+                           scores != nullptr))
+    plan.sparse_waves = -1;
   if (lib.make_plan((int32_t)batch, (int32_t)hq, (int32_t)hkv, (int32_t)d, (int32_t)rows, max_items, &plan) != TD_OK)
     return false;
   const float scale = (float)(1.0 / std::sqrt((double)d));

@@ -140,6 +140,30 @@ def test_regular_calls_are_served_natively(cuda, monkeypatch):
     assert max(served["prefill"] for served in calls.values()) == 2, calls  # prompts whose plan wants no scratch
 
 
+@pytest.mark.parametrize("mode", ["per_head", "group_sum"])
+def test_slices_follow_the_tensors_they_are_of(mode):
+    """Slices of a batched controller's tensors are kept while those stay: one that is exchanged, or another batch size,
+    and they are made again."""
+    from tidaldecode_amd.utils import batch_controller as bc
+
+    c = bc.BatchInferenceController(1, 4, 64, 16, 8, 100, 3, torch.float16, "cpu", num_kv_heads=2, select_mode=mode)
+    kinds = [bc._positions_of, bc._full_of, bc._sparse_of, bc._select_of] + ([bc._sums_of] if mode == "group_sum" else [])
+
+    def agree():
+        for of in kinds:
+            kept, now = c._kept(of), of(c)
+            for a, b in zip(kept if isinstance(kept, tuple) else (kept,), now if isinstance(now, tuple) else (now,)):
+                assert a.data_ptr() == b.data_ptr() and a.shape == b.shape and a.stride() == b.stride(), of
+
+    agree()
+    c.add_sequences([20, 30])
+    agree()
+    for name in ("qk_product", "lse", "page_table", "_meta", "score_sum", "score_bound", "_table_starts", "_list_starts"):
+        if getattr(c, name) is not None:
+            setattr(c, name, getattr(c, name).clone())
+            agree()
+
+
 @pytest.mark.gpu
 def test_launches_leave_the_interpreters_lock(cuda, monkeypatch):
     """Every call that was served, once more with PyGILState_Check (1 where its thread holds the lock, which

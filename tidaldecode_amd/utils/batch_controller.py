@@ -288,9 +288,9 @@ class BatchInferenceController:
         at = self._kept_of
         if at is None or at[0] != self.batch or at[1] is not self.qk_product or at[2] is not self.lse or \
                 at[3] is not self.page_table or at[4] is not self._meta or at[5] is not self.score_sum or \
-                at[6] is not self.score_bound:
+                at[6] is not self.score_bound or at[7] is not self._table_starts or at[8] is not self._list_starts:
             self._kept_of = (self.batch, self.qk_product, self.lse, self.page_table, self._meta, self.score_sum,
-                             self.score_bound)
+                             self.score_bound, self._table_starts, self._list_starts)
             self._kept_views = {}
         views = self._kept_views.get(of)
         if views is None:

@@ -325,3 +325,24 @@ def test_prefill_without_layers(cuda):
     model.layers.clear()
     ids = torch.randint(0, 1000, (9,), device=cuda)
     assert _close(model.prefill(ids), _reference_logits(model, ids))
+
+
+@pytest.mark.parametrize("form", ["width", "transposed", "strided", "regular"])
+def test_prefill_takes_any_vocabulary_head(cuda, form):
+    """Heads that the one-row product does not take (a width that is no multiple of 8, columns that lie together, rows
+    that are not aligned) are multiplied by the library's, as they always were."""
+    from tidaldecode_amd import _kernels
+    from tidaldecode_amd.llama import TidalLlama
+
+    model = TidalLlama(_small(hidden_size=100 if form == "width" else 256), cuda, seed=1)
+    if form == "transposed":
+        model.lm_head = model.lm_head.t().contiguous().t()
+    if form == "strided":
+        model.lm_head = torch.nn.functional.pad(model.lm_head, (0, 4))[:, :256]
+    assert _kernels.gemv_fits(model.lm_head) == (form == "regular")
+    ids = torch.randint(0, model.config.vocab_size, (70,), generator=torch.Generator().manual_seed(2)).to(cuda)
+    logits = []
+    for model.use_gemv in (True, False):
+        model.tidal_init(16, 100)
+        logits.append(model.prefill(ids))
+    assert torch.equal(*logits) if form != "regular" else (logits[0] - logits[1]).abs().max() <= 0.05

@@ -232,6 +232,13 @@ def rope_append_prompt(qkv: torch.Tensor, num_qo_heads: int, past_kv_len: int, k
     return q
 
 
+def gemv_fits(weight: torch.Tensor) -> bool:
+    """Whether ``gemv`` takes the weight: aligned rows of 8 to 30720 elements, a multiple of 8 of them."""
+    return weight.dim() == 2 and weight.dtype in (torch.float16, torch.bfloat16) and weight.stride(1) == 1 and \
+        8 <= weight.size(1) <= 30720 and weight.size(1) % 8 == 0 and weight.stride(0) % 8 == 0 and \
+        weight.stride(0) >= weight.size(1) and weight.data_ptr() % 16 == 0
+
+
 def gemv(weight: torch.Tensor, x: torch.Tensor, *, norm_weight: Optional[torch.Tensor] = None,
          eps: float = 1e-5, gated: bool = False, residual: Optional[torch.Tensor] = None,
          pair_gated: bool = False, out: Optional[torch.Tensor] = None) -> torch.Tensor:

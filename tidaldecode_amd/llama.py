@@ -180,7 +180,8 @@ class TidalLlama:
         h = self._rms(x[-1:], self.norm) if mlp is None else \
             _kernels.add_rms_norm(x[-1:], mlp[-1:], self.norm, c.rms_norm_eps)
         # (one row: 262 MB of 32000 x 4096 weights in 41 us, which the library's product takes 60 for)
-        logits = _kernels.gemv(self.lm_head, h.view(-1)).view(1, -1) if self.use_gemv else h @ self.lm_head.t()
+        logits = _kernels.gemv(self.lm_head, h.view(-1)).view(1, -1) \
+            if self.use_gemv and _kernels.gemv_fits(self.lm_head) else h @ self.lm_head.t()
         torch.cuda.synchronize()
         ctrl.prefill_latency.append(time.perf_counter() - t0)
         return logits[0]

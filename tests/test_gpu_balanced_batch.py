@@ -20,16 +20,17 @@ def _lens(kind, batch, hi):
 
 @pytest.fixture(params=["planned", "balanced"])
 def launch(request, monkeypatch):
-    """As the planner decides, and balanced also where it takes even chunks (up to 64 sequences)."""
+    """As the planner decides, and balanced also where it takes even chunks or short lists (up to 64 sequences)."""
     from tidaldecode_amd import _kernels
+    from tidaldecode_amd.utils import batch_controller
 
     if request.param == "planned":
-        return
+        return request.param
     wrapper = _kernels.BatchDecodeWithPagedKVCachePyTorchWrapper
     planned = wrapper._plan
 
     def plan_of(self, batch, rows, items, short_list=True):
-        plan = planned(self, batch, rows, items, short_list)
+        plan = planned(self, batch, rows, items, False)
         heads, kv, d = self._geom[:3]
         group = next(g for g in (2, 4, 8) if heads // kv <= g or g == 8)
         hrows = kv * -(-(heads // kv) // group)
@@ -45,7 +46,9 @@ def launch(request, monkeypatch):
             return lambda *a: False
 
     monkeypatch.setattr(wrapper, "_plan", plan_of)
-    monkeypatch.setattr(_kernels, "host_calls", Declines())
+    for module in (_kernels, batch_controller):
+        monkeypatch.setattr(module, "host_calls", Declines())
+    return request.param
 
 
 @pytest.mark.parametrize("heads,kv,d,page,dtype", [(32, 8, 128, 16, torch.bfloat16), (28, 4, 128, 16, torch.float16),
@@ -54,6 +57,7 @@ def launch(request, monkeypatch):
 @pytest.mark.parametrize("kind,batch,hi", [("mixed", 2, 700), ("mixed", 16, 3000), ("one long", 9, 5000),
                                            ("equal", 5, 129), ("mixed", 64, 300), ("mixed", 65, 300)])
 def test_batches(cuda, launch, heads, kv, d, page, dtype, kind, batch, hi):
+    from tidaldecode_amd import _kernels
     from tidaldecode_amd.utils import BatchInferenceController
 
     lens = _lens(kind, batch, hi)
@@ -65,6 +69,7 @@ def test_batches(cuda, launch, heads, kv, d, page, dtype, kind, batch, hi):
     pool = c.buf_layer(0)
     for step in range(2):  # the second on tickets and partials the first has used
         o = c.attend_full(q, 0, output_qk_product=True)
+    assert launch == "planned" or _kernels.last_decode_kernel().startswith("streaming")
     rows = c.qk_product.view(batch, heads, -1)
     tol = 2e-3 if dtype == torch.float16 else 1e-2
     for b, n in enumerate(lens):
@@ -82,6 +87,7 @@ def test_batches(cuda, launch, heads, kv, d, page, dtype, kind, batch, hi):
 @pytest.mark.parametrize("batch,hi", [(3, 900), (16, 2000)])
 def test_fused_step_of_a_batch(cuda, launch, batch, hi):
     """With the new tokens folded into the launch: the same outputs, logits and cache as the separate calls."""
+    from tidaldecode_amd import _kernels
     from tidaldecode_amd.utils import BatchInferenceController
 
     heads, kv, d, page = 32, 8, 128, 16
@@ -100,6 +106,7 @@ def test_fused_step_of_a_batch(cuda, launch, batch, hi):
         else:
             c.rope_append(q, k, v, 0)
             o = c.attend_full(q, 0, output_qk_product=True)
+        assert launch == "planned" or _kernels.last_decode_kernel().startswith("streaming")
         out.append((o.float(), c.qk_product.clone(), c.pool.buf.float()))
     (o0, l0, p0), (o1, l1, p1) = out
     # a rotated element may differ by one bf16 step between the kernels: 2^-8 of values up to 5

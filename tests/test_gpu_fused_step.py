@@ -25,7 +25,8 @@ def _ulp_close(a, b, dtype):
                                               (28, 4, 4, "slots"),
                                               # 12 heads per KV head: two head rows (8 + 4) per KV head
                                               (24, 2, 2, "slots"), (24, 2, 1, "pages")])
-def test_fused_equals_separate(cuda, dtype, hq, hkv, rows, mode):
+@pytest.mark.parametrize("waves", [0, -1])    # as the library prefers, and on the streaming kernel
+def test_fused_equals_separate(cuda, dtype, hq, hkv, rows, mode, waves):
     from oracle import tidal_oracle as orc
     from tidaldecode_amd import _kernels
 
@@ -69,6 +70,7 @@ def test_fused_equals_separate(cuda, dtype, hq, hkv, rows, mode):
     stride = npg * page
     w = _kernels.BatchDecodeWithPagedKVCachePyTorchWrapper(0)
     w.begin_forward(None, hq, hkv, d, page, torch.empty(0, dtype=dtype))
+    w.sparse_waves = waves
 
     def run(fused):
         pl = pool.clone()
@@ -83,6 +85,7 @@ def test_fused_equals_separate(cuda, dtype, hq, hkv, rows, mode):
         else:
             _kernels.rope_append_decode(qq, knew, vnew, pl, positions, dst, 0, 1.0, theta)
             w.forward(qq, o, pl, idx, indptr, ll, li, scores, index_kind=kind, n_list=n_list)
+        assert _kernels.last_decode_kernel() == ("short-list" if waves == 0 and hq // hkv <= 8 else "streaming")
         torch.cuda.synchronize()
         return o, pl, scores
 

@@ -10,19 +10,27 @@ pytestmark = pytest.mark.gpu
 SHAPES = [(4, 4, 64), (14, 2, 64), (8, 2, 64), (4, 2, 64), (14, 2, 128), (6, 2, 128), (4, 4, 128)]
 
 
-def _wrapper(hq, hkv, d, page, dtype, layout=0):
+# waves of a workgroup, tokens of a split and whether it merges in the launch: as planned, and such that every wave of
+# a long list takes several tiles (rows of eight lanes: of 64 tokens, else of 32)
+PLANNED = (0, 0, -1)
+TILES = [(4, 1024, 0), (4, 2048, 1), (8, 1024, 1), (8, 2048, 0)]
+
+
+def _wrapper(hq, hkv, d, page, dtype, layout=0, shape=PLANNED):
     from tidaldecode_amd import _kernels
 
     w = _kernels.BatchDecodeWithPagedKVCachePyTorchWrapper(layout)
     w.begin_forward(None, hq, hkv, d, page, torch.empty(0, dtype=dtype))
+    w.sparse_waves, w.chunk_tokens, w.fused_merge = shape
+    assert shape == PLANNED or w.chunk_tokens >= 2 * w.sparse_waves * 4096 // d
     return w
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("hq,hkv,d", SHAPES)
 @pytest.mark.parametrize("per_query_head", [False, True])
-@pytest.mark.parametrize("layout", [0, 1])
-def test_slot_lists_with_the_new_token(cuda, dtype, hq, hkv, d, per_query_head, layout):
+@pytest.mark.parametrize("layout,shape", [(0, PLANNED), (1, PLANNED)] + [(0, x) for x in TILES])
+def test_slot_lists_with_the_new_token(cuda, dtype, hq, hkv, d, per_query_head, layout, shape):
     from oracle import tidal_oracle as orc
     from tidaldecode_amd import _kernels
 
@@ -37,10 +45,10 @@ def test_slot_lists_with_the_new_token(cuda, dtype, hq, hkv, d, per_query_head, 
     cos, sin = _kernels.rope_table(torch.tensor([n - 1], **dev), d, 1.0, theta)
     slot = int(case.slots_of(torch.tensor([n - 1]))[0])
     fresh = (knew.to(dtype).to(cuda), vnew.to(dtype).to(cuda), cos, sin, torch.tensor([slot], **dev))
-    w = _wrapper(hq, hkv, d, page, dtype, layout)
+    w = _wrapper(hq, hkv, d, page, dtype, layout, shape)
     qd = q.to(dtype).to(cuda)
     g = torch.Generator().manual_seed(hq)
-    for k in (1, 31, 33, 64, 65, 129, 256, 257, 513, 1300, 2600):
+    for k in (1, 31, 33, 64, 65, 129, 256, 257, 513, 1300, 2600) if shape == PLANNED else (1, 257, 513, 1300, 2600):
         pos = torch.stack([torch.randperm(n - 1, generator=g)[: k - 1] for _ in range(rows)])
         pos = torch.cat([pos, torch.full((rows, 1), n - 1)], 1)[:, torch.randperm(k, generator=g)]
         pool, o = case.pool.to(cuda), torch.full_like(qd, float("nan"))
@@ -60,8 +68,8 @@ def test_slot_lists_with_the_new_token(cuda, dtype, hq, hkv, d, per_query_head, 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("hq,hkv,d", SHAPES)
-@pytest.mark.parametrize("page", [1, 16, 32])
-def test_pages_of_the_whole_sequence_with_logits(cuda, dtype, hq, hkv, d, page):
+@pytest.mark.parametrize("page,shape", [(1, PLANNED), (16, PLANNED), (32, PLANNED)] + [(16, x) for x in TILES])
+def test_pages_of_the_whole_sequence_with_logits(cuda, dtype, hq, hkv, d, page, shape):
     from oracle import tidal_oracle as orc
     from tidaldecode_amd import _kernels
 
@@ -69,7 +77,7 @@ def test_pages_of_the_whole_sequence_with_logits(cuda, dtype, hq, hkv, d, page):
         case = PagedCase(n, hkv, d, page, dtype, seed=n)
         q = randn((hq, d), n + 1, dtype)
         logits = orc.attn_logits(q, case.k)
-        w = _wrapper(hq, hkv, d, page, dtype)
+        w = _wrapper(hq, hkv, d, page, dtype, shape=shape)
         qd = q.to(dtype).to(cuda).unsqueeze(0)
         for scores_dtype in (torch.float32, dtype):
             o = torch.full_like(qd, float("nan"))
@@ -88,7 +96,8 @@ def test_pages_of_the_whole_sequence_with_logits(cuda, dtype, hq, hkv, d, page):
 
 
 @pytest.mark.parametrize("hq,hkv,d", [(4, 4, 128), (14, 2, 64)])
-def test_page_lists_of_a_ragged_batch(cuda, hq, hkv, d):
+@pytest.mark.parametrize("shape", [PLANNED, (4, 512, 0), (4, 512, 1)])
+def test_page_lists_of_a_ragged_batch(cuda, hq, hkv, d, shape):
     """Lists of pages per query head, the forced last page, counts on the device."""
     from oracle import tidal_oracle as orc
     from tidaldecode_amd import _kernels
@@ -113,7 +122,7 @@ def test_page_lists_of_a_ragged_batch(cuda, hq, hkv, d):
     q = randn((len(cases), hq, d), 9, dtype)
     qd = q.to(dtype).to(cuda)
     o = torch.full_like(qd, float("nan"))
-    w = _wrapper(hq, hkv, d, page, dtype)
+    w = _wrapper(hq, hkv, d, page, dtype, shape=shape)
     w.forward(qd, o, pool, idx.to(torch.int32).to(cuda), torch.tensor([i * width for i in range(len(cases) + 1)], **dev),
               torch.tensor([c.last_page_len for c in cases], **dev),
               torch.tensor([int(c.page_table[-1]) + b for c, b in zip(cases, base)], **dev), None,

@@ -104,9 +104,10 @@ _SHAPES = [(8, 8, 128, 16, "NHD", "per_head"), (8, 2, 64, 4, "HND", "group_sum")
 
 def _use(monkeypatch, calls):
     from tidaldecode_amd import utils as ops
+    from tidaldecode_amd.utils import batch_controller
 
-    monkeypatch.setattr(_kernels, "host_calls", calls)
-    monkeypatch.setattr(ops, "host_calls", calls)
+    for module in (_kernels, ops, batch_controller):
+        monkeypatch.setattr(module, "host_calls", calls)
 
 
 @pytest.mark.gpu
@@ -117,6 +118,47 @@ def test_same_bits_as_the_python_path(cuda, monkeypatch, dtype, shape):
     _use(monkeypatch, _Off())
     b, _ = _workload(cuda, dtype, *shape)
     assert len(a) == len(b)
+    for x, y in zip(a, b):
+        assert x.dtype == y.dtype and x.shape == y.shape and torch.equal(x, y)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mode", ["per_head", "group_sum"])
+@pytest.mark.parametrize("fused", [False, True])
+def test_batches_are_served_natively_with_the_same_bits(cuda, monkeypatch, mode, fused):
+    from tidaldecode_amd.utils import BatchInferenceController
+
+    def workload(calls):
+        _use(monkeypatch, calls)
+        g = torch.Generator(device=cuda).manual_seed(3)
+        c = BatchInferenceController(2, 8, 128, 16, 40, 700, 3, torch.bfloat16, cuda, num_kv_heads=2, select_mode=mode,
+                                     page_order_seed=5)
+        c.pool.buf.normal_(generator=g)
+        c.add_sequences([600, 33, 150])
+        out = []
+        for _ in range(2):
+            c.begin_step()
+            cos, sin = c.rope_table()
+            for layer in range(2):
+                q, k, v = (torch.randn((3, h, 128), generator=g, device=cuda).bfloat16() for h in (8, 2, 2))
+                if not fused:
+                    c.rope_append(q, k, v, layer)
+                fresh = (k, v, cos, sin) if fused else None
+                if layer == 0:
+                    out.append(c.attend_full(q, 0, output_qk_product=True, fresh=fresh))
+                    c.select()
+                else:
+                    out.append(c.attend_sparse(q, 1, fresh=fresh))
+            out += [c.qk_product.clone(), c.lse.clone(), c.topk_dindices_buffer.clone()]
+        torch.cuda.synchronize()
+        return out + [c.pool.buf]
+
+    recorder = _Recorder()
+    a, b = workload(recorder), workload(_Off())
+    names = [name for name, _ in recorder.served]
+    # (the first attention needs its workspace made)
+    assert names.count("topk") == 2 and 3 <= names.count("attend") <= 4, names
+    assert names.count("score_reduce") == (2 if mode == "group_sum" else 0)
     for x, y in zip(a, b):
         assert x.dtype == y.dtype and x.shape == y.shape and torch.equal(x, y)
 
@@ -137,7 +179,7 @@ def test_regular_calls_are_served_natively(cuda, monkeypatch):
         assert served["topk"] == 2 and served["estimate"] == 2 and served["gemv"] == 3, (shape, served)
         assert served["attend"] >= 2 and served["forward"] == 2, (shape, served)
         assert served["score_reduce"] == (2 if shape[-1] == "group_sum" else 0), (shape, served)
-    assert max(served["prefill"] for served in calls.values()) == 2, calls  # prompts whose plan wants no scratch
+    assert max(served["prefill"] for served in calls.values()) == 2, calls  # two layers of a prompt
 
 
 @pytest.mark.parametrize("mode", ["per_head", "group_sum"])

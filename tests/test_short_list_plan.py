@@ -18,9 +18,7 @@ def test_plans(hq, hkv, d, batch):
             assert p.sparse_waves in (4, 8) and p.sparse_rows == 8
             assert p.chunk_tokens % (p.sparse_waves * 4096 // d) == 0
             assert 1 <= p.max_splits <= 64 and (p.max_splits - 1) * p.chunk_tokens < items <= p.max_splits * p.chunk_tokens
-            single = p.workspace_bytes - (1 << 20)  # what one split takes, within the rounding of the two arrays
-            assert p.workspace_bytes <= SCRATCH or single // p.max_splits + (1 << 20) > SCRATCH or p.max_splits == 1 or \
-                items > 16384 // 2, (rows, items, p.max_splits, p.workspace_bytes)
+            assert p.workspace_bytes <= SCRATCH or p.max_splits == 1, (rows, items, p.max_splits, p.workspace_bytes)
             # quotients by the product with 2^32 / chunk, rounded up, which the kernel forms
             magic = ((1 << 32) + p.chunk_tokens - 1) // p.chunk_tokens
             for n in (1, items // 2 + 1, items):

@@ -692,8 +692,8 @@ __device__ __forceinline__ void attend_share(const DecodeParams& p, const int hr
       // at one piece, fall on different banks.  Dot products, which this replaces, take 4 QPG instructions per
       // row and lane and a reduction over the row; eight heads of 128 were bound by them, and so were rows of
       // eight lanes, whose values were weighted on the vector ALU as well.  bf16, logits out, three layers
-      // (two of them full), us, before -> now: 28/4 heads x 128 at 4140 tokens 81.8 -> 65.6, at 60000 148 ->
-      // 120; x 64 81.3 -> 55.7 and 138 -> 91.6; 32/8 heads x 64 at 16000 75.6 -> 68.2.  Two and four heads of
+      // (two of them full, lists of 1024 per KV head), us, before -> now: 28/4 heads x 128 at 60000 tokens 145 -> 115;
+      // x 64 139 -> 93; 32/8 heads x 64 at 16000 76.6 -> 61.3.  Two and four heads of
       // 128 are bound by the loads and lose 1 - 3 % to the detour; a third tile of loads in flight costs them 9 %
       // and eight heads 17 % at 60000 tokens.
       auto place = [](int r, int c) { return r * (D * 2) + 16 * (c ^ (LPR == 16 ? r : (r >> 1) & 7)); };
@@ -1098,7 +1098,8 @@ __global__ __launch_bounds__(NT) void merge_partials_kernel(const DecodeParams p
 // Instantiated shapes (tile_rows = K/V load instructions per wave tile):
 //   one query head per head row: head_dim 64/128/256, 8 waves x {2, 4} rows or 16 waves x 4 rows;
 //   2, 4 or 8 query heads per head row (KV rows shared inside a GQA group): head_dim 64 and 128
-//   (256: 2 or 4), 8 waves x 4 rows; head_dim 128 on the matrix cores, the others on the vector ALU.
+//   (256: 2 or 4), 8 waves x 4 rows; weighted values on the matrix cores (256: on the vector ALU), and scores too
+//   for 8 heads and for head_dim 64.
 static bool shape_supported(int head_dim, int qpg, int nw, int rows = 4) {
   if (qpg == 1)
     return (head_dim == 64 || head_dim == 128 || head_dim == 256) &&

@@ -584,9 +584,9 @@ extern "C" int td_decode_attn(const td_paged_kv* kv, const td_index_list* list,
   }
   if (fresh && !p.lean)
     return fail(TD_ERR_UNSUPPORTED,
-                "td_decode_attn: outside the short-list kernel (token-slot lists of up to %lld entries, "
-                "head_dim 128, no score output) the fused decode step needs a power-of-two page_size and "
-                "a pool below 4 GiB (page_size %d, pool %lld bytes); use td_rope_append_decode first",
+                "td_decode_attn: the fused decode step needs a power-of-two page_size and a pool below 4 GiB, but for "
+                "token-slot lists of up to %lld entries at head_dim 128 without score output, one per query head "
+                "(groups of a power of two) or per 2, 4 or 8 of them (page_size %d, pool %lld bytes); use td_rope_append_decode first",
                 (long long)kSparseMaxItems, kv->page_size, (long long)(kv->max_pages * p.page_stride * 2));
   if (kv->dtype == TD_F16)
     rc = launch_decode_f16(p, D, qpg, plan->waves_per_block, plan->tile_rows, page_mode, scores != nullptr,

@@ -3,9 +3,9 @@
 //
 // A decode step of a short context is bound by its host: a Python entry point spends 8 to 14 us in
 // tensor attribute reads, ctypes structures and argument conversion for a kernel of 5 us.  Every
-// function here returns True after it has launched, and False, having done nothing, for whatever it
-// does not recognise as regular (an argument of another kind, a check that fails, a workspace that
-// has to be allocated): the caller then goes on in Python, which raises the errors and handles the
+// function here returns True, or the output it made, after it has launched, and False, having launched nothing, for
+// whatever it does not recognise as regular (an argument of another kind, a check that fails, a handle's workspace
+// that has to grow): the caller then goes on in Python, which raises the errors and handles the
 // rest.  Nothing is kept between calls; the only state is the table of function addresses.
 #include <Python.h>
 #include <ATen/ATen.h>

@@ -1,19 +1,21 @@
-// Sparse-layer decode attention for gfx950 (MI355X): the short-list form of decode_attn_kernel,
-// for head_dim 128, one query head per head row, token-slot lists, power-of-two pages and a pool
-// below 4 GiB.  Same arguments, same split workspace and the same results as decode_attn_kernel;
+// Sparse-layer decode attention for gfx950 (MI355X): the short-list form of decode_attn_kernel, for head_dim 64 and
+// 128, one query head per list walk or up to eight that share one, token-slot or page lists, with or without logits.
+// Pools of 4 GiB and more and pages that are no power of two: head_dim 128, token-slot lists, no logits.  Same
+// arguments, same split workspace and the same results as decode_attn_kernel;
 // what differs is the shape of the work, chosen for launches that move a few tens of MiB and are
 // bound by dependent round trips and instruction issue rather than by bandwidth:
 //
-//   * a wave owns 4 U tokens (U = 8 or 16 K rows and as many V rows per lane: 64 or 128 VGPRs of
-//     loads), all of them in flight at once, K rows first so that q.k runs while V arrives;
+//   * a wave owns 4 U tokens, 8 U at head_dim 64 (U = 8 or 16 K rows and as many V rows per lane: 64 or 128
+//     VGPRs of loads), all of them in flight at once, K rows first so that q.k runs while V arrives;
 //   * the list entry of a token is loaded once, by the lane that owns the token; its byte offset
-//     reaches the 16 lanes of a row through DPP row broadcasts (one instruction per row);
-//   * q.k partial sums are reduce-scattered over the 16 lanes of a row, so that after U partial
+//     reaches the 16 (8) lanes of a row through DPP row broadcasts (one or two instructions per row);
+//   * one head: q.k partial sums are reduce-scattered over the lanes of a row, so that after U partial
 //     dot products a lane holds the complete logit of ONE token and the softmax arithmetic runs
 //     once per token instead of once per lane; the probabilities go back through row broadcasts;
-//   * the maximum is wave-uniform per tile, so the four lane groups add up without rescaling;
-//   * the workgroup's waves meet once in LDS, then wave 0 alone publishes the partial, takes the
-//     ticket and, if it is the last of its head row, merges the partials (no further barrier).
+//   * shared rows: both products on the matrix cores, the keys through the wave's own LDS into operand layout;
+//   * the maximum is wave-uniform per tile, so the lane groups add up without rescaling;
+//   * the workgroup's waves meet once in LDS, then wave j alone publishes the partials of the heads j, j + NW, ..,
+//     takes their tickets and, where it is the last of a head, merges the partials (no further barrier).
 //
 // Semantics follow kernels/include/decode/decode_attn.cuh:432-658 of the reference
 // (BatchDecodeWithPagedKVCacheKernel) including the forced last page (decode_page.cuh:320-346).

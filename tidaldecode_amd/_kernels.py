@@ -152,11 +152,33 @@ def _cut_columns(m: int, n: int, k: int) -> int:
 def _row_splits(m: int, n: int, k: int) -> int:
     """Cuts of the inner dimension with which td_gemm_rows takes a product [m, k] x [n, k]^T, 0: the library's.  One
     tile of rows, few enough columns that the library leaves the chip idle, workgroups for all 256 compute units
-    with eight steps of 128 each (measured at the kernel; 80 rows of 6144 columns are where it draws level)."""
-    if not 17 <= m <= 144 or n > 8192 or n % 64 or k % 128 or k < 2048 or k > 1 << 20 or (n > 4096 and m <= 80):
+    with eight steps of 128 each, and a size where it is the faster one.
+
+    Measured on one MI355X, cold weights, 42 row counts and 31 weights of 64 to 8192 columns and inner dimensions of
+    2048 to 28672, both types; time here over the library's, by rows.  Up to 48: 0.6 to 1.07, but for 32 rows of
+    4096 x 8192 1.2.  49 to 63: from k = 5632 on 0.7 to 1.01, 1024 x 8192 1.14, 4096 x 4096 0.97 to 1.07, 3072 x 3072
+    1.14.  64 to 80: 0.47 to 0.95 of what is taken, 1024 x 8192 1.07, 4096 x 2048 1.05.  81 to 112 and 128: 0.4 to 1.06,
+    2048 x 5632 1.05, 4096 x 2048 1.4.  113 to 127, where the library has a tile of its own and eight blocks of 16 rows
+    are multiplied as nine here: 0.5 to 0.97 of deep products, 4096 x 4096 1.2, 4096 x 8192 1.05.  129 and more: 0.47 to
+    1.0 (6144 x 4096 fp16 1.06), 3584 x 3584 1.04, 4096 x 2048 1.37.  More than 6144 columns of no deeper product:
+    7168 x 5120 0.97 to 1.09, 8192 x 4096 1.0 to 1.16, 8192 x 8192 1.0 to 1.33."""
+    if not 17 <= m <= 144 or n > 8192 or n % 64 or k % 128 or k < 2048 or k > 1 << 20 or (n > 4096 and m <= 80) or \
+            (n > 6144 and 2 * k < 3 * n):
         return 0
+    if m <= 48:
+        faster = n >= 512 and (m > 32 or n <= 3072 or k % 8192 != 0)
+    elif m < 64:
+        faster = k >= 5632 and n >= 2048
+    elif m <= 80:
+        faster = k >= 3072 and n >= 2048
+    elif m <= 112 or m == 128:
+        faster = n * k >= 12 << 20
+    elif m < 128:
+        faster = k >= 6144 and k > 2 * n and n >= 2048
+    else:
+        faster = n * k >= 1 << 24
     splits = min(256 // (n // 64), k // 1024, 8)
-    return splits if splits > 1 else 0
+    return splits if faster and splits > 1 else 0
 
 
 def _served_directly(x: torch.Tensor, weight: torch.Tensor) -> bool:

@@ -50,14 +50,18 @@ struct DecodeParams {
                      // of 3 runs as 4, 5-7 as 8; the padding heads have q = 0 and are never stored)
   int32_t subs;      // head rows per KV head on the shared-row kernels: groups above 8 are cut
                      // into rows of 8 query heads (the last one padded)
+  int32_t num_kv_heads;
+  // (What a launch needs first lies together from here to `scale_log2`, with no word between that it does not: scalar
+  // loads come in blocks of up to eight words, and a register that a block fills for nothing is given out again,
+  // behind a wait for the block.  With two such words the short lists without a new token waited twice, 0.2 us.)
   // index list
   const int32_t* idx;
   int32_t idx_row_stride;  // 0 for a shared row
   int32_t idx_cols;        // elements a row holds (the caller's row stride; 0: unknown): reads stop there
   int32_t idx_per_kv;      // 1: rows are per KV head while QPG == 1
+  int32_t n_list_host;
   const int32_t* indptr;
   const int32_t* count_arr;  // per-sequence entry counts of a padded table (else indptr differences)
-  int32_t n_list_host;
   const int32_t* last_len_arr;
   const int32_t* last_idx_arr;
   int32_t last_len;
@@ -65,9 +69,7 @@ struct DecodeParams {
   // split
   int32_t chunk_tokens;
   uint32_t chunk_magic;  // 2^32 / chunk_tokens, rounded up: exact for the short-list kernel's up to 2^16 tokens
-  int32_t num_kv_heads;
   uint32_t kv_magic;    // 2^24 / q_per_kv, rounded up
-  int32_t list_shift;   // short-list kernel: log2 of the tokens a list entry stands for
   int32_t max_splits;
   int32_t fused_merge;
   float scale_log2;  // sm_scale * log2(e)
@@ -81,6 +83,7 @@ struct DecodeParams {
   int32_t* ws_cnt;  // [batch * head rows] ticket counters, ticket_stride words apart
   int32_t ticket_stride;
   int32_t batch, slots;  // balanced launches: sequences, and workgroups per head row
+  int32_t list_shift;    // short-list kernel: log2 of the tokens a list entry stands for
   // the token being decoded (FRESH kernels): un-rotated k, v, its rotary cos/sin and its slot
   const void* fresh_k;
   const void* fresh_v;

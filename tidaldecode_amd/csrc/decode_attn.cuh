@@ -270,9 +270,10 @@ __device__ __forceinline__ int seq_items(const DecodeParams& p, int b, SeqList& 
 // of a weight above 0 is above 0 (fp16: of 2^-39 and more): an infinite value times a remainder of 0, or of the other
 // sign, would give NaN.  fp16 weights are taken times kWeightScale, or those below 2^-25 would vanish beside a
 // denominator that counts them.  Head_dim 64 takes kWhole, and short lists in fp16 do: their values met fp32 weights or
-// a single part before they came to the matrix cores in two.  The third product costs 1 - 3 %: one layer, rounded |
-// whole, us: 28/4 heads x 64, bf16, lists of 4096 7.20 | 7.31, 60000 tokens 24.9 | 25.3; 32/8 heads x 64, fp16, 60000
-// tokens 37.1 | 37.5; 32/8 heads x 128, fp16, lists of 4096 8.2 | 8.4.
+// a single part before they came to the matrix cores in two.  The third part costs a launch 2 % (its arithmetic; the four
+// sums by turns instead of part after part change nothing), one of 300 tokens, which is a chain of latencies, 6: one
+// layer, rounded | whole, us: 16/8 heads x 64, bf16, logits out, 300 tokens 5.50 | 5.88, 2000 7.28 | 7.50; 28/4 x 64 300
+// 5.87 | 6.07, 60000 24.9 | 25.3; 32/8 x 64, fp16, 60000 37.1 | 37.5; 32/8 heads x 128, fp16, lists of 4096 8.2 | 8.4.
 enum WeightParts { kRounded = 2, kWhole = 3 };
 template <typename T, WeightParts PARTS>
 constexpr float kWeightScale = PARTS == kWhole && std::is_same<T, F16>::value ? 32768.f : 1.f;

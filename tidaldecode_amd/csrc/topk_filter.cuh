@@ -624,6 +624,8 @@ static bool filter_fits(int len, int k, int threads) {
 // bf16, 512 rows 3000 -> 1024 | 15.1 | 10.7, 8192 -> 2048 18.2 | 12.8, 8192 -> 2500 18.3 | 14.1 and 18.6 | 16.2, 5000
 // -> 2500 18.7 | 16.5 and 18.9 | 17.2, 8192 -> 4096 20.9 | 20.7 and 21.3 | 21.7.  bf16 rows of up to kMidLen: 128 rows
 // 8193 -> 512 10.4 | 9.6, 10240 -> 800 10.7 | 10.4, -> 1000 10.7 | 10.8; 256 rows 9000 -> 1500 12.9 | 12.6.
+// (Over 480 shapes of more than 256 rows, 3000 to 10240 long: 0.68 to 1.0, but bf16 rows of 3000 to 4600 -> 1800 to 2500,
+// whose survivors just pass a multiple of four a thread, 0.84 to 1.06, and 512 fp32 rows of 8193 -> 3300 23.2 | 25.2.)
 // Rows of up to 2048 elements gain at any k (bf16 1500 -> 1024, a tie and as many survivors as there can be, 0.96),
 // rows of more than 65536, which the slices read again in every pass, too.
 static bool filter_pays(int len, int k, int rows, bool half) {
